@@ -648,24 +648,17 @@ def main(argv=None) -> int:
                                                       not args.no_autotune, fixed, qmap)
     mlups = n_cells * args.steps / (ms_total * 1e-3) / 1e6
     ms_step = ms_total / args.steps
-    pp = tun["pipe_planes"]
-    # dominant kernel: the bulk launch over the regular blocks (every cell fluid); the face cells are
-    # stepped by it when it applies the face rules itself, else by the face-cell kernel
-    face_in_bulk = args.stream == "ab" and pp > 1 and not tun["face_kernel"]
-    bulk_cells = (info["n_regular"] + info["n_interior"]) * 16 ** 3 - (0 if face_in_bulk else info["n_face_cells"])
+    # dominant kernel: AB pattern, the two-cells-per-lane kernel over every block; AA pattern, the pipelined
+    # kernels over the regular blocks
+    ab = args.stream == "ab"
+    bulk_cells = n_fluid if ab and qmap is None else (info["n_regular"] + info["n_interior"]) * 16 ** 3
     achieved = bytes_per_lup("f32") * bulk_cells / (ms_kernel * 1e-3) / 1e9
     step_gbs = bytes_per_lup("f32") * n_fluid / (ms_step * 1e-3) / 1e9
     area = np.pi * (D / 2) ** 2
     cd = float(F[0] / (0.5 * U_IN ** 2 * area))
 
     # (the collision's unit-rate form: the reference's default rates omega_bulk = omega_3 = omega_4 = 1)
-    if args.stream == "ab" and pp > 1 and tun.get("pair_kernel") and not tun["face_kernel"]:
-        kernel = (f"k_step_pair32<{pp}, true, 1> + k_step_pair32<{pp}, true, 0>" if tun["pair_kernel"] == 2
-                  else f"k_step_pair32<{pp}, true, 1>")
-    elif args.stream == "ab" and pp > 1:
-        kernel = f"k_step_pipe<StF32, {pp}, {2 if tun['face_kernel'] else 1}, true, false>"
-    else:
-        kernel = "k_step<StF32, regular>"
+    kernel = "k_step_two<StF32, true, false, 0>" if ab else "k_step_pipe_aa<StF32>"
     traffic = measured_traffic(kernel)
 
     out = {
@@ -700,18 +693,10 @@ def main(argv=None) -> int:
         ms_t16, ms_k16, _, F16, tun16, _ = gpu_leg(grid, "f16s", args.stream, args.steps, args.warmup,
                                                    not args.no_autotune, fixed, qmap)
         m16 = n_cells * args.steps / (ms_t16 * 1e-3) / 1e6
-        face16 = args.stream == "ab" and tun16["pipe_planes"] > 1 and not tun16["face_kernel"]
-        bulk16 = (info["n_regular"] + info["n_interior"]) * 16 ** 3 - (0 if face16 else info["n_face_cells"])
+        bulk16 = bulk_cells
         a16 = bytes_per_lup("f16s") * bulk16 / (ms_k16 * 1e-3) / 1e9
         s16 = bytes_per_lup("f16s") * n_fluid / (ms_t16 / args.steps * 1e-3) / 1e9
-        pp16 = tun16["pipe_planes"]
-        if args.stream == "ab" and pp16 > 1 and tun16.get("pair_kernel") and not tun16["face_kernel"]:
-            k16 = (f"k_step_pair<StF16S, {pp16}, true, 1> + k_step_pair<StF16S, {pp16}, true, 0>"
-                   if tun16["pair_kernel"] == 2 else f"k_step_pair<StF16S, {pp16}, true, 1>")
-        elif args.stream == "ab" and pp16 > 1:
-            k16 = f"k_step_pipe<StF16S, {pp16}, {2 if tun16['face_kernel'] else 1}, true, false>"
-        else:
-            k16 = "k_step<StF16S, regular>"
+        k16 = "k_step_two<StF16S, true, false, 0>" if ab else "k_step_pipe_aa<StF16S>"
         traffic16 = measured_traffic(k16, "step_f16_256_hbm_traffic.md")
         out["fp16_shifted"] = {"value": round(m16, 1), "unit": "MLUPS", "ms_per_step": round(ms_t16 / args.steps, 4),
                                "speedup_vs_f32": round(m16 / mlups, 3), "tuning": tun16,
@@ -746,12 +731,10 @@ def main(argv=None) -> int:
         ms_tw, ms_kw, _, Fw, tunw, _ = gpu_leg(grid, "f32", args.stream, args.steps, args.warmup,
                                                not args.no_autotune, fixed, qmap, wale=True)
         mw = n_cells * args.steps / (ms_tw * 1e-3) / 1e6
-        facew = args.stream == "ab" and tunw["pipe_planes"] > 1
-        bulkw = (info["n_regular"] + info["n_interior"]) * 16 ** 3 - (0 if facew else info["n_face_cells"])
+        bulkw = bulk_cells
         bw = bytes_per_lup("f32", wale=True)
         aw = bw * bulkw / (ms_kw * 1e-3) / 1e9
-        ppw = min(tunw["pipe_planes"], 8)
-        kw = f"k_step_pipe<StF32, {ppw}, 1, true, true>" if facew else "k_step<StF32, regular, wale>"
+        kw = "k_step_two<StF32, true, true, 0>" if ab else "k_step<StF32, regular, wale>"
         out["wale_on"] = {"value": round(mw, 1), "unit": "MLUPS", "ms_per_step": round(ms_tw / args.steps, 4),
                           "vs_wale_off": round(mw / mlups, 3), "c_wale": 0.2, "inlet_turbulence": 0.01,
                           "tuning": tunw, "cd_transient": round(float(Fw[0] / (0.5 * U_IN ** 2 * area)), 5),

@@ -176,12 +176,16 @@ int oal_plan_destroy(OalPlan* plan);
  * the host arrays of f, rho and u. */
 int oal_level_cells(const OalPlan* plan, int level, int64_t* n_cells);
 
-/* Replaces: nothing (introspection).  How a level's blocks split over the step kernels: blocks on
- * a regular lexicographic grid with no boundary rule or solid link (n_regular, one arithmetic-address
- * launch; in the AB pattern also whole blocks on a domain face with no solid near), other blocks
- * with no boundary rule (n_interior), and the boundary blocks of both kinds plus the regular blocks
- * that overhang the extent (n_partial), launched on a second stream that overlaps the bulk launches.
- * The bulk launches that oal_time_steps times (ms_kernel) cover the n_regular and n_interior blocks. */
+/* Replaces: nothing (introspection).  A level's blocks by kind: on a regular lexicographic grid with no
+ * boundary rule or solid link (n_regular; in the AB pattern also whole blocks on a domain face with no
+ * solid near), other blocks with no boundary rule (n_interior), boundary blocks of both, and regular
+ * blocks that overhang the extent (n_partial) or hold sponge cells (n_sponge).  The AB pattern with FP32
+ * arithmetic steps them in one launch of the two-cells-per-lane kernel, but for blocks with an absent
+ * neighbour inside the extent, under the exact specular z wall or the transverse freestream, next to
+ * solid cells with OAL_BB_REFERENCE, or whose neighbours lie 4 GiB of populations apart; these, and in
+ * FP64 and the AA pattern the boundary blocks, are launched on a second stream that overlaps the bulk
+ * launches.  The bulk launches that oal_time_steps times (ms_kernel) are the two-cells-per-lane kernel's,
+ * or the n_regular and n_interior blocks'. */
 typedef struct OalLevelInfo {
     int64_t n_cells;         /* n_blocks * bs^3 (of the caller's blocks, 8^3 ones included; the
                                 kernel counts below are of the library's 16^3 blocks) */
@@ -191,23 +195,19 @@ typedef struct OalLevelInfo {
     int32_t n_interior;
     int32_t n_boundary_regular;
     int32_t n_boundary;
-    int32_t n_face_cells;    /* AB pattern: cells of regular blocks on a domain face; the bulk kernel
-                                applies their rules itself or leaves them to the face-cell kernel
-                                (OalTuning.face_kernel) */
+    int32_t n_face_cells;    /* AB pattern: cells of regular blocks on a domain face (FP64: stepped by the
+                                face-cell kernel) */
     int32_t n_ghost_blocks;  /* refined plans: blocks the library adds around the level (filled from
                                 the coarser level, not stepped; not part of n_blocks or n_cells) */
     int32_t n_covered_blocks;/* refined plans: blocks of n_blocks whose children exist (written by
                                 restriction, not stepped) */
-    int32_t n_partial;       /* AB pattern: regular blocks that overhang the extent, no solid near (the
-                                pipelined kernel with the face rules at the extent's last cells, on the
-                                second stream; in a domain whose block layers span 2 GiB or more they
-                                are boundary blocks) */
-    int32_t n_sponge;        /* AB pattern: regular blocks with sponge cells and no solid near (the
-                                pipelined kernel's sponge form, on the second stream) */
+    int32_t n_partial;       /* AB pattern, FP32 arithmetic: regular blocks that overhang the extent, no solid
+                                near (in a domain whose block layers span 2 GiB or more they count as
+                                boundary blocks) */
+    int32_t n_sponge;        /* AB pattern, FP32 arithmetic: regular blocks with sponge cells and no solid
+                                near */
     int32_t n_solid_regular; /* of n_boundary_regular: blocks whose only flag is a solid cell near, away
-                                from the domain faces (FP32 arithmetic, halfway bounce-back: the
-                                pipelined kernel's solid-link form on steps that do not collect the
-                                force) */
+                                from the domain faces */
 } OalLevelInfo;
 int oal_level_info(const OalPlan* plan, int level, OalLevelInfo* info);
 
@@ -332,8 +332,7 @@ int oal_set_bouzidi(OalPlan* plan, int level, const uint16_t* q_map, int32_t ff_
  * [x,y,z,b], values in [0, 1]; NULL (or all zero) removes it.  A cell with sp > 0 has its density and
  * velocity blended toward (1, u_inlet) before the collision uses them, rho (1 - sp) + sp and
  * u (1 - sp) + (u_inlet, 0, 0) sp; with blend_distributions 1 (SPONGE_BLEND_DISTRIBUTIONS,
- * src/io/config_loader.jl:1312) its populations are blended toward the inlet equilibrium too.  Blocks
- * holding a nonzero strength are stepped by the general kernels.  Requires the AB pattern and a level
+ * src/io/config_loader.jl:1312) its populations are blended toward the inlet equilibrium too.  Requires the AB pattern and a level
  * without interpolated bounce-back; drops captured step graphs. */
 int oal_set_sponge(OalPlan* plan, int level, const float* sponge, int32_t blend_distributions);
 
@@ -391,27 +390,23 @@ int oal_time_steps(OalPlan* plan, int level, int n, int flags, double* ms_total,
  * 8 TB/s datasheet peak. */
 int oal_copy_bandwidth(int device, int64_t bytes, int reps, double* gbs);
 
-/* Launch shape of the step kernels.  pipe_planes: z-planes of a 16^3 block one workgroup of the
- * interior kernel walks with its next plane's loads in flight (1 = one plane per workgroup, no
- * pipelining; 2, 4, 8 or 16).  overlap: 1 = boundary and face launches on a second stream,
- * concurrent with the bulk launch; 0 = every launch in order on the plan's stream.  face_kernel
- * (pull/AB pattern, blocks on a domain face): 0 = the pipelined kernel applies the domain-face rules
- * itself; 1 = it skips the cells on the faces and a separate face-cell kernel steps them.  graph:
- * 1 = oal_step on the plan's own stream (stream NULL) replays a hipGraph of one (coarse) step,
- * captured on first use for each arrangement of the levels' buffers, with the step index read from
- * device memory (a step that collects the force runs as ordinary launches); 0 = the host issues
+/* Launch shape of the step kernels.  pipe_planes (AA pattern, FP32 arithmetic): z-planes of a 16^3
+ * block one workgroup of the regular blocks' kernel walks with its next plane's loads in flight (1 = one
+ * plane per workgroup, no pipelining; 2, 4 or 8; 16 runs as 8).  overlap: 1 = the boundary and face
+ * launches on a second stream, concurrent with the bulk launch; 0 = every launch in order on the plan's
+ * stream.  face_kernel, pair_kernel: accepted and reported, without effect (the AB pattern with FP32
+ * arithmetic has one kernel, two cells per lane with the face rules in it; FP64 steps the face cells in
+ * their own kernel).  graph: 1 = oal_step on the plan's own stream (stream NULL) replays a hipGraph of one
+ * (coarse) step, captured on first use for each arrangement of the levels' buffers, with the step index
+ * read from device memory (a step that collects the force runs as ordinary launches); 0 = the host issues
  * every launch.  Refined plans start with graph 1, one-level plans with 0.  Setting the tuning drops
- * the captured graphs. */
+ * the captured graphs.  Every shape gives the same bits. */
 typedef struct {
     int32_t pipe_planes;
     int32_t overlap;
     int32_t face_kernel;
     int32_t graph;
-    int32_t pair_kernel;   /* FP32 and 16-bit storage, AB pattern, pipe_planes > 1, face_kernel 0, no WALE: the
-                              regular blocks step two cells per lane (8-byte FP32 / 4-byte 16-bit words holding
-                              both): 1 in one launch (the FP32 default), 2 with the blocks on a domain face in a
-                              launch of their own (the 16-bit default); 0 = one cell per lane; the same bits
-                              every way */
+    int32_t pair_kernel;
     int32_t reserved[3];
 } OalTuning;
 

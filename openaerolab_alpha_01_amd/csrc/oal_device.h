@@ -359,7 +359,11 @@ struct CellRates {
 // SPONGE: the sponge blend (kernel_cumulant.jl:428-446) of a cell with q.sponge > 0: rho and u blended
 // toward (1, u_inlet) before the collision uses them, and with q.sponge_blend the populations toward the
 // inlet equilibrium, the transform then summing the blended populations.
-template <class T, bool UNIT = false, bool SPONGE = false>
+//
+// LDS_LIMITER: the positivity limiter's populations pass through LDS in a rolled loop (workgroups of 128
+// lanes, each lane its own column).  Unrolled, its 54 equilibria raise the kernel from 90 to 168 registers,
+// which every wave would pay for a branch that few cells take.
+template <class T, bool UNIT = false, bool SPONGE = false, bool LDS_LIMITER = false>
 __device__ __forceinline__ void collide_cell(T (&f)[27], const CellRates<T>& q, const CollParams& p,
                                              T& rho_o, T& ux_o, T& uy_o, T& uz_o) {
     T A[27];
@@ -607,18 +611,43 @@ __device__ __forceinline__ void collide_cell(T (&f)[27], const CellRates<T>& q, 
         const T fmin = fmn(fmn(fmn(fmn(m9[0], m9[1]), m9[2]), fmn(fmn(m9[3], m9[4]), m9[5])),
                            fmn(fmn(m9[6], m9[7]), m9[8]));
         if (fmin < T(0) && A[0] == A[0]) {
-            T alpha = T(1);
+            if constexpr (LDS_LIMITER) {
+                __shared__ T lim[27][128];
+                const int t = threadIdx.x;
 #pragma unroll
-            for (int k = 0; k < 27; ++k) {
-                const T fe = feq_auto(rb, uxe, uye, uze, wgt<T>(k), T(dcx(k)), T(dcy(k)), T(dcz(k)), p.compressible);
-                const T fn = A[k] - fe;
-                if (fn < T(0) && fe > T(1e-15f)) alpha = mn(alpha, fe / (fe - fn + T(1e-15f)));
-            }
-            alpha = mx(alpha, T(0));
+                for (int k = 0; k < 27; ++k) lim[k][t] = A[k];
+                auto fe_of = [&](int k) {
+                    return feq_auto(rb, uxe, uye, uze, wgt_rt<T>(k), T(k % 3 - 1), T((k / 3) % 3 - 1), T(k / 9 - 1), p.compressible);
+                };
+                T alpha = T(1);
+#pragma unroll 1
+                for (int k = 0; k < 27; ++k) {
+                    const T fe = fe_of(k);
+                    const T fn = lim[k][t] - fe;
+                    if (fn < T(0) && fe > T(1e-15f)) alpha = mn(alpha, fe / (fe - fn + T(1e-15f)));
+                }
+                alpha = mx(alpha, T(0));
+#pragma unroll 1
+                for (int k = 0; k < 27; ++k) {
+                    const T fe = fe_of(k);
+                    lim[k][t] = fe + alpha * (lim[k][t] - fe);
+                }
 #pragma unroll
-            for (int k = 0; k < 27; ++k) {
-                const T fe = feq_auto(rb, uxe, uye, uze, wgt<T>(k), T(dcx(k)), T(dcy(k)), T(dcz(k)), p.compressible);
-                A[k] = fe + alpha * (A[k] - fe);
+                for (int k = 0; k < 27; ++k) A[k] = lim[k][t];
+            } else {
+                T alpha = T(1);
+#pragma unroll
+                for (int k = 0; k < 27; ++k) {
+                    const T fe = feq_auto(rb, uxe, uye, uze, wgt<T>(k), T(dcx(k)), T(dcy(k)), T(dcz(k)), p.compressible);
+                    const T fn = A[k] - fe;
+                    if (fn < T(0) && fe > T(1e-15f)) alpha = mn(alpha, fe / (fe - fn + T(1e-15f)));
+                }
+                alpha = mx(alpha, T(0));
+#pragma unroll
+                for (int k = 0; k < 27; ++k) {
+                    const T fe = feq_auto(rb, uxe, uye, uze, wgt<T>(k), T(dcx(k)), T(dcy(k)), T(dcz(k)), p.compressible);
+                    A[k] = fe + alpha * (A[k] - fe);
+                }
             }
         }
     }

@@ -44,7 +44,7 @@ struct DevDomain {
 struct StepArgs {
     const void* fin;             // populations read this step
     void* fout;                  // populations written (== fin for the AA pattern)
-    const int32_t* nbr_bm;       // [32 * nb] block-major neighbour rows, 0-based, -1 = none
+    const int32_t* nbr_bm;       // [32 * nb] block-major neighbour rows, 0-based, -1 = none; entry 27: the lowest
     const int32_t* borg;         // [3 * nb] block origin in cells
     const int32_t* bdom;         // [nb] domain index
     const uint32_t* bflags;      // [nb]
@@ -60,23 +60,19 @@ struct StepArgs {
     const int32_t* blist_boundary_regular;  // [n_boundary_regular] boundary blocks with lexicographic neighbours
     const int32_t* blist_boundary;   // [n_boundary] the other blocks
     uint32_t n_regular, n_interior, n_boundary_regular, n_boundary;
-    uint32_t n_boundary_regular_solid;   // blocks at the head of blist_boundary_regular whose only flag is BF_SOLID
-    const int32_t* blist_partial;    // [n_partial] AB pattern: regular blocks that overhang the extent, no solid near
-    uint32_t n_partial;
-    const int32_t* blist_sponge;     // [n_sponge] AB pattern: regular blocks with sponge cells, no solid near
-    uint32_t n_sponge;
-    // the regular list split (AB pattern): blocks on no domain face, and whole blocks on a domain face
-    const int32_t* blist_regular_plain;
-    uint32_t n_regular_plain;
-    const int32_t* blist_regular_face;
-    uint32_t n_regular_face;
+    // the two-cells-per-lane kernel's blocks (AB pattern, FP32 arithmetic; blist_boundary_regular and
+    // blist_boundary then hold the blocks it does not take): without sponge cells, with sponge cells, and
+    // the former split into those with solid links near and the others
+    const int32_t* blist_two;
+    const int32_t* blist_two_sponge;
+    const int32_t* blist_two_links;
+    const int32_t* blist_two_free;
+    uint32_t n_two, n_two_sponge, n_two_links, n_two_free;
     const int32_t* lslot;        // [nb] link-mask slot of a block with solid cells near, -1 = none
     const uint32_t* lmask;       // [n_lslots * BS3] per cell: bit k source of direction k solid, bit 27 cell solid
     const uint32_t* face_cells;  // [n_face] AB pattern: cells of regular-list blocks with a source outside the extent
     uint32_t n_face;
     int32_t regular_face;        // AB pattern: the blocks of this launch may lie on a domain face (set per launch)
-    int32_t face_kernel;         // 1: the pipelined kernel skips face cells and the face-cell kernel steps
-                                 // them; 0: it applies the face rules itself
     const int32_t* oslot;        // [nb] AA pattern: outlet side-buffer slot of the block, -1 = none
     void* obuf;                  // [n_oslots * 9 * BS2] AA pattern: outlet-face populations with cx = -1
     uint32_t ncell;              // cells of the level (the stride of the velocity fields' components)
@@ -90,7 +86,6 @@ struct StepArgs {
     int32_t parity;              // AA pattern: 1 odd step (neighbour slots), 0 even step (own slots)
     int32_t pipe_planes;         // planes per workgroup of the pipelined interior kernel (1 = off; divides 16)
     int32_t face_x;              // a domain of the level has the exact specular z wall, or the transverse freestream is on
-    int32_t pair_kernel;         // FP32 / 16-bit storage: regular blocks two cells per lane (pipelined shapes)
     // interpolated bounce-back: per link-mask slot, [27][BS3] Float16 bits of the wall distance q of the
     // link from a cell along c_k (units of |c_k|); null = halfway bounce-back on every solid link
     const uint16_t* qmap;
@@ -105,12 +100,10 @@ struct StepArgs {
     __device__ __forceinline__ int32_t step() const { return ts_dev ? ts_dev[0] * ts_mul + ts_add : time_step; }
 };
 
-// Whether a domain's block grid fits the 32-bit offsets of the two-cells-per-lane kernels (populations
-// of `esize` bytes, one buffer resource per block): two layers of blocks, two rows and three blocks
-// below 4 GiB
-inline bool pair_fits(int nbx, int nby, int esize = 2) {
-    const uint64_t blk = 27ull * BS3 * (uint64_t)esize;
-    return 2ull * (uint64_t)nbx * (uint64_t)nby * blk + (2ull * (uint64_t)nbx + 3ull) * blk < (1ull << 32);
+// Whether the two-cells-per-lane kernel's 32-bit byte offsets span a block's neighbours (block indices lo to
+// hi, populations of `esize` bytes)
+inline bool two_fits(int64_t lo, int64_t hi, uint64_t esize) {
+    return (uint64_t)(hi - lo + 1) * 27ull * BS3 * esize < (1ull << 32);
 }
 
 struct ReduceArgs {
@@ -140,6 +133,12 @@ hipError_t launch_step_f16s(int stream_mode, bool wale, const StepArgs& a, hipSt
                             hipEvent_t bulk0, hipEvent_t bulk1);
 hipError_t launch_step_bf16s(int stream_mode, bool wale, const StepArgs& a, hipStream_t stream, hipStream_t side,
                              hipEvent_t bulk0, hipEvent_t bulk1);
+// the two-cells-per-lane step kernel over a.blist (a.n_items workgroups): oal_two_<storage>.hip
+void launch_two_f32(bool wale, int extra, const StepArgs& a, hipStream_t stream);
+void launch_two_f16s(bool wale, int extra, const StepArgs& a, hipStream_t stream);
+void launch_two_bf16s(bool wale, int extra, const StepArgs& a, hipStream_t stream);
+// and over the n blocks of a list, by storage code
+void launch_two(int storage, bool wale, int extra, const int32_t* list, uint32_t n, hipStream_t stream, const StepArgs& a);
 hipError_t launch_copy16(const void* src, void* dst, size_t bytes, hipStream_t stream);
 // Host arrays of init / conversion / macro output cover the first nhost cells of a level (the caller's
 // blocks); the device arrays have ncell cells per direction.

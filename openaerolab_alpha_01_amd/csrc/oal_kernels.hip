@@ -18,6 +18,18 @@ hipError_t launch_step(int storage, int stream_mode, bool wale, const StepArgs& 
     }
 }
 
+void launch_two(int storage, bool wale, int extra, const int32_t* list, uint32_t n, hipStream_t stream, const StepArgs& a) {
+    if (!n) return;
+    StepArgs r = a;
+    r.blist = list;
+    r.n_items = n * PLANES;
+    switch (storage) {
+        case 0: launch_two_f32(wale, extra, r, stream); break;
+        case 2: launch_two_f16s(wale, extra, r, stream); break;
+        default: launch_two_bf16s(wale, extra, r, stream); break;
+    }
+}
+
 // ------------------------------------------------------------------------------------------------
 // Bandwidth probe: a streaming 16-byte copy, the measured HBM ceiling of the roofline
 // ------------------------------------------------------------------------------------------------

@@ -97,17 +97,19 @@ struct Level {
     DevBuf<int32_t> oslot;             // AA: outlet side-buffer slot per block
     DevBuf<int32_t> blist_rg, blist_in, blist_br, blist_bd;  // block lists per kernel kind
     uint32_t n_regular = 0, n_interior = 0, n_boundary_regular = 0, n_boundary = 0;
-    uint32_t n_br_solid = 0;   // blocks at the head of the regular boundary list whose only flag is BF_SOLID
-    DevBuf<int32_t> blist_pr;          // regular blocks that overhang the extent (pipelined, AB)
-    DevBuf<int32_t> blist_sp;          // regular blocks with sponge cells, no solid near (pipelined, AB)
-    uint32_t n_sponge = 0;
-    uint32_t n_partial = 0;
-    // the regular blocks split in two (AB), for the kernels that step the ones on a domain face apart
-    DevBuf<int32_t> blist_rp, blist_rf;   // plain (no face) and on a domain face, each in lexicographic order
-    uint32_t n_regular_face = 0;          // (n_regular counts them too)
+    uint32_t n_br_solid = 0;   // regular boundary blocks whose only flag is BF_SOLID
+    uint32_t n_partial = 0;            // regular blocks that overhang the extent, no solid near (AB)
+    uint32_t n_sponge = 0;             // regular blocks with sponge cells, no solid near (AB)
     DevBuf<uint32_t> face_cells;       // AB: face cells of the regular-list blocks
     uint32_t n_face = 0;
     bool regular_face = false;         // AB: the regular list holds blocks on a domain face
+    // the two-cells-per-lane kernel's blocks (AB pattern, FP32 arithmetic): without and with sponge cells,
+    // the former also split by solid links near (interpolated bounce-back); the boundary blocks it does not
+    // take, with and without lexicographic neighbours
+    DevBuf<int32_t> blist_tw, blist_ts, blist_tl, blist_tn, blist_xr, blist_xb;
+    uint32_t n_two = 0, n_two_sponge = 0, n_two_links = 0, n_two_free = 0, n_rest_regular = 0, n_rest = 0;
+    std::vector<char> two_fit_h;       // a block's neighbours lie within that kernel's 32-bit offsets
+    bool two() const { return ab && fp32; }
     DevBuf<int32_t> lslot;             // link-mask slot per block
     DevBuf<uint32_t> lmask;            // per-cell solid-link masks of blocks near solid cells
     std::vector<int32_t> lslot_h;      // host copy of lslot
@@ -155,7 +157,7 @@ struct Level {
     std::vector<uint32_t> flags_h;
     std::vector<char> regular_h, near_h;
     std::vector<int32_t> borg_h, bdom_h;
-    bool ab = true, pipe_ok = true;
+    bool ab = true, fp32 = true, bb_halfway = true;
     bool tfs = false;                // transverse freestream on the y and z faces
     // sponge (kernel_cumulant.jl:428-446): per sponge slot [BS3] strengths of the blocks that hold a
     // nonzero one (empty: no sponge)
@@ -182,7 +184,8 @@ struct Level {
     void release() {
         nbr.release(); borg.release(); bdom.release(); dom_item0.release(); dom_block0.release();
         bflags.release(); solid.release(); doms.release(); fA.release(); fB.release(); velA.release(); velB.release();
-        fpart.release(); mpart.release(); red_out.release(); guard.release(); oslot.release(); obuf.release(); blist_rg.release(); blist_in.release(); blist_br.release(); blist_bd.release(); blist_pr.release(); blist_sp.release(); blist_rp.release(); blist_rf.release(); face_cells.release();
+        blist_tw.release(); blist_ts.release(); blist_tl.release(); blist_tn.release(); blist_xr.release(); blist_xb.release();
+        fpart.release(); mpart.release(); red_out.release(); guard.release(); oslot.release(); obuf.release(); blist_rg.release(); blist_in.release(); blist_br.release(); blist_bd.release(); face_cells.release();
         lslot.release(); lmask.release(); qmap.release(); sponge.release(); sslot.release();
         g_src.release(); g_dst.release(); g_slot.release(); g_w.release(); g_m.release();
         r_src.release(); r_dst.release(); r_slot.release(); r_w.release(); r_m.release();
@@ -242,8 +245,8 @@ int upload(DevBuf<T>& d, const std::vector<T>& h) {
 
 // Host tables of one level, built and validated before any device call
 struct HostLevel {
-    std::vector<int32_t> borg, bdom, nbr, nbr_bm, oslot, blist_rg, blist_in, blist_br, blist_bd, blist_pr, blist_sp, blist_rp, blist_rf,
-        lslot;
+    std::vector<int32_t> borg, bdom, nbr, nbr_bm, oslot, blist_rg, blist_in, blist_br, blist_bd,
+        blist_tw, blist_ts, blist_tl, blist_tn, blist_xr, blist_xb, lslot;
     std::vector<uint32_t> lmask;
     std::vector<uint32_t> face_cells;
     int32_t n_oslots = 0;
@@ -254,8 +257,9 @@ struct HostLevel {
 // The block lists of a level's step kernels from its block flags (L.flags_h) and the host tables kept
 // for that purpose; rebuilt when the flags change (a sponge field marks its blocks).
 void build_lists(Level& L, HostLevel& H) {
-    H.blist_rg.clear(); H.blist_rp.clear(); H.blist_rf.clear(); H.blist_in.clear();
-    H.blist_br.clear(); H.blist_bd.clear(); H.blist_pr.clear(); H.blist_sp.clear(); H.face_cells.clear();
+    H.blist_rg.clear(); H.blist_in.clear(); H.blist_br.clear(); H.blist_bd.clear(); H.face_cells.clear();
+    L.n_partial = L.n_sponge = 0;
+    for (auto* l : {&H.blist_tw, &H.blist_ts, &H.blist_tl, &H.blist_tn, &H.blist_xr, &H.blist_xb}) l->clear();
     L.regular_face = false;
     const std::vector<uint32_t>& flags = L.flags_h;
     // blocks on a face whose rule the pipelined kernels do not apply (the exact specular z wall reads
@@ -275,14 +279,24 @@ void build_lists(Level& L, HostLevel& H) {
         if (flags[b] & BF_INACTIVE) continue;   // never stepped
         const bool regular = L.regular_h[b] != 0;
         const bool special = (flags[b] & BF_EDGE) && special_face(b, dm);
+        // the two-cells-per-lane kernel takes every block but those with an absent neighbour inside the
+        // extent, those under the exact specular z wall or the transverse freestream, those near solid
+        // cells with the reference's reflection, and those whose neighbours its 32-bit offsets do not span
+        // (4 GiB of populations: the wraps of periodic levels and the ghosts of octree levels beyond that)
+        if ((flags[b] & BF_MISSING) || special || !L.two_fit_h[b] || ((flags[b] & BF_SOLID) && !L.bb_halfway)) {
+            (regular ? H.blist_xr : H.blist_xb).push_back((int32_t)b);
+        } else if (flags[b] & BF_SPONGE) {
+            H.blist_ts.push_back((int32_t)b);
+        } else {
+            H.blist_tw.push_back((int32_t)b);
+            ((flags[b] & BF_SOLID) ? H.blist_tl : H.blist_tn).push_back((int32_t)b);
+        }
         if (flags[b] == 0) {
             (regular ? H.blist_rg : H.blist_in).push_back((int32_t)b);
-            if (regular) H.blist_rp.push_back((int32_t)b);
         } else if (L.ab && regular && flags[b] == BF_EDGE && !special) {
             // AB pattern: a whole block on a domain face, no solid near, joins the regular list; the
             // cells on its faces (sources outside the extent) go to the face-cell list
             H.blist_rg.push_back((int32_t)b);
-            H.blist_rf.push_back((int32_t)b);
             L.regular_face = true;
             const int o[3] = {L.borg_h[3 * b], L.borg_h[3 * b + 1], L.borg_h[3 * b + 2]};
             bool lo[3], hi[3];
@@ -298,39 +312,31 @@ void build_lists(Level& L, HostLevel& H) {
                         for (int a = 0; a < 3; ++a) face = face || (lo[a] && l[a] == 0) || (hi[a] && l[a] == BS - 1);
                         if (face) H.face_cells.push_back(b * BS3 + (uint32_t)(x + BS * (y + BS * z)));
                     }
-        } else if (L.ab && L.pipe_ok && regular && flags[b] == (BF_EDGE | BF_PARTIAL) && L.near_h[L.bdom_h[b]] && !special) {
-            // AB pattern: a block that overhangs the extent, no solid near: the pipelined kernel with the
-            // face rules at the extent's last cells (in a domain whose block layers span 2 GiB or more the
-            // one-plane boundary kernel, whose addresses are 64-bit)
-            H.blist_pr.push_back((int32_t)b);
-        } else if (L.ab && L.pipe_ok && regular && (flags[b] & BF_SPONGE) && !(flags[b] & ~(BF_SPONGE | BF_EDGE | BF_PARTIAL)) &&
+        } else if (L.ab && L.fp32 && regular && flags[b] == (BF_EDGE | BF_PARTIAL) && L.near_h[L.bdom_h[b]] && !special) {
+            ++L.n_partial;
+        } else if (L.ab && L.fp32 && regular && (flags[b] & BF_SPONGE) && !(flags[b] & ~(BF_SPONGE | BF_EDGE | BF_PARTIAL)) &&
                    L.near_h[L.bdom_h[b]] && !special) {
-            // AB pattern: a block with sponge cells and no solid near (whole or overhanging the extent):
-            // the pipelined kernel's sponge form, with the face rules at the extent's last cells
-            H.blist_sp.push_back((int32_t)b);
+            ++L.n_sponge;
         } else {
             (regular ? H.blist_br : H.blist_bd).push_back((int32_t)b);
         }
     }
-    // the regular boundary blocks whose only flag is a solid cell near first (the pipelined kernel's
-    // solid-link form takes them where it applies)
-    {
-        const auto mid = std::stable_partition(H.blist_br.begin(), H.blist_br.end(),
-                                               [&](int32_t b) { return flags[b] == BF_SOLID; });
-        L.n_br_solid = (uint32_t)(mid - H.blist_br.begin());
-    }
+    L.n_br_solid = (uint32_t)std::count_if(H.blist_br.begin(), H.blist_br.end(), [&](int32_t b) { return flags[b] == BF_SOLID; });
     L.n_face = (uint32_t)H.face_cells.size();
-    L.n_regular_face = (uint32_t)H.blist_rf.size();
     L.n_regular = (uint32_t)H.blist_rg.size();
     L.n_interior = (uint32_t)H.blist_in.size();
     L.n_boundary_regular = (uint32_t)H.blist_br.size();
-    L.n_partial = (uint32_t)H.blist_pr.size();
-    L.n_sponge = (uint32_t)H.blist_sp.size();
     L.n_boundary = (uint32_t)H.blist_bd.size();
+    L.n_two = (uint32_t)H.blist_tw.size();
+    L.n_two_sponge = (uint32_t)H.blist_ts.size();
+    L.n_two_links = (uint32_t)H.blist_tl.size();
+    L.n_two_free = (uint32_t)H.blist_tn.size();
+    L.n_rest_regular = (uint32_t)H.blist_xr.size();
+    L.n_rest = (uint32_t)H.blist_xb.size();
 }
 
 // Host-side construction of one level's tables from the reference-convention descriptor.
-int prepare_level(const OalLevelDesc& d, const OalCollision& coll, bool ab, bool pipe_ok, size_t sbytes, Level& L, HostLevel& H,
+int prepare_level(const OalLevelDesc& d, const OalCollision& coll, bool ab, bool fp32, bool bb_halfway, size_t sbytes, Level& L, HostLevel& H,
                   const std::vector<uint8_t>* inactive = nullptr) {
     if (d.n_blocks <= 0) return fail(OAL_ERR_ARG, "level with no blocks");
     if (!d.map_x || !d.map_y || !d.map_z || !d.neighbor_table) return fail(OAL_ERR_ARG, "level block arrays missing");
@@ -488,18 +494,33 @@ int prepare_level(const OalLevelDesc& d, const OalCollision& coll, bool ab, bool
         }
         L.regular_h[b] = regular ? 1 : 0;
     }
+    // block-major copy of the neighbour table: one 32-entry row per block (scalar loads)
+    H.nbr_bm.assign((size_t)nb * 32, -1);
+    // (entry 27: the lowest index among them, the base of the two-cells-per-lane kernel's 32-bit byte
+    // offsets, which must reach the highest)
+    L.two_fit_h.assign(nb, 0);
+    for (uint32_t b = 0; b < nb; ++b) {
+        int32_t lo = (int32_t)b, hi = (int32_t)b;
+        for (int k = 0; k < 27; ++k) {
+            const int32_t n = k == 13 ? (int32_t)b : nbr[(size_t)k * nb + b];
+            H.nbr_bm[(size_t)b * 32 + k] = n;
+            if (n >= 0) {
+                lo = std::min(lo, n);
+                hi = std::max(hi, n);
+            }
+        }
+        H.nbr_bm[(size_t)b * 32 + 27] = lo;
+        L.two_fit_h[b] = two_fits(lo, hi, (uint64_t)sbytes) ? 1 : 0;
+    }
     L.near_h = near;
     L.flags_h = flags;
     L.borg_h = borg;
     L.bdom_h = bdom;
     L.ab = ab;
-    L.pipe_ok = pipe_ok;
+    L.fp32 = fp32;
+    L.bb_halfway = bb_halfway;
     L.tfs = coll.transverse_freestream != 0;
     build_lists(L, H);
-    // block-major copy of the neighbour table: one 32-entry row per block (scalar loads)
-    H.nbr_bm.assign((size_t)nb * 32, -1);
-    for (uint32_t b = 0; b < nb; ++b)
-        for (int k = 0; k < 27; ++k) H.nbr_bm[(size_t)b * 32 + k] = k == 13 ? (int32_t)b : nbr[(size_t)k * nb + b];
     // blocks holding an outlet face (x = extent - 1 of a non-periodic x axis): AA side-buffer slots
     H.oslot.assign(nb, -1);
     for (uint32_t b = 0; b < nb; ++b) {
@@ -973,7 +994,9 @@ int upload_level(OalPlan* p, Level& L, const HostLevel& H) {
         return rc;
     if (!H.solid.empty() && (rc = upload(L.solid, H.solid))) return rc;
     if ((rc = upload(L.blist_rg, H.blist_rg)) || (rc = upload(L.blist_in, H.blist_in)) ||
-        (rc = upload(L.blist_br, H.blist_br)) || (rc = upload(L.blist_bd, H.blist_bd)) || (rc = upload(L.blist_pr, H.blist_pr)) || (rc = upload(L.blist_sp, H.blist_sp)) || (rc = upload(L.blist_rp, H.blist_rp)) || (rc = upload(L.blist_rf, H.blist_rf)) ||
+        (rc = upload(L.blist_br, H.blist_br)) || (rc = upload(L.blist_bd, H.blist_bd)) ||
+        (rc = upload(L.blist_tw, H.blist_tw)) || (rc = upload(L.blist_ts, H.blist_ts)) || (rc = upload(L.blist_tl, H.blist_tl)) ||
+        (rc = upload(L.blist_tn, H.blist_tn)) || (rc = upload(L.blist_xr, H.blist_xr)) || (rc = upload(L.blist_xb, H.blist_xb)) ||
         (rc = upload(L.lslot, H.lslot)) || (rc = upload(L.lmask, H.lmask)) || (rc = upload(L.face_cells, H.face_cells)))
         return rc;
     if (p->stream_mode == OAL_STREAM_AA) {
@@ -1021,29 +1044,14 @@ StepArgs make_args(OalPlan* p, Level& L, int32_t time_step, bool want_force) {
     a.blist_boundary_regular = L.blist_br.p;
     a.blist_boundary = L.blist_bd.p;
     a.n_regular = L.n_regular;
-    a.blist_regular_plain = L.blist_rp.p;
-    a.n_regular_plain = L.n_regular - L.n_regular_face;
-    a.blist_regular_face = L.blist_rf.p;
-    a.n_regular_face = L.n_regular_face;
-    a.blist_partial = L.blist_pr.p;
-    a.blist_sponge = L.blist_sp.p;
-    a.n_sponge = L.n_sponge;
-    a.n_partial = L.n_partial;
     a.n_interior = L.n_interior;
     a.n_boundary_regular = L.n_boundary_regular;
     a.n_boundary = L.n_boundary;
-    a.n_boundary_regular_solid = L.pipe_ok ? L.n_br_solid : 0;
     a.lslot = L.lslot.p;
     a.lmask = L.lmask.p;
     a.face_cells = L.face_cells.p;
     a.n_face = L.n_face;
     a.regular_face = L.regular_face ? 1 : 0;
-    // the in-kernel face rules address by signed 32-bit byte offsets from a block: a domain whose
-    // layer of blocks (plus a row and a block) spans 2 GiB or more takes the face-cell kernel
-    bool near = true;
-    for (const DevDomain& dm : L.doms_h)
-        near = near && ((uint64_t)dm.nbx * dm.nby + dm.nbx + 1) * 27u * BS3 * (uint64_t)storage_bytes(p->storage) < (1ull << 31);
-    a.face_kernel = (p->face_kernel || !near) ? 1 : 0;
     a.face_x = p->cp.tfs ? 1 : 0;
     for (const DevDomain& dm : L.doms_h) a.face_x |= dm.zwall == 1 ? 1 : 0;
     a.obuf = L.obuf.p;
@@ -1063,10 +1071,20 @@ StepArgs make_args(OalPlan* p, Level& L, int32_t time_step, bool want_force) {
     }
     a.parity = p->stream_mode == OAL_STREAM_AA ? (L.aa_phase == 0 ? 1 : 0) : 0;
     a.pipe_planes = p->pipe_planes;
-    // (two cells per lane where the level's block grid fits its 32-bit offsets)
-    bool pair_ok = p->pair_kernel != 0;
-    for (const DevDomain& dm : L.doms_h) pair_ok = pair_ok && pair_fits(dm.nbx, dm.nby, p->storage == OAL_F32 ? 4 : 2);
-    a.pair_kernel = pair_ok ? p->pair_kernel : 0;
+    a.blist_two = L.blist_tw.p;
+    a.n_two = L.n_two;
+    a.blist_two_sponge = L.blist_ts.p;
+    a.n_two_sponge = L.n_two_sponge;
+    a.blist_two_links = L.blist_tl.p;
+    a.n_two_links = L.n_two_links;
+    a.blist_two_free = L.blist_tn.p;
+    a.n_two_free = L.n_two_free;
+    if (L.two()) {   // the boundary kernels keep the blocks it does not take
+        a.blist_boundary_regular = L.blist_xr.p;
+        a.n_boundary_regular = L.n_rest_regular;
+        a.blist_boundary = L.blist_xb.p;
+        a.n_boundary = L.n_rest;
+    }
     a.qmap = L.qmap.p;
     a.sponge = L.has_sponge ? L.sponge.p : nullptr;
     a.sslot = L.sslot.p;
@@ -1085,8 +1103,9 @@ int level_step(OalPlan* p, int level, int32_t time_step, int flags, hipStream_t 
     if (want_force && !L.has_solid) return fail(OAL_ERR_STATE, "force requested on a level without obstacle cells");
     StepArgs a = make_args(p, L, time_step, want_force);
     // side-stream work: boundary blocks, face cells and the blocks that overhang the extent
-    const bool split = p->overlap && L.n_regular + L.n_interior > 0 &&
-                       L.n_boundary_regular + L.n_boundary + L.n_face + L.n_partial + L.n_sponge > 0;
+    const bool split = p->overlap && (L.two() ? a.n_two + a.n_two_sponge > 0 && a.n_boundary_regular + a.n_boundary > 0
+                                              : L.n_regular + L.n_interior > 0 &&
+                                                    L.n_boundary_regular + L.n_boundary + L.n_face > 0);
     if (split) {
         // fork: the side stream starts after everything queued on s, then s waits for the side stream
         OAL_HIP(hipEventRecord(p->fork, s));
@@ -1531,8 +1550,8 @@ int oal_plan_create(const OalPlanDesc* desc, OalPlan** out) {
             for (int b = 0; b < o.nb(); ++b) inactive[b] = o.status[b] != OCT_STEPPED;
         }
         // the pipelined kernels cover FP32-arithmetic storage
-        const bool pipe_ok = desc->storage != OAL_F64;
-        const int rc = prepare_level(d, desc->collision, desc->stream_mode == OAL_STREAM_AB, pipe_ok,
+        const bool fp32 = desc->storage != OAL_F64;
+        const int rc = prepare_level(d, desc->collision, desc->stream_mode == OAL_STREAM_AB, fp32, desc->bb_mode == OAL_BB_HALFWAY,
                                      storage_bytes(desc->storage), p->levels[l],
                                      host[l], ml ? &inactive : nullptr);
         if (rc) return bail(rc);
@@ -1731,7 +1750,7 @@ int oal_level_info(const OalPlan* p, int level, OalLevelInfo* info) {
     info->n_regular = (int32_t)L.n_regular;
     info->n_partial = (int32_t)L.n_partial;
     info->n_sponge = (int32_t)L.n_sponge;
-    info->n_solid_regular = L.pipe_ok ? (int32_t)L.n_br_solid : 0;
+    info->n_solid_regular = L.fp32 ? (int32_t)L.n_br_solid : 0;
     info->n_interior = (int32_t)L.n_interior;
     info->n_boundary_regular = (int32_t)L.n_boundary_regular;
     info->n_boundary = (int32_t)L.n_boundary;
@@ -1960,7 +1979,7 @@ int oal_time_steps(OalPlan* p, int level, int n, int flags, double* ms_total, do
     OAL_HIP(hipSetDevice(p->device));
     OAL_HIP(hipStreamSynchronize(p->stream));
     const Level& L = p->levels[level];
-    const bool bulk = L.n_regular + L.n_interior > 0;
+    const bool bulk = L.two() ? L.n_two + L.n_two_sponge > 0 : L.n_regular + L.n_interior > 0;
     if (bulk) {
         while (p->bulk_ev.size() < 2 * (size_t)n) {
             hipEvent_t e = nullptr;
@@ -2083,8 +2102,10 @@ static int set_sponge_lib(OalPlan* p, int level, const float* sponge, int32_t bl
     auto re = [](auto& d, const auto& h) { d.release(); return upload(d, h); };
     int rc;
     if ((rc = re(L.bflags, L.flags_h)) || (rc = re(L.blist_rg, H.blist_rg)) || (rc = re(L.blist_in, H.blist_in)) ||
-        (rc = re(L.blist_br, H.blist_br)) || (rc = re(L.blist_bd, H.blist_bd)) || (rc = re(L.blist_pr, H.blist_pr)) || (rc = re(L.blist_sp, H.blist_sp)) ||
-        (rc = re(L.blist_rp, H.blist_rp)) || (rc = re(L.blist_rf, H.blist_rf)) || (rc = re(L.face_cells, H.face_cells)) ||
+        (rc = re(L.blist_br, H.blist_br)) || (rc = re(L.blist_bd, H.blist_bd)) ||
+       
+        (rc = re(L.blist_tw, H.blist_tw)) || (rc = re(L.blist_ts, H.blist_ts)) || (rc = re(L.blist_tl, H.blist_tl)) ||
+        (rc = re(L.blist_tn, H.blist_tn)) || (rc = re(L.blist_xr, H.blist_xr)) || (rc = re(L.blist_xb, H.blist_xb)) || (rc = re(L.face_cells, H.face_cells)) ||
         (rc = re(L.sponge, vals)) || (rc = re(L.sslot, slot)))
         return rc;
     L.has_sponge = !vals.empty();

@@ -60,6 +60,9 @@ enum : int {
     SRC_TFS = 9      // transverse freestream: own population blended toward feq(1, u_inlet)  :323-339
 };
 
+// what a level needs beside the plain step in the two-cells-per-lane kernel
+enum : int { TWO_PLAIN = 0, TWO_SPONGE = 1, TWO_BFL = 2 };
+
 enum : int { PAT_AB = 0, PAT_AA_EVEN = 1, PAT_AA_ODD = 2 };
 
 // Uniform (per-workgroup) and per-lane state of one cell
@@ -191,9 +194,8 @@ struct RegAddr {
 
 // Faces of non-periodic axes that a block of the regular list touches.  Such blocks are whole (not
 // partial), so a face is where the block's origin is 0 or its far side is the extent.  Cells on a face
-// have sources outside the extent: the pipelined kernel applies their rules itself (FACE_RULES) or
-// skips these cells (FACE_SKIP), the one-plane regular kernel skips them; the face-cell kernel steps
-// the skipped cells.
+// have sources outside the extent: the one-plane regular kernel skips them and the face-cell kernel steps
+// them (FP64).
 struct FaceBits {
     bool xlo, xhi, ylo, yhi, zlo, zhi;
 };
@@ -685,415 +687,9 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(step_wa
     if (a.fpart) wg_sum3(F0 * dm->force_scale, F1 * dm->force_scale, F2 * dm->force_scale, a.fpart, item);
 }
 
-// Regular interior blocks, pull/AB pattern, software-pipelined over z: a workgroup walks `a.pipe_planes`
-// consecutive planes of one block and issues the loads of the next plane before the collision of the
-// current one, so every wave keeps a plane of loads in flight while it computes.
-//
-// Vector-memory loads and stores share one completion counter on gfx950, and with both pending the
-// compiler may only wait for all of them.  The schedule is therefore: wait for everything at the top of
-// an iteration (the current plane's loads and the previous plane's stores, both issued one collision
-// earlier), issue the next plane's loads, then collide and store the current plane from registers that
-// are already complete.  Prefetched values stay in their storage form until the collision uses them.
-template <class SP>
-__device__ __forceinline__ void reg_load_raw(const StepArgs& a, const RegAddr<SP>& ra, int z, typename SP::raw (&r)[27]) {
-    using st = typename SP::st;
-    for_dirs([&](auto kc) {
-        constexpr int K = decltype(kc)::value;
-        r[K] = SP::ld_raw((const st*)(ra.base(a.fin, K, z, dcz(K)) + ra.v[dcx(K) + 1][dcy(K) + 1]));
-    });
-}
-
 __device__ __forceinline__ void wait_all_vmem() {
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0), expcnt and lgkmcnt left open
     __builtin_amdgcn_sched_barrier(0);
-}
-
-// inlet: the equilibrium at (1, u_inlet + noise) for the directions entering through x = 0
-struct InletRule {
-    bool on;          // this lane's cell lies on the inlet face
-    float u_in;
-    int gy, gz;       // the cell's global y and z (the noise position)
-};
-
-// WALE in the pipelined kernel (AB pattern, regular blocks: no solid cell in the block or its halo, the
-// neighbour blocks at lexicographic offsets).  The previous step's velocity at the six face neighbours
-// (x+, x-, y+, y-, z+, z-) of a lane's cell is loaded before the next plane's populations, so that the
-// collision waits for these loads only; a neighbour across a non-periodic domain face is the cell
-// itself (physics_utils.jl:1981-2035, 2217-2233, the rule of wale_of).
-template <class T>
-struct PipeWale {
-    T u[6][3];
-};
-template <class T>
-struct PipeWaleRates {
-    T tau, amr_scale;           // of the domain, read before the first store
-};
-template <class SP, bool UNIT, bool WALE = false, bool SPONGE = false>
-__device__ __forceinline__ void reg_collide_store(const StepArgs& a, const RegAddr<SP>& ra, const CellRates<typename SP::T>& q0,
-                                                  int z, uint32_t cell, const typename SP::raw (&r)[27],
-                                                  const InletRule* inlet = nullptr, bool store = true,
-                                                  const PipeWale<typename SP::T>* wv = nullptr,
-                                                  const PipeWaleRates<typename SP::T>* wr = nullptr, uint32_t vidx = 0,
-                                                  typename SP::T sponge = typename SP::T(0)) {
-    using T = typename SP::T;
-    using st = typename SP::st;
-    CellRates<T> q = q0;
-    if constexpr (SPONGE) q.sponge = sponge;
-    if constexpr (WALE) {
-        const T h = T(0.5);
-        const auto& u = wv->u;
-        const T nu_eddy = wale_nu(h * (u[0][0] - u[1][0]), h * (u[2][0] - u[3][0]), h * (u[4][0] - u[5][0]),
-                                  h * (u[0][1] - u[1][1]), h * (u[2][1] - u[3][1]), h * (u[4][1] - u[5][1]),
-                                  h * (u[0][2] - u[1][2]), h * (u[2][2] - u[3][2]), h * (u[4][2] - u[5][2]), T(a.cp.c_wale));
-        cell_rates<T>(nu_eddy, wr->tau, wr->amr_scale, T(a.cp.nu_sgs_bg), a.cp.adaptive_omega4, T(a.cp.lambda),
-                      T(a.cp.omega_4), q.omega1, q.omega4_diag);
-    }
-    T f[27];
-    for_dirs([&](auto kc) {
-        constexpr int K = decltype(kc)::value;
-        f[K] = SP::from_raw(r[K], wgt<T>(K));
-    });
-    if (inlet && inlet->on) {
-        CellCtx c{};
-        c.gy = inlet->gy;
-        c.gz = inlet->gz;
-        for_dirs([&](auto kc) {
-            constexpr int K = decltype(kc)::value;
-            if constexpr (dcx(K) > 0)
-                f[K] = boundary_value<K, T>(SRC_INLET, a, c, inlet->u_in, a.step(), [&](auto) { return T(0); });
-        });
-    }
-    T rho_o, ux_o, uy_o, uz_o;
-    collide_cell<T, UNIT, SPONGE>(f, q, a.cp, rho_o, ux_o, uy_o, uz_o);
-    const bool dith = SP::dithered && a.cp.dither;
-    const uint32_t hc = SP::dithered ? round_cell(round_key(a.step()), cell) : 0u;
-    if (store) {
-        for_dirs([&](auto kc) {
-            constexpr int K = decltype(kc)::value;
-            SP::sto_r((st*)(ra.base(a.fout, K, z, 0) + ra.v[1][1]), f[K], wgt<T>(K), round_bits(hc, K), dith);
-        });
-        if constexpr (WALE) {
-            T* vo = (T*)a.vel_out;
-            vo[vidx] = ux_o; vo[a.ncell + vidx] = uy_o; vo[2 * (size_t)a.ncell + vidx] = uz_o;
-        }
-    }
-}
-
-// Domain-face rules inside the pipelined kernel (AB pattern).  A source outside the extent is replaced
-// by a population of the cell's own state (kernel_cumulant.jl:233-345, the order of classify): the
-// rules only change the address a lane reads, except at the inlet, whose equilibrium replaces the
-// loaded value after conversion.
-struct FaceRules {
-    bool xl, xh, yl, yh;          // per lane: the cell lies on the x-min / x-max / y-min / y-max face
-    bool zlo, zhi;                // the block touches the z-min / z-max face (uniform)
-    bool zwall, ymin_wall;        // no-slip variants of the z faces and of the y-min face (uniform)
-    // blocks that overhang the extent (FACE_PARTIAL): the planes of the z faces inside the block
-    // (-1: none) and, per lane, a cell beyond the extent in x or y (its in-plane source offsets all
-    // point at its own cell; never stored)
-    int zlo_plane, zhi_plane;
-    bool dead;
-};
-
-// Gather with the domain-face rules.  Every read is addressed by its byte offset from the start of
-// the own block, formed in 32-bit arithmetic modulo 2^32 and read as a signed offset: the host uses
-// this form only where a layer of blocks spans less than 2 GiB, so every offset read is exact.  The rules pick, per lane, one
-// of a few candidate offsets that are all computed (uniform parts in scalar registers), so that the
-// choice is a select rather than a branch.
-template <class SP, bool PARTIAL = false>
-__device__ __forceinline__ void reg_load_raw_face(const StepArgs& a, const RegAddr<SP>& ra, const FaceRules& fr, int z,
-                                                  typename SP::raw (&r)[27]) {
-    using st = typename SP::st;
-    const char* f0 = (const char*)a.fin + ra.blk0 * (int64_t)sizeof(st);   // the own block (uniform)
-    const uint32_t nbytes = BS3 * (uint32_t)sizeof(st);                    // one direction slot
-    uint32_t zs[3];                                           // plane shift of sources with cz = -1, 0, 1
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        const int sz = z - (q - 1);
-        const int dz = sz < 0 ? -1 : (sz >= BS ? 1 : 0);
-        zs[q] = (uint32_t)((dz * ra.plane_elems + (int64_t)(sz - BS * dz - ra.zref) * BS2) * (int64_t)sizeof(st));
-    }
-    const bool zlo = PARTIAL ? z == fr.zlo_plane : (fr.zlo && z == 0);       // uniform
-    const bool zhi = PARTIAL ? z == fr.zhi_plane : (fr.zhi && z == BS - 1);
-    // uniform parts pass through readfirstlane, which the optimiser cannot see through: it must not
-    // fold them into per-lane sums and hoist 27 of those out of the plane loop
-    auto uni = [](uint32_t u) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)u); };
-    const uint32_t v11 = (uint32_t)ra.v[1][1];
-    for_dirs([&](auto kc) {
-        constexpr int K = decltype(kc)::value;
-        constexpr int cx = dcx(K), cy = dcy(K), cz = dcz(K);
-        uint32_t o = (uint32_t)ra.v[cx + 1][cy + 1] + uni((uint32_t)K * nbytes + zs[cz + 1]);
-        auto own = [&](uint32_t slot) { return v11 + uni(slot * nbytes + zs[1]); };
-        // lowest precedence first; each later rule overrides (kernel_cumulant.jl:233-345)
-        if constexpr (cz != 0) {
-            const bool zo = cz > 0 ? zlo : zhi;
-            const uint32_t o_z = own(fr.zwall ? dopp(K) : dmir_z(K));
-            o = zo ? o_z : o;                                               // z faces
-            if constexpr (cy != 0) {
-                const bool yo = cy > 0 ? fr.yl : fr.yh;
-                const uint32_t o_y = own(cy > 0 && fr.ymin_wall ? dopp(K) : dmir_y(K));
-                o = (yo && !(zo && fr.zwall)) ? o_y : o;                    // y faces, below no-slip z walls
-            }
-        } else if constexpr (cy != 0) {
-            const bool yo = cy > 0 ? fr.yl : fr.yh;
-            const uint32_t o_y = own(cy > 0 && fr.ymin_wall ? dopp(K) : dmir_y(K));
-            o = yo ? o_y : o;
-        }
-        if constexpr (cx != 0) {
-            const uint32_t o_x = own(K);
-            o = (cx > 0 ? fr.xl : fr.xh) ? o_x : o;    // outlet: own population; inlet: any valid address
-        }
-        r[K] = SP::ld_raw((const st*)(f0 + (int32_t)o));   // within +-2 GiB of the own block
-    });
-}
-
-// FACE: how blocks on a domain face are handled.  FACE_PARTIAL: blocks that overhang the extent, with
-// the face rules at the extent's last cells and the cells beyond it neither read through nor stored.
-// FACE_SOLID: blocks of the regular grid whose only flag is a solid cell in or next to them, away from
-// the domain faces: halfway bounce-back (the source of a solid link is the cell's own slot opp K of the
-// previous step) chosen per lane by address, the link masks loaded two planes ahead
-enum : int { FACE_NONE = 0, FACE_RULES = 1, FACE_SKIP = 2, FACE_PARTIAL = 3, FACE_SOLID = 4 };
-
-// Register budget: with one plane of populations in flight beside the collision of another the kernel
-// fits the 168 VGPRs of 3 waves per SIMD; the in-kernel face rules add per-lane address selects and
-// scalar offsets that only fit the 256 VGPRs of 2 waves.
-#ifndef OAL_FACE_RULES_WAVES
-#define OAL_FACE_RULES_WAVES 2
-#endif
-// (the 16-bit forms' conversions and rounding need more registers: 2 waves for every form of theirs)
-// (WALE's velocity gather as well)
-template <class SP, int FACE, bool WALE = false>
-constexpr int pipe_waves() {
-    return FACE == FACE_RULES || FACE == FACE_PARTIAL || FACE == FACE_SOLID || SP::dithered || WALE ? OAL_FACE_RULES_WAVES : 3;
-}
-
-// UNIT: the collision form for the unit rates omega_bulk = omega_3 = omega_4 = 1 (a separate kernel, so
-// that each form keeps its own register allocation).  WALE: the eddy viscosity from the previous step's
-// velocity, and this step's velocity written.
-// SPONGE: blocks with sponge cells (kernel_cumulant.jl:428-446), each cell's strength loaded with its
-// populations
-template <class SP, int NP, int FACE, bool UNIT, bool WALE = false, bool SPONGE = false>
-__global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(pipe_waves<SP, FACE, WALE>(), pipe_waves<SP, FACE, WALE>())))
-k_step_pipe(const StepArgs a) {
-    using T = typename SP::T;
-    using st = typename SP::st;
-    // the loop bound stays a run-time value (equal to NP): with a constant bound the prefetch
-    // conditions fold away, the scheduler mixes the next plane's loads into the collision and the
-    // kernel spills
-    const int np = a.pipe_planes;
-    constexpr uint32_t groups = (uint32_t)(PLANES / NP);
-    const PipeItem it = pipe_item<false>(groups, np);
-    const uint32_t b = (uint32_t)a.blist[it.pos];
-    const int z0 = it.z0;
-    // FACE_PARTIAL: planes from zmax on lie beyond the extent and are neither read nor stepped (the
-    // loop bound itself stays z0 + np: a bound the compiler can narrow lets it reorder the prefetch)
-    int zmax = BS;
-    if constexpr (FACE == FACE_PARTIAL || FACE == FACE_RULES) {
-        // (FACE_RULES: whole blocks, zmax >= BS; the guard it adds to every plane keeps the compiler from
-        // hoisting the next plane's address arithmetic, which spills at 2 to 8 planes)
-        const DevDomain* d0 = a.doms + a.bdom[b];
-        zmax = d0->ext[2] - a.borg[3 * b + 2];
-        if (FACE == FACE_PARTIAL && z0 >= zmax) return;
-    }
-    CellCtx c;
-    c.b = b;
-    c.lx = threadIdx.x & (BS - 1);
-    c.ly = threadIdx.x >> 4;
-    c.z = z0;
-    c.own = b * BS3 + (uint32_t)z0 * BS2 + (uint32_t)c.ly * BS + (uint32_t)c.lx;
-    const DevDomain* dm = a.doms + a.bdom[b];
-    RegAddr<SP> ra;
-    ra.init(c, dm->nbx, dm->nby);   // offsets of plane z0
-    // every domain parameter is read before the first store: reads issued after stores to the
-    // population arrays could not be proven independent of them
-    CellRates<T> q;
-    if constexpr (sizeof(T) == 8) { q.omega1 = dm->omega1_d; q.omega4_diag = dm->omega4d_d; }
-    else { q.omega1 = dm->omega1; q.omega4_diag = dm->omega4d; }
-    q.forced = dm->forced != 0;
-    q.Fx = T(dm->F[0]); q.Fy = T(dm->F[1]); q.Fz = T(dm->F[2]);
-    const float* sp_cells = nullptr;
-    if constexpr (SPONGE) {
-        q.sponge = T(0);
-        q.sponge_u = T(dm->u_in);
-        q.sponge_blend = a.sponge_blend;
-        if (a.bflags[b] & BF_SPONGE) sp_cells = a.sponge + (size_t)a.sslot[b] * BS3 + (c.own - b * BS3 - (uint32_t)z0 * BS2);
-    }
-    // the strength of the lane's cell in plane z (0 outside the sponge)
-    auto sp_load = [&](int z) -> T {
-        if constexpr (SPONGE) return sp_cells ? T(sp_cells[(uint32_t)z * BS2]) : T(0);
-        else return T(0);
-    };
-    // blocks on a domain face: FACE_RULES applies the face rules here, FACE_SKIP leaves the face cells
-    // to the face-cell kernel
-    FaceRules fr{};
-    InletRule in{};
-    bool lane_face = false;
-    FaceBits fskip{};
-    if constexpr (FACE == FACE_SKIP) {
-        fskip = face_bits(a, b, dm);
-        lane_face = face_lane(fskip, c.lx, c.ly);
-    }
-    auto live = [&](int z) { return FACE != FACE_SKIP || !(lane_face || face_plane(fskip, z)); };
-    if constexpr (FACE == FACE_PARTIAL) {
-        const int gx = a.borg[3 * b] + c.lx, gy = a.borg[3 * b + 1] + c.ly, oz = a.borg[3 * b + 2];
-        fr.xl = !dm->per[0] && gx == 0;
-        fr.xh = !dm->per[0] && gx == dm->ext[0] - 1;
-        fr.yl = !dm->per[1] && gy == 0;
-        fr.yh = !dm->per[1] && gy == dm->ext[1] - 1;
-        fr.zlo_plane = (!dm->per[2] && oz == 0) ? 0 : -1;
-        fr.zhi_plane = (!dm->per[2] && dm->ext[2] - 1 - oz < BS) ? dm->ext[2] - 1 - oz : -1;
-        fr.dead = gx >= dm->ext[0] || gy >= dm->ext[1];
-        if (fr.dead) {
-            // a cell beyond the extent reads only its own column (its x / y sources may lie in blocks
-            // that do not exist); the z rules keep its reads inside the level as for every lane
-            const int32_t v11 = ra.v[1][1];
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-#pragma unroll
-                for (int j = 0; j < 3; ++j) ra.v[i][j] = v11;
-        }
-        fr.zwall = dm->zwall != 0;
-        fr.ymin_wall = dm->ymin_wall == 1;
-        in.on = fr.xl;
-        in.u_in = dm->u_in;
-        in.gy = gy;
-        in.gz = oz;      // + z per plane
-    }
-    if constexpr (FACE == FACE_RULES) {
-        const FaceBits fb = face_bits(a, b, dm);
-        fr.xl = fb.xlo && c.lx == 0;
-        fr.xh = fb.xhi && c.lx == BS - 1;
-        fr.yl = fb.ylo && c.ly == 0;
-        fr.yh = fb.yhi && c.ly == BS - 1;
-        fr.zlo = fb.zlo;
-        fr.zhi = fb.zhi;
-        fr.zwall = dm->zwall != 0;
-        fr.ymin_wall = dm->ymin_wall == 1;
-        in.on = fr.xl;
-        in.u_in = dm->u_in;
-        in.gy = a.borg[3 * b + 1] + c.ly;
-        in.gz = a.borg[3 * b + 2];      // + z per plane
-    }
-    // WALE: the x / y neighbours' cell offsets of the lane (0: across a domain face, the cell itself),
-    // the block layer, and the domain's rates
-    int32_t wxp = 0, wxm = 0, wyp = 0, wym = 0, wlayer = 0;
-    PipeWaleRates<T> wr{};
-    if constexpr (WALE) {
-        const int32_t row = dm->nbx * BS3 - (BS - 1) * BS;
-        wxp = fr.xh ? 0 : (c.lx < BS - 1 ? 1 : BS3 - (BS - 1));
-        wxm = fr.xl ? 0 : (c.lx > 0 ? -1 : -(BS3 - (BS - 1)));
-        wyp = fr.yh ? 0 : (c.ly < BS - 1 ? BS : row);
-        wym = fr.yl ? 0 : (c.ly > 0 ? -BS : -row);
-        if constexpr (FACE == FACE_PARTIAL) {
-            if (fr.dead) { wxp = 0; wxm = 0; wyp = 0; wym = 0; }
-        }
-        wlayer = dm->nbx * dm->nby * BS3;
-        wr.tau = T(dm->tau);
-        wr.amr_scale = T(dm->amr_scale);
-    }
-    // the six neighbours' velocities of the lane's cell in plane z
-    auto wale_load = [&](int z, PipeWale<T>& w) {
-        const T* v = (const T*)a.vel_in;
-        const uint32_t own = c.own + (uint32_t)(z - z0) * BS2;
-        bool zl = false, zh = false;
-        if constexpr (FACE == FACE_RULES) { zl = fr.zlo && z == 0; zh = fr.zhi && z == BS - 1; }
-        if constexpr (FACE == FACE_PARTIAL) { zl = z == fr.zlo_plane; zh = z == fr.zhi_plane; }
-        const int32_t zp = zh ? 0 : (z < BS - 1 ? BS2 : wlayer - (BS - 1) * BS2);
-        const int32_t zm = zl ? 0 : (z > 0 ? -BS2 : -(wlayer - (BS - 1) * BS2));
-        const int32_t off[6] = {wxp, wxm, wyp, wym, zp, zm};
-#pragma unroll
-        for (int q6 = 0; q6 < 6; ++q6) {
-            const uint32_t i = (uint32_t)((int32_t)own + off[q6]);
-            w.u[q6][0] = v[i]; w.u[q6][1] = v[a.ncell + i]; w.u[q6][2] = v[2 * (size_t)a.ncell + i];
-        }
-    };
-    // FACE_SOLID: the solid-link masks of the lane's cell (bit 27: the cell itself is solid)
-    const uint32_t* lm_cells = nullptr;
-    if constexpr (FACE == FACE_SOLID) lm_cells = a.lmask + (size_t)a.lslot[b] * BS3 + (c.own - b * BS3 - (uint32_t)z0 * BS2);
-    auto lm_load = [&](int z) -> uint32_t {
-        if constexpr (FACE == FACE_SOLID) return z < z0 + np ? lm_cells[(uint32_t)z * BS2] : 0u;
-        else return 0u;
-    };
-    uint32_t lm_cur = 0;   // FACE_SOLID: the mask of the plane the next load() reads
-    auto load = [&](const RegAddr<SP>& r, int z, typename SP::raw (&dst)[27]) {
-        if constexpr (FACE == FACE_RULES) { if (z < zmax) reg_load_raw_face<SP>(a, r, fr, z, dst); }
-        else if constexpr (FACE == FACE_PARTIAL) { if (z < zmax) reg_load_raw_face<SP, true>(a, r, fr, z, dst); }
-        else if constexpr (FACE == FACE_SOLID) {
-            using st = typename SP::st;
-            const uint32_t m = lm_cur;
-            for_dirs([&](auto kc) {
-                constexpr int K = decltype(kc)::value;
-                const char* pr = r.base(a.fin, K, z, dcz(K)) + r.v[dcx(K) + 1][dcy(K) + 1];
-                const char* ps = r.base(a.fin, dopp(K), z, 0) + r.v[1][1];
-                dst[K] = SP::ld_raw((const st*)(((m >> K) & 1u) ? ps : pr));
-            });
-        }
-        else if (live(z)) reg_load_raw<SP>(a, r, z, dst);
-    };
-    const uint32_t cell0 = dm->cell0;   // read before the first store, as every domain parameter
-    auto collide = [&](const RegAddr<SP>& r, int z, const typename SP::raw (&src)[27], const PipeWale<T>& w, T sp,
-                       uint32_t lm) {
-        const uint32_t vidx = c.own + (uint32_t)(z - z0) * BS2;
-        const uint32_t cell = vidx - cell0;
-        if constexpr (FACE == FACE_SOLID) {
-            // a solid cell is not stepped (halfway bounce-back)
-            reg_collide_store<SP, UNIT, WALE, SPONGE>(a, r, q, z, cell, src, nullptr, !((lm >> 27) & 1u), &w, &wr, vidx, sp);
-            return;
-        }
-        if constexpr (FACE == FACE_RULES) {
-            if (z >= zmax) return;
-            InletRule iz = in;
-            iz.gz += z;
-            reg_collide_store<SP, UNIT, WALE, SPONGE>(a, r, q, z, cell, src, &iz, true, &w, &wr, vidx, sp);
-        } else if constexpr (FACE == FACE_PARTIAL) {
-            if (z >= zmax) return;
-            InletRule iz = in;
-            iz.gz += z;
-            reg_collide_store<SP, UNIT, WALE, SPONGE>(a, r, q, z, cell, src, &iz, !fr.dead, &w, &wr, vidx, sp);
-        } else if (live(z)) {
-            reg_collide_store<SP, UNIT, WALE, SPONGE>(a, r, q, z, cell, src, nullptr, true, &w, &wr, vidx, sp);
-        }
-    };
-    // WALE: the plane's neighbour velocities, issued before the next plane's populations
-    auto wale_pre = [&](int z, PipeWale<T>& w) {
-        if constexpr (WALE) {
-            if (z < zmax && live(z)) wale_load(z, w);
-            __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    // the per-lane offsets stay those of plane z0; later planes shift the uniform base
-    typename SP::raw fa[27], fb[27];
-    T spa = T(0), spb = T(0);
-    uint32_t lma = 0, lmb = 0, lmn = 0;   // FACE_SOLID: the masks of the planes in fa / fb, and the next one's
-    PipeWale<T> wv;
-    if constexpr (FACE == FACE_SOLID) {
-        lma = lm_load(z0);
-        wait_all_vmem();
-        lm_cur = lma;
-    }
-    load(ra, z0, fa);
-    if constexpr (SPONGE) spa = sp_load(z0);
-    if constexpr (FACE == FACE_SOLID) lmn = lm_load(z0 + 1);
-    for (int z = z0; z < z0 + np; z += 2) {
-        wait_all_vmem();
-        wale_pre(z, wv);
-        if (z + 1 < z0 + np) {
-            if constexpr (FACE == FACE_SOLID) { lmb = lmn; lm_cur = lmb; }
-            load(ra, z + 1, fb);
-            if constexpr (SPONGE) spb = sp_load(z + 1);
-            if constexpr (FACE == FACE_SOLID) lmn = lm_load(z + 2);
-        }
-        collide(ra, z, fa, wv, spa, lma);
-        if (z + 1 >= z0 + np) break;
-        wait_all_vmem();
-        wale_pre(z + 1, wv);
-        if (z + 2 < z0 + np) {
-            if constexpr (FACE == FACE_SOLID) { lma = lmn; lm_cur = lma; }
-            load(ra, z + 2, fa);
-            if constexpr (SPONGE) spa = sp_load(z + 2);
-            if constexpr (FACE == FACE_SOLID) lmn = lm_load(z + 3);
-        }
-        collide(ra, z + 1, fb, wv, spb, lmb);
-    }
 }
 
 // The in-place AA pattern on the regular blocks (no domain face, no solid near; neighbour blocks at
@@ -1102,9 +698,11 @@ k_step_pipe(const StepArgs a) {
 // slot opp k of x - c_k and writes f*_k to slot k of x + c_k.  Either way a lane reads and writes the
 // same 27 slots and no other lane touches them, so the next plane's prefetch never meets a store of the
 // current plane.  The storage rounding of f*_k takes the bits of (cell, k, step) as in every pattern.
-// (the odd half-step's two-sided addressing needs the 2-wave register budget)
+// Register budget: one plane of populations in flight beside the collision of another; the odd
+// half-step's two-sided addressing and the 16-bit forms' conversions fit the 256 VGPRs of 2 waves per
+// SIMD only, the other forms the 168 of 3
 template <class SP, int PAT>
-constexpr int pipe_aa_waves() { return PAT == PAT_AA_ODD ? OAL_FACE_RULES_WAVES : pipe_waves<SP, FACE_NONE>(); }
+constexpr int pipe_aa_waves() { return PAT == PAT_AA_ODD || SP::dithered ? 2 : 3; }
 
 template <class SP, int NP, int PAT, bool UNIT>
 __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(pipe_aa_waves<SP, PAT>(), pipe_aa_waves<SP, PAT>())))
@@ -1205,80 +803,14 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(step_wa
     step_cell<SP, PAT_AB, WALE, true>(a, c, dm, true, false, F0, F1, F2);
 }
 
-}  // namespace oal
-
-#include "oal_step_pair.h"
-#include "oal_step_pair32.h"
-
-namespace oal {
-
-// (WALE: the face-rule form for every whole block; the forms without rules spill with WALE's gather)
-template <class SP, int NP, bool UNIT, bool WALE>
-static void launch_pipe_u(int face, dim3 grid, hipStream_t s, const StepArgs& r) {
-    if constexpr (WALE) {
-        if (face == FACE_PARTIAL) {
-            if constexpr (NP <= 8) hipLaunchKernelGGL((k_step_pipe<SP, NP, FACE_PARTIAL, UNIT, true>), grid, dim3(WG), 0, s, r);
-        } else {
-            hipLaunchKernelGGL((k_step_pipe<SP, NP, FACE_RULES, UNIT, true>), grid, dim3(WG), 0, s, r);
-        }
-    } else {
-        if (face == FACE_RULES) hipLaunchKernelGGL((k_step_pipe<SP, NP, FACE_RULES, UNIT, false>), grid, dim3(WG), 0, s, r);
-        else if (face == FACE_SKIP) hipLaunchKernelGGL((k_step_pipe<SP, NP, FACE_SKIP, UNIT, false>), grid, dim3(WG), 0, s, r);
-        else if (face == FACE_PARTIAL) {
-            if constexpr (NP <= 8) hipLaunchKernelGGL((k_step_pipe<SP, NP, FACE_PARTIAL, UNIT, false>), grid, dim3(WG), 0, s, r);
-        }
-        else if (face == FACE_SOLID) {
-            if constexpr (NP <= 8) hipLaunchKernelGGL((k_step_pipe<SP, NP, FACE_SOLID, UNIT, false>), grid, dim3(WG), 0, s, r);
-        }
-        else hipLaunchKernelGGL((k_step_pipe<SP, NP, FACE_NONE, UNIT, false>), grid, dim3(WG), 0, s, r);
-    }
-}
-// (the WALE forms come in 2, 4 and 8 planes; the launch caps the planes at 8)
-template <class SP, int NP>
-static void launch_pipe_sponge(dim3 grid, hipStream_t s, const StepArgs& r) {
-    if (r.cp.unit) hipLaunchKernelGGL((k_step_pipe<SP, NP, FACE_PARTIAL, true, false, true>), grid, dim3(WG), 0, s, r);
-    else hipLaunchKernelGGL((k_step_pipe<SP, NP, FACE_PARTIAL, false, false, true>), grid, dim3(WG), 0, s, r);
-}
-
-template <class SP, int NP, bool WALE = false>
-static void launch_pipe(int face, dim3 grid, hipStream_t s, const StepArgs& r) {
-    if constexpr (!WALE || NP <= 8) {
-        if (r.cp.unit) launch_pipe_u<SP, NP, true, WALE>(face, grid, s, r);
-        else launch_pipe_u<SP, NP, false, WALE>(face, grid, s, r);
-    }
-}
-
-// One step of a level: launches over disjoint block lists (regular, other interior, regular boundary,
-// boundary), each compiled for its own register budget, plus, in the AB pattern, the face cells that
-// the regular kernels skip.  The boundary and face launches go to `side` (when given) so that they
-// overlap the bandwidth-bound bulk launch; the caller joins the two streams.
+// the boundary lists on the one-plane kernel
 template <class SP, int PAT, bool WALE>
-static hipError_t launch_pat(const StepArgs& a, hipStream_t stream, hipStream_t side, hipEvent_t bulk0, hipEvent_t bulk1) {
+static void launch_boundary(const StepArgs& a, hipStream_t bs) {
     StepArgs r = a;
-    hipStream_t bs = side ? side : stream;
-    // (a q-map exists only in the AB pattern)
     const bool bfl = PAT == PAT_AB && a.qmap != nullptr;
-    // regular-grid blocks whose only flag is a solid cell near (at the head of the list): the pipelined
-    // kernel's solid-link form where it applies (AB pattern, FP32 arithmetic, halfway bounce-back, no
-    // q-map, WALE or force), the rest on the one-plane kernel
-    uint32_t br_first = 0;
-    if constexpr (PAT == PAT_AB && !WALE && sizeof(typename SP::T) == 4) {
-        if (a.n_boundary_regular_solid && !bfl && !a.fpart && a.cp.bb_mode == 1 && a.pipe_planes > 1) {
-            StepArgs rs = r;
-            rs.blist = a.blist_boundary_regular;
-            rs.pipe_planes = a.pipe_planes > 8 ? 8 : a.pipe_planes;
-            const dim3 g(a.n_boundary_regular_solid * (PLANES / rs.pipe_planes));
-            switch (rs.pipe_planes) {
-                case 2: launch_pipe<SP, 2>(FACE_SOLID, g, bs, rs); break;
-                case 4: launch_pipe<SP, 4>(FACE_SOLID, g, bs, rs); break;
-                default: launch_pipe<SP, 8>(FACE_SOLID, g, bs, rs); break;
-            }
-            br_first = a.n_boundary_regular_solid;
-        }
-    }
-    if (a.n_boundary_regular > br_first) {
-        r.blist = a.blist_boundary_regular + br_first;
-        const dim3 g((a.n_boundary_regular - br_first) * PLANES);
+    if (a.n_boundary_regular) {
+        r.blist = a.blist_boundary_regular;
+        const dim3 g(a.n_boundary_regular * PLANES);
         if constexpr (PAT == PAT_AB) {
             if (bfl && a.face_x) hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_BOUNDARY_REGULAR, true>), g, dim3(WG), 0, bs, r);
             else if (bfl) hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_BOUNDARY_REGULAR, true, false, false>), g, dim3(WG), 0, bs, r);
@@ -1306,119 +838,58 @@ static hipError_t launch_pat(const StepArgs& a, hipStream_t stream, hipStream_t 
             else hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_BOUNDARY, false, false, false>), g, dim3(WG), 0, bs, r);
         }
     }
-    // face cells: the pipelined kernel applies the face rules itself, the one-plane regular kernel
-    // leaves them to the face-cell kernel
-    constexpr bool pipe_capable = PAT == PAT_AB && sizeof(typename SP::T) == 4;
-    if constexpr (PAT == PAT_AB) {
-        // (the pair kernel applies the rules too; with WALE the pipelined kernel always does)
-        const bool piped = pipe_capable && a.pipe_planes > 1;
-        if (a.n_face && (!piped || (a.face_kernel && !WALE)))
-            hipLaunchKernelGGL((k_face<SP, WALE>), dim3((a.n_face + WG - 1) / WG), dim3(WG), 0, bs, a);
+}
+
+// One step of a level: launches over disjoint block lists.
+//   AB pattern, FP32 arithmetic: the two-cells-per-lane kernel for every block but a few kinds, those on
+//     the one-plane boundary kernel.
+//   AB pattern, FP64, and the AA pattern: regular, other interior, regular boundary and boundary blocks,
+//     each on a kernel compiled for its own register budget, and in the AB pattern the face cells that the
+//     regular kernel skips.
+// The boundary and face launches go to `side` (when given) so that they overlap the bulk launch; the
+// caller joins the two streams.
+template <class SP, int PAT, bool WALE>
+static hipError_t launch_pat(const StepArgs& a, hipStream_t stream, hipStream_t side, hipEvent_t bulk0, hipEvent_t bulk1) {
+    hipStream_t bs = side ? side : stream;
+    launch_boundary<SP, PAT, WALE>(a, bs);
+    constexpr bool two = PAT == PAT_AB && sizeof(typename SP::T) == 4;
+    if constexpr (PAT == PAT_AB && !two) {
+        if (a.n_face) hipLaunchKernelGGL((k_face<SP, WALE>), dim3((a.n_face + WG - 1) / WG), dim3(WG), 0, bs, a);
     }
     if (bulk0) {
         const hipError_t e = hipEventRecord(bulk0, stream);
         if (e != hipSuccess) return e;
     }
-    // regular blocks (no force on them): one launch in lexicographic order, so that neighbouring blocks,
-    // which share halo rows, stay close in the sweep; the 16-bit storage forms step them two cells per
-    // lane (the face rules applied in the kernel)
-    auto launch_regular = [&](const int32_t* list, uint32_t n, bool face, bool pair) {
-        r.blist = list;
-        r.regular_face = face ? 1 : 0;
-        if constexpr (pipe_capable) {
-            // (WALE: at most 8 planes per workgroup)
-            r.pipe_planes = WALE && a.pipe_planes > 8 ? 8 : a.pipe_planes;
-            const dim3 g(n * (PLANES / (r.pipe_planes > 1 ? r.pipe_planes : 1)));
-            if constexpr (SP::dithered && !WALE) {
-                if (pair) {
-                    launch_pair<SP>(a.pipe_planes, face, g, stream, r);
-                    return;
-                }
-            } else if constexpr (SP::code == StF32::code && !WALE) {
-                if (pair) {
-                    launch_pair32<SP>(a.pipe_planes, face, g, stream, r);
-                    return;
-                }
-            }
-            const int fc = !face ? FACE_NONE : (a.face_kernel && !WALE ? FACE_SKIP : FACE_RULES);
-            switch (r.pipe_planes) {
-                case 2: launch_pipe<SP, 2, WALE>(fc, g, stream, r); break;
-                case 4: launch_pipe<SP, 4, WALE>(fc, g, stream, r); break;
-                case 8: launch_pipe<SP, 8, WALE>(fc, g, stream, r); break;
-                case 16: launch_pipe<SP, 16, WALE>(fc, g, stream, r); break;
-                default: hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_REGULAR>), g, dim3(WG), 0, stream, r); break;
-            }
-        } else if constexpr (PAT != PAT_AB && !WALE && sizeof(typename SP::T) == 4) {
-            // the AA pattern's regular blocks (none on a domain face): pipelined over z, 2 to 8 planes
-            r.pipe_planes = a.pipe_planes > 8 ? 8 : a.pipe_planes;
-            const dim3 g(n * (PLANES / (r.pipe_planes > 1 ? r.pipe_planes : 1)));
-            switch (r.pipe_planes) {
-                case 2: launch_pipe_aa<SP, 2, PAT>(g, stream, r); break;
-                case 4: launch_pipe_aa<SP, 4, PAT>(g, stream, r); break;
-                case 8: launch_pipe_aa<SP, 8, PAT>(g, stream, r); break;
-                default: hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_REGULAR>), g, dim3(WG), 0, stream, r); break;
-            }
+    if constexpr (two) {
+        if (a.qmap) {   // interpolated bounce-back: its form of the kernel where there are solid links
+            launch_two(SP::code, WALE, TWO_BFL, a.blist_two_links, a.n_two_links, stream, a);
+            launch_two(SP::code, WALE, TWO_PLAIN, a.blist_two_free, a.n_two_free, stream, a);
         } else {
-            hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_REGULAR>), dim3(n * PLANES), dim3(WG), 0, stream, r);
+            launch_two(SP::code, WALE, TWO_PLAIN, a.blist_two, a.n_two, stream, a);
+            launch_two(SP::code, WALE, TWO_SPONGE, a.blist_two_sponge, a.n_two_sponge, stream, a);
         }
-    };
-    const bool pair = pipe_capable && (SP::dithered || SP::code == StF32::code) && !WALE && a.pair_kernel &&
-                      a.pipe_planes > 1 && !(a.regular_face && a.face_kernel);
-    if (pair && a.pair_kernel == 2) {
-        // the blocks on a domain face and the others apart (the latter with the smaller register budget)
-        if (a.n_regular_face) launch_regular(a.blist_regular_face, a.n_regular_face, true, true);
-        if (a.n_regular_plain) launch_regular(a.blist_regular_plain, a.n_regular_plain, false, true);
-    } else if (a.n_regular) {
-        launch_regular(a.blist_regular, a.n_regular, a.regular_face != 0, pair);
-    }
-    if (a.n_partial) {
-        // regular blocks that overhang the extent (listed only where the pipelined kernel applies); at
-        // most 8 planes per workgroup (the 16-plane form of this kernel spills); on the side stream
-        // with the boundary launches, overlapping the bulk launch
-        r.blist = a.blist_partial;
-        if constexpr (pipe_capable) {
-            StepArgs rp = r;
-            rp.pipe_planes = a.pipe_planes > 8 ? 8 : a.pipe_planes;
-            const dim3 g(a.n_partial * (PLANES / (rp.pipe_planes > 1 ? rp.pipe_planes : 1)));
-            switch (rp.pipe_planes) {
-                case 2: launch_pipe<SP, 2, WALE>(FACE_PARTIAL, g, bs, rp); break;
-                case 4: launch_pipe<SP, 4, WALE>(FACE_PARTIAL, g, bs, rp); break;
-                case 8: launch_pipe<SP, 8, WALE>(FACE_PARTIAL, g, bs, rp); break;
-                default: hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_BOUNDARY_REGULAR>), g, dim3(WG), 0, bs, rp); break;
-            }
-        } else {
-            hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_BOUNDARY_REGULAR>), dim3(a.n_partial * PLANES), dim3(WG), 0,
-                               bs, r);
-        }
-    }
-    if (a.n_sponge) {
-        // regular blocks with sponge cells and no solid near (AB pattern): the pipelined kernel's sponge
-        // form (without WALE; at most 8 planes per workgroup), else the one-plane kernel's; on the side
-        // stream with the boundary launches
-        StepArgs rs = r;
-        rs.blist = a.blist_sponge;
-        bool piped = false;
-        if constexpr (pipe_capable && !WALE) {
-            if (a.pipe_planes > 1) {
-                rs.pipe_planes = a.pipe_planes > 8 ? 8 : a.pipe_planes;
-                const dim3 g(a.n_sponge * (PLANES / rs.pipe_planes));
-                switch (rs.pipe_planes) {
-                    case 2: launch_pipe_sponge<SP, 2>(g, bs, rs); break;
-                    case 4: launch_pipe_sponge<SP, 4>(g, bs, rs); break;
-                    default: launch_pipe_sponge<SP, 8>(g, bs, rs); break;
+    } else {
+        StepArgs r = a;
+        if (a.n_regular) {
+            r.blist = a.blist_regular;
+            if constexpr (PAT != PAT_AB && !WALE && sizeof(typename SP::T) == 4) {
+                // the AA pattern's regular blocks (none on a domain face): pipelined over z, 2 to 8 planes
+                r.pipe_planes = a.pipe_planes > 8 ? 8 : a.pipe_planes;
+                const dim3 g(a.n_regular * (PLANES / (r.pipe_planes > 1 ? r.pipe_planes : 1)));
+                switch (r.pipe_planes) {
+                    case 2: launch_pipe_aa<SP, 2, PAT>(g, stream, r); break;
+                    case 4: launch_pipe_aa<SP, 4, PAT>(g, stream, r); break;
+                    case 8: launch_pipe_aa<SP, 8, PAT>(g, stream, r); break;
+                    default: hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_REGULAR>), g, dim3(WG), 0, stream, r); break;
                 }
-                piped = true;
+            } else {
+                hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_REGULAR>), dim3(a.n_regular * PLANES), dim3(WG), 0, stream, r);
             }
         }
-        if (!piped) {
-            const dim3 g(a.n_sponge * PLANES);
-            if (a.face_x) hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_BOUNDARY_REGULAR, false, true>), g, dim3(WG), 0, bs, rs);
-            else hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_BOUNDARY_REGULAR, false, true, false>), g, dim3(WG), 0, bs, rs);
+        if (a.n_interior) {
+            r.blist = a.blist_interior;
+            hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_INTERIOR>), dim3(a.n_interior * PLANES), dim3(WG), 0, stream, r);
         }
-    }
-    if (a.n_interior) {
-        r.blist = a.blist_interior;
-        hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_INTERIOR>), dim3(a.n_interior * PLANES), dim3(WG), 0, stream, r);
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess || !bulk1) return e;
