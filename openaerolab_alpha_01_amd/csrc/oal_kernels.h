@@ -40,11 +40,36 @@ struct DevDomain {
     int32_t pad;
 };
 
+// All a workgroup of the two-cells-per-lane kernel reads about its block, one record per entry of a block
+// list: one round of scalar loads in place of a chain (list entry, block tables, domain).  Neighbour
+// offsets are in bytes of populations from the lowest block among the neighbours and the block (absent:
+// the block's own), so that 32 bits reach every one.
+struct TwoRec {
+    uint32_t off[27];          // by (dx + 1) + 3 (dy + 1) + 9 (dz + 1); [13]: the block itself
+    uint32_t base;             // the lowest block
+    uint32_t block;
+    uint32_t flags;            // BF_* and TR_*
+    int32_t org[3];
+    int32_t lslot, sslot;      // link-mask and sponge slots
+    int32_t ext[3];
+    float u_in, omega1, omega4d, F[3], tau, amr_scale, force_scale;
+    uint32_t cell0;
+    uint32_t face[6];          // neighbour blocks x+, x-, y+, y-, z+, z- (WALE; absent: the block itself)
+    uint32_t pad[10];
+};
+static_assert(sizeof(TwoRec) == 256, "a record is four cache lines of the scalar cache");
+enum : uint32_t {
+    TR_PER_X = 1u << 8, TR_PER_Y = 1u << 9, TR_PER_Z = 1u << 10,   // periodic axes
+    TR_ZWALL = 1u << 11, TR_YMIN = 1u << 12,                       // no-slip z faces, no-slip y-min face
+    TR_FORCED = 1u << 13,
+    TR_ABSENT = 1u << 16       // shifted by 0..5: the face neighbour is absent
+};
+
 // arguments of the fused stream-collide kernels
 struct StepArgs {
     const void* fin;             // populations read this step
     void* fout;                  // populations written (== fin for the AA pattern)
-    const int32_t* nbr_bm;       // [32 * nb] block-major neighbour rows, 0-based, -1 = none; entry 27: the lowest
+    const int32_t* nbr_bm;       // [32 * nb] block-major neighbour rows, 0-based, -1 = none
     const int32_t* borg;         // [3 * nb] block origin in cells
     const int32_t* bdom;         // [nb] domain index
     const uint32_t* bflags;      // [nb]
@@ -63,10 +88,12 @@ struct StepArgs {
     // the two-cells-per-lane kernel's blocks (AB pattern, FP32 arithmetic; blist_boundary_regular and
     // blist_boundary then hold the blocks it does not take): without sponge cells, with sponge cells, and
     // the former split into those with solid links near and the others
-    const int32_t* blist_two;
-    const int32_t* blist_two_sponge;
-    const int32_t* blist_two_links;
-    const int32_t* blist_two_free;
+    const TwoRec* rec;           // the records of this launch (set per launch)
+    const TwoRec* two;
+    const TwoRec* two_sponge;
+    const TwoRec* two_links;
+    const TwoRec* two_free;
+    int32_t two_keep;            // the level's population buffers stay in the memory-side cache between steps
     uint32_t n_two, n_two_sponge, n_two_links, n_two_free;
     const int32_t* lslot;        // [nb] link-mask slot of a block with solid cells near, -1 = none
     const uint32_t* lmask;       // [n_lslots * BS3] per cell: bit k source of direction k solid, bit 27 cell solid
@@ -106,6 +133,10 @@ inline bool two_fits(int64_t lo, int64_t hi, uint64_t esize) {
     return (uint64_t)(hi - lo + 1) * 27ull * BS3 * esize < (1ull << 32);
 }
 
+// Population bytes of a level (both buffers) up to which the two-cells-per-lane kernel's stores are left in
+// the memory-side cache
+constexpr uint64_t TWO_KEEP_BYTES = 192ull << 20;
+
 struct ReduceArgs {
     const double* part;          // [n_items * 4]
     const int32_t* dom_item0;    // [n_domains + 1] first item of each domain
@@ -133,12 +164,12 @@ hipError_t launch_step_f16s(int stream_mode, bool wale, const StepArgs& a, hipSt
                             hipEvent_t bulk0, hipEvent_t bulk1);
 hipError_t launch_step_bf16s(int stream_mode, bool wale, const StepArgs& a, hipStream_t stream, hipStream_t side,
                              hipEvent_t bulk0, hipEvent_t bulk1);
-// the two-cells-per-lane step kernel over a.blist (a.n_items workgroups): oal_two_<storage>.hip
+// the two-cells-per-lane step kernel over a.rec (a.n_items workgroups): oal_two_<storage>.hip
 void launch_two_f32(bool wale, int extra, const StepArgs& a, hipStream_t stream);
 void launch_two_f16s(bool wale, int extra, const StepArgs& a, hipStream_t stream);
 void launch_two_bf16s(bool wale, int extra, const StepArgs& a, hipStream_t stream);
 // and over the n blocks of a list, by storage code
-void launch_two(int storage, bool wale, int extra, const int32_t* list, uint32_t n, hipStream_t stream, const StepArgs& a);
+void launch_two(int storage, bool wale, int extra, const TwoRec* rec, uint32_t n, hipStream_t stream, const StepArgs& a);
 hipError_t launch_copy16(const void* src, void* dst, size_t bytes, hipStream_t stream);
 // Host arrays of init / conversion / macro output cover the first nhost cells of a level (the caller's
 // blocks); the device arrays have ncell cells per direction.

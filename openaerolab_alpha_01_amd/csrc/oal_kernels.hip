@@ -18,10 +18,10 @@ hipError_t launch_step(int storage, int stream_mode, bool wale, const StepArgs& 
     }
 }
 
-void launch_two(int storage, bool wale, int extra, const int32_t* list, uint32_t n, hipStream_t stream, const StepArgs& a) {
+void launch_two(int storage, bool wale, int extra, const TwoRec* rec, uint32_t n, hipStream_t stream, const StepArgs& a) {
     if (!n) return;
     StepArgs r = a;
-    r.blist = list;
+    r.rec = rec;
     r.n_items = n * PLANES;
     switch (storage) {
         case 0: launch_two_f32(wale, extra, r, stream); break;

@@ -106,9 +106,12 @@ struct Level {
     // the two-cells-per-lane kernel's blocks (AB pattern, FP32 arithmetic): without and with sponge cells,
     // the former also split by solid links near (interpolated bounce-back); the boundary blocks it does not
     // take, with and without lexicographic neighbours
-    DevBuf<int32_t> blist_tw, blist_ts, blist_tl, blist_tn, blist_xr, blist_xb;
+    DevBuf<TwoRec> rec_tw, rec_ts, rec_tl, rec_tn;
+    DevBuf<int32_t> blist_xr, blist_xb;
     uint32_t n_two = 0, n_two_sponge = 0, n_two_links = 0, n_two_free = 0, n_rest_regular = 0, n_rest = 0;
     std::vector<char> two_fit_h;       // a block's neighbours lie within that kernel's 32-bit offsets
+    std::vector<int32_t> nbr_h;        // [32 * nb] neighbour rows (the device's nbr)
+    uint32_t esize = 4;                // bytes of a stored population
     bool two() const { return ab && fp32; }
     DevBuf<int32_t> lslot;             // link-mask slot per block
     DevBuf<uint32_t> lmask;            // per-cell solid-link masks of blocks near solid cells
@@ -184,7 +187,7 @@ struct Level {
     void release() {
         nbr.release(); borg.release(); bdom.release(); dom_item0.release(); dom_block0.release();
         bflags.release(); solid.release(); doms.release(); fA.release(); fB.release(); velA.release(); velB.release();
-        blist_tw.release(); blist_ts.release(); blist_tl.release(); blist_tn.release(); blist_xr.release(); blist_xb.release();
+        rec_tw.release(); rec_ts.release(); rec_tl.release(); rec_tn.release(); blist_xr.release(); blist_xb.release();
         fpart.release(); mpart.release(); red_out.release(); guard.release(); oslot.release(); obuf.release(); blist_rg.release(); blist_in.release(); blist_br.release(); blist_bd.release(); face_cells.release();
         lslot.release(); lmask.release(); qmap.release(); sponge.release(); sslot.release();
         g_src.release(); g_dst.release(); g_slot.release(); g_w.release(); g_m.release();
@@ -247,6 +250,7 @@ int upload(DevBuf<T>& d, const std::vector<T>& h) {
 struct HostLevel {
     std::vector<int32_t> borg, bdom, nbr, nbr_bm, oslot, blist_rg, blist_in, blist_br, blist_bd,
         blist_tw, blist_ts, blist_tl, blist_tn, blist_xr, blist_xb, lslot;
+    std::vector<TwoRec> rec_tw, rec_ts, rec_tl, rec_tn;
     std::vector<uint32_t> lmask;
     std::vector<uint32_t> face_cells;
     int32_t n_oslots = 0;
@@ -333,6 +337,51 @@ void build_lists(Level& L, HostLevel& H) {
     L.n_two_free = (uint32_t)H.blist_tn.size();
     L.n_rest_regular = (uint32_t)H.blist_xr.size();
     L.n_rest = (uint32_t)H.blist_xb.size();
+}
+
+// The records of the two-cells-per-lane kernel's block lists; slot: the sponge slots (empty: none)
+void build_two_recs(const Level& L, HostLevel& H, const std::vector<int32_t>& sslot) {
+    auto make = [&](const std::vector<int32_t>& list, std::vector<TwoRec>& out) {
+        out.assign(list.size(), TwoRec{});
+        for (size_t i = 0; i < list.size(); ++i) {
+            const uint32_t b = (uint32_t)list[i];
+            const int32_t* nt = L.nbr_h.data() + (size_t)b * 32;
+            const DevDomain& dm = L.doms_h[L.bdom_h[b]];
+            TwoRec& r = out[i];
+            uint32_t lo = b;
+            for (int k = 0; k < 27; ++k)
+                if (nt[k] >= 0) lo = std::min(lo, (uint32_t)nt[k]);
+            for (int k = 0; k < 27; ++k) r.off[k] = ((nt[k] < 0 ? b : (uint32_t)nt[k]) - lo) * (27u * BS3 * L.esize);
+            r.base = lo;
+            r.block = b;
+            r.flags = L.flags_h[b] | (dm.per[0] ? TR_PER_X : 0u) | (dm.per[1] ? TR_PER_Y : 0u) | (dm.per[2] ? TR_PER_Z : 0u) |
+                      (dm.zwall != 0 ? TR_ZWALL : 0u) | (dm.ymin_wall == 1 ? TR_YMIN : 0u) | (dm.forced ? TR_FORCED : 0u);
+            for (int a = 0; a < 3; ++a) {
+                r.org[a] = L.borg_h[3 * b + a];
+                r.ext[a] = dm.ext[a];
+                r.F[a] = dm.F[a];
+            }
+            r.lslot = L.lslot_h[b];
+            r.sslot = sslot.empty() ? -1 : sslot[b];
+            r.u_in = dm.u_in;
+            r.omega1 = dm.omega1;
+            r.omega4d = dm.omega4d;
+            r.tau = dm.tau;
+            r.amr_scale = dm.amr_scale;
+            r.force_scale = dm.force_scale;
+            r.cell0 = dm.cell0;
+            const int fk[6] = {14, 12, 16, 10, 22, 4};
+            for (int f = 0; f < 6; ++f) {
+                r.face[f] = nt[fk[f]] < 0 ? b : (uint32_t)nt[fk[f]];
+                if (nt[fk[f]] < 0) r.flags |= TR_ABSENT << f;
+            }
+        }
+    };
+    if (!L.two()) return;
+    make(H.blist_tw, H.rec_tw);
+    make(H.blist_ts, H.rec_ts);
+    make(H.blist_tl, H.rec_tl);
+    make(H.blist_tn, H.rec_tn);
 }
 
 // Host-side construction of one level's tables from the reference-convention descriptor.
@@ -496,9 +545,10 @@ int prepare_level(const OalLevelDesc& d, const OalCollision& coll, bool ab, bool
     }
     // block-major copy of the neighbour table: one 32-entry row per block (scalar loads)
     H.nbr_bm.assign((size_t)nb * 32, -1);
-    // (entry 27: the lowest index among them, the base of the two-cells-per-lane kernel's 32-bit byte
-    // offsets, which must reach the highest)
+    // (and whether the two-cells-per-lane kernel's 32-bit byte offsets, from the lowest index among them,
+    // reach the highest)
     L.two_fit_h.assign(nb, 0);
+    L.esize = (uint32_t)sbytes;
     for (uint32_t b = 0; b < nb; ++b) {
         int32_t lo = (int32_t)b, hi = (int32_t)b;
         for (int k = 0; k < 27; ++k) {
@@ -509,9 +559,9 @@ int prepare_level(const OalLevelDesc& d, const OalCollision& coll, bool ab, bool
                 hi = std::max(hi, n);
             }
         }
-        H.nbr_bm[(size_t)b * 32 + 27] = lo;
         L.two_fit_h[b] = two_fits(lo, hi, (uint64_t)sbytes) ? 1 : 0;
     }
+    if (ab && fp32) L.nbr_h = H.nbr_bm;
     L.near_h = near;
     L.flags_h = flags;
     L.borg_h = borg;
@@ -582,6 +632,7 @@ int prepare_level(const OalLevelDesc& d, const OalCollision& coll, bool ab, bool
                     m[(z * BS + y) * BS + x] = bits;
                 }
     }
+    build_two_recs(L, H, {});
     return OAL_OK;
 }
 
@@ -995,8 +1046,8 @@ int upload_level(OalPlan* p, Level& L, const HostLevel& H) {
     if (!H.solid.empty() && (rc = upload(L.solid, H.solid))) return rc;
     if ((rc = upload(L.blist_rg, H.blist_rg)) || (rc = upload(L.blist_in, H.blist_in)) ||
         (rc = upload(L.blist_br, H.blist_br)) || (rc = upload(L.blist_bd, H.blist_bd)) ||
-        (rc = upload(L.blist_tw, H.blist_tw)) || (rc = upload(L.blist_ts, H.blist_ts)) || (rc = upload(L.blist_tl, H.blist_tl)) ||
-        (rc = upload(L.blist_tn, H.blist_tn)) || (rc = upload(L.blist_xr, H.blist_xr)) || (rc = upload(L.blist_xb, H.blist_xb)) ||
+        (rc = upload(L.rec_tw, H.rec_tw)) || (rc = upload(L.rec_ts, H.rec_ts)) || (rc = upload(L.rec_tl, H.rec_tl)) ||
+        (rc = upload(L.rec_tn, H.rec_tn)) || (rc = upload(L.blist_xr, H.blist_xr)) || (rc = upload(L.blist_xb, H.blist_xb)) ||
         (rc = upload(L.lslot, H.lslot)) || (rc = upload(L.lmask, H.lmask)) || (rc = upload(L.face_cells, H.face_cells)))
         return rc;
     if (p->stream_mode == OAL_STREAM_AA) {
@@ -1071,13 +1122,14 @@ StepArgs make_args(OalPlan* p, Level& L, int32_t time_step, bool want_force) {
     }
     a.parity = p->stream_mode == OAL_STREAM_AA ? (L.aa_phase == 0 ? 1 : 0) : 0;
     a.pipe_planes = p->pipe_planes;
-    a.blist_two = L.blist_tw.p;
+    a.two = L.rec_tw.p;
     a.n_two = L.n_two;
-    a.blist_two_sponge = L.blist_ts.p;
+    a.two_keep = 2ull * L.fA.n <= TWO_KEEP_BYTES ? 1 : 0;
+    a.two_sponge = L.rec_ts.p;
     a.n_two_sponge = L.n_two_sponge;
-    a.blist_two_links = L.blist_tl.p;
+    a.two_links = L.rec_tl.p;
     a.n_two_links = L.n_two_links;
-    a.blist_two_free = L.blist_tn.p;
+    a.two_free = L.rec_tn.p;
     a.n_two_free = L.n_two_free;
     if (L.two()) {   // the boundary kernels keep the blocks it does not take
         a.blist_boundary_regular = L.blist_xr.p;
@@ -2099,13 +2151,14 @@ static int set_sponge_lib(OalPlan* p, int level, const float* sponge, int32_t bl
     drop_graphs(p);
     HostLevel H;
     build_lists(L, H);
+    build_two_recs(L, H, slot);
     auto re = [](auto& d, const auto& h) { d.release(); return upload(d, h); };
     int rc;
     if ((rc = re(L.bflags, L.flags_h)) || (rc = re(L.blist_rg, H.blist_rg)) || (rc = re(L.blist_in, H.blist_in)) ||
         (rc = re(L.blist_br, H.blist_br)) || (rc = re(L.blist_bd, H.blist_bd)) ||
        
-        (rc = re(L.blist_tw, H.blist_tw)) || (rc = re(L.blist_ts, H.blist_ts)) || (rc = re(L.blist_tl, H.blist_tl)) ||
-        (rc = re(L.blist_tn, H.blist_tn)) || (rc = re(L.blist_xr, H.blist_xr)) || (rc = re(L.blist_xb, H.blist_xb)) || (rc = re(L.face_cells, H.face_cells)) ||
+        (rc = re(L.rec_tw, H.rec_tw)) || (rc = re(L.rec_ts, H.rec_ts)) || (rc = re(L.rec_tl, H.rec_tl)) ||
+        (rc = re(L.rec_tn, H.rec_tn)) || (rc = re(L.blist_xr, H.blist_xr)) || (rc = re(L.blist_xb, H.blist_xb)) || (rc = re(L.face_cells, H.face_cells)) ||
         (rc = re(L.sponge, vals)) || (rc = re(L.sslot, slot)))
         return rc;
     L.has_sponge = !vals.empty();

@@ -862,11 +862,11 @@ static hipError_t launch_pat(const StepArgs& a, hipStream_t stream, hipStream_t 
     }
     if constexpr (two) {
         if (a.qmap) {   // interpolated bounce-back: its form of the kernel where there are solid links
-            launch_two(SP::code, WALE, TWO_BFL, a.blist_two_links, a.n_two_links, stream, a);
-            launch_two(SP::code, WALE, TWO_PLAIN, a.blist_two_free, a.n_two_free, stream, a);
+            launch_two(SP::code, WALE, TWO_BFL, a.two_links, a.n_two_links, stream, a);
+            launch_two(SP::code, WALE, TWO_PLAIN, a.two_free, a.n_two_free, stream, a);
         } else {
-            launch_two(SP::code, WALE, TWO_PLAIN, a.blist_two, a.n_two, stream, a);
-            launch_two(SP::code, WALE, TWO_SPONGE, a.blist_two_sponge, a.n_two_sponge, stream, a);
+            launch_two(SP::code, WALE, TWO_PLAIN, a.two, a.n_two, stream, a);
+            launch_two(SP::code, WALE, TWO_SPONGE, a.two_sponge, a.n_two_sponge, stream, a);
         }
     } else {
         StepArgs r = a;

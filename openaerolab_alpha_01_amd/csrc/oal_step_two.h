@@ -20,14 +20,18 @@
 // after decoding.
 //
 // Bound and shape.  The plane's 27 words are all in flight together and nothing is kept for a next plane,
-// so a lane needs 97 to 126 registers and four waves share a SIMD; their loads overlap other waves'
+// so a lane needs 97 to 125 registers and four waves share a SIMD; their loads overlap other waves'
 // collisions.  That needs the rare limiter out of the registers (collide_cell's LDS form): with it inline
-// the kernel takes 168 and spills.  Bound: HBM in FP32, VALU issue in the 16-bit forms.  Measured against
-// walking four planes of a block per workgroup with the next plane's words in flight (two waves per SIMD,
-// a launch per kind of block, the default shape before): 256^3 sphere box FP32 667 -> 644 us per step, FP16
-// 467 -> 453 us; WALE 192 x 160 x 160 FP32 295 -> 243 us, WALE 200 x 120 x 104 FP16 200 -> 114 us; WALE
-// 100 x 60 x 44 75 -> 26 us (that shape left 48 workgroups per launch); 12 ragged boxes with solids and
-// sponges FP16 813 -> 542 us.  Blocks run fastest: x-neighbour blocks share the lines of the row ends.
+// the kernel takes 168 and spills.  Bound: HBM in FP32 (256^3: 5.9 TB/s of 6.0 that a copy reaches counting
+// 216 bytes per cell), VALU issue in the 16-bit forms (about 760 instructions per cell, 97 % of the issue
+// slots).  Measured against walking four planes of a block per workgroup with the next plane's words in
+// flight (two waves per SIMD, a launch per kind of block, the default shape before): 256^3 sphere box FP32
+// 667 -> 633 us per step, FP16 467 -> 370 us; WALE 192 x 160 x 160 FP32 295 -> 232 us, WALE 200 x 120 x 104
+// FP16 200 -> 93 us; WALE 100 x 60 x 44 75 -> 20 us (that shape left 48 workgroups per launch); 12 ragged
+// boxes with solids and sponges FP16 813 -> 460 us.  Blocks run fastest: x-neighbour blocks share the lines
+// of the row ends.  One record per block (TwoRec) in place of a chain of table reads: FP16 256^3 453 -> 372
+// us, 48 x 32 x 32 13.5 -> 10.8 us.  Stores written through at device scope: 48 x 32 x 32 10.8 -> 10.2 us,
+// WALE 100 x 60 x 44 25.3 -> 20.9 us without the non-temporal hint (which 256^3 needs: 635 against 681 us).
 #pragma once
 
 #include "oal_step.h"
@@ -61,14 +65,18 @@ struct Two {   // 16-bit forms: A in the low half
     __device__ static __forceinline__ uint32_t b(word w) { return w >> 16; }
     __device__ static __forceinline__ word set_a(word w, uint32_t c) { return (w & 0xffff0000u) | c; }
     __device__ static __forceinline__ word set_b(word w, uint32_t c) { return (w & 0xffffu) | (c << 16); }
+    // the x-neighbour block's cell of the lane at j = 0 (its last pair, the cell in the high half), at j = 7
+    // (its first pair, the cell in the low half)
+    static constexpr uint32_t end_first = (BS - 2) * es, end_last = 0;
+    __device__ static __forceinline__ uint32_t lde(__amdgpu_buffer_rsrc_t r, uint32_t v) { return ld2(r, v, 0); }
     // (left lane's B, own A); end: the x-neighbour block's cell of the lane at j = 0
     __device__ static __forceinline__ word from_left(word w, bool first, uint32_t end) {
-        const uint32_t l = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x111, 0xf, 0xf, false);
-        return __builtin_amdgcn_alignbyte(w, first ? end << 16 : l, 2);
+        const uint32_t l = (uint32_t)__builtin_amdgcn_mov_dpp((int)w, 0x111, 0xf, 0xf, true);
+        return __builtin_amdgcn_alignbyte(w, first ? end : l, 2);
     }
     // (own B, right lane's A)
     __device__ static __forceinline__ word from_right(word w, bool last, uint32_t end) {
-        const uint32_t r = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w, 0x101, 0xf, 0xf, false);
+        const uint32_t r = (uint32_t)__builtin_amdgcn_mov_dpp((int)w, 0x101, 0xf, 0xf, true);
         return __builtin_amdgcn_alignbyte(last ? end : r, w, 2);
     }
     __device__ static __forceinline__ float dec_a(word w, float wk) { return SP::dec_lo(w, wk); }
@@ -96,12 +104,14 @@ struct Two<StF32> {
     __device__ static __forceinline__ uint32_t b(word w) { return w.y; }
     __device__ static __forceinline__ word set_a(word w, uint32_t c) { w.x = c; return w; }
     __device__ static __forceinline__ word set_b(word w, uint32_t c) { w.y = c; return w; }
+    static constexpr uint32_t end_first = (BS - 1) * es, end_last = 0;
+    __device__ static __forceinline__ uint32_t lde(__amdgpu_buffer_rsrc_t r, uint32_t v) { return ld1(r, v); }
     __device__ static __forceinline__ word from_left(word w, bool first, uint32_t end) {
-        const uint32_t l = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w.y, 0x111, 0xf, 0xf, false);
+        const uint32_t l = (uint32_t)__builtin_amdgcn_mov_dpp((int)w.y, 0x111, 0xf, 0xf, true);
         return word{first ? end : l, w.x};
     }
     __device__ static __forceinline__ word from_right(word w, bool last, uint32_t end) {
-        const uint32_t r = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w.x, 0x101, 0xf, 0xf, false);
+        const uint32_t r = (uint32_t)__builtin_amdgcn_mov_dpp((int)w.x, 0x101, 0xf, 0xf, true);
         return word{w.y, last ? end : r};
     }
     __device__ static __forceinline__ float dec_a(word w, float) { return __uint_as_float(w.x); }
@@ -118,6 +128,8 @@ struct TwoFaces {
     bool zl, zh;            // uniform: the plane lies on the z-min / z-max face
     bool zwall, ymin_wall;  // no-slip variants of the z faces and of the y-min face
 };
+// a lane's cells: on the inlet (A), on the outlet, stepped (inside the extent and not solid)
+enum : uint32_t { LF_INLET = 1, LF_OUTLET_A = 2, LF_OUTLET_B = 4, LF_LIVE_A = 8, LF_LIVE_B = 16 };
 // is the source of direction K beyond a y or z face, and which own population does the rule take
 // (precedence: no-slip z wall, no-slip y-min wall, y mirror, z mirror)?
 template <int K>
@@ -147,12 +159,14 @@ __device__ __forceinline__ void two_sum3(double v0, double v1, double v2, double
     }
 }
 
-#ifndef OAL_TWO_STORE_AUX
-#define OAL_TWO_STORE_AUX 2   // the non-temporal hint
-#endif
+// Cache policy of the stores (gfx950's sc and nt bits): written through at device scope, so that the
+// kernel's end has no dirty lines to write back; non-temporal too where the level's two population buffers
+// exceed TWO_KEEP_BYTES (below that the next step reads them from the 256 MB memory-side cache).
+enum : int { TWO_ST_KEEP = 16, TWO_ST_STREAM = 18 };
 
-template <class SP, bool UNIT, bool WALE, int EXTRA>
-__global__ void __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(4)))
+// DITH: stochastic rounding (the 16-bit forms)
+template <class SP, bool UNIT, bool WALE, int EXTRA, bool DITH>
+__global__ void __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(EXTRA == TWO_BFL || (EXTRA == TWO_SPONGE && !(UNIT && !WALE)) ? 3 : 4)))
 k_step_two(const StepArgs a) {
     using W = Two<SP>;
     using word = typename W::word;
@@ -162,52 +176,57 @@ k_step_two(const StepArgs a) {
     const uint32_t litem = xcd_item(blockIdx.x, gridDim.x);
     const uint32_t nblk = gridDim.x / PLANES;
     const uint32_t zi = litem / nblk;
-    const uint32_t b = (uint32_t)a.blist[litem - zi * nblk];
+    // (constant address space: read by scalar loads wherever a field is used)
+    const auto& R = ((const __attribute__((address_space(4))) TwoRec*)a.rec)[litem - zi * nblk];
+    const uint32_t b = R.block;
     const int z = (int)zi;
-    const uint32_t flags = a.bflags[b];
-    const DevDomain* dm = a.doms + a.bdom[b];
-    const int ox = a.borg[3 * b], oy = a.borg[3 * b + 1], gz = a.borg[3 * b + 2] + z;
-    if (gz >= dm->ext[2]) return;                // a plane beyond the extent
+    const uint32_t flags = R.flags;
+    const int ox = R.org[0], oy = R.org[1], gz = R.org[2] + z;
+    if (gz >= R.ext[2]) return;                  // a plane beyond the extent
     const int jx = (int)(threadIdx.x & 7u), ly = (int)(threadIdx.x >> 3);
-    const int32_t* nt = a.nbr_bm + (size_t)b * 32;
-    const uint32_t nb0 = (uint32_t)nt[27];       // lowest block index among the neighbours and the block
-    // byte offset of a neighbour block (an absent one, never a source: the block itself)
-    auto boff = [&](int dx, int dy, int dz) -> uint32_t {
-        const int32_t n = nt[(dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)];
-        return ((n < 0 ? b : (uint32_t)n) - nb0) * blk;
-    };
-    const __amdgpu_buffer_rsrc_t fin = buf_at((const char*)a.fin + (size_t)nb0 * blk);
+    auto boff = [&](int dx, int dy, int dz) -> uint32_t { return R.off[(dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)]; };
+    const __amdgpu_buffer_rsrc_t fin = buf_at((const char*)a.fin + (size_t)R.base * blk);
     const uint32_t row = (uint32_t)ly * (BS * es) + (uint32_t)jx * (2 * es);
     const uint32_t zown = (uint32_t)z * (BS2 * es);
-    const uint32_t own0 = (b - nb0) * blk;       // uniform
+    const uint32_t own0 = R.off[13];             // uniform
     const bool first = jx == 0, last = jx == 7;
 
     const bool edge = (flags & BF_EDGE) != 0;
     TwoFaces fc{};
-    bool xl = false, xha = false, xhb = false, lva = true, lvb = true;
+    // what the lane's cells are, in a vector register: as booleans each would hold a scalar register pair
+    // through the kernel, and the scalar registers spill
+    uint32_t lf = LF_LIVE_A | LF_LIVE_B;
     if (edge) {
         const int gy = oy + ly, ga = ox + 2 * jx;
-        fc.yl = !dm->per[1] && gy == 0;
-        fc.yh = !dm->per[1] && gy == dm->ext[1] - 1;
-        fc.zl = !dm->per[2] && gz == 0;
-        fc.zh = !dm->per[2] && gz == dm->ext[2] - 1;
-        fc.zwall = dm->zwall != 0;
-        fc.ymin_wall = dm->ymin_wall == 1;
-        xl = !dm->per[0] && ga == 0;
-        xha = !dm->per[0] && ga == dm->ext[0] - 1;
-        xhb = !dm->per[0] && ga + 1 == dm->ext[0] - 1;
-        lva = gy < dm->ext[1] && ga < dm->ext[0];
-        lvb = gy < dm->ext[1] && ga + 1 < dm->ext[0];
+        const bool px = (flags & TR_PER_X) != 0, py = (flags & TR_PER_Y) != 0, pz = (flags & TR_PER_Z) != 0;
+        fc.yl = !py && gy == 0;
+        fc.yh = !py && gy == R.ext[1] - 1;
+        fc.zl = !pz && gz == 0;
+        fc.zh = !pz && gz == R.ext[2] - 1;
+        fc.zwall = (flags & TR_ZWALL) != 0;
+        fc.ymin_wall = (flags & TR_YMIN) != 0;
+        lf = !px && ga == 0 ? LF_INLET : 0u;
+        lf |= !px && ga == R.ext[0] - 1 ? LF_OUTLET_A : 0u;
+        lf |= !px && ga + 1 == R.ext[0] - 1 ? LF_OUTLET_B : 0u;
+        lf |= gy < R.ext[1] && ga < R.ext[0] ? LF_LIVE_A : 0u;
+        lf |= gy < R.ext[1] && ga + 1 < R.ext[0] ? LF_LIVE_B : 0u;
     }
+    asm("" : "+v"(lf));
+    auto is = [&](uint32_t f) { return (lf & f) != 0; };
     // solid links of the two cells (bit k: the source of direction k is solid; bit 27: the cell is)
     uint32_t lma = 0, lmb = 0;
     if (flags & BF_SOLID) {
-        const u32x2 m = *(const u32x2*)(a.lmask + (size_t)a.lslot[b] * BS3 + (uint32_t)z * BS2 + (uint32_t)ly * BS + 2u * (uint32_t)jx);
+        const u32x2 m = *(const u32x2*)(a.lmask + (size_t)R.lslot * BS3 + (uint32_t)z * BS2 + (uint32_t)ly * BS + 2u * (uint32_t)jx);
         lma = m.x;
         lmb = m.y;
-        lva = lva && !((lma >> 27) & 1u);
-        lvb = lvb && !((lmb >> 27) & 1u);
+        if ((lma >> 27) & 1u) lf &= ~LF_LIVE_A;
+        if ((lmb >> 27) & 1u) lf &= ~LF_LIVE_B;
     }
+
+    // a wave with nothing to step (rows beyond the extent, the inside of a solid) ends here, unless the
+    // workgroup sums the force
+    const bool want_force = a.fpart != nullptr && (flags & BF_SOLID);
+    if (!want_force && __builtin_amdgcn_ballot_w64(is(LF_LIVE_A | LF_LIVE_B)) == 0) return;
 
     // WALE: the previous step's velocity of the pair and of its neighbour pairs, requested first
     u32x2 vo[3], vyp[3], vym[3], vzp[3], vzm[3];
@@ -216,15 +235,15 @@ k_step_two(const StepArgs a) {
     if constexpr (WALE) {
         const __amdgpu_buffer_rsrc_t vr = buf_at(a.vel_in);
         const uint32_t comp = a.ncell * 4u;
-        auto cell0 = [&](int32_t n) { return (uint32_t)n * (BS3 * 4u); };
+        auto at = [&](uint32_t n) { return n * (BS3 * 4u); };
         const uint32_t loc = (uint32_t)(ly * BS + 2 * jx) * 4u, zc = (uint32_t)z * (BS2 * 4u);
-        const uint32_t own = cell0((int32_t)b) + zc + loc;
-        const int32_t nyp = nt[13 + 3], nym = nt[13 - 3], nzp = nt[13 + 9], nzm = nt[13 - 9];
+        const uint32_t own = at(b) + zc + loc;
+        auto absent = [&](int f) { return ((flags >> f) & TR_ABSENT) != 0; };   // (uniform)
         const bool cp = ly == BS - 1, cm = ly == 0;
-        uint32_t oyp = cp ? (nyp < 0 ? own : cell0(nyp) + zc + loc - (BS - 1) * BS * 4u) : own + BS * 4u;
-        uint32_t oym = cm ? (nym < 0 ? own : cell0(nym) + zc + loc + (BS - 1) * BS * 4u) : own - BS * 4u;
-        uint32_t ozp = z == BS - 1 ? (nzp < 0 ? own : cell0(nzp) + loc) : own + BS2 * 4u;
-        uint32_t ozm = z == 0 ? (nzm < 0 ? own : cell0(nzm) + (BS - 1) * BS2 * 4u + loc) : own - BS2 * 4u;
+        uint32_t oyp = cp ? (absent(2) ? own : at(R.face[2]) + zc + loc - (BS - 1) * BS * 4u) : own + BS * 4u;
+        uint32_t oym = cm ? (absent(3) ? own : at(R.face[3]) + zc + loc + (BS - 1) * BS * 4u) : own - BS * 4u;
+        uint32_t ozp = z == BS - 1 ? (absent(4) ? own : at(R.face[4]) + loc) : own + BS2 * 4u;
+        uint32_t ozm = z == 0 ? (absent(5) ? own : at(R.face[5]) + (BS - 1) * BS2 * 4u + loc) : own - BS2 * 4u;
         if (edge) {
             oyp = fc.yh ? own : oyp;
             oym = fc.yl ? own : oym;
@@ -242,10 +261,9 @@ k_step_two(const StepArgs a) {
             vend[q] = 0;
         }
         if (first || last) {
-            const int32_t nx = first ? nt[12] : nt[14];
-            no_end = nx < 0;
+            no_end = first ? absent(1) : absent(0);
             // (-x block's cell 15 of the row, +x block's cell 0)
-            const uint32_t oe = no_end ? own : cell0(nx) + zc + (uint32_t)(ly * BS + (first ? BS - 1 : 0)) * 4u;
+            const uint32_t oe = no_end ? own : at(first ? R.face[1] : R.face[0]) + zc + (uint32_t)(ly * BS + (first ? BS - 1 : 0)) * 4u;
 #pragma unroll
             for (int q = 0; q < 3; ++q) vend[q] = __builtin_amdgcn_raw_buffer_load_b32(vr, (int)oe, (int)(q * comp), 0);
         }
@@ -253,7 +271,7 @@ k_step_two(const StepArgs a) {
     float spa = 0.0f, spb = 0.0f;
     if constexpr (EXTRA == TWO_SPONGE) {
         if (flags & BF_SPONGE) {
-            const float* sp = a.sponge + (size_t)a.sslot[b] * BS3 + (uint32_t)z * BS2 + (uint32_t)ly * BS + 2u * (uint32_t)jx;
+            const float* sp = a.sponge + (size_t)R.sslot * BS3 + (uint32_t)z * BS2 + (uint32_t)ly * BS + 2u * (uint32_t)jx;
             spa = sp[0];
             spb = sp[1];
         }
@@ -282,7 +300,7 @@ k_step_two(const StepArgs a) {
             v[k][i] = c + r + (uint32_t)jx * (2 * es);
             // row ends: direction (+1, cy, cz) from the -x block's cell 15 at j = 0, (-1, cy, cz) from the
             // +x block's cell 0 at j = 7 (slots 2 apart)
-            ve[k][i] = (first ? m + (BS - 1) * es + 2 * slot : p) + r;
+            ve[k][i] = (first ? m + W::end_first + 2 * slot : p + W::end_last) + r;
         }
     }
     word s[27];
@@ -312,40 +330,40 @@ k_step_two(const StepArgs a) {
         for_dirs([&](auto kc) {
             constexpr int K = decltype(kc)::value;
             constexpr int cy = dcy(K), cz = dcz(K);
-            if constexpr (dcx(K) < 0) e9[K / 3] = W::ld1(fin, ve[cz + 1][cy + 1] + (uint32_t)K * slot + zs[cz + 1]);
+            if constexpr (dcx(K) < 0) e9[K / 3] = W::lde(fin, ve[cz + 1][cy + 1] + (uint32_t)K * slot + zs[cz + 1]);
         });
     }
 
     // WALE: the eddy viscosity of both cells, while the populations are in flight
     CellRates<float> qa;
-    qa.forced = dm->forced != 0;
-    qa.Fx = dm->F[0]; qa.Fy = dm->F[1]; qa.Fz = dm->F[2];
-    qa.omega1 = dm->omega1;
-    qa.omega4_diag = dm->omega4d;
+    qa.forced = (flags & TR_FORCED) != 0;
+    qa.Fx = R.F[0]; qa.Fy = R.F[1]; qa.Fz = R.F[2];
+    qa.omega1 = R.omega1;
+    qa.omega4_diag = R.omega4d;
     if constexpr (EXTRA == TWO_SPONGE) {
-        qa.sponge_u = dm->u_in;
+        qa.sponge_u = R.u_in;
         qa.sponge_blend = a.sponge_blend;
     }
     float om1b = qa.omega1, om4b = qa.omega4_diag;
-    const uint32_t cell0 = dm->cell0;
-    const float u_in = dm->u_in, force_scale = dm->force_scale;
+    const uint32_t cell0 = R.cell0;
+    const float u_in = R.u_in, force_scale = R.force_scale;
     if constexpr (WALE) {
-        const float tau = dm->tau, amr = dm->amr_scale;
+        const float tau = R.tau, amr = R.amr_scale;
         auto f32 = [](uint32_t u) { return __uint_as_float(u); };
         float ga[3][3], gb[3][3];
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             const float A = f32(vo[q].x), B = f32(vo[q].y);
-            const uint32_t l = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)vo[q].y, 0x111, 0xf, 0xf, false);
-            const uint32_t r = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)vo[q].x, 0x101, 0xf, 0xf, false);
+            const uint32_t l = (uint32_t)__builtin_amdgcn_mov_dpp((int)vo[q].y, 0x111, 0xf, 0xf, true);
+            const uint32_t r = (uint32_t)__builtin_amdgcn_mov_dpp((int)vo[q].x, 0x101, 0xf, 0xf, true);
             float axm = first ? f32(vend[q]) : f32(l), bxp = last ? f32(vend[q]) : f32(r);
             float axp = B, bxm = A;
             float ayp = f32(vyp[q].x), aym = f32(vym[q].x), azp = f32(vzp[q].x), azm = f32(vzm[q].x);
             float byp = f32(vyp[q].y), bym = f32(vym[q].y), bzp = f32(vzp[q].y), bzm = f32(vzm[q].y);
             // across a face, beside an absent block or a solid cell: the cell itself
-            axm = (xl || (first && no_end)) ? A : axm;
-            axp = xha ? A : axp;
-            bxp = (xhb || (last && no_end)) ? B : bxp;
+            axm = (is(LF_INLET) || (first && no_end)) ? A : axm;
+            axp = is(LF_OUTLET_A) ? A : axp;
+            bxp = (is(LF_OUTLET_B) || (last && no_end)) ? B : bxp;
             if (flags & BF_SOLID) {
                 axp = (lma >> 12) & 1u ? A : axp; axm = (lma >> 14) & 1u ? A : axm;
                 ayp = (lma >> 10) & 1u ? A : ayp; aym = (lma >> 16) & 1u ? A : aym;
@@ -364,25 +382,30 @@ k_step_two(const StepArgs a) {
     }
 
     // the sources of the pair
-    for_dirs([&](auto kc) {
-        constexpr int K = decltype(kc)::value;
-        constexpr int cx = dcx(K), cy = dcy(K), cz = dcz(K);
-        if constexpr (cx != 0) {
-            word w;
-            if constexpr (cx > 0) w = W::from_left(s[K], first, e9[K / 3]);
-            else w = W::from_right(s[K], last, e9[K / 3]);
-            if constexpr (cy != 0 || cz != 0) {
-                int j;
-                const bool face = two_row_rule<K>(fc, j);
-                if constexpr (es == 4) { w.x = face ? s[K].x : w.x; w.y = face ? s[K].y : w.y; }
-                else w = face ? s[K] : w;
+    auto sources = [&](auto rules) {
+        for_dirs([&](auto kc) {
+            constexpr int K = decltype(kc)::value;
+            constexpr int cx = dcx(K), cy = dcy(K), cz = dcz(K);
+            if constexpr (cx != 0) {
+                word w;
+                if constexpr (cx > 0) w = W::from_left(s[K], first, e9[K / 3]);
+                else w = W::from_right(s[K], last, e9[K / 3]);
+                if constexpr (decltype(rules)::value && (cy != 0 || cz != 0)) {
+                    int j;
+                    const bool face = two_row_rule<K>(fc, j);
+                    if constexpr (es == 4) { w.x = face ? s[K].x : w.x; w.y = face ? s[K].y : w.y; }
+                    else w = face ? s[K] : w;
+                }
+                s[K] = w;
             }
-            s[K] = w;
-        }
-    });
+        });
+    };
+    if (edge) sources(std::true_type{});
+    else sources(std::false_type{});
     // second pass: solid links and the outlet, in waves that hold one
     const uint32_t links = lma | lmb;
-    if (__builtin_amdgcn_ballot_w64((links & 0x7ffffffu) != 0 || xha || xhb) != 0) {
+    if (__builtin_amdgcn_ballot_w64((links & 0x7ffffffu) != 0 || is(LF_OUTLET_A | LF_OUTLET_B)) != 0) {
+        const bool xha = is(LF_OUTLET_A), xhb = is(LF_OUTLET_B);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
             uint32_t ra[9], rb[9];
@@ -409,10 +432,8 @@ k_step_two(const StepArgs a) {
 
     // collide A, then B; each cell's result takes its half of the words
     const uint32_t ca = b * BS3 + (uint32_t)z * BS2 + (uint32_t)ly * BS + 2u * (uint32_t)jx;
-    const bool dith = SP::dithered && a.cp.dither;
-    const uint32_t key = SP::dithered ? round_key(a.step()) : 0u;
+    const uint32_t key = DITH ? round_key(a.step()) : 0u;
     double F0 = 0.0, F1 = 0.0, F2 = 0.0;
-    const bool want_force = a.fpart != nullptr && (flags & BF_SOLID);
     float va[3], vb[3];
     CellCtx cc{};
     cc.b = b;
@@ -446,7 +467,7 @@ k_step_two(const StepArgs a) {
         constexpr int K = decltype(kc)::value;
         f[K] = W::dec_a(s[K], wgt<float>(K));
     });
-    if (xl) {
+    if (is(LF_INLET)) {
         for_dirs([&](auto kc) {
             constexpr int K = decltype(kc)::value;
             if constexpr (dcx(K) > 0)
@@ -454,39 +475,32 @@ k_step_two(const StepArgs a) {
         });
     }
     if constexpr (EXTRA == TWO_BFL) {
-        if (lva && (lma & 0x7ffffffu)) bfl(f, ca, lma, xha, xl);
+        if (is(LF_LIVE_A) && (lma & 0x7ffffffu)) bfl(f, ca, lma, is(LF_OUTLET_A), is(LF_INLET));
     }
     if constexpr (EXTRA == TWO_SPONGE) qa.sponge = spa;
     collide_cell<float, UNIT, EXTRA == TWO_SPONGE, true>(f, qa, a.cp, rho_o, va[0], va[1], va[2]);
     {
-        const uint32_t hc = SP::dithered ? round_cell(key, ca - cell0) : 0u;
+        const uint32_t hc = DITH ? round_cell(key, ca - cell0) : 0u;
         for_dirs([&](auto kc) {
             constexpr int K = decltype(kc)::value;
             if constexpr (es == 4) s[K].x = __float_as_uint(f[K]);
         });
         if constexpr (es == 2) {
-            if (dith) {
-                for_dirs([&](auto kc) {
-                    constexpr int K = decltype(kc)::value;
-                    s[K] = SP::template put<false>(s[K], f[K], wgt<float>(K), round_bits(hc, K), true);
-                });
-            } else {
-                for_dirs([&](auto kc) {
-                    constexpr int K = decltype(kc)::value;
-                    s[K] = SP::template put<false>(s[K], f[K], wgt<float>(K), 0u, false);
-                });
-            }
+            for_dirs([&](auto kc) {
+                constexpr int K = decltype(kc)::value;
+                s[K] = SP::template put<false>(s[K], f[K], wgt<float>(K), DITH ? round_bits(hc, K) : 0u, DITH);
+            });
         }
     }
     if constexpr (EXTRA != TWO_BFL)
-        if (want_force && lva) link_force(std::integral_constant<int, 0>{}, lma);
+        if (want_force && is(LF_LIVE_A)) link_force(std::integral_constant<int, 0>{}, lma);
     __builtin_amdgcn_sched_barrier(0);
     for_dirs([&](auto kc) {
         constexpr int K = decltype(kc)::value;
         f[K] = W::dec_b(s[K], wgt<float>(K));
     });
     if constexpr (EXTRA == TWO_BFL) {
-        if (lvb && (lmb & 0x7ffffffu)) bfl(f, ca + 1u, lmb, xhb, false);
+        if (is(LF_LIVE_B) && (lmb & 0x7ffffffu)) bfl(f, ca + 1u, lmb, is(LF_OUTLET_B), false);
     }
     CellRates<float> qb = qa;
     qb.omega1 = om1b;
@@ -494,50 +508,41 @@ k_step_two(const StepArgs a) {
     if constexpr (EXTRA == TWO_SPONGE) qb.sponge = spb;
     collide_cell<float, UNIT, EXTRA == TWO_SPONGE, true>(f, qb, a.cp, rho_o, vb[0], vb[1], vb[2]);
     {
-        const uint32_t hc = SP::dithered ? round_cell(key, ca + 1u - cell0) : 0u;
+        const uint32_t hc = DITH ? round_cell(key, ca + 1u - cell0) : 0u;
         for_dirs([&](auto kc) {
             constexpr int K = decltype(kc)::value;
             if constexpr (es == 4) s[K].y = __float_as_uint(f[K]);
         });
         if constexpr (es == 2) {
-            if (dith) {
-                for_dirs([&](auto kc) {
-                    constexpr int K = decltype(kc)::value;
-                    s[K] = SP::template put<true>(s[K], f[K], wgt<float>(K), round_bits(hc, K), true);
-                });
-            } else {
-                for_dirs([&](auto kc) {
-                    constexpr int K = decltype(kc)::value;
-                    s[K] = SP::template put<true>(s[K], f[K], wgt<float>(K), 0u, false);
-                });
-            }
+            for_dirs([&](auto kc) {
+                constexpr int K = decltype(kc)::value;
+                s[K] = SP::template put<true>(s[K], f[K], wgt<float>(K), DITH ? round_bits(hc, K) : 0u, DITH);
+            });
         }
     }
     if constexpr (EXTRA != TWO_BFL)
-        if (want_force && lvb) link_force(std::integral_constant<int, 1>{}, lmb);
+        if (want_force && is(LF_LIVE_B)) link_force(std::integral_constant<int, 1>{}, lmb);
 
-    // store: the whole words where both cells of every lane of the wave step
-    const __amdgpu_buffer_rsrc_t fo = buf_at((char*)a.fout + (size_t)nb0 * blk);
+    // store
+    const __amdgpu_buffer_rsrc_t fo = buf_at((char*)a.fout + (size_t)R.base * blk);
     const uint32_t vown = own0 + row;
-    const bool both = lva && lvb;
-    if (__builtin_amdgcn_ballot_w64(!both) == 0) {
-        for_dirs([&](auto kc) {
-            constexpr int K = decltype(kc)::value;
-            W::template st2<OAL_TWO_STORE_AUX>(s[K], fo, vown, (uint32_t)K * slot + zown);
-        });
-    } else {
+    const bool lva = is(LF_LIVE_A), lvb = is(LF_LIVE_B), both = lva && lvb;
+    auto store = [&](auto aux) {
+        constexpr int AUX = decltype(aux)::value;
         if (both) {
             for_dirs([&](auto kc) {
                 constexpr int K = decltype(kc)::value;
-                W::template st2<OAL_TWO_STORE_AUX>(s[K], fo, vown, (uint32_t)K * slot + zown);
+                W::template st2<AUX>(s[K], fo, vown, (uint32_t)K * slot + zown);
             });
         } else if (lva || lvb) {
             for_dirs([&](auto kc) {
                 constexpr int K = decltype(kc)::value;
-                W::template st1<OAL_TWO_STORE_AUX>(lva ? W::a(s[K]) : W::b(s[K]), fo, vown + (lva ? 0u : es), (uint32_t)K * slot + zown);
+                W::template st1<AUX>(lva ? W::a(s[K]) : W::b(s[K]), fo, vown + (lva ? 0u : es), (uint32_t)K * slot + zown);
             });
         }
-    }
+    };
+    if (a.two_keep) store(std::integral_constant<int, TWO_ST_KEEP>{});
+    else store(std::integral_constant<int, TWO_ST_STREAM>{});
     if constexpr (WALE) {
         float* vout = (float*)a.vel_out;
 #pragma unroll
@@ -552,23 +557,31 @@ k_step_two(const StepArgs a) {
 }
 
 // the blocks of one list, one plane per workgroup
-template <class SP, bool UNIT>
+template <class SP, bool UNIT, bool DITH>
 static void launch_two_u(bool wale, int extra, dim3 g, hipStream_t s, const StepArgs& r) {
     if (wale) {
-        if (extra == TWO_SPONGE) hipLaunchKernelGGL((k_step_two<SP, UNIT, true, TWO_SPONGE>), g, dim3(TWG), 0, s, r);
-        else if (extra == TWO_BFL) hipLaunchKernelGGL((k_step_two<SP, UNIT, true, TWO_BFL>), g, dim3(TWG), 0, s, r);
-        else hipLaunchKernelGGL((k_step_two<SP, UNIT, true, TWO_PLAIN>), g, dim3(TWG), 0, s, r);
+        if (extra == TWO_SPONGE) hipLaunchKernelGGL((k_step_two<SP, UNIT, true, TWO_SPONGE, DITH>), g, dim3(TWG), 0, s, r);
+        else if (extra == TWO_BFL) hipLaunchKernelGGL((k_step_two<SP, UNIT, true, TWO_BFL, DITH>), g, dim3(TWG), 0, s, r);
+        else hipLaunchKernelGGL((k_step_two<SP, UNIT, true, TWO_PLAIN, DITH>), g, dim3(TWG), 0, s, r);
     } else {
-        if (extra == TWO_SPONGE) hipLaunchKernelGGL((k_step_two<SP, UNIT, false, TWO_SPONGE>), g, dim3(TWG), 0, s, r);
-        else if (extra == TWO_BFL) hipLaunchKernelGGL((k_step_two<SP, UNIT, false, TWO_BFL>), g, dim3(TWG), 0, s, r);
-        else hipLaunchKernelGGL((k_step_two<SP, UNIT, false, TWO_PLAIN>), g, dim3(TWG), 0, s, r);
+        if (extra == TWO_SPONGE) hipLaunchKernelGGL((k_step_two<SP, UNIT, false, TWO_SPONGE, DITH>), g, dim3(TWG), 0, s, r);
+        else if (extra == TWO_BFL) hipLaunchKernelGGL((k_step_two<SP, UNIT, false, TWO_BFL, DITH>), g, dim3(TWG), 0, s, r);
+        else hipLaunchKernelGGL((k_step_two<SP, UNIT, false, TWO_PLAIN, DITH>), g, dim3(TWG), 0, s, r);
     }
 }
 template <class SP>
 static void launch_two_sp(bool wale, int extra, const StepArgs& r, hipStream_t s) {
     const dim3 g(r.n_items);
-    if (r.cp.unit) launch_two_u<SP, true>(wale, extra, g, s, r);
-    else launch_two_u<SP, false>(wale, extra, g, s, r);
+    auto go = [&](auto dith) {
+        if (r.cp.unit) launch_two_u<SP, true, decltype(dith)::value>(wale, extra, g, s, r);
+        else launch_two_u<SP, false, decltype(dith)::value>(wale, extra, g, s, r);
+    };
+    if constexpr (SP::dithered) {
+        if (r.cp.dither) go(std::true_type{});
+        else go(std::false_type{});
+    } else {
+        go(std::false_type{});
+    }
 }
 
 }  // namespace oal
