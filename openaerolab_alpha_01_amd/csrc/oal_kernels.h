@@ -181,6 +181,10 @@ hipError_t launch_convert_out(int storage, const void* f, void* dst, int dst_dty
                               int permute, hipStream_t stream);
 hipError_t launch_macro(int storage, const void* f, double* rho, double* u, uint32_t ncell, uint32_t nhost, int permute,
                         void* vel, hipStream_t stream);
+// rho and u of the caller's cells [c0, c0 + n) as [4][n] into out (pinned host memory); map: the library cell
+// of each caller cell, or null
+hipError_t launch_macro_out(int storage, const void* f, const uint32_t* map, uint32_t c0, uint32_t n, int permute, double* out,
+                            hipStream_t stream);
 // Level transfers of a refined plan.  gather: the working-precision populations of each listed cell
 // (bit 31 set = not blended in time) of fnew, or of (1 - w1) fold + w1 fnew when fold is given, in
 // records of XFER_STRIDE values; for the 16-bit forms without fold, records of the stored codes

@@ -192,6 +192,41 @@ hipError_t launch_macro(int storage, const void* f, double* rho, double* u, uint
     }
 }
 
+// The same for a range of the caller's cells [c0, c0 + n), written as [4][n] (rho, ux, uy, uz) into pinned
+// host memory over the link; map: the library cell of each caller cell (levels in 8^3 blocks), or null.
+template <class SP>
+__global__ void __launch_bounds__(WG) k_macro_out(const typename SP::st* f, const uint32_t* map, uint32_t c0, uint32_t n,
+                                                  int permute, double* out) {
+    using T = typename SP::T;
+    const uint32_t i = blockIdx.x * WG + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t cell = map ? map[c0 + i] : c0 + i;
+    double dr = 0.0, jx = 0.0, jy = 0.0, jz = 0.0;
+#pragma unroll
+    for (int k = 0; k < 27; ++k) {
+        const double s = (double)SP::ld(f + pop_index(cell, permute ? 26 - k : k), wgt<T>(k)) - (double)wgt<T>(k);
+        dr += s; jx += s * dcx(k); jy += s * dcy(k); jz += s * dcz(k);
+    }
+    const double r = 1.0 + dr;
+    out[i] = r;
+    out[n + i] = jx / r;
+    out[2 * (size_t)n + i] = jy / r;
+    out[3 * (size_t)n + i] = jz / r;
+}
+
+hipError_t launch_macro_out(int storage, const void* f, const uint32_t* map, uint32_t c0, uint32_t n, int permute, double* out,
+                            hipStream_t s) {
+    const dim3 g((n + WG - 1) / WG);
+    switch (storage) {
+        case 0: hipLaunchKernelGGL((k_macro_out<StF32>), g, dim3(WG), 0, s, (const float*)f, map, c0, n, permute, out); break;
+        case 1: hipLaunchKernelGGL((k_macro_out<StF64>), g, dim3(WG), 0, s, (const double*)f, map, c0, n, permute, out); break;
+        case 2: hipLaunchKernelGGL((k_macro_out<StF16S>), g, dim3(WG), 0, s, (const _Float16*)f, map, c0, n, permute, out); break;
+        case 3: hipLaunchKernelGGL((k_macro_out<StBF16S>), g, dim3(WG), 0, s, (const uint16_t*)f, map, c0, n, permute, out); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
 // ------------------------------------------------------------------------------------------------
 // AA pattern: outlet side buffer from a state in stored form (after upload / initialisation), the
 // copy the even step makes of every outlet-face population with cx = -1
