@@ -150,8 +150,11 @@ struct ReduceArgs {
 // interior block lists), the kernels that carry most of the cells.
 hipError_t launch_step(int storage, int stream_mode, bool wale, const StepArgs& a, hipStream_t stream, hipStream_t side,
                        hipEvent_t bulk0 = nullptr, hipEvent_t bulk1 = nullptr);
-// values per gathered donor record of the level transfers: 27 populations padded to 28 (16-byte rows)
-constexpr int XFER_STRIDE = 28;
+// values per gathered donor record of the level transfers: 27 populations padded to 32 in FP32 (one cache
+// line), to 28 in FP64 (16-byte rows); buffers hold XFER_STRIDE
+template <class T>
+constexpr int xfer_stride() { return sizeof(T) == 4 ? 32 : 28; }
+constexpr int XFER_STRIDE = 32;
 
 // p[0] = v, in stream order (the step index of a replayed step graph)
 hipError_t launch_set_i32(int32_t* p, int32_t v, hipStream_t stream);
@@ -187,7 +190,7 @@ hipError_t launch_macro_out(int storage, const void* f, const uint32_t* map, uin
                             hipStream_t stream);
 // Level transfers of a refined plan.  gather: the working-precision populations of each listed cell
 // (bit 31 set = not blended in time) of fnew, or of (1 - w1) fold + w1 fnew when fold is given, in
-// records of XFER_STRIDE values; for the 16-bit forms without fold, records of the stored codes
+// records of xfer_stride() values; for the 16-bit forms without fold, records of the stored codes
 // (raw, decoded by the rebuild, which must then be told `raw`).  rebuild: for each target cell, the weighted sum of the gathered populations over its
 // 64 stencil nodes (slot[64 * i + node], -1 = unused; weight w[...]: cell-major), its second-order
 // non-equilibrium moments set to scale * keep times their value, written to f; with vel (WALE), the

@@ -415,52 +415,56 @@ template <> struct Vec16<double> {
 // the rebuild; the decoded values are the ones a float record would hold.
 constexpr int XFER_RAW_STRIDE = 32;
 
-// gather: a few lanes per donor, each writing one 16-byte piece of its record (the pieces of a
-// wavefront's donors are contiguous): RAW, 4 lanes of 8 codes; float records, 7 lanes of 4 values;
-// double records, 14 lanes of 2
-template <class SP, bool RAW>
-constexpr int xfer_gather_lanes() {
-    return RAW ? XFER_RAW_STRIDE / 8 : XFER_STRIDE / Vec16<typename SP::T>::n;
-}
+// gather: one lane per donor, so that a direction's loads run over consecutive cells (donors ascend), all
+// 27 in flight; the records leave through LDS as 16-byte pieces in order.  RAW: the stored codes.
 template <class SP, bool RAW>
 __global__ void __launch_bounds__(WG) k_xfer_gather(const typename SP::st* fnew, const typename SP::st* fold,
-                                                    const uint32_t* cells, uint32_t n, uint32_t ncell, typename SP::T w1,
-                                                    typename SP::T* out) {
+                                                    const uint32_t* cells, uint32_t n, typename SP::T w1, typename SP::T* out) {
     using T = typename SP::T;
-    constexpr int Q = xfer_gather_lanes<SP, RAW>();
-    const uint32_t t = blockIdx.x * WG + threadIdx.x;
-    if (t >= n * (uint32_t)Q) return;
-    const uint32_t i = t / Q;
-    const int q = (int)(t - i * Q);
+    constexpr int RW = RAW ? XFER_RAW_STRIDE / 2 : xfer_stride<T>() * (int)sizeof(T) / 4;   // 32-bit words of a record
+    constexpr int P = RW / 4;                                                             // its 16-byte pieces
+    __shared__ uint4 sh[WG / 64][64][P + 1];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t i0 = blockIdx.x * WG + (uint32_t)wave * 64u;
+    if (i0 >= n) return;
+    const uint32_t i = i0 + (uint32_t)lane < n ? i0 + (uint32_t)lane : n - 1;
     const uint32_t e = cells[i];
     const uint32_t c = e & 0x7fffffffu;
+    uint32_t w[RW];
+#pragma unroll
+    for (int k = 0; k < RW; ++k) w[k] = 0;
     if constexpr (RAW) {
-        uint32_t h[8];
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const int k = 8 * q + r;
-            h[r] = k < 27 ? (uint32_t)SP::ld_raw(fnew + pop_index(c, k)) : 0u;
-        }
-        reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(out) + (size_t)i * XFER_RAW_STRIDE)[q] =
-            make_uint4(h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16));
-        return;
+        uint32_t h[27];
+        for_dirs([&](auto kc) { constexpr int K = decltype(kc)::value; h[K] = SP::ld_raw(fnew + pop_index(c, K)); });
+        for_dirs([&](auto kc) { constexpr int K = decltype(kc)::value; w[K / 2] |= h[K] << (16 * (K % 2)); });
+    } else {
+        const bool blend = fold && !(e >> 31);
+        typename SP::raw a[27], b[27];
+        for_dirs([&](auto kc) { constexpr int K = decltype(kc)::value; a[K] = SP::ld_raw(fnew + pop_index(c, K)); });
+        if (fold) for_dirs([&](auto kc) { constexpr int K = decltype(kc)::value; b[K] = SP::ld_raw(fold + pop_index(c, K)); });
+        for_dirs([&](auto kc) {
+            constexpr int K = decltype(kc)::value;
+            T x = SP::from_raw(a[K], wgt<T>(K));
+            if (blend) x = SP::from_raw(b[K], wgt<T>(K)) * (T(1) - w1) + x * w1;
+            if constexpr (sizeof(T) == 4) {
+                w[K] = __float_as_uint((float)x);
+            } else {
+                const uint64_t u = (uint64_t)__double_as_longlong((double)x);
+                w[2 * K] = (uint32_t)u;
+                w[2 * K + 1] = (uint32_t)(u >> 32);
+            }
+        });
     }
-    using V = typename Vec16<T>::type;
-    constexpr int VN = Vec16<T>::n;
-    const bool blend = fold && !(e >> 31);
-    V v;
 #pragma unroll
-    for (int r = 0; r < VN; ++r) {
-        const int k = VN * q + r;
-        T x = T(0);
-        if (k < 27) {
-            const T w = wgt_rt<T>(k);
-            x = SP::ld(fnew + pop_index(c, k), w);
-            if (blend) x = SP::ld(fold + pop_index(c, k), w) * (T(1) - w1) + x * w1;
-        }
-        v[r] = x;
+    for (int p = 0; p < P; ++p) sh[wave][lane][p] = make_uint4(w[4 * p], w[4 * p + 1], w[4 * p + 2], w[4 * p + 3]);
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t pieces = (n - i0 < 64u ? n - i0 : 64u) * P;
+    uint4* o = reinterpret_cast<uint4*>(out) + (size_t)i0 * P;
+#pragma unroll
+    for (int q = 0; q < P; ++q) {
+        const uint32_t t = (uint32_t)(q * 64 + lane);
+        if (t < pieces) o[t] = sh[wave][t / P][t % P];
     }
-    reinterpret_cast<V*>(out + (size_t)i * XFER_STRIDE)[q] = v;
 }
 
 // sum of a value over the 16 lanes of a DPP row, as a fixed pairwise tree: lanes l and l xor 1, then
@@ -493,76 +497,14 @@ __device__ __forceinline__ bool row_any(bool b) {
     return ((m >> (threadIdx.x & 48u)) & 0xffffull) != 0;
 }
 
-// rebuild: 16 lanes (one DPP row) per written cell, lane j summing stencil nodes 4j .. 4j + 3 in node
-// order from zero, the 16 partial sums then added as a pairwise tree (row_sum); every lane forms the
-// moments, lane j rebuilds and stores directions j and j + 16.  Stencils are cell-major: slot[i][64],
-// wt[i][64].
-template <class SP, bool RAW>
-__global__ void __launch_bounds__(WG) k_xfer_rebuild(typename SP::st* f, uint32_t ncell, const uint32_t* tcells, uint32_t n,
-                                                     const int32_t* slot, const float* wt, const typename SP::T* m,
-                                                     typename SP::T scale, typename SP::T keep, typename SP::T* vel) {
-    using T = typename SP::T;
-    const uint32_t i = blockIdx.x * (WG / 16) + (threadIdx.x >> 4);
-    const int j = (int)(threadIdx.x & 15);
-    if (i >= n) return;   // whole rows: the lanes of a live cell stay together
-    const int4 s4 = *reinterpret_cast<const int4*>(slot + (size_t)i * 64 + 4 * j);
-    const float4 w4 = *reinterpret_cast<const float4*>(wt + (size_t)i * 64 + 4 * j);
-    const int32_t sr[4] = {s4.x, s4.y, s4.z, s4.w};
-    const T wn[4] = {T(w4.x), T(w4.y), T(w4.z), T(w4.w)};
-    T acc[27];
-#pragma unroll
-    for (int k = 0; k < 27; ++k) acc[k] = T(0);
-    if constexpr (RAW) {
-        uint4 rec[4][4];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const uint4* row = reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(m) +
-                                                              (size_t)(sr[g] >= 0 ? sr[g] : 0) * XFER_RAW_STRIDE);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) rec[g][q] = row[q];
-        }
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const bool use = sr[g] >= 0;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint32_t wd[4] = {rec[g][q].x, rec[g][q].y, rec[g][q].z, rec[g][q].w};
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int k = 8 * q + e;
-                    if (k < 27) {
-                        const T add = acc[k] + wn[g] * SP::from_raw((wd[e >> 1] >> (16 * (e & 1))) & 0xffffu, wgt<T>(k));
-                        acc[k] = use ? add : acc[k];
-                    }
-                }
-            }
-        }
-    } else {
-        using V = typename Vec16<T>::type;
-        constexpr int VN = Vec16<T>::n;
-        V rec[4][XFER_STRIDE / VN];
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const V* row = reinterpret_cast<const V*>(m + (size_t)(sr[g] >= 0 ? sr[g] : 0) * XFER_STRIDE);
-#pragma unroll
-            for (int q = 0; q < XFER_STRIDE / VN; ++q) rec[g][q] = row[q];
-        }
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const bool use = sr[g] >= 0;
-#pragma unroll
-            for (int q = 0; q < XFER_STRIDE / VN; ++q)
-#pragma unroll
-                for (int e = 0; e < VN; ++e)
-                    if (q * VN + e < 27) {
-                        const T add = acc[q * VN + e] + wn[g] * rec[g][q][e];
-                        acc[q * VN + e] = use ? add : acc[q * VN + e];
-                    }
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < 27; ++k) acc[k] = row_sum(acc[k]);
-    // moments of the interpolated state (every lane)
+// moments of an interpolated state: density, velocity and the change of its second-order non-equilibrium
+// moments
+template <class T>
+struct XferMoments {
+    T rho, ux, uy, uz, dxx, dyy, dzz, dxy, dxz, dyz, tr, usq;
+};
+template <class T>
+__device__ __forceinline__ XferMoments<T> xfer_moments(const T (&acc)[27], T scale, T keep) {
     T rho = T(0), jx = T(0), jy = T(0), jz = T(0), pxx = T(0), pyy = T(0), pzz = T(0), pxy = T(0), pxz = T(0), pyz = T(0);
     for_dirs([&](auto kc) {
         constexpr int K = decltype(kc)::value;
@@ -596,6 +538,64 @@ __global__ void __launch_bounds__(WG) k_xfer_rebuild(typename SP::st* f, uint32_
     const T dxy = sk * qxy - qxy, dxz = sk * qxz - qxz, dyz = sk * qyz - qyz;
     const T tr = (dxx + dyy) + dzz;
     const T usq = (ux * ux + uy * uy) + uz * uz;
+    return XferMoments<T>{rho, ux, uy, uz, dxx, dyy, dzz, dxy, dxz, dyz, tr, usq};
+}
+// one population of the rebuilt cell (a: the interpolated one) and of its equilibrium
+template <class T>
+__device__ __forceinline__ void xfer_value(const XferMoments<T>& q, T a, T w, T cx, T cy, T cz, T& out, T& eq) {
+    const T third = T(1.0 / 3.0);
+    const T cac = ((cx * cx * q.dxx + cy * cy * q.dyy) + cz * cz * q.dzz) + T(2) * ((cx * cy * q.dxy + cx * cz * q.dxz) + cy * cz * q.dyz);
+    out = a + (w * T(4.5)) * (cac - q.tr * third);
+    const T cu = (cx * q.ux + cy * q.uy) + cz * q.uz;
+    eq = (w * q.rho) * (((T(1) + T(3) * cu) + T(4.5) * cu * cu) - T(1.5) * q.usq);
+}
+
+// rebuild, FP64: 16 lanes (one DPP row) per written cell, lane j summing stencil nodes 4j .. 4j + 3 in node
+// order from zero, the 16 partial sums then added as a pairwise tree (row_sum); every lane forms the
+// moments, lane j rebuilds and stores directions j and j + 16.  Stencils are cell-major: slot[i][64],
+// wt[i][64].
+template <class SP>
+__global__ void __launch_bounds__(WG) k_xfer_rebuild_row(typename SP::st* f, uint32_t ncell, const uint32_t* tcells, uint32_t n,
+                                                     const int32_t* slot, const float* wt, const typename SP::T* m,
+                                                     typename SP::T scale, typename SP::T keep, typename SP::T* vel) {
+    using T = typename SP::T;
+    const uint32_t i = blockIdx.x * (WG / 16) + (threadIdx.x >> 4);
+    const int j = (int)(threadIdx.x & 15);
+    if (i >= n) return;   // whole rows: the lanes of a live cell stay together
+    const int4 s4 = *reinterpret_cast<const int4*>(slot + (size_t)i * 64 + 4 * j);
+    const float4 w4 = *reinterpret_cast<const float4*>(wt + (size_t)i * 64 + 4 * j);
+    const int32_t sr[4] = {s4.x, s4.y, s4.z, s4.w};
+    const T wn[4] = {T(w4.x), T(w4.y), T(w4.z), T(w4.w)};
+    T acc[27];
+#pragma unroll
+    for (int k = 0; k < 27; ++k) acc[k] = T(0);
+    {
+        using V = typename Vec16<T>::type;
+        constexpr int VN = Vec16<T>::n;
+        constexpr int ST = xfer_stride<T>();
+        V rec[4][ST / VN];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const V* row = reinterpret_cast<const V*>(m + (size_t)(sr[g] >= 0 ? sr[g] : 0) * ST);
+#pragma unroll
+            for (int q = 0; q < ST / VN; ++q) rec[g][q] = row[q];
+        }
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const bool use = sr[g] >= 0;
+#pragma unroll
+            for (int q = 0; q < ST / VN; ++q)
+#pragma unroll
+                for (int e = 0; e < VN; ++e)
+                    if (q * VN + e < 27) {
+                        const T add = acc[q * VN + e] + wn[g] * rec[g][q][e];
+                        acc[q * VN + e] = use ? add : acc[q * VN + e];
+                    }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 27; ++k) acc[k] = row_sum(acc[k]);
+    const XferMoments<T> m0 = xfer_moments<T>(acc, scale, keep);
     // lane j: directions j and j + 16
     T out[2], eq[2];
     bool bad = false;
@@ -608,10 +608,7 @@ __global__ void __launch_bounds__(WG) k_xfer_rebuild(typename SP::st* f, uint32_
             T a = acc[0];
 #pragma unroll
             for (int kk = 1; kk < 27; ++kk) a = kk == k ? acc[kk] : a;
-            const T cac = ((cx * cx * dxx + cy * cy * dyy) + cz * cz * dzz) + T(2) * ((cx * cy * dxy + cx * cz * dxz) + cy * cz * dyz);
-            out[h] = a + (w * T(4.5)) * (cac - tr * third);
-            const T cu = (cx * ux + cy * uy) + cz * uz;
-            eq[h] = (w * rho) * (((T(1) + T(3) * cu) + T(4.5) * cu * cu) - T(1.5) * usq);
+            xfer_value(m0, a, w, cx, cy, cz, out[h], eq[h]);
             bad = bad || out[h] < T(1e-6) * w;
         }
     }
@@ -625,9 +622,179 @@ __global__ void __launch_bounds__(WG) k_xfer_rebuild(typename SP::st* f, uint32_
     // WALE: the written cell's velocity (that of the interpolated state, which the rescale and the
     // equilibrium fallback keep) for the receiving level's gradient gather
     if (vel && j == 0) {
-        vel[c] = ux;
-        vel[ncell + c] = uy;
-        vel[2 * (size_t)ncell + c] = uz;
+        vel[c] = m0.ux;
+        vel[ncell + c] = m0.uy;
+        vel[2 * (size_t)ncell + c] = m0.uz;
+    }
+}
+
+// rebuild, FP32 arithmetic: a wave sums one written cell at a time with all lanes, and rebuilds up to
+// XFER_CELLS of them together.
+//   Sums: the lanes of a record are neighbours (8 of 16 bytes for float records, 4 for stored codes), so
+//   that a load instruction reads whole lines; the lanes of a group sum its stencil nodes 4j .. 4j + 3 in
+//   node order from zero (float records: two such partial sums per group), and the 16 partial sums add as
+//   a pairwise tree: the low bits of j within a DPP row (rotations by 8 and by 4 lanes, the second on
+//   values alike in the first's lanes), the high bits over the wave's four rows through LDS.
+//   Cells: two lanes per cell read its 27 sums, form the moments and write half the directions each.
+// Bound: VALU issue (64 x 27 multiplies and adds per cell, unfused, in a fixed order).  Against 16 lanes per
+// cell with one record per lane, all of them forming the moments: a 75 000-cell fill from FP16 levels 53 -> 43
+// us, a 4-level octree step 1668 -> 1571 us.
+constexpr int XFER_CELLS = 16;   // written cells per wave, at most
+constexpr int XWG = 256;         // lanes of a workgroup
+template <class SP, bool RAW>
+__global__ void __launch_bounds__(XWG) k_xfer_rebuild(typename SP::st* f, uint32_t ncell, const uint32_t* tcells, uint32_t n,
+                                                     uint32_t per, const int32_t* slot, const float* wt, const float* m,
+                                                     float scale, float keep, float* vel) {
+    constexpr int V = RAW ? 8 : 4;            // directions per lane
+    constexpr int NODES = RAW ? 4 : 8;        // nodes per lane
+    constexpr int H = NODES / 4;              // partial sums per lane
+    __shared__ float sums[XWG / 64][XFER_CELLS][4 * 32 + 4];   // [cell][row][direction], padded off the banks
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const uint32_t i0 = (blockIdx.x * (XWG / 64) + (uint32_t)wave) * per;
+    if (i0 >= n) return;
+    const int cnt = (int)(n - i0 < per ? n - i0 : per);
+    const int q = RAW ? lane & 3 : lane & 7;
+    // group of nodes: its low bits in lane bit 3 (then 2), the high ones in the row
+    const int g = RAW ? ((lane >> 3) & 1) | (((lane >> 2) & 1) << 1) | ((lane >> 4) << 2) : lane >> 3;
+    float wk[V];
+#pragma unroll
+    for (int e = 0; e < V; ++e) wk[e] = wgt_rt<float>(V * q + e < 27 ? V * q + e : 13);
+    // a quad's lanes read the nodes of its group, one (RAW) or two (lane and lane + 4) each, and pass them on
+    // by quad broadcasts
+    const uint32_t mine = (uint32_t)(g * NODES + (lane & 3));
+    struct Stencil {
+        uint32_t r[H];        // record in 16-byte units (unused nodes: record 0)
+        float w[H];
+        bool some;            // an unused node
+    };
+    auto stencil = [&](int d, Stencil& t) {
+        const size_t o = (size_t)(i0 + (uint32_t)(d < cnt ? d : cnt - 1)) * 64 + mine;
+        t.some = false;
+#pragma unroll
+        for (int h = 0; h < H; ++h) {
+            const int32_t sv = slot[o + 4 * h];
+            t.r[h] = sv < 0 ? 0xffffffffu : (uint32_t)sv * (RAW ? 4u : 8u);
+            t.w[h] = wt[o + 4 * h];
+        }
+    };
+    const uint4* mq = reinterpret_cast<const uint4*>(m) + q;
+    auto records = [&](const Stencil& t, uint4 (&rec)[NODES]) {
+        for_each_dir(std::make_integer_sequence<int, NODES>{}, [&](auto ec) {
+            constexpr int E = decltype(ec)::value;
+            const uint32_t r = (uint32_t)__builtin_amdgcn_mov_dpp((int)t.r[E / 4], (E & 3) * 0x55, 0xf, 0xf, false);
+            rec[E] = mq[r == 0xffffffffu ? 0u : r];
+        });
+    };
+    Stencil sa, sb, sc{};
+    uint4 ra[NODES], rb[NODES];
+    stencil(0, sa);
+    stencil(1, sb);
+    records(sa, ra);
+    auto one = [&](int d, const Stencil& t, uint4 (&rec)[NODES]) {
+        float acc[H][V];
+        bool some = false;
+#pragma unroll
+        for (int h = 0; h < H; ++h) some = some || t.r[h] == 0xffffffffu;
+        auto add = [&](auto check) {
+#pragma unroll
+            for (int h = 0; h < H; ++h)
+#pragma unroll
+                for (int e = 0; e < V; ++e) acc[h][e] = 0.0f;
+            for_each_dir(std::make_integer_sequence<int, NODES>{}, [&](auto ec) {
+                constexpr int E = decltype(ec)::value;
+                const uint32_t wd[4] = {rec[E].x, rec[E].y, rec[E].z, rec[E].w};
+                const float w = dpp_get<(E & 3) * 0x55>(t.w[E / 4]);
+                bool use = true;
+                if constexpr (decltype(check)::value)
+                    use = (uint32_t)__builtin_amdgcn_mov_dpp((int)t.r[E / 4], (E & 3) * 0x55, 0xf, 0xf, false) != 0xffffffffu;
+#pragma unroll
+                for (int k = 0; k < V; ++k) {
+                    float x;
+                    if constexpr (RAW) x = SP::from_raw((wd[k >> 1] >> (16 * (k & 1))) & 0xffffu, wk[k]);
+                    else x = __uint_as_float(wd[k]);
+                    const float v = acc[E / 4][k] + w * x;
+                    if constexpr (decltype(check)::value) acc[E / 4][k] = use ? v : acc[E / 4][k];
+                    else acc[E / 4][k] = v;
+                }
+            });
+        };
+        if (__builtin_amdgcn_ballot_w64(some) == 0) add(std::false_type{});
+        else add(std::true_type{});
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            float t;
+            if constexpr (RAW) {
+                t = acc[0][k];
+                t = t + dpp_get<0x128>(t);    // row_ror:8
+                t = t + dpp_get<0x124>(t);    // row_ror:4
+            } else {
+                t = acc[0][k] + acc[1][k];
+                t = t + dpp_get<0x128>(t);
+            }
+            acc[0][k] = t;
+        }
+        if ((lane & 15) < (RAW ? 4 : 8)) {
+            float4* o = reinterpret_cast<float4*>(&sums[wave][d][(lane >> 4) * 32 + V * q]);
+#pragma unroll
+            for (int k = 0; k < V / 4; ++k) o[k] = make_float4(acc[0][4 * k], acc[0][4 * k + 1], acc[0][4 * k + 2], acc[0][4 * k + 3]);
+        }
+    };
+    // the next cell's records and the stencil after it are in flight during a cell's sums
+    for (int d = 0; d < cnt; d += 2) {
+        stencil(d + 2, sc);
+        records(sb, rb);
+        one(d, sa, ra);
+        if (d + 1 >= cnt) break;
+        sa = sc;
+        stencil(d + 3, sc);
+        records(sa, ra);
+        one(d + 1, sb, rb);
+        sb = sc;
+    }
+    __builtin_amdgcn_wave_barrier();
+    // two lanes per cell, for a direction and its opposite: c c is the same and c u changes its sign
+    const int d = lane >> 1;
+    const bool opp = lane & 1;
+    if (d >= cnt) return;
+    float acc[27];
+    {
+        const float* b = &sums[wave][d][0];
+#pragma unroll
+        for (int k = 0; k < 7; ++k) {
+            const float4 r0 = *reinterpret_cast<const float4*>(b + 4 * k), r1 = *reinterpret_cast<const float4*>(b + 32 + 4 * k);
+            const float4 r2 = *reinterpret_cast<const float4*>(b + 64 + 4 * k), r3 = *reinterpret_cast<const float4*>(b + 96 + 4 * k);
+            acc[4 * k] = (r0.x + r1.x) + (r2.x + r3.x);
+            acc[4 * k + 1] = (r0.y + r1.y) + (r2.y + r3.y);
+            acc[4 * k + 2] = (r0.z + r1.z) + (r2.z + r3.z);
+            if (k < 6) acc[4 * k + 3] = (r0.w + r1.w) + (r2.w + r3.w);
+        }
+    }
+    const XferMoments<float> m0 = xfer_moments<float>(acc, scale, keep);
+    float out[14], eq[14];
+    bool bad = false;
+    for_each_dir(std::make_integer_sequence<int, 14>{}, [&](auto kc) {
+        constexpr int K = decltype(kc)::value;
+        constexpr float w = wgt<float>(K);
+        XferMoments<float> q0 = m0;
+        // (c -> -c: the signs of c u only)
+        q0.ux = opp ? -m0.ux : m0.ux;
+        q0.uy = opp ? -m0.uy : m0.uy;
+        q0.uz = opp ? -m0.uz : m0.uz;
+        xfer_value(q0, opp ? acc[26 - K] : acc[K], w, (float)dcx(K), (float)dcy(K), (float)dcz(K), out[K], eq[K]);
+        bad = bad || out[K] < 1e-6f * w;
+    });
+    bad = ((__builtin_amdgcn_ballot_w64(bad) >> (lane & 62)) & 3ull) != 0;
+    const uint32_t c = tcells[i0 + (uint32_t)d];
+    for_each_dir(std::make_integer_sequence<int, 14>{}, [&](auto kc) {
+        constexpr int K = decltype(kc)::value;
+        if (K < 13 || !opp) SP::sto(f + pop_index(c, opp ? 26 - K : K), bad ? eq[K] : out[K], wgt<float>(K));
+    });
+    // WALE: the written cell's velocity (that of the interpolated state, which the rescale and the
+    // equilibrium fallback keep) for the receiving level's gradient gather
+    if (vel && !opp) {
+        vel[c] = m0.ux;
+        vel[ncell + c] = m0.uy;
+        vel[2 * (size_t)ncell + c] = m0.uz;
     }
 }
 
@@ -642,22 +809,31 @@ hipError_t launch_set_i32(int32_t* p, int32_t v, hipStream_t s) {
 
 
 template <class SP, bool RAW>
-static hipError_t xfer_sp(const void* fnew, const void* fold, const uint32_t* cells, uint32_t n, uint32_t ncell, double w1,
-                          void* out, hipStream_t s) {
+static hipError_t xfer_sp(const void* fnew, const void* fold, const uint32_t* cells, uint32_t n, double w1, void* out,
+                          hipStream_t s) {
     using T = typename SP::T;
     if (!n) return hipSuccess;
-    constexpr uint32_t Q = (uint32_t)xfer_gather_lanes<SP, RAW>();
-    hipLaunchKernelGGL((k_xfer_gather<SP, RAW>), dim3((n * Q + WG - 1) / WG), dim3(WG), 0, s, (const typename SP::st*)fnew,
-                       (const typename SP::st*)fold, cells, n, ncell, T(w1), (T*)out);
+    hipLaunchKernelGGL((k_xfer_gather<SP, RAW>), dim3((n + WG - 1) / WG), dim3(WG), 0, s, (const typename SP::st*)fnew,
+                       (const typename SP::st*)fold, cells, n, T(w1), (T*)out);
     return hipGetLastError();
 }
 template <class SP, bool RAW>
 static hipError_t rebuild_sp(void* f, uint32_t ncell, const uint32_t* tcells, uint32_t n, const int32_t* slot, const float* w,
                              const void* m, double scale, double keep, void* vel, hipStream_t s) {
     using T = typename SP::T;
+    using st = typename SP::st;
     if (!n) return hipSuccess;
-    hipLaunchKernelGGL((k_xfer_rebuild<SP, RAW>), dim3((n + WG / 16 - 1) / (WG / 16)), dim3(WG), 0, s, (typename SP::st*)f, ncell, tcells, n,
-                       slot, w, (const T*)m, T(scale), T(keep), (T*)vel);
+    if constexpr (sizeof(T) == 8) {
+        hipLaunchKernelGGL((k_xfer_rebuild_row<SP>), dim3((n + WG / 16 - 1) / (WG / 16)), dim3(WG), 0, s, (st*)f, ncell, tcells, n,
+                           slot, w, (const T*)m, T(scale), T(keep), (T*)vel);
+    } else {
+        // written cells per wave: fewer where 32 would leave less than two waves per SIMD (2048 of them)
+        uint32_t per = n / 2048u;
+        per = per < 1u ? 1u : (per > (uint32_t)XFER_CELLS ? (uint32_t)XFER_CELLS : per);
+        const uint32_t waves = (n + per - 1) / per;
+        hipLaunchKernelGGL((k_xfer_rebuild<SP, RAW>), dim3((waves + XWG / 64 - 1) / (XWG / 64)), dim3(XWG), 0, s, (st*)f, ncell, tcells,
+                           n, per, slot, w, (const float*)m, (float)scale, (float)keep, (float*)vel);
+    }
     return hipGetLastError();
 }
 
@@ -666,12 +842,12 @@ hipError_t launch_xfer_gather(int storage, const void* fnew, const void* fold, c
                                uint32_t ncell, double w1, void* out, hipStream_t s) {
     const bool raw = fold == nullptr;
     switch (storage) {
-        case 0: return xfer_sp<StF32, false>(fnew, fold, cells, n, ncell, w1, out, s);
-        case 1: return xfer_sp<StF64, false>(fnew, fold, cells, n, ncell, w1, out, s);
-        case 2: return raw ? xfer_sp<StF16S, true>(fnew, fold, cells, n, ncell, w1, out, s)
-                           : xfer_sp<StF16S, false>(fnew, fold, cells, n, ncell, w1, out, s);
-        case 3: return raw ? xfer_sp<StBF16S, true>(fnew, fold, cells, n, ncell, w1, out, s)
-                           : xfer_sp<StBF16S, false>(fnew, fold, cells, n, ncell, w1, out, s);
+        case 0: return xfer_sp<StF32, false>(fnew, fold, cells, n, w1, out, s);
+        case 1: return xfer_sp<StF64, false>(fnew, fold, cells, n, w1, out, s);
+        case 2: return raw ? xfer_sp<StF16S, true>(fnew, fold, cells, n, w1, out, s)
+                           : xfer_sp<StF16S, false>(fnew, fold, cells, n, w1, out, s);
+        case 3: return raw ? xfer_sp<StBF16S, true>(fnew, fold, cells, n, w1, out, s)
+                           : xfer_sp<StBF16S, false>(fnew, fold, cells, n, w1, out, s);
         default: return hipErrorInvalidValue;
     }
 }

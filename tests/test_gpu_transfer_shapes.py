@@ -1,0 +1,22 @@
+"""Level transfers on enough cells that a wave of the rebuild takes several of them (5 per wave in the fill,
+3 in the full restriction, the last wave short), with complete stencils and, around the sphere, incomplete
+ones: every level's populations bit for bit the oracle's refined run."""
+import pytest
+import test_gpu_octree as T
+
+from openaerolab_alpha_01_amd.geometry import sphere_octree
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("storage,wale", [("f32", 0.2), ("f16s", 0.0), ("bf16s", 0.2)])
+def test_many_transferred_cells(oracle, storage, wale):
+    from oracle import octree
+    # 2 refined coarse blocks: 64 x 32 x 32 fine cells, 10760 ghost cells around them, 8192 covered cells
+    cfg = dict(grids=lambda: sphere_octree((64, 48, 48), 2, (64.0, 48.0, 48.0), 6.0, (2,)), tau=0.55, u_inlet=0.04,
+               u0=(0.04, 0.0, 0.0), wale=dict(c_wale=wale) if wale else {})
+    grids, run, plan = T.run_both(oracle, octree, "many cells", storage, 1, cfg=cfg)
+    assert plan.level_info(1)["n_blocks"] == 16
+    for l in range(2):
+        T.compare_level(oracle, plan, run, storage, l)
+    plan.close()
