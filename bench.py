@@ -648,17 +648,16 @@ def main(argv=None) -> int:
                                                       not args.no_autotune, fixed, qmap)
     mlups = n_cells * args.steps / (ms_total * 1e-3) / 1e6
     ms_step = ms_total / args.steps
-    # dominant kernel: AB pattern, the two-cells-per-lane kernel over every block; AA pattern, the pipelined
-    # kernels over the regular blocks
+    # dominant kernel: the two-cells-per-lane kernel over every block (AA pattern: its odd half-step)
     ab = args.stream == "ab"
-    bulk_cells = n_fluid if ab and qmap is None else (info["n_regular"] + info["n_interior"]) * 16 ** 3
+    bulk_cells = n_fluid if qmap is None else (info["n_regular"] + info["n_interior"]) * 16 ** 3
     achieved = bytes_per_lup("f32") * bulk_cells / (ms_kernel * 1e-3) / 1e9
     step_gbs = bytes_per_lup("f32") * n_fluid / (ms_step * 1e-3) / 1e9
     area = np.pi * (D / 2) ** 2
     cd = float(F[0] / (0.5 * U_IN ** 2 * area))
 
     # (the collision's unit-rate form: the reference's default rates omega_bulk = omega_3 = omega_4 = 1)
-    kernel = "k_step_two<StF32, true, false, 0>" if ab else "k_step_pipe_aa<StF32>"
+    kernel = "k_step_two<StF32, true, false, 0>" if ab else "k_step_two<StF32, true, false, 0, odd>"
     traffic = measured_traffic(kernel)
 
     out = {
@@ -696,7 +695,7 @@ def main(argv=None) -> int:
         bulk16 = bulk_cells
         a16 = bytes_per_lup("f16s") * bulk16 / (ms_k16 * 1e-3) / 1e9
         s16 = bytes_per_lup("f16s") * n_fluid / (ms_t16 / args.steps * 1e-3) / 1e9
-        k16 = "k_step_two<StF16S, true, false, 0>" if ab else "k_step_pipe_aa<StF16S>"
+        k16 = "k_step_two<StF16S, true, false, 0>" if ab else "k_step_two<StF16S, true, false, 0, odd>"
         traffic16 = measured_traffic(k16, "step_f16_256_hbm_traffic.md")
         out["fp16_shifted"] = {"value": round(m16, 1), "unit": "MLUPS", "ms_per_step": round(ms_t16 / args.steps, 4),
                                "speedup_vs_f32": round(m16 / mlups, 3), "tuning": tun16,
@@ -723,8 +722,7 @@ def main(argv=None) -> int:
                              "population_bytes": 27 * 4 * n_cells, "population_bytes_ab": 2 * 27 * 4 * n_cells,
                              "step_achieved_gbs": round(sa, 1), "step_frac": round(sa / HBM_PEAK_GBS, 4),
                              "tuning": {k: tuna[k] for k in ("pipe_planes", "overlap", "face_kernel")},
-                             "blocks": {"pipelined_regular": infoa["n_regular"],
-                                        "one_plane_boundary": infoa["n_boundary_regular"] + infoa["n_boundary"]},
+                             "blocks": {k: infoa[k] for k in ("n_blocks", "n_regular", "n_boundary_regular", "n_boundary")},
                              "cd_transient": round(float(Fa[0] / (0.5 * U_IN ** 2 * area)), 5)}
     if not args.no_wale_leg:
         # the reference's production collision on the same workload: WALE (c_wale 0.2) and inlet noise (0.01)

@@ -390,13 +390,11 @@ int oal_time_steps(OalPlan* plan, int level, int n, int flags, double* ms_total,
  * 8 TB/s datasheet peak. */
 int oal_copy_bandwidth(int device, int64_t bytes, int reps, double* gbs);
 
-/* Launch shape of the step kernels.  pipe_planes (AA pattern, FP32 arithmetic): z-planes of a 16^3
- * block one workgroup of the regular blocks' kernel walks with its next plane's loads in flight (1 = one
- * plane per workgroup, no pipelining; 2, 4 or 8; 16 runs as 8).  overlap: 1 = the boundary and face
- * launches on a second stream, concurrent with the bulk launch; 0 = every launch in order on the plan's
- * stream.  face_kernel, pair_kernel: accepted and reported, without effect (the AB pattern with FP32
- * arithmetic has one kernel, two cells per lane with the face rules in it; FP64 steps the face cells in
- * their own kernel).  graph: 1 = oal_step on the plan's own stream (stream NULL) replays a hipGraph of one
+/* Launch shape of the step kernels.  overlap: 1 = the boundary and face launches on a second stream,
+ * concurrent with the bulk launch; 0 = every launch in order on the plan's stream.  pipe_planes,
+ * face_kernel, pair_kernel: accepted and reported, without effect (with FP32 arithmetic one kernel, two
+ * cells per lane and one plane per workgroup with the face rules in it, steps both patterns; FP64 steps
+ * the face cells in their own kernel).  graph: 1 = oal_step on the plan's own stream (stream NULL) replays a hipGraph of one
  * (coarse) step, captured on first use for each arrangement of the levels' buffers, with the step index
  * read from device memory (a step that collects the force runs as ordinary launches); 0 = the host issues
  * every launch.  Refined plans start with graph 1, one-level plans with 0.  Setting the tuning drops

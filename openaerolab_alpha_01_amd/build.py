@@ -77,12 +77,15 @@ def build_oracle(verbose: bool = False) -> Path:
 
 def scratch_kernels(report: str) -> list[tuple[str, int]]:
     """(kernel, bytes per lane) of every kernel that the compiler's resource-usage remarks show with
-    scratch (register spills)"""
+    scratch (register spills).  A frame no larger than the spilled scalar registers, in a kernel that spills
+    no vector register, holds their slots only: scalars are kept in lanes of a vector register and the
+    frame is never accessed."""
     out = []
     for block in report.split("remark: Function Name: ")[1:]:
         name = block.split()[0]
         m = re.search(r"ScratchSize \[bytes/lane\]: (\d+)", block)
-        if m and int(m.group(1)) > 0:
+        sgpr, vgpr = (int((re.search(rf"{r} Spill: (\d+)", block) or [0, 0])[1]) for r in ("SGPRs", "VGPRs"))
+        if m and int(m.group(1)) > (0 if vgpr else 4 * sgpr):
             out.append((name, int(m.group(1))))
     return out
 

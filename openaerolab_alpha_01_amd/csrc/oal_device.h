@@ -243,7 +243,7 @@ struct CollParams {
     int32_t adaptive_omega4, limiter, compressible, bb_mode;
     float c_wale, nu_sgs_bg, inlet_turb;
     int32_t dither;   // 16-bit storage forms: stochastic rounding of the step's stores
-    int32_t unit;     // omega_bulk = omega_3 = omega_4 = 1: the pipelined kernels use the UNIT collision
+    int32_t unit;     // omega_bulk = omega_3 = omega_4 = 1: the step kernels use the UNIT collision
     int32_t tfs;      // transverse freestream at the y and z faces
     float tfs_blend;
 };
@@ -326,6 +326,13 @@ __host__ __device__ inline void cell_rates(T nu_eddy, T tau, T amr_scale, T nu_b
         const T lo = a_val < T(0.01f) ? T(0.01f) : a_val;
         omega4_diag = T(2) < lo ? T(2) : lo;
     }
+}
+
+// 27 words of LDS per lane for the rare branches of the two-cells-per-lane kernel (workgroups of 128 lanes;
+// word k of a lane at [k * 128 + lane]): one array for all of them
+__device__ __forceinline__ uint32_t* two_lds() {
+    __shared__ uint32_t words[27 * 128];
+    return words;
 }
 
 // Per-cell constants of the collision
@@ -612,10 +619,9 @@ __device__ __forceinline__ void collide_cell(T (&f)[27], const CellRates<T>& q, 
                            fmn(fmn(m9[6], m9[7]), m9[8]));
         if (fmin < T(0) && A[0] == A[0]) {
             if constexpr (LDS_LIMITER) {
-                __shared__ T lim[27][128];
-                const int t = threadIdx.x;
+                T* lim = (T*)two_lds() + threadIdx.x;
 #pragma unroll
-                for (int k = 0; k < 27; ++k) lim[k][t] = A[k];
+                for (int k = 0; k < 27; ++k) lim[k * 128] = A[k];
                 auto fe_of = [&](int k) {
                     return feq_auto(rb, uxe, uye, uze, wgt_rt<T>(k), T(k % 3 - 1), T((k / 3) % 3 - 1), T(k / 9 - 1), p.compressible);
                 };
@@ -623,17 +629,17 @@ __device__ __forceinline__ void collide_cell(T (&f)[27], const CellRates<T>& q, 
 #pragma unroll 1
                 for (int k = 0; k < 27; ++k) {
                     const T fe = fe_of(k);
-                    const T fn = lim[k][t] - fe;
+                    const T fn = lim[k * 128] - fe;
                     if (fn < T(0) && fe > T(1e-15f)) alpha = mn(alpha, fe / (fe - fn + T(1e-15f)));
                 }
                 alpha = mx(alpha, T(0));
 #pragma unroll 1
                 for (int k = 0; k < 27; ++k) {
                     const T fe = fe_of(k);
-                    lim[k][t] = fe + alpha * (lim[k][t] - fe);
+                    lim[k * 128] = fe + alpha * (lim[k * 128] - fe);
                 }
 #pragma unroll
-                for (int k = 0; k < 27; ++k) A[k] = lim[k][t];
+                for (int k = 0; k < 27; ++k) A[k] = lim[k * 128];
             } else {
                 T alpha = T(1);
 #pragma unroll

@@ -50,12 +50,12 @@ struct TwoRec {
     uint32_t block;
     uint32_t flags;            // BF_* and TR_*
     int32_t org[3];
-    int32_t lslot, sslot;      // link-mask and sponge slots
+    int32_t lslot, sslot, oslot;   // link-mask, sponge and outlet-copy slots
     int32_t ext[3];
     float u_in, omega1, omega4d, F[3], tau, amr_scale, force_scale;
     uint32_t cell0;
     uint32_t face[6];          // neighbour blocks x+, x-, y+, y-, z+, z- (WALE; absent: the block itself)
-    uint32_t pad[10];
+    uint32_t pad[9];
 };
 static_assert(sizeof(TwoRec) == 256, "a record is four cache lines of the scalar cache");
 enum : uint32_t {
@@ -111,7 +111,6 @@ struct StepArgs {
     const int32_t* ts_dev;
     int32_t ts_mul, ts_add;
     int32_t parity;              // AA pattern: 1 odd step (neighbour slots), 0 even step (own slots)
-    int32_t pipe_planes;         // planes per workgroup of the pipelined interior kernel (1 = off; divides 16)
     int32_t face_x;              // a domain of the level has the exact specular z wall, or the transverse freestream is on
     // interpolated bounce-back: per link-mask slot, [27][BS3] Float16 bits of the wall distance q of the
     // link from a cell along c_k (units of |c_k|); null = halfway bounce-back on every solid link

@@ -116,7 +116,7 @@ struct Level {
     std::vector<char> two_fit_h;       // a block's neighbours lie within that kernel's 32-bit offsets
     std::vector<int32_t> nbr_h;        // [32 * nb] neighbour rows (the device's nbr)
     uint32_t esize = 4;                // bytes of a stored population
-    bool two() const { return ab && fp32; }
+    bool two() const { return fp32; }
     DevBuf<int32_t> lslot;             // link-mask slot per block
     DevBuf<uint32_t> lmask;            // per-cell solid-link masks of blocks near solid cells
     std::vector<int32_t> lslot_h;      // host copy of lslot
@@ -239,10 +239,11 @@ struct FieldStage {
 
 struct OalPlan {
     int device = 0;
-    int pipe_planes = 4;   // planes per workgroup of the pipelined interior kernel
     bool overlap = true;   // boundary and face launches on the side stream
-    bool face_kernel = false;   // face cells by the face-cell kernel instead of rules in the pipelined one
-    int pair_kernel = 2;        // FP32 / 16-bit storage: regular blocks two cells per lane (1 one launch, 2 face blocks apart)
+    // launch-shape fields kept as the caller set them; no kernel reads them
+    int pipe_planes = 4;
+    bool face_kernel = false;
+    int pair_kernel = 2;
     int storage = OAL_F32;
     int stream_mode = OAL_STREAM_AB;
     int bb_mode = OAL_BB_HALFWAY;
@@ -305,7 +306,7 @@ void build_lists(Level& L, HostLevel& H) {
     for (auto* l : {&H.blist_tw, &H.blist_ts, &H.blist_tl, &H.blist_tn, &H.blist_xr, &H.blist_xb}) l->clear();
     L.regular_face = false;
     const std::vector<uint32_t>& flags = L.flags_h;
-    // blocks on a face whose rule the pipelined kernels do not apply (the exact specular z wall reads
+    // blocks on a face whose rule the two-cells kernel does not apply (the exact specular z wall reads
     // another cell of the wall row; the transverse freestream blends): the general kernels step them
     auto special_face = [&](uint32_t b, const DevDomain& dm) {
         bool lo[3], hi[3];
@@ -402,6 +403,7 @@ void build_two_recs(const Level& L, HostLevel& H, const std::vector<int32_t>& ss
             }
             r.lslot = L.lslot_h[b];
             r.sslot = sslot.empty() ? -1 : sslot[b];
+            r.oslot = H.oslot.empty() ? -1 : H.oslot[b];
             r.u_in = dm.u_in;
             r.omega1 = dm.omega1;
             r.omega4d = dm.omega4d;
@@ -600,7 +602,7 @@ int prepare_level(const OalLevelDesc& d, const OalCollision& coll, bool ab, bool
         }
         L.two_fit_h[b] = two_fits(lo, hi, (uint64_t)sbytes) ? 1 : 0;
     }
-    if (ab && fp32) L.nbr_h = H.nbr_bm;
+    if (fp32) L.nbr_h = H.nbr_bm;
     L.near_h = near;
     L.flags_h = flags;
     L.borg_h = borg;
@@ -1109,7 +1111,7 @@ int upload_level(OalPlan* p, Level& L, const HostLevel& H) {
     if (L.fpart.alloc((size_t)L.n_items * 4) != hipSuccess || L.mpart.alloc((size_t)nb * 4) != hipSuccess ||
         L.red_out.alloc((size_t)L.n_domains * 4) != hipSuccess || L.guard.alloc(1) != hipSuccess)
         return fail(OAL_ERR_NOMEM, "reduction buffer allocation failed");
-    // force partials start at zero: the pipelined interior kernel (no solid links) never writes them
+    // force partials start at zero: blocks without solid links never write them
     OAL_HIP(hipMemset(L.fpart.p, 0, (size_t)L.n_items * 4 * sizeof(double)));
     return OAL_OK;
 }
@@ -1161,7 +1163,6 @@ StepArgs make_args(OalPlan* p, Level& L, int32_t time_step, bool want_force) {
         a.ts_add = 0;
     }
     a.parity = p->stream_mode == OAL_STREAM_AA ? (L.aa_phase == 0 ? 1 : 0) : 0;
-    a.pipe_planes = p->pipe_planes;
     a.two = L.rec_tw.p;
     a.n_two = L.n_two;
     a.two_keep = 2ull * L.fA.n <= TWO_KEEP_BYTES ? 1 : 0;
@@ -1641,7 +1642,7 @@ int oal_plan_create(const OalPlanDesc* desc, OalPlan** out) {
             inactive.resize(o.nb());
             for (int b = 0; b < o.nb(); ++b) inactive[b] = o.status[b] != OCT_STEPPED;
         }
-        // the pipelined kernels cover FP32-arithmetic storage
+        // the two-cells kernel covers FP32-arithmetic storage
         const bool fp32 = desc->storage != OAL_F64;
         const int rc = prepare_level(d, desc->collision, desc->stream_mode == OAL_STREAM_AB, fp32, desc->bb_mode == OAL_BB_HALFWAY,
                                      storage_bytes(desc->storage), p->levels[l],

@@ -2,8 +2,7 @@
 // units oal_step_<storage>.hip so that the four storage forms compile in parallel.
 //
 // Work decomposition of the step kernels: one work-item per cell, one workgroup per 16 x 16 plane of
-// a 16^3 block (256 lanes = 4 wavefronts of 16 x 4 cells), or per several planes in the pipelined
-// kernels.  Populations are block-major: each block holds its 27 direction arrays of 4096 cells
+// a 16^3 block (256 lanes = 4 wavefronts of 16 x 4 cells).  Populations are block-major: each block holds its 27 direction arrays of 4096 cells
 // contiguously (pop_index), so the 64 lanes of a wavefront touch 4 consecutive 64-byte rows of each
 // of the block's direction arrays.  A workgroup's block, plane, domain and neighbour-block indices are
 // uniform, which keeps them in scalar registers.
@@ -25,27 +24,6 @@ __device__ __forceinline__ uint32_t xcd_item(uint32_t i, uint32_t n) {
     return x < r ? x * (q + 1u) + j : r * (q + 1u) + (x - r) * q + j;
 }
 
-// The list position and first plane of a pipelined workgroup (the grid holds n_blocks * groups
-// workgroups, groups = planes per block / planes per workgroup).  BLOCKS_FASTEST walks the blocks
-// fastest, so that x-neighbour blocks, which share the rows of each other's x-shifted accesses, run at
-// the same time on the same L2: on a 256^3 level the two-cells-per-lane FP32 kernel 627 -> 615 us and
-// the AA odd half-step's reads 1.14 -> 1.06 of the algorithmic bytes.  The others walk each block's
-// planes fastest (the WALE kernel 835 us against 859, the AA even half-step faster too).
-struct PipeItem {
-    uint32_t pos;
-    int z0;
-};
-template <bool BLOCKS_FASTEST>
-__device__ __forceinline__ PipeItem pipe_item(uint32_t groups, int np) {
-    const uint32_t litem = xcd_item(blockIdx.x, gridDim.x);
-    if constexpr (BLOCKS_FASTEST) {
-        const uint32_t nblk = gridDim.x / groups;
-        return PipeItem{litem % nblk, (int)(litem / nblk) * np};
-    } else {
-        return PipeItem{litem / groups, (int)(litem % groups) * np};
-    }
-}
-
 // how the population arriving in one direction is obtained
 enum : int {
     SRC_REG = 0,     // pulled from the source cell
@@ -61,7 +39,8 @@ enum : int {
 };
 
 // what a level needs beside the plain step in the two-cells-per-lane kernel
-enum : int { TWO_PLAIN = 0, TWO_SPONGE = 1, TWO_BFL = 2 };
+// (or which half-step of the AA pattern)
+enum : int { TWO_PLAIN = 0, TWO_SPONGE = 1, TWO_BFL = 2, TWO_AA_EVEN = 3, TWO_AA_ODD = 4 };
 
 enum : int { PAT_AB = 0, PAT_AA_EVEN = 1, PAT_AA_ODD = 2 };
 
@@ -687,95 +666,6 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(step_wa
     if (a.fpart) wg_sum3(F0 * dm->force_scale, F1 * dm->force_scale, F2 * dm->force_scale, a.fpart, item);
 }
 
-__device__ __forceinline__ void wait_all_vmem() {
-    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0), expcnt and lgkmcnt left open
-    __builtin_amdgcn_sched_barrier(0);
-}
-
-// The in-place AA pattern on the regular blocks (no domain face, no solid near; neighbour blocks at
-// lexicographic offsets), software-pipelined over z as k_step_pipe.  The even half-step reads each
-// population from the cell's own slot k and writes f*_k to its own slot opp k; the odd half-step reads
-// slot opp k of x - c_k and writes f*_k to slot k of x + c_k.  Either way a lane reads and writes the
-// same 27 slots and no other lane touches them, so the next plane's prefetch never meets a store of the
-// current plane.  The storage rounding of f*_k takes the bits of (cell, k, step) as in every pattern.
-// Register budget: one plane of populations in flight beside the collision of another; the odd
-// half-step's two-sided addressing and the 16-bit forms' conversions fit the 256 VGPRs of 2 waves per
-// SIMD only, the other forms the 168 of 3
-template <class SP, int PAT>
-constexpr int pipe_aa_waves() { return PAT == PAT_AA_ODD || SP::dithered ? 2 : 3; }
-
-template <class SP, int NP, int PAT, bool UNIT>
-__global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(pipe_aa_waves<SP, PAT>(), pipe_aa_waves<SP, PAT>())))
-k_step_pipe_aa(const StepArgs a) {
-    using T = typename SP::T;
-    using st = typename SP::st;
-    const int np = a.pipe_planes;   // (a run-time bound, as in k_step_pipe)
-    constexpr uint32_t groups = (uint32_t)(PLANES / NP);
-    const PipeItem it = pipe_item<PAT == PAT_AA_ODD>(groups, np);
-    const uint32_t b = (uint32_t)a.blist[it.pos];
-    const int z0 = it.z0;
-    CellCtx c;
-    c.b = b;
-    c.lx = threadIdx.x & (BS - 1);
-    c.ly = threadIdx.x >> 4;
-    c.z = z0;
-    c.own = b * BS3 + (uint32_t)z0 * BS2 + (uint32_t)c.ly * BS + (uint32_t)c.lx;
-    const DevDomain* dm = a.doms + a.bdom[b];
-    RegAddr<SP> ra;
-    ra.init(c, dm->nbx, dm->nby);
-    CellRates<T> q;
-    if constexpr (sizeof(T) == 8) { q.omega1 = dm->omega1_d; q.omega4_diag = dm->omega4d_d; }
-    else { q.omega1 = dm->omega1; q.omega4_diag = dm->omega4d; }
-    q.forced = dm->forced != 0;
-    q.Fx = T(dm->F[0]); q.Fy = T(dm->F[1]); q.Fz = T(dm->F[2]);
-    const uint32_t cell0 = dm->cell0;
-    const uint32_t key = SP::dithered ? round_key(a.step()) : 0u;
-    auto load = [&](int z, typename SP::raw (&r)[27]) {
-        for_dirs([&](auto kc) {
-            constexpr int K = decltype(kc)::value;
-            if constexpr (PAT == PAT_AA_EVEN)
-                r[K] = SP::ld_raw((const st*)(ra.base(a.fin, K, z, 0) + ra.v[1][1]));
-            else
-                r[K] = SP::ld_raw((const st*)(ra.base(a.fin, dopp(K), z, dcz(K)) + ra.v[dcx(K) + 1][dcy(K) + 1]));
-        });
-    };
-    auto collide = [&](int z, const typename SP::raw (&r)[27]) {
-        T f[27];
-        for_dirs([&](auto kc) {
-            constexpr int K = decltype(kc)::value;
-            f[K] = SP::from_raw(r[K], wgt<T>(K));
-        });
-        T rho_o, ux_o, uy_o, uz_o;
-        collide_cell<T, UNIT>(f, q, a.cp, rho_o, ux_o, uy_o, uz_o);
-        const bool dith = SP::dithered && a.cp.dither;
-        const uint32_t hc = SP::dithered ? round_cell(key, c.own + (uint32_t)(z - z0) * BS2 - cell0) : 0u;
-        for_dirs([&](auto kc) {
-            constexpr int K = decltype(kc)::value;
-            st* p;
-            if constexpr (PAT == PAT_AA_EVEN) p = (st*)(ra.base(a.fout, dopp(K), z, 0) + ra.v[1][1]);
-            else p = (st*)(ra.base(a.fout, K, z, -dcz(K)) + ra.v[1 - dcx(K)][1 - dcy(K)]);
-            SP::sto_r(p, f[K], wgt<T>(K), round_bits(hc, K), dith);
-        });
-    };
-    typename SP::raw fa[27], fb[27];
-    load(z0, fa);
-    for (int z = z0; z < z0 + np; z += 2) {
-        wait_all_vmem();
-        if (z + 1 < z0 + np) load(z + 1, fb);
-        collide(z, fa);
-        if (z + 1 >= z0 + np) break;
-        wait_all_vmem();
-        if (z + 2 < z0 + np) load(z + 2, fa);
-        collide(z + 1, fb);
-    }
-}
-
-template <class SP, int NP, int PAT>
-static void launch_pipe_aa(dim3 grid, hipStream_t s, const StepArgs& r) {
-    if (r.cp.unit) hipLaunchKernelGGL((k_step_pipe_aa<SP, NP, PAT, true>), grid, dim3(WG), 0, s, r);
-    else hipLaunchKernelGGL((k_step_pipe_aa<SP, NP, PAT, false>), grid, dim3(WG), 0, s, r);
-}
-
 // Face cells of the regular-list blocks (AB pattern): one lane per listed cell, the general path with
 // the domain-face rules.  These blocks hold no solid cell and no solid link, so no force is summed.
 template <class SP, bool WALE>
@@ -841,18 +731,17 @@ static void launch_boundary(const StepArgs& a, hipStream_t bs) {
 }
 
 // One step of a level: launches over disjoint block lists.
-//   AB pattern, FP32 arithmetic: the two-cells-per-lane kernel for every block but a few kinds, those on
-//     the one-plane boundary kernel.
-//   AB pattern, FP64, and the AA pattern: regular, other interior, regular boundary and boundary blocks,
-//     each on a kernel compiled for its own register budget, and in the AB pattern the face cells that the
-//     regular kernel skips.
+//   FP32 arithmetic: the two-cells-per-lane kernel for every block but a few kinds, those on the one-plane
+//     boundary kernel.
+//   FP64: regular, other interior, regular boundary and boundary blocks, each on a kernel compiled for its
+//     own register budget, and in the AB pattern the face cells that the regular kernel skips.
 // The boundary and face launches go to `side` (when given) so that they overlap the bulk launch; the
 // caller joins the two streams.
 template <class SP, int PAT, bool WALE>
 static hipError_t launch_pat(const StepArgs& a, hipStream_t stream, hipStream_t side, hipEvent_t bulk0, hipEvent_t bulk1) {
     hipStream_t bs = side ? side : stream;
     launch_boundary<SP, PAT, WALE>(a, bs);
-    constexpr bool two = PAT == PAT_AB && sizeof(typename SP::T) == 4;
+    constexpr bool two = sizeof(typename SP::T) == 4;
     if constexpr (PAT == PAT_AB && !two) {
         if (a.n_face) hipLaunchKernelGGL((k_face<SP, WALE>), dim3((a.n_face + WG - 1) / WG), dim3(WG), 0, bs, a);
     }
@@ -861,7 +750,9 @@ static hipError_t launch_pat(const StepArgs& a, hipStream_t stream, hipStream_t 
         if (e != hipSuccess) return e;
     }
     if constexpr (two) {
-        if (a.qmap) {   // interpolated bounce-back: its form of the kernel where there are solid links
+        if constexpr (PAT != PAT_AB) {
+            launch_two(SP::code, WALE, PAT == PAT_AA_EVEN ? TWO_AA_EVEN : TWO_AA_ODD, a.two, a.n_two, stream, a);
+        } else if (a.qmap) {   // interpolated bounce-back: its form of the kernel where there are solid links
             launch_two(SP::code, WALE, TWO_BFL, a.two_links, a.n_two_links, stream, a);
             launch_two(SP::code, WALE, TWO_PLAIN, a.two_free, a.n_two_free, stream, a);
         } else {
@@ -872,19 +763,7 @@ static hipError_t launch_pat(const StepArgs& a, hipStream_t stream, hipStream_t 
         StepArgs r = a;
         if (a.n_regular) {
             r.blist = a.blist_regular;
-            if constexpr (PAT != PAT_AB && !WALE && sizeof(typename SP::T) == 4) {
-                // the AA pattern's regular blocks (none on a domain face): pipelined over z, 2 to 8 planes
-                r.pipe_planes = a.pipe_planes > 8 ? 8 : a.pipe_planes;
-                const dim3 g(a.n_regular * (PLANES / (r.pipe_planes > 1 ? r.pipe_planes : 1)));
-                switch (r.pipe_planes) {
-                    case 2: launch_pipe_aa<SP, 2, PAT>(g, stream, r); break;
-                    case 4: launch_pipe_aa<SP, 4, PAT>(g, stream, r); break;
-                    case 8: launch_pipe_aa<SP, 8, PAT>(g, stream, r); break;
-                    default: hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_REGULAR>), g, dim3(WG), 0, stream, r); break;
-                }
-            } else {
-                hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_REGULAR>), dim3(a.n_regular * PLANES), dim3(WG), 0, stream, r);
-            }
+            hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_REGULAR>), dim3(a.n_regular * PLANES), dim3(WG), 0, stream, r);
         }
         if (a.n_interior) {
             r.blist = a.blist_interior;

@@ -1,4 +1,4 @@
-// The step kernel of the FP32-arithmetic forms in the AB pattern, two cells per lane; a
+// The step kernel of the FP32-arithmetic forms, two cells per lane; a
 // translation unit per storage form (oal_two_<storage>.hip).
 //
 // One workgroup of 128 lanes steps one 16 x 16 plane of a block; a lane steps the cells (2j, 2j + 1) of
@@ -19,6 +19,10 @@
 // (the own population k) replace one cell of a pair; the inlet equilibrium replaces A's value at x = 0
 // after decoding.
 //
+// AA pattern (one population buffer, two half-steps): the even one reads population k of a cell from its own
+// slot k and writes it to the own slot opp k; the odd one gathers from slot opp k of x - c_k and scatters to
+// slot k of x + c_k (two_scatter).  Both are one launch over every block.
+//
 // Bound and shape.  The plane's 27 words are all in flight together and nothing is kept for a next plane,
 // so a lane needs 97 to 125 registers and four waves share a SIMD; their loads overlap other waves'
 // collisions.  That needs the rare limiter out of the registers (collide_cell's LDS form): with it inline
@@ -32,6 +36,8 @@
 // of the row ends.  One record per block (TwoRec) in place of a chain of table reads: FP16 256^3 453 -> 372
 // us, 48 x 32 x 32 13.5 -> 10.8 us.  Stores written through at device scope: 48 x 32 x 32 10.8 -> 10.2 us,
 // WALE 100 x 60 x 44 25.3 -> 20.9 us without the non-temporal hint (which 256^3 needs: 635 against 681 us).
+// AA 192 x 160 x 160 FP32, sphere: 340 -> 204 us per step against a pipelined kernel for the blocks off the
+// faces and a one-plane kernel for the rest (a third of the blocks); 5.2 TB/s of the pair's 216 bytes per cell.
 #pragma once
 
 #include "oal_step.h"
@@ -162,11 +168,110 @@ __device__ __forceinline__ void two_sum3(double v0, double v1, double v2, double
 // Cache policy of the stores (gfx950's sc and nt bits): written through at device scope, so that the
 // kernel's end has no dirty lines to write back; non-temporal too where the level's two population buffers
 // exceed TWO_KEEP_BYTES (below that the next step reads them from the 256 MB memory-side cache).
-enum : int { TWO_ST_KEEP = 16, TWO_ST_STREAM = 18 };
+// The AA odd half-step's stores are ordinary ones: the words at the row ends are completed in the cache by
+// two workgroups (192 x 160 x 160 FP32: 204 us per step, 213 non-temporal, 271 written through).
+enum : int { TWO_ST_KEEP = 16, TWO_ST_STREAM = 18, TWO_ST_SCATTER = 0 };
+
+// The writes of the AA pattern's odd half-step: population K of a cell goes to slot K of x + c_K.  The word
+// a lane stores for direction K is the aligned pair of the row (y + cy, z + cz), whose two cells come from
+// its own pair and, for cx != 0, the neighbouring lane's; at the row ends one cell goes to the x-neighbour
+// block alone.  Where x + c_K does not step (beyond a face, solid), the rule of direction J = opp K is
+// evaluated from the fresh state and stored in the own slot J, which the even half-step reads; an inlet
+// link is left to the even half-step.  A lane's rows are its own in both passes, and of the words at the
+// row ends each workgroup reads and writes its own cells only, so no access meets another's.
+template <class SP, class REC, class WORD>
+__device__ __forceinline__ void two_scatter(const REC& R, __amdgpu_buffer_rsrc_t fo, int z, int jx, int ly, bool edge,
+                                            const TwoFaces& fc, uint32_t lf, uint32_t lma, uint32_t lmb, const WORD (&s)[27]) {
+    using W = Two<SP>;
+    constexpr uint32_t es = W::es, slot = BS3 * es;
+    constexpr int AUX = TWO_ST_SCATTER;
+    asm("" : "+v"(ly), "+v"(jx));   // the offsets are formed again here: kept from the gather they would cost 18 registers
+    const bool first = jx == 0, last = jx == 7;
+    const uint32_t own = R.off[13] + (uint32_t)ly * (BS * es) + (uint32_t)jx * (2 * es) + (uint32_t)z * (BS2 * es);
+    // the pair's offset in the row (y + cy, z + cz), and the x-neighbour block's cell next to the row's end
+    auto row_of = [&](int cy, int cz, uint32_t& v, uint32_t& e) {
+        const REC* p = &R;
+        asm("" : "+s"(p));   // (six offsets at a time: all 27 would spill the scalar registers)
+        auto boff = [&](int dx, int dy, int dz) -> uint32_t { return p->off[(dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)]; };
+        const int tz = z + cz;
+        const int dz = tz < 0 ? -1 : (tz >= BS ? 1 : 0);
+        const bool cross = cy > 0 ? ly == BS - 1 : (cy < 0 ? ly == 0 : false);
+        const uint32_t r = (uint32_t)((ly + cy) & (BS - 1)) * (BS * es) + (uint32_t)(tz & (BS - 1)) * (BS2 * es);
+        const uint32_t c0 = boff(0, 0, dz), c1 = boff(0, cy, dz), m0 = boff(-1, 0, dz), m1 = boff(-1, cy, dz), p0 = boff(1, 0, dz),
+                       p1 = boff(1, cy, dz);
+        v = (cross ? c1 : c0) + r + (uint32_t)jx * (2 * es);
+        e = (first ? (cross ? m1 : m0) + (BS - 1) * es : (cross ? p1 : p0)) + r;
+    };
+    // K: the cells whose x + c_K steps
+    uint32_t ra = (lf & LF_LIVE_A) ? 0x7ffffffu : 0u, rb = (lf & LF_LIVE_B) ? 0x7ffffffu : 0u;
+    const uint32_t la = ra, lb = rb;
+    const bool special = edge || (R.flags & BF_SOLID);
+    if (special) {
+        for_dirs([&](auto kc) {
+            constexpr int K = decltype(kc)::value, J = dopp(K);
+            int j;
+            const bool row = two_row_rule<J>(fc, j);
+            const bool xa = (dcx(K) < 0 && (lf & LF_INLET)) || (dcx(K) > 0 && (lf & LF_OUTLET_A));
+            const bool xb = dcx(K) > 0 && (lf & LF_OUTLET_B);
+            if (row || xa || ((lma >> J) & 1u)) ra &= ~(1u << K);
+            if (row || xb || ((lmb >> J) & 1u)) rb &= ~(1u << K);
+        });
+    }
+    // of the pair left and right of this one in the row
+    const uint32_t rl0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)rb, 0x111, 0xf, 0xf, true);
+    const uint32_t rr0 = (uint32_t)__builtin_amdgcn_mov_dpp((int)ra, 0x101, 0xf, 0xf, true);
+    const uint32_t rl = first ? 0u : rl0, rr = last ? 0u : rr0;
+    for_dirs([&](auto cc) {
+        constexpr int C = decltype(cc)::value;
+        if constexpr (C < 9) {
+            constexpr int cy = C % 3 - 1, cz = C / 3 - 1, K0 = 3 * C;   // directions (cx, cy, cz) = K0 + cx + 1
+            __builtin_amdgcn_sched_barrier(0);   // (the offsets of one row at a time)
+            uint32_t v, e;
+            row_of(cy, cz, v, e);
+            auto put = [&](const WORD& w, uint32_t lo, uint32_t hi, int k) {
+                if (lo & hi & 1u) W::template st2<AUX>(w, fo, v, (uint32_t)k * slot);
+                else if (lo & 1u) W::template st1<AUX>(W::a(w), fo, v, (uint32_t)k * slot);
+                else if (hi & 1u) W::template st1<AUX>(W::b(w), fo, v + es, (uint32_t)k * slot);
+            };
+            put(s[K0 + 1], ra >> (K0 + 1), rb >> (K0 + 1), K0 + 1);
+            put(W::from_left(s[K0 + 2], first, 0u), rl >> (K0 + 2), ra >> (K0 + 2), K0 + 2);
+            put(W::from_right(s[K0], last, 0u), rb >> K0, rr >> K0, K0);
+            // B to the +x block's cell 0, A to the -x block's cell 15
+            if (first ? (ra >> K0) & 1u : (last ? (rb >> (K0 + 2)) & 1u : 0u))
+                W::template st1<AUX>(first ? W::a(s[K0]) : W::b(s[K0 + 2]), fo, e + (first ? (uint32_t)K0 : (uint32_t)K0 + 2) * slot, 0);
+        }
+    });
+    // the rules' writes, one cell of the pairs after the other: its codes through LDS, a rolled loop over the
+    // directions that some lane needs (unrolled, the choices among the 27 words spill)
+    uint32_t wa = la & ~ra, wb = lb & ~rb;
+    if (lf & LF_INLET) wa &= ~0x1249249u;         // (directions with cx < 0: bits 0, 3, 6, ...)
+    if (special && __builtin_amdgcn_ballot_w64((wa | wb) != 0) != 0) {
+        uint32_t* lds = two_lds() + threadIdx.x;
+        for (int half = 0; half < 2; ++half) {
+            const uint32_t w = half ? wb : wa;
+            const bool outlet = (lf & (half ? LF_OUTLET_B : LF_OUTLET_A)) != 0;
+            for_dirs([&](auto kc) {
+                constexpr int K = decltype(kc)::value;
+                lds[K * TWG] = half ? W::b(s[K]) : W::a(s[K]);
+            });
+#pragma unroll 1
+            for (int k = 0; k < 27; ++k) {
+                const bool mine = (w >> k) & 1u;
+                if (__builtin_amdgcn_ballot_w64(mine) == 0) continue;
+                const int j = 26 - k, cx = k % 3 - 1, cyj = 1 - (k / 3) % 3, czj = 1 - k / 9;
+                const bool zf = (czj > 0 && fc.zl) || (czj < 0 && fc.zh), yf = (cyj > 0 && fc.yl) || (cyj < 0 && fc.yh);
+                const bool wall = (fc.zwall && zf) || (fc.ymin_wall && cyj > 0 && fc.yl);
+                // the rule of direction j: its own population, the opposite one (walls and solid links), the mirrors
+                const int src = outlet && cx > 0 ? j : (wall || !(zf || yf)) ? k : yf ? j - 6 * cyj : j - 18 * czj;
+                if (mine) W::template st1<AUX>(lds[src * TWG], fo, own + (uint32_t)half * es, (uint32_t)j * slot);
+            }
+        }
+    }
+}
 
 // DITH: stochastic rounding (the 16-bit forms)
-template <class SP, bool UNIT, bool WALE, int EXTRA, bool DITH>
-__global__ void __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(EXTRA == TWO_BFL || (EXTRA == TWO_SPONGE && !(UNIT && !WALE)) ? 3 : 4)))
+template <class SP, bool UNIT, bool WALE, int EXTRA, bool DITH, int PAT>
+__global__ void __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(PAT == PAT_AA_ODD && SP::dithered ? 2 : EXTRA == TWO_BFL || PAT == PAT_AA_ODD || (EXTRA == TWO_SPONGE && !(UNIT && !WALE)) ? 3 : 4)))
 k_step_two(const StepArgs a) {
     using W = Two<SP>;
     using word = typename W::word;
@@ -300,22 +405,29 @@ k_step_two(const StepArgs a) {
             v[k][i] = c + r + (uint32_t)jx * (2 * es);
             // row ends: direction (+1, cy, cz) from the -x block's cell 15 at j = 0, (-1, cy, cz) from the
             // +x block's cell 0 at j = 7 (slots 2 apart)
-            ve[k][i] = (first ? m + W::end_first + 2 * slot : p + W::end_last) + r;
+            ve[k][i] = (first ? m + W::end_first + (PAT == PAT_AA_ODD ? -2u * slot : 2 * slot) : p + W::end_last) + r;
         }
     }
+    // the slot direction K is read from: in the odd half-step of the AA pattern opp K of the source cell
+    constexpr auto rd = [](int k) { return (uint32_t)(PAT == PAT_AA_ODD ? dopp(k) : k); };
     word s[27];
     uint32_t e9[9];
 #pragma unroll
     for (int q = 0; q < 9; ++q) e9[q] = 0;
-    if (edge) {
+    if constexpr (PAT == PAT_AA_EVEN) {   // every population in the cell's own slot
+        for_dirs([&](auto kc) {
+            constexpr int K = decltype(kc)::value;
+            s[K] = W::ld2(fin, own0 + row, (uint32_t)K * slot + zown);
+        });
+    } else if (edge) {
         for_dirs([&](auto kc) {
             constexpr int K = decltype(kc)::value;
             constexpr int cy = dcy(K), cz = dcz(K);
-            uint32_t o = v[cz + 1][cy + 1] + (uint32_t)K * slot + zs[cz + 1];
+            uint32_t o = v[cz + 1][cy + 1] + rd(K) * slot + zs[cz + 1];
             if constexpr (cy != 0 || cz != 0) {
                 int j;
                 const bool face = two_row_rule<K>(fc, j);
-                o = face ? own0 + row + (uint32_t)j * slot + zown : o;
+                o = face ? own0 + row + rd(j) * slot + zown : o;
             }
             s[K] = W::ld2(fin, o, 0);
         });
@@ -323,14 +435,14 @@ k_step_two(const StepArgs a) {
         for_dirs([&](auto kc) {
             constexpr int K = decltype(kc)::value;
             constexpr int cy = dcy(K), cz = dcz(K);
-            s[K] = W::ld2(fin, v[cz + 1][cy + 1], (uint32_t)K * slot + zs[cz + 1]);
+            s[K] = W::ld2(fin, v[cz + 1][cy + 1], rd(K) * slot + zs[cz + 1]);
         });
     }
-    if (first || last) {
+    if (PAT != PAT_AA_EVEN && (first || last)) {
         for_dirs([&](auto kc) {
             constexpr int K = decltype(kc)::value;
             constexpr int cy = dcy(K), cz = dcz(K);
-            if constexpr (dcx(K) < 0) e9[K / 3] = W::lde(fin, ve[cz + 1][cy + 1] + (uint32_t)K * slot + zs[cz + 1]);
+            if constexpr (dcx(K) < 0) e9[K / 3] = W::lde(fin, ve[cz + 1][cy + 1] + rd(K) * slot + zs[cz + 1]);
         });
     }
 
@@ -400,11 +512,15 @@ k_step_two(const StepArgs a) {
             }
         });
     };
-    if (edge) sources(std::true_type{});
-    else sources(std::false_type{});
+    if constexpr (PAT != PAT_AA_EVEN) {
+        if (edge) sources(std::true_type{});
+        else sources(std::false_type{});
+    }
+    // AA pattern: the lane's row in the outlet copies (9 populations with cx = -1 per row, by (y, z))
+    const uint32_t ocopy = PAT == PAT_AB ? 0u : (uint32_t)R.oslot * (9 * BS2 * es) + (uint32_t)(ly * BS + z) * es;
     // second pass: solid links and the outlet, in waves that hold one
     const uint32_t links = lma | lmb;
-    if (__builtin_amdgcn_ballot_w64((links & 0x7ffffffu) != 0 || is(LF_OUTLET_A | LF_OUTLET_B)) != 0) {
+    if (PAT != PAT_AA_EVEN && __builtin_amdgcn_ballot_w64((links & 0x7ffffffu) != 0 || is(LF_OUTLET_A | LF_OUTLET_B)) != 0) {
         const bool xha = is(LF_OUTLET_A), xhb = is(LF_OUTLET_B);
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
@@ -415,8 +531,15 @@ k_step_two(const StepArgs a) {
                     const bool oa = dcx(K) < 0 && xha, ob = dcx(K) < 0 && xhb;
                     ra[K % 9] = 0;
                     rb[K % 9] = 0;
-                    if (((lma >> K) & 1u) || oa) ra[K % 9] = W::ld1(fin, own0 + row + zown + (oa ? (uint32_t)K : (uint32_t)dopp(K)) * slot);
-                    if (((lmb >> K) & 1u) || ob) rb[K % 9] = W::ld1(fin, own0 + row + es + zown + (ob ? (uint32_t)K : (uint32_t)dopp(K)) * slot);
+                    if constexpr (PAT == PAT_AB) {
+                        if (((lma >> K) & 1u) || oa) ra[K % 9] = W::ld1(fin, own0 + row + zown + (oa ? (uint32_t)K : (uint32_t)dopp(K)) * slot);
+                        if (((lmb >> K) & 1u) || ob) rb[K % 9] = W::ld1(fin, own0 + row + es + zown + (ob ? (uint32_t)K : (uint32_t)dopp(K)) * slot);
+                    } else {   // the outlet from the even half-step's copy
+                        if ((lma >> K) & 1u) ra[K % 9] = W::ld1(fin, own0 + row + zown + (uint32_t)K * slot);
+                        if ((lmb >> K) & 1u) rb[K % 9] = W::ld1(fin, own0 + row + es + zown + (uint32_t)K * slot);
+                        if (oa) ra[K % 9] = W::ld1(buf_at(a.obuf), ocopy + (uint32_t)(K / 3) * (BS2 * es));
+                        if (ob) rb[K % 9] = W::ld1(buf_at(a.obuf), ocopy + (uint32_t)(K / 3) * (BS2 * es));
+                    }
                 }
             });
             for_dirs([&](auto kc) {
@@ -527,22 +650,38 @@ k_step_two(const StepArgs a) {
     const __amdgpu_buffer_rsrc_t fo = buf_at((char*)a.fout + (size_t)R.base * blk);
     const uint32_t vown = own0 + row;
     const bool lva = is(LF_LIVE_A), lvb = is(LF_LIVE_B), both = lva && lvb;
-    auto store = [&](auto aux) {
-        constexpr int AUX = decltype(aux)::value;
-        if (both) {
+    if constexpr (PAT == PAT_AA_ODD) {
+        two_scatter<SP>(R, fo, z, jx, ly, edge, fc, lf, lma, lmb, s);
+    } else {
+        // (the even half-step writes population K to the own slot opp K)
+        constexpr auto wr = [](int k) { return (uint32_t)(PAT == PAT_AA_EVEN ? dopp(k) : k); };
+        auto store = [&](auto aux) {
+            constexpr int AUX = decltype(aux)::value;
+            if (both) {
+                for_dirs([&](auto kc) {
+                    constexpr int K = decltype(kc)::value;
+                    W::template st2<AUX>(s[K], fo, vown, wr(K) * slot + zown);
+                });
+            } else if (lva || lvb) {
+                for_dirs([&](auto kc) {
+                    constexpr int K = decltype(kc)::value;
+                    W::template st1<AUX>(lva ? W::a(s[K]) : W::b(s[K]), fo, vown + (lva ? 0u : es), wr(K) * slot + zown);
+                });
+            }
+        };
+        if (a.two_keep) store(std::integral_constant<int, TWO_ST_KEEP>{});
+        else store(std::integral_constant<int, TWO_ST_STREAM>{});
+    }
+    if constexpr (PAT == PAT_AA_EVEN) {
+        // the outlet row's populations with cx = -1, which the odd half-step's neighbours overwrite
+        if (is(LF_OUTLET_A | LF_OUTLET_B) && (is(LF_OUTLET_A) ? lva : lvb)) {
             for_dirs([&](auto kc) {
                 constexpr int K = decltype(kc)::value;
-                W::template st2<AUX>(s[K], fo, vown, (uint32_t)K * slot + zown);
-            });
-        } else if (lva || lvb) {
-            for_dirs([&](auto kc) {
-                constexpr int K = decltype(kc)::value;
-                W::template st1<AUX>(lva ? W::a(s[K]) : W::b(s[K]), fo, vown + (lva ? 0u : es), (uint32_t)K * slot + zown);
+                if constexpr (dcx(K) < 0)
+                    W::template st1<0>(is(LF_OUTLET_A) ? W::a(s[K]) : W::b(s[K]), buf_at(a.obuf), ocopy + (uint32_t)(K / 3) * (BS2 * es), 0);
             });
         }
-    };
-    if (a.two_keep) store(std::integral_constant<int, TWO_ST_KEEP>{});
-    else store(std::integral_constant<int, TWO_ST_STREAM>{});
+    }
     if constexpr (WALE) {
         float* vout = (float*)a.vel_out;
 #pragma unroll
@@ -557,30 +696,30 @@ k_step_two(const StepArgs a) {
 }
 
 // the blocks of one list, one plane per workgroup
-template <class SP, bool UNIT, bool DITH>
-static void launch_two_u(bool wale, int extra, dim3 g, hipStream_t s, const StepArgs& r) {
-    if (wale) {
-        if (extra == TWO_SPONGE) hipLaunchKernelGGL((k_step_two<SP, UNIT, true, TWO_SPONGE, DITH>), g, dim3(TWG), 0, s, r);
-        else if (extra == TWO_BFL) hipLaunchKernelGGL((k_step_two<SP, UNIT, true, TWO_BFL, DITH>), g, dim3(TWG), 0, s, r);
-        else hipLaunchKernelGGL((k_step_two<SP, UNIT, true, TWO_PLAIN, DITH>), g, dim3(TWG), 0, s, r);
-    } else {
-        if (extra == TWO_SPONGE) hipLaunchKernelGGL((k_step_two<SP, UNIT, false, TWO_SPONGE, DITH>), g, dim3(TWG), 0, s, r);
-        else if (extra == TWO_BFL) hipLaunchKernelGGL((k_step_two<SP, UNIT, false, TWO_BFL, DITH>), g, dim3(TWG), 0, s, r);
-        else hipLaunchKernelGGL((k_step_two<SP, UNIT, false, TWO_PLAIN, DITH>), g, dim3(TWG), 0, s, r);
-    }
+template <class SP, bool UNIT, bool DITH, bool WALE>
+static void launch_two_w(int extra, dim3 g, hipStream_t s, const StepArgs& r) {
+    if (extra == TWO_SPONGE) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_SPONGE, DITH, PAT_AB>), g, dim3(TWG), 0, s, r);
+    else if (extra == TWO_BFL) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_BFL, DITH, PAT_AB>), g, dim3(TWG), 0, s, r);
+    else if (extra == TWO_AA_EVEN) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_PLAIN, DITH, PAT_AA_EVEN>), g, dim3(TWG), 0, s, r);
+    else if (extra == TWO_AA_ODD) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_PLAIN, DITH, PAT_AA_ODD>), g, dim3(TWG), 0, s, r);
+    else hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_PLAIN, DITH, PAT_AB>), g, dim3(TWG), 0, s, r);
 }
 template <class SP>
 static void launch_two_sp(bool wale, int extra, const StepArgs& r, hipStream_t s) {
     const dim3 g(r.n_items);
-    auto go = [&](auto dith) {
-        if (r.cp.unit) launch_two_u<SP, true, decltype(dith)::value>(wale, extra, g, s, r);
-        else launch_two_u<SP, false, decltype(dith)::value>(wale, extra, g, s, r);
+    auto go = [&](auto unit, auto dith) {
+        if (wale) launch_two_w<SP, decltype(unit)::value, decltype(dith)::value, true>(extra, g, s, r);
+        else launch_two_w<SP, decltype(unit)::value, decltype(dith)::value, false>(extra, g, s, r);
+    };
+    auto rates = [&](auto dith) {
+        if (r.cp.unit) go(std::true_type{}, dith);
+        else go(std::false_type{}, dith);
     };
     if constexpr (SP::dithered) {
-        if (r.cp.dither) go(std::true_type{});
-        else go(std::false_type{});
+        if (r.cp.dither) rates(std::true_type{});
+        else rates(std::false_type{});
     } else {
-        go(std::false_type{});
+        rates(std::false_type{});
     }
 }
 
