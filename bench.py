@@ -581,12 +581,11 @@ def main(argv=None) -> int:
     ap.add_argument("--no-copy-bw", action="store_true", help="skip the copy-bandwidth reference measurement")
     ap.add_argument("--no-autotune", action="store_true", help="keep the default launch shape")
     ap.add_argument("--pipe-planes", type=int, default=None, choices=[1, 2, 4, 8, 16],
-                    help="fixed planes per workgroup of the bulk kernel (implies --no-autotune)")
+                    help="fixed, without effect on the kernels (implies --no-autotune)")
     ap.add_argument("--overlap", type=int, default=None, choices=[0, 1],
                     help="fixed: boundary launches on a second stream (1) or in order (0) (implies --no-autotune)")
     ap.add_argument("--face-kernel", type=int, default=None, choices=[0, 1],
-                    help="fixed: face cells by a separate kernel (1) or by the bulk kernel's rules (0) "
-                         "(implies --no-autotune)")
+                    help="fixed, without effect on the kernels (implies --no-autotune)")
     ap.add_argument("--validate", action="store_true",
                     help="accuracy run instead of the benchmark: Cd and L2(u) of FP32 / FP16 / BF16 vs FP64")
     ap.add_argument("--val-steps", type=int, default=20000)

@@ -195,8 +195,7 @@ typedef struct OalLevelInfo {
     int32_t n_interior;
     int32_t n_boundary_regular;
     int32_t n_boundary;
-    int32_t n_face_cells;    /* AB pattern: cells of regular blocks on a domain face (FP64: stepped by the
-                                face-cell kernel) */
+    int32_t n_face_cells;    /* AB pattern: cells of regular blocks on a domain face */
     int32_t n_ghost_blocks;  /* refined plans: blocks the library adds around the level (filled from
                                 the coarser level, not stepped; not part of n_blocks or n_cells) */
     int32_t n_covered_blocks;/* refined plans: blocks of n_blocks whose children exist (written by
@@ -393,11 +392,11 @@ int oal_copy_bandwidth(int device, int64_t bytes, int reps, double* gbs);
 /* Launch shape of the step kernels.  overlap: 1 = the boundary and face launches on a second stream,
  * concurrent with the bulk launch; 0 = every launch in order on the plan's stream.  pipe_planes,
  * face_kernel, pair_kernel: accepted and reported, without effect (with FP32 arithmetic one kernel, two
- * cells per lane and one plane per workgroup with the face rules in it, steps both patterns; FP64 steps
- * the face cells in their own kernel).  graph: 1 = oal_step on the plan's own stream (stream NULL) replays a hipGraph of one
- * (coarse) step, captured on first use for each arrangement of the levels' buffers, with the step index
- * read from device memory (a step that collects the force runs as ordinary launches); 0 = the host issues
- * every launch.  Refined plans start with graph 1, one-level plans with 0.  Setting the tuning drops
+ * cells per lane and one plane per workgroup with the face rules in it, steps both patterns; likewise one
+ * cell per lane in FP64 with the AB pattern).  graph: 1 = oal_step on the plan's own stream (stream NULL)
+ * replays a hipGraph of one (coarse) step, captured on first use for each arrangement of the levels'
+ * buffers, with the step index read from device memory (a step that collects the force runs as ordinary
+ * launches); 0 = the host issues every launch.  Refined plans start with graph 1, one-level plans with 0.  Setting the tuning drops
  * the captured graphs.  Every shape gives the same bits. */
 typedef struct {
     int32_t pipe_planes;

@@ -40,7 +40,7 @@ struct DevDomain {
     int32_t pad;
 };
 
-// All a workgroup of the two-cells-per-lane kernel reads about its block, one record per entry of a block
+// All a workgroup of a one-launch step kernel (k_step_two, k_step_one) reads about its block, one record per entry of a block
 // list: one round of scalar loads in place of a chain (list entry, block tables, domain).  Neighbour
 // offsets are in bytes of populations from the lowest block among the neighbours and the block (absent:
 // the block's own), so that 32 bits reach every one.
@@ -55,7 +55,9 @@ struct TwoRec {
     float u_in, omega1, omega4d, F[3], tau, amr_scale, force_scale;
     uint32_t cell0;
     uint32_t face[6];          // neighbour blocks x+, x-, y+, y-, z+, z- (WALE; absent: the block itself)
-    uint32_t pad[9];
+    uint32_t pad0;
+    double omega1_d, omega4d_d;   // FP64 form
+    uint32_t pad[4];
 };
 static_assert(sizeof(TwoRec) == 256, "a record is four cache lines of the scalar cache");
 enum : uint32_t {
@@ -85,8 +87,8 @@ struct StepArgs {
     const int32_t* blist_boundary_regular;  // [n_boundary_regular] boundary blocks with lexicographic neighbours
     const int32_t* blist_boundary;   // [n_boundary] the other blocks
     uint32_t n_regular, n_interior, n_boundary_regular, n_boundary;
-    // the two-cells-per-lane kernel's blocks (AB pattern, FP32 arithmetic; blist_boundary_regular and
-    // blist_boundary then hold the blocks it does not take): without sponge cells, with sponge cells, and
+    // the one-launch kernels' blocks (FP32 arithmetic, and FP64 in the AB pattern; blist_boundary_regular and
+    // blist_boundary then hold the blocks they do not take): without sponge cells, with sponge cells, and
     // the former split into those with solid links near and the others
     const TwoRec* rec;           // the records of this launch (set per launch)
     const TwoRec* two;
@@ -97,9 +99,6 @@ struct StepArgs {
     uint32_t n_two, n_two_sponge, n_two_links, n_two_free;
     const int32_t* lslot;        // [nb] link-mask slot of a block with solid cells near, -1 = none
     const uint32_t* lmask;       // [n_lslots * BS3] per cell: bit k source of direction k solid, bit 27 cell solid
-    const uint32_t* face_cells;  // [n_face] AB pattern: cells of regular-list blocks with a source outside the extent
-    uint32_t n_face;
-    int32_t regular_face;        // AB pattern: the blocks of this launch may lie on a domain face (set per launch)
     const int32_t* oslot;        // [nb] AA pattern: outlet side-buffer slot of the block, -1 = none
     void* obuf;                  // [n_oslots * 9 * BS2] AA pattern: outlet-face populations with cx = -1
     uint32_t ncell;              // cells of the level (the stride of the velocity fields' components)
@@ -172,6 +171,8 @@ void launch_two_f16s(bool wale, int extra, const StepArgs& a, hipStream_t stream
 void launch_two_bf16s(bool wale, int extra, const StepArgs& a, hipStream_t stream);
 // and over the n blocks of a list, by storage code
 void launch_two(int storage, bool wale, int extra, const TwoRec* rec, uint32_t n, hipStream_t stream, const StepArgs& a);
+// the one-cell-per-lane FP64 step kernel over n records: oal_one_f64.hip
+void launch_one_f64(bool wale, const TwoRec* rec, uint32_t n, const StepArgs& a, hipStream_t stream);
 hipError_t launch_copy16(const void* src, void* dst, size_t bytes, hipStream_t stream);
 // Host arrays of init / conversion / macro output cover the first nhost cells of a level (the caller's
 // blocks); the device arrays have ncell cells per direction.

@@ -104,10 +104,8 @@ struct Level {
     uint32_t n_br_solid = 0;   // regular boundary blocks whose only flag is BF_SOLID
     uint32_t n_partial = 0;            // regular blocks that overhang the extent, no solid near (AB)
     uint32_t n_sponge = 0;             // regular blocks with sponge cells, no solid near (AB)
-    DevBuf<uint32_t> face_cells;       // AB: face cells of the regular-list blocks
-    uint32_t n_face = 0;
-    bool regular_face = false;         // AB: the regular list holds blocks on a domain face
-    // the two-cells-per-lane kernel's blocks (AB pattern, FP32 arithmetic): without and with sponge cells,
+    uint32_t n_face = 0;               // AB: face cells of the regular-list blocks
+    // the one-launch kernels' blocks (FP32 arithmetic, and FP64 in the AB pattern): without and with sponge cells,
     // the former also split by solid links near (interpolated bounce-back); the boundary blocks it does not
     // take, with and without lexicographic neighbours
     DevBuf<TwoRec> rec_tw, rec_ts, rec_tl, rec_tn;
@@ -116,7 +114,7 @@ struct Level {
     std::vector<char> two_fit_h;       // a block's neighbours lie within that kernel's 32-bit offsets
     std::vector<int32_t> nbr_h;        // [32 * nb] neighbour rows (the device's nbr)
     uint32_t esize = 4;                // bytes of a stored population
-    bool two() const { return fp32; }
+    bool two() const { return fp32 || ab; }
     DevBuf<int32_t> lslot;             // link-mask slot per block
     DevBuf<uint32_t> lmask;            // per-cell solid-link masks of blocks near solid cells
     std::vector<int32_t> lslot_h;      // host copy of lslot
@@ -193,7 +191,7 @@ struct Level {
         nbr.release(); borg.release(); bdom.release(); dom_item0.release(); dom_block0.release();
         bflags.release(); solid.release(); doms.release(); fA.release(); fB.release(); velA.release(); velB.release();
         rec_tw.release(); rec_ts.release(); rec_tl.release(); rec_tn.release(); blist_xr.release(); blist_xb.release();
-        fpart.release(); mpart.release(); red_out.release(); guard.release(); oslot.release(); obuf.release(); blist_rg.release(); blist_in.release(); blist_br.release(); blist_bd.release(); face_cells.release();
+        fpart.release(); mpart.release(); red_out.release(); guard.release(); oslot.release(); obuf.release(); blist_rg.release(); blist_in.release(); blist_br.release(); blist_bd.release();
         c8map_d.release(); lslot.release(); lmask.release(); qmap.release(); sponge.release(); sslot.release();
         g_src.release(); g_dst.release(); g_slot.release(); g_w.release(); g_m.release();
         r_src.release(); r_dst.release(); r_slot.release(); r_w.release(); r_m.release();
@@ -292,7 +290,6 @@ struct HostLevel {
         blist_tw, blist_ts, blist_tl, blist_tn, blist_xr, blist_xb, lslot;
     std::vector<TwoRec> rec_tw, rec_ts, rec_tl, rec_tn;
     std::vector<uint32_t> lmask;
-    std::vector<uint32_t> face_cells;
     int32_t n_oslots = 0;
     std::vector<uint32_t> flags;
     std::vector<uint8_t> solid;
@@ -301,10 +298,9 @@ struct HostLevel {
 // The block lists of a level's step kernels from its block flags (L.flags_h) and the host tables kept
 // for that purpose; rebuilt when the flags change (a sponge field marks its blocks).
 void build_lists(Level& L, HostLevel& H) {
-    H.blist_rg.clear(); H.blist_in.clear(); H.blist_br.clear(); H.blist_bd.clear(); H.face_cells.clear();
-    L.n_partial = L.n_sponge = 0;
+    H.blist_rg.clear(); H.blist_in.clear(); H.blist_br.clear(); H.blist_bd.clear();
+    L.n_partial = L.n_sponge = L.n_face = 0;
     for (auto* l : {&H.blist_tw, &H.blist_ts, &H.blist_tl, &H.blist_tn, &H.blist_xr, &H.blist_xb}) l->clear();
-    L.regular_face = false;
     const std::vector<uint32_t>& flags = L.flags_h;
     // blocks on a face whose rule the two-cells kernel does not apply (the exact specular z wall reads
     // another cell of the wall row; the transverse freestream blends): the general kernels step them
@@ -323,11 +319,13 @@ void build_lists(Level& L, HostLevel& H) {
         if (flags[b] & BF_INACTIVE) continue;   // never stepped
         const bool regular = L.regular_h[b] != 0;
         const bool special = (flags[b] & BF_EDGE) && special_face(b, dm);
-        // the two-cells-per-lane kernel takes every block but those with an absent neighbour inside the
+        // the one-launch kernels take every block but those with an absent neighbour inside the
         // extent, those under the exact specular z wall or the transverse freestream, those near solid
-        // cells with the reference's reflection, and those whose neighbours its 32-bit offsets do not span
+        // cells with the reference's reflection, and those whose neighbours their 32-bit offsets do not span
         // (4 GiB of populations: the wraps of periodic levels and the ghosts of octree levels beyond that)
-        if ((flags[b] & BF_MISSING) || special || !L.two_fit_h[b] || ((flags[b] & BF_SOLID) && !L.bb_halfway)) {
+        // (the FP64 form has none with a sponge)
+        if ((flags[b] & BF_MISSING) || special || !L.two_fit_h[b] || ((flags[b] & BF_SOLID) && !L.bb_halfway) ||
+            (!L.fp32 && (flags[b] & BF_SPONGE))) {
             (regular ? H.blist_xr : H.blist_xb).push_back((int32_t)b);
         } else if (flags[b] & BF_SPONGE) {
             H.blist_ts.push_back((int32_t)b);
@@ -338,10 +336,8 @@ void build_lists(Level& L, HostLevel& H) {
         if (flags[b] == 0) {
             (regular ? H.blist_rg : H.blist_in).push_back((int32_t)b);
         } else if (L.ab && regular && flags[b] == BF_EDGE && !special) {
-            // AB pattern: a whole block on a domain face, no solid near, joins the regular list; the
-            // cells on its faces (sources outside the extent) go to the face-cell list
+            // AB pattern: a whole block on a domain face, no solid near, counts as regular
             H.blist_rg.push_back((int32_t)b);
-            L.regular_face = true;
             const int o[3] = {L.borg_h[3 * b], L.borg_h[3 * b + 1], L.borg_h[3 * b + 2]};
             bool lo[3], hi[3];
             for (int a = 0; a < 3; ++a) {
@@ -354,7 +350,7 @@ void build_lists(Level& L, HostLevel& H) {
                         const int l[3] = {x, y, z};
                         bool face = false;
                         for (int a = 0; a < 3; ++a) face = face || (lo[a] && l[a] == 0) || (hi[a] && l[a] == BS - 1);
-                        if (face) H.face_cells.push_back(b * BS3 + (uint32_t)(x + BS * (y + BS * z)));
+                        L.n_face += face ? 1u : 0u;
                     }
         } else if (L.ab && L.fp32 && regular && flags[b] == (BF_EDGE | BF_PARTIAL) && L.near_h[L.bdom_h[b]] && !special) {
             ++L.n_partial;
@@ -366,7 +362,6 @@ void build_lists(Level& L, HostLevel& H) {
         }
     }
     L.n_br_solid = (uint32_t)std::count_if(H.blist_br.begin(), H.blist_br.end(), [&](int32_t b) { return flags[b] == BF_SOLID; });
-    L.n_face = (uint32_t)H.face_cells.size();
     L.n_regular = (uint32_t)H.blist_rg.size();
     L.n_interior = (uint32_t)H.blist_in.size();
     L.n_boundary_regular = (uint32_t)H.blist_br.size();
@@ -377,9 +372,11 @@ void build_lists(Level& L, HostLevel& H) {
     L.n_two_free = (uint32_t)H.blist_tn.size();
     L.n_rest_regular = (uint32_t)H.blist_xr.size();
     L.n_rest = (uint32_t)H.blist_xb.size();
+    // FP64 with interpolated bounce-back: the general kernel steps the blocks with solid links too
+    if (!L.fp32) H.blist_xb.insert(H.blist_xb.end(), H.blist_tl.begin(), H.blist_tl.end());
 }
 
-// The records of the two-cells-per-lane kernel's block lists; slot: the sponge slots (empty: none)
+// The records of the one-launch kernels' block lists; slot: the sponge slots (empty: none)
 void build_two_recs(const Level& L, HostLevel& H, const std::vector<int32_t>& sslot) {
     auto make = [&](const std::vector<int32_t>& list, std::vector<TwoRec>& out) {
         out.assign(list.size(), TwoRec{});
@@ -407,6 +404,8 @@ void build_two_recs(const Level& L, HostLevel& H, const std::vector<int32_t>& ss
             r.u_in = dm.u_in;
             r.omega1 = dm.omega1;
             r.omega4d = dm.omega4d;
+            r.omega1_d = dm.omega1_d;
+            r.omega4d_d = dm.omega4d_d;
             r.tau = dm.tau;
             r.amr_scale = dm.amr_scale;
             r.force_scale = dm.force_scale;
@@ -602,7 +601,7 @@ int prepare_level(const OalLevelDesc& d, const OalCollision& coll, bool ab, bool
         }
         L.two_fit_h[b] = two_fits(lo, hi, (uint64_t)sbytes) ? 1 : 0;
     }
-    if (fp32) L.nbr_h = H.nbr_bm;
+    if (fp32 || ab) L.nbr_h = H.nbr_bm;
     L.near_h = near;
     L.flags_h = flags;
     L.borg_h = borg;
@@ -1090,7 +1089,7 @@ int upload_level(OalPlan* p, Level& L, const HostLevel& H) {
         (rc = upload(L.blist_br, H.blist_br)) || (rc = upload(L.blist_bd, H.blist_bd)) ||
         (rc = upload(L.rec_tw, H.rec_tw)) || (rc = upload(L.rec_ts, H.rec_ts)) || (rc = upload(L.rec_tl, H.rec_tl)) ||
         (rc = upload(L.rec_tn, H.rec_tn)) || (rc = upload(L.blist_xr, H.blist_xr)) || (rc = upload(L.blist_xb, H.blist_xb)) ||
-        (rc = upload(L.lslot, H.lslot)) || (rc = upload(L.lmask, H.lmask)) || (rc = upload(L.face_cells, H.face_cells)))
+        (rc = upload(L.lslot, H.lslot)) || (rc = upload(L.lmask, H.lmask)))
         return rc;
     if (p->stream_mode == OAL_STREAM_AA) {
         if ((rc = upload(L.oslot, H.oslot))) return rc;
@@ -1142,9 +1141,6 @@ StepArgs make_args(OalPlan* p, Level& L, int32_t time_step, bool want_force) {
     a.n_boundary = L.n_boundary;
     a.lslot = L.lslot.p;
     a.lmask = L.lmask.p;
-    a.face_cells = L.face_cells.p;
-    a.n_face = L.n_face;
-    a.regular_face = L.regular_face ? 1 : 0;
     a.face_x = p->cp.tfs ? 1 : 0;
     for (const DevDomain& dm : L.doms_h) a.face_x |= dm.zwall == 1 ? 1 : 0;
     a.obuf = L.obuf.p;
@@ -1176,7 +1172,7 @@ StepArgs make_args(OalPlan* p, Level& L, int32_t time_step, bool want_force) {
         a.blist_boundary_regular = L.blist_xr.p;
         a.n_boundary_regular = L.n_rest_regular;
         a.blist_boundary = L.blist_xb.p;
-        a.n_boundary = L.n_rest;
+        a.n_boundary = L.n_rest + (!L.fp32 && L.qmap.p ? L.n_two_links : 0);
     }
     a.qmap = L.qmap.p;
     a.sponge = L.has_sponge ? L.sponge.p : nullptr;
@@ -1195,10 +1191,10 @@ int level_step(OalPlan* p, int level, int32_t time_step, int flags, hipStream_t 
     const bool want_force = (flags & OAL_STEP_FORCE) != 0;
     if (want_force && !L.has_solid) return fail(OAL_ERR_STATE, "force requested on a level without obstacle cells");
     StepArgs a = make_args(p, L, time_step, want_force);
-    // side-stream work: boundary blocks, face cells and the blocks that overhang the extent
+    // side-stream work: the boundary lists
     const bool split = p->overlap && (L.two() ? a.n_two + a.n_two_sponge > 0 && a.n_boundary_regular + a.n_boundary > 0
                                               : L.n_regular + L.n_interior > 0 &&
-                                                    L.n_boundary_regular + L.n_boundary + L.n_face > 0);
+                                                    L.n_boundary_regular + L.n_boundary > 0);
     if (split) {
         // fork: the side stream starts after everything queued on s, then s waits for the side stream
         OAL_HIP(hipEventRecord(p->fork, s));
@@ -2283,7 +2279,7 @@ static int set_sponge_lib(OalPlan* p, int level, const float* sponge, int32_t bl
         (rc = re(L.blist_br, H.blist_br)) || (rc = re(L.blist_bd, H.blist_bd)) ||
        
         (rc = re(L.rec_tw, H.rec_tw)) || (rc = re(L.rec_ts, H.rec_ts)) || (rc = re(L.rec_tl, H.rec_tl)) ||
-        (rc = re(L.rec_tn, H.rec_tn)) || (rc = re(L.blist_xr, H.blist_xr)) || (rc = re(L.blist_xb, H.blist_xb)) || (rc = re(L.face_cells, H.face_cells)) ||
+        (rc = re(L.rec_tn, H.rec_tn)) || (rc = re(L.blist_xr, H.blist_xr)) || (rc = re(L.blist_xb, H.blist_xb)) ||
         (rc = re(L.sponge, vals)) || (rc = re(L.sslot, slot)))
         return rc;
     L.has_sponge = !vals.empty();

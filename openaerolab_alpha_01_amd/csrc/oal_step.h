@@ -171,34 +171,6 @@ struct RegAddr {
     }
 };
 
-// Faces of non-periodic axes that a block of the regular list touches.  Such blocks are whole (not
-// partial), so a face is where the block's origin is 0 or its far side is the extent.  Cells on a face
-// have sources outside the extent: the one-plane regular kernel skips them and the face-cell kernel steps
-// them (FP64).
-struct FaceBits {
-    bool xlo, xhi, ylo, yhi, zlo, zhi;
-};
-
-__device__ __forceinline__ FaceBits face_bits(const StepArgs& a, uint32_t b, const DevDomain* dm) {
-    const int ox = a.borg[3 * b], oy = a.borg[3 * b + 1], oz = a.borg[3 * b + 2];
-    FaceBits f;
-    f.xlo = !dm->per[0] && ox == 0;
-    f.xhi = !dm->per[0] && ox + BS == dm->ext[0];
-    f.ylo = !dm->per[1] && oy == 0;
-    f.yhi = !dm->per[1] && oy + BS == dm->ext[1];
-    f.zlo = !dm->per[2] && oz == 0;
-    f.zhi = !dm->per[2] && oz + BS == dm->ext[2];
-    return f;
-}
-
-__device__ __forceinline__ bool face_lane(const FaceBits& f, int lx, int ly) {
-    return (f.xlo && lx == 0) || (f.xhi && lx == BS - 1) || (f.ylo && ly == 0) || (f.yhi && ly == BS - 1);
-}
-
-__device__ __forceinline__ bool face_plane(const FaceBits& f, int z) {
-    return (f.zlo && z == 0) || (f.zhi && z == BS - 1);
-}
-
 // Population J of this cell's own post-collision state of the previous step: slot (x, J) after an
 // AB step, slot (x, opp J) after an AA even step.
 template <class SP, int PAT, int J>
@@ -643,14 +615,7 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(step_wa
     double F0 = 0.0, F1 = 0.0, F2 = 0.0;
     c.lmask = 0;
     if constexpr (SEL == SEL_REGULAR) {
-        bool live = true;
-        if constexpr (PAT == PAT_AB) {
-            if (a.regular_face) {
-                const FaceBits fb = face_bits(a, b, dm);
-                live = !(face_lane(fb, c.lx, c.ly) || face_plane(fb, c.z));
-            }
-        }
-        step_cell<SP, PAT, WALE, false, true>(a, c, dm, live, false, F0, F1, F2);
+        step_cell<SP, PAT, WALE, false, true>(a, c, dm, true, false, F0, F1, F2);
     } else if constexpr (SEL == SEL_INTERIOR) {
         step_cell<SP, PAT, WALE, false>(a, c, dm, true, false, F0, F1, F2);
     } else {
@@ -664,33 +629,6 @@ __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(step_wa
             step_cell<SP, PAT, WALE, true, false, BFL, SPONGE, FX>(a, c, dm, active, solid_own, F0, F1, F2);
     }
     if (a.fpart) wg_sum3(F0 * dm->force_scale, F1 * dm->force_scale, F2 * dm->force_scale, a.fpart, item);
-}
-
-// Face cells of the regular-list blocks (AB pattern): one lane per listed cell, the general path with
-// the domain-face rules.  These blocks hold no solid cell and no solid link, so no force is summed.
-template <class SP, bool WALE>
-__global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(step_waves<SP, PAT_AB, WALE>()))) k_face(const StepArgs a) {
-    const uint32_t i = blockIdx.x * WG + threadIdx.x;
-    if (i >= a.n_face) return;
-    const uint32_t own = a.face_cells[i];
-    const uint32_t b = own / BS3, loc = own % BS3;
-    CellCtx c;
-    c.b = b;
-    c.own = own;
-    c.lx = (int)(loc & (BS - 1));
-    c.ly = (int)((loc >> 4) & (BS - 1));
-    c.z = (int)(loc >> 8);
-    c.flags = a.bflags[b];
-    const DevDomain* dm = a.doms + a.bdom[b];
-    c.ext0 = dm->ext[0]; c.ext1 = dm->ext[1]; c.ext2 = dm->ext[2];
-    c.per0 = dm->per[0]; c.per1 = dm->per[1]; c.per2 = dm->per[2];
-    c.zwall = dm->zwall; c.ymin_wall = dm->ymin_wall;
-    c.gx = a.borg[3 * b] + c.lx;
-    c.gy = a.borg[3 * b + 1] + c.ly;
-    c.gz = a.borg[3 * b + 2] + c.z;
-    c.lmask = 0;
-    double F0 = 0.0, F1 = 0.0, F2 = 0.0;
-    step_cell<SP, PAT_AB, WALE, true>(a, c, dm, true, false, F0, F1, F2);
 }
 
 // the boundary lists on the one-plane kernel
@@ -733,18 +671,16 @@ static void launch_boundary(const StepArgs& a, hipStream_t bs) {
 // One step of a level: launches over disjoint block lists.
 //   FP32 arithmetic: the two-cells-per-lane kernel for every block but a few kinds, those on the one-plane
 //     boundary kernel.
-//   FP64: regular, other interior, regular boundary and boundary blocks, each on a kernel compiled for its
-//     own register budget, and in the AB pattern the face cells that the regular kernel skips.
-// The boundary and face launches go to `side` (when given) so that they overlap the bulk launch; the
+//   FP64, AB pattern: likewise the one-cell-per-lane kernel.
+//   FP64, AA pattern: regular, other interior, regular boundary and boundary blocks, each on a kernel
+//     compiled for its own register budget.
+// The boundary launches go to `side` (when given) so that they overlap the bulk launch; the
 // caller joins the two streams.
 template <class SP, int PAT, bool WALE>
 static hipError_t launch_pat(const StepArgs& a, hipStream_t stream, hipStream_t side, hipEvent_t bulk0, hipEvent_t bulk1) {
     hipStream_t bs = side ? side : stream;
     launch_boundary<SP, PAT, WALE>(a, bs);
     constexpr bool two = sizeof(typename SP::T) == 4;
-    if constexpr (PAT == PAT_AB && !two) {
-        if (a.n_face) hipLaunchKernelGGL((k_face<SP, WALE>), dim3((a.n_face + WG - 1) / WG), dim3(WG), 0, bs, a);
-    }
     if (bulk0) {
         const hipError_t e = hipEventRecord(bulk0, stream);
         if (e != hipSuccess) return e;
@@ -759,6 +695,9 @@ static hipError_t launch_pat(const StepArgs& a, hipStream_t stream, hipStream_t 
             launch_two(SP::code, WALE, TWO_PLAIN, a.two, a.n_two, stream, a);
             launch_two(SP::code, WALE, TWO_SPONGE, a.two_sponge, a.n_two_sponge, stream, a);
         }
+    } else if constexpr (PAT == PAT_AB) {   // (with interpolated bounce-back the boundary lists hold the links)
+        if (a.qmap) launch_one_f64(WALE, a.two_free, a.n_two_free, a, stream);
+        else launch_one_f64(WALE, a.two, a.n_two, a, stream);
     } else {
         StepArgs r = a;
         if (a.n_regular) {

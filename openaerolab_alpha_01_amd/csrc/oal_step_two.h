@@ -134,6 +134,18 @@ struct TwoFaces {
     bool zl, zh;            // uniform: the plane lies on the z-min / z-max face
     bool zwall, ymin_wall;  // no-slip variants of the z faces and of the y-min face
 };
+template <class REC>
+__device__ __forceinline__ TwoFaces two_faces(const REC& R, uint32_t flags, int gy, int gz) {
+    const bool py = (flags & TR_PER_Y) != 0, pz = (flags & TR_PER_Z) != 0;
+    TwoFaces fc;
+    fc.yl = !py && gy == 0;
+    fc.yh = !py && gy == R.ext[1] - 1;
+    fc.zl = !pz && gz == 0;
+    fc.zh = !pz && gz == R.ext[2] - 1;
+    fc.zwall = (flags & TR_ZWALL) != 0;
+    fc.ymin_wall = (flags & TR_YMIN) != 0;
+    return fc;
+}
 // a lane's cells: on the inlet (A), on the outlet, stepped (inside the extent and not solid)
 enum : uint32_t { LF_INLET = 1, LF_OUTLET_A = 2, LF_OUTLET_B = 4, LF_LIVE_A = 8, LF_LIVE_B = 16 };
 // is the source of direction K beyond a y or z face, and which own population does the rule take
@@ -303,13 +315,8 @@ k_step_two(const StepArgs a) {
     uint32_t lf = LF_LIVE_A | LF_LIVE_B;
     if (edge) {
         const int gy = oy + ly, ga = ox + 2 * jx;
-        const bool px = (flags & TR_PER_X) != 0, py = (flags & TR_PER_Y) != 0, pz = (flags & TR_PER_Z) != 0;
-        fc.yl = !py && gy == 0;
-        fc.yh = !py && gy == R.ext[1] - 1;
-        fc.zl = !pz && gz == 0;
-        fc.zh = !pz && gz == R.ext[2] - 1;
-        fc.zwall = (flags & TR_ZWALL) != 0;
-        fc.ymin_wall = (flags & TR_YMIN) != 0;
+        const bool px = (flags & TR_PER_X) != 0;
+        fc = two_faces(R, flags, gy, gz);
         lf = !px && ga == 0 ? LF_INLET : 0u;
         lf |= !px && ga == R.ext[0] - 1 ? LF_OUTLET_A : 0u;
         lf |= !px && ga + 1 == R.ext[0] - 1 ? LF_OUTLET_B : 0u;

@@ -1,4 +1,4 @@
-"""The two-cells-per-lane step kernel (both patterns) at the extents where its pairs, row ends and rules
+"""The two-cells-per-lane step kernel (both patterns) and the FP64 one at the extents where pairs, row ends and rules
 can go wrong, against the oracle bit for bit."""
 import numpy as np
 import pytest
@@ -50,4 +50,26 @@ def test_two_cells_per_lane(oracle, storage, case, stream):
         got = plan.download_f(dtype=np.float32 if storage == "f32" else np.float64)
         want = f_or if storage == "f32" else oracle.to_unshifted(storage, f_or)
         assert np.array_equal(got[..., live], want[..., live])
+    plan.close()
+
+
+@pytest.mark.parametrize("limiter", [1, 2])
+@pytest.mark.parametrize("case", list(CASES))
+def test_one_cell_per_lane_fp64(oracle, case, limiter):
+    """The FP64 kernel (AB pattern) on the same extents, without and with the positivity limiter's form."""
+    cfg = CASES[case]
+    grid = uniform_grid(cfg["n"], periodic=cfg.get("periodic", (False, False, False)))
+    if "solid" in cfg:
+        grid.solid = sphere_mask(grid, *cfg["solid"])
+    okw = dict(cfg["okw"], limiter=limiter)
+    rho, u = fields(grid, seed=29, u0=(okw.get("u_inlet", 0.0), 0, 0))
+    force_steps = (2,) if "solid" in cfg else ()
+    f_or, forces, _ = oracle_run(oracle, grid, "f64", 3, okw, rho, u, force_steps=force_steps)
+    plan = gpu_plan(grid, "f64", okw)
+    plan.init_equilibrium(rho, u)
+    for t in range(3):
+        plan.level_step(0, t, force=t in force_steps)
+    if force_steps:
+        np.testing.assert_allclose(plan.force()[0], forces[0], rtol=1e-11, atol=1e-14)
+    compare(oracle, plan, "f64", f_or, grid)
     plan.close()
