@@ -92,6 +92,15 @@ __host__ __device__ __forceinline__ size_t pop_index(uint32_t cell, int k) {
     return ((size_t)(cell >> 12) * 27u + (size_t)k) * 4096u + (cell & 4095u);
 }
 
+// a constant held in a vector register: FP32 instructions that read vector registers and literals only issue
+// every second cycle, with a scalar register among the operands every fourth (measured: 2.7 against 4.4
+// cycles per wave), and one literal is all that an instruction takes
+__device__ __forceinline__ float in_vgpr(float x) {
+    asm("" : "+v"(x));
+    return x;
+}
+constexpr int dnorm(int k) { return (dcx(k) != 0) + (dcy(k) != 0) + (dcz(k) != 0); }
+
 struct StF32 {
     using st = float;
     using T = float;
@@ -154,13 +163,18 @@ struct StF16S {
         return __builtin_fmaf(dec(enc(shifted(f, w), r, sr)), inv_scale, w);
     }
     // packed pairs (two cells along x in one 32-bit word, the lower cell in the low half): decode one
-    // half, or replace one half by a cell's rounded value (the same rounding as sto_r)
+    // half, or replace one half by a cell's rounded value (the same rounding as sto_r) given 2^N f, N = |cx| +
+    // |cy| + |cz| (collide_cell's SCALED form; the factor's exact inverse goes into the encoding's own)
     __device__ static __forceinline__ T dec_lo(uint32_t p, T w) { return __builtin_fmaf(dec((uint16_t)p), inv_scale, w); }
     __device__ static __forceinline__ T dec_hi(uint32_t p, T w) { return __builtin_fmaf(dec((uint16_t)(p >> 16)), inv_scale, w); }
-    template <bool HI>
-    __device__ static __forceinline__ uint32_t put(uint32_t old, T f, T w, uint32_t r, bool sr) {
+    template <int K>
+    __device__ static __forceinline__ float unscaled(T f) {
+        return __builtin_fmaf(f, in_vgpr(scale / float(1 << dnorm(K))), -(wgt<T>(K) * scale));
+    }
+    template <bool HI, int K>
+    __device__ static __forceinline__ uint32_t put(uint32_t old, T f, uint32_t r, bool sr) {
         typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-        const float x = shifted(f, w);
+        const float x = unscaled<K>(f);
         if (sr) return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_sr_f16_f32(__builtin_bit_cast(h2, old), x, r, HI));
         const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)x);
         return HI ? (old & 0xffffu) | (h << 16) : (old & 0xffff0000u) | h;
@@ -201,11 +215,16 @@ struct StBF16S {
     }
     __device__ static __forceinline__ T dec_lo(uint32_t p, T w) { return __uint_as_float(p << 16) + w; }
     __device__ static __forceinline__ T dec_hi(uint32_t p, T w) { return __uint_as_float(p & 0xffff0000u) + w; }
-    template <bool HI>
-    __device__ static __forceinline__ uint32_t put(uint32_t old, T f, T w, uint32_t r, bool sr) {
+    template <int K>
+    __device__ static __forceinline__ float unscaled(T f) {
+        return __builtin_fmaf(f, in_vgpr(1.0f / float(1 << dnorm(K))), -wgt<T>(K));
+    }
+    template <bool HI, int K>
+    __device__ static __forceinline__ uint32_t put(uint32_t old, T f, uint32_t r, bool sr) {
         typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-        if (sr) return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_sr_bf16_f32(__builtin_bit_cast(b2, old), f - w, r, HI));
-        const uint32_t h = f32_to_bf16_rne(f - w);
+        const float x = unscaled<K>(f);
+        if (sr) return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_sr_bf16_f32(__builtin_bit_cast(b2, old), x, r, HI));
+        const uint32_t h = f32_to_bf16_rne(x);
         return HI ? (old & 0xffffu) | (h << 16) : (old & 0xffff0000u) | h;
     }
 };
@@ -370,7 +389,12 @@ struct CellRates {
 // LDS_LIMITER: the positivity limiter's populations pass through LDS in a rolled loop (workgroups of 128
 // lanes, each lane its own column).  Unrolled, its 54 equilibria raise the kernel from 90 to 168 registers,
 // which every wave would pay for a branch that few cells take.
-template <class T, bool UNIT = false, bool SPONGE = false, bool LDS_LIMITER = false>
+//
+// SCALED: on return f[k] is the population times 2^(|cx| + |cy| + |cz|): the backward passes leave out their
+// halvings (f-, f+ = (m2 -+ m1) / 2: a power of two per pass, which commutes with every rounding), 27 of about
+// 750 instructions per cell, for the 16-bit forms, whose encoding multiplies anyway (with the encoding's factors
+// in vector registers, 256^3 FP16: 376 -> 371 us per step).
+template <class T, bool UNIT = false, bool SPONGE = false, bool LDS_LIMITER = false, bool SCALED = false>
 __device__ __forceinline__ void collide_cell(T (&f)[27], const CellRates<T>& q, const CollParams& p,
                                              T& rho_o, T& ux_o, T& uy_o, T& uz_o) {
     T A[27];
@@ -564,15 +588,23 @@ __device__ __forceinline__ void collide_cell(T (&f)[27], const CellRates<T>& q, 
     }
 
     // backward passes z, y, x: (k0, k1, k2) -> (f-, f0, f+) about u
+    auto halves = [](T& fm, T& fp, T m1, T m2) {
+        if constexpr (SCALED) {
+            fm = m2 - m1;
+            fp = m2 + m1;
+        } else {
+            const T h = T(0.5) * m1;
+            fm = fmx(T(0.5), m2, -h);
+            fp = fmx(T(0.5), m2, h);
+        }
+    };
     auto back = [&](int i0, int i1, int i2, T u) {
         const T uu = u * u, t = T(2) * u;
         const T a = A[i0], b = A[i1], c = A[i2];
         const T m1 = fmx(u, a, b);
         const T m2 = fmx(uu, a, fmx(t, b, c));
-        const T h = T(0.5) * m1;
-        A[i0] = fmx(T(0.5), m2, -h);
+        halves(A[i0], A[i2], m1, m2);
         A[i1] = a - m2;
-        A[i2] = fmx(T(0.5), m2, h);
     };
     if constexpr (UNIT) {
         // the z pass with its known zeros: rows (r, r + 9, r + 18) with r even have k1 = 0 (1st, 3rd and
@@ -583,19 +615,15 @@ __device__ __forceinline__ void collide_cell(T (&f)[27], const CellRates<T>& q, 
             const T a = A[r2], c = A[r2 + 18];
             const T m1 = u * a;
             const T m2 = fmx(uu, a, c);
-            const T h = T(0.5) * m1;
-            A[r2] = fmx(T(0.5), m2, -h);
+            halves(A[r2], A[r2 + 18], m1, m2);
             A[r2 + 9] = a - m2;
-            A[r2 + 18] = fmx(T(0.5), m2, h);
         }
 #pragma unroll
         for (int r2 = 1; r2 < 9; r2 += 2) {
             const T b = A[r2 + 9];
             const T m2 = t * b;
-            const T h = T(0.5) * b;
-            A[r2] = fmx(T(0.5), m2, -h);
+            halves(A[r2], A[r2 + 18], b, m2);
             A[r2 + 9] = -m2;
-            A[r2 + 18] = fmx(T(0.5), m2, h);
         }
     } else {
 #pragma unroll
@@ -617,7 +645,11 @@ __device__ __forceinline__ void collide_cell(T (&f)[27], const CellRates<T>& q, 
         for (int i = 0; i < 9; ++i) m9[i] = fmn(fmn(A[3 * i], A[3 * i + 1]), A[3 * i + 2]);
         const T fmin = fmn(fmn(fmn(fmn(m9[0], m9[1]), m9[2]), fmn(fmn(m9[3], m9[4]), m9[5])),
                            fmn(fmn(m9[6], m9[7]), m9[8]));
-        if (fmin < T(0) && A[0] == A[0]) {
+        if (fmin < T(0) && A[0] == A[0]) {   // (the test holds for scaled values too)
+            if constexpr (SCALED) {
+#pragma unroll
+                for (int k = 0; k < 27; ++k) A[k] *= T(1) / T(1 << dnorm(k));
+            }
             if constexpr (LDS_LIMITER) {
                 T* lim = (T*)two_lds() + threadIdx.x;
 #pragma unroll
@@ -655,6 +687,10 @@ __device__ __forceinline__ void collide_cell(T (&f)[27], const CellRates<T>& q, 
                     A[k] = fe + alpha * (A[k] - fe);
                 }
             }
+            if constexpr (SCALED) {
+#pragma unroll
+                for (int k = 0; k < 27; ++k) A[k] *= T(1 << dnorm(k));
+            }
         }
     }
     if (q.forced) {   // Guo term of the force density (kernel_cumulant.jl:889-905)
@@ -665,7 +701,7 @@ __device__ __forceinline__ void collide_cell(T (&f)[27], const CellRates<T>& q, 
             const T cu = cxf * uxe + cyf * uye + czf * uze;
             const T ft = wgt<T>(k) * T(3) * ((cxf - ux + T(3) * cu * cxf) * q.Fx + (cyf - uy + T(3) * cu * cyf) * q.Fy +
                                              (czf - uz + T(3) * cu * czf) * q.Fz);
-            A[k] = A[k] + g * ft;
+            A[k] = SCALED ? fmx(T(1 << dnorm(k)), g * ft, A[k]) : A[k] + g * ft;
         }
     }
 #pragma unroll

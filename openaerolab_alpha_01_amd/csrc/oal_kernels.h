@@ -135,6 +135,14 @@ inline bool two_fits(int64_t lo, int64_t hi, uint64_t esize) {
 // the memory-side cache
 constexpr uint64_t TWO_KEEP_BYTES = 192ull << 20;
 
+// Blocks up to which a level in the AB pattern with FP32 arithmetic takes the one-cell-per-lane kernel (half as
+// many with WALE): twice the waves with half the work each.  128 blocks fill the chip's wave slots in either
+// form; measured (us per step, one against two cells per lane), FP32: 8 blocks 6.7 / 9.6, 64 11.0 / 13.2,
+// 216 31.6 / 34.3, 512 84 / 87, 1000 161 / 162, 4096 653 / 634; FP16: 8 7.3 / 13.4, 216 26.8 / 29.4,
+// 512 56.9 / 63.4, 640 68.6 / 67.8, 4096 385 / 370; WALE FP32: 8 9.4 / 11.6, 216 38.9 / 40.9, 294 63.4 / 62.2,
+// 1000 202 / 193; WALE FP16: 216 35.5 / 37.3, 343 49.9 / 49.0, 1000 146 / 126.
+constexpr uint32_t ONE_BLOCKS = 512;
+
 struct ReduceArgs {
     const double* part;          // [n_items * 4]
     const int32_t* dom_item0;    // [n_domains + 1] first item of each domain
@@ -171,8 +179,12 @@ void launch_two_f16s(bool wale, int extra, const StepArgs& a, hipStream_t stream
 void launch_two_bf16s(bool wale, int extra, const StepArgs& a, hipStream_t stream);
 // and over the n blocks of a list, by storage code
 void launch_two(int storage, bool wale, int extra, const TwoRec* rec, uint32_t n, hipStream_t stream, const StepArgs& a);
-// the one-cell-per-lane FP64 step kernel over n records: oal_one_f64.hip
-void launch_one_f64(bool wale, const TwoRec* rec, uint32_t n, const StepArgs& a, hipStream_t stream);
+// likewise the one-cell-per-lane step kernel (AB pattern): oal_one_<storage>.hip
+void launch_one_f32(bool wale, const StepArgs& a, hipStream_t stream);
+void launch_one_f64(bool wale, const StepArgs& a, hipStream_t stream);
+void launch_one_f16s(bool wale, const StepArgs& a, hipStream_t stream);
+void launch_one_bf16s(bool wale, const StepArgs& a, hipStream_t stream);
+void launch_one(int storage, bool wale, const TwoRec* rec, uint32_t n, hipStream_t stream, const StepArgs& a);
 hipError_t launch_copy16(const void* src, void* dst, size_t bytes, hipStream_t stream);
 // Host arrays of init / conversion / macro output cover the first nhost cells of a level (the caller's
 // blocks); the device arrays have ncell cells per direction.

@@ -670,7 +670,7 @@ static void launch_boundary(const StepArgs& a, hipStream_t bs) {
 
 // One step of a level: launches over disjoint block lists.
 //   FP32 arithmetic: the two-cells-per-lane kernel for every block but a few kinds, those on the one-plane
-//     boundary kernel.
+//     boundary kernel; on small levels in the AB pattern the one-cell-per-lane kernel in its place.
 //   FP64, AB pattern: likewise the one-cell-per-lane kernel.
 //   FP64, AA pattern: regular, other interior, regular boundary and boundary blocks, each on a kernel
 //     compiled for its own register budget.
@@ -692,12 +692,13 @@ static hipError_t launch_pat(const StepArgs& a, hipStream_t stream, hipStream_t 
             launch_two(SP::code, WALE, TWO_BFL, a.two_links, a.n_two_links, stream, a);
             launch_two(SP::code, WALE, TWO_PLAIN, a.two_free, a.n_two_free, stream, a);
         } else {
-            launch_two(SP::code, WALE, TWO_PLAIN, a.two, a.n_two, stream, a);
+            if (a.n_two <= (WALE ? ONE_BLOCKS / 2 : ONE_BLOCKS)) launch_one(SP::code, WALE, a.two, a.n_two, stream, a);
+            else launch_two(SP::code, WALE, TWO_PLAIN, a.two, a.n_two, stream, a);
             launch_two(SP::code, WALE, TWO_SPONGE, a.two_sponge, a.n_two_sponge, stream, a);
         }
     } else if constexpr (PAT == PAT_AB) {   // (with interpolated bounce-back the boundary lists hold the links)
-        if (a.qmap) launch_one_f64(WALE, a.two_free, a.n_two_free, a, stream);
-        else launch_one_f64(WALE, a.two, a.n_two, a, stream);
+        if (a.qmap) launch_one(SP::code, WALE, a.two_free, a.n_two_free, stream, a);
+        else launch_one(SP::code, WALE, a.two, a.n_two, stream, a);
     } else {
         StepArgs r = a;
         if (a.n_regular) {

@@ -27,8 +27,8 @@
 // so a lane needs 97 to 125 registers and four waves share a SIMD; their loads overlap other waves'
 // collisions.  That needs the rare limiter out of the registers (collide_cell's LDS form): with it inline
 // the kernel takes 168 and spills.  Bound: HBM in FP32 (256^3: 5.9 TB/s of 6.0 that a copy reaches counting
-// 216 bytes per cell), VALU issue in the 16-bit forms (about 760 instructions per cell, 97 % of the issue
-// slots).  Measured against walking four planes of a block per workgroup with the next plane's words in
+// 216 bytes per cell), in the 16-bit forms VALU and HBM alike (256^3 FP16: about 720 instructions per cell, half of them
+// issued every second cycle, the others every fourth or eighth, some 70 % of the time; 4.9 TB/s).  Measured against walking four planes of a block per workgroup with the next plane's words in
 // flight (two waves per SIMD, a launch per kind of block, the default shape before): 256^3 sphere box FP32
 // 667 -> 633 us per step, FP16 467 -> 370 us; WALE 192 x 160 x 160 FP32 295 -> 232 us, WALE 200 x 120 x 104
 // FP16 200 -> 93 us; WALE 100 x 60 x 44 75 -> 20 us (that shape left 48 workgroups per launch); 12 ragged
@@ -36,6 +36,7 @@
 // of the row ends.  One record per block (TwoRec) in place of a chain of table reads: FP16 256^3 453 -> 372
 // us, 48 x 32 x 32 13.5 -> 10.8 us.  Stores written through at device scope: 48 x 32 x 32 10.8 -> 10.2 us,
 // WALE 100 x 60 x 44 25.3 -> 20.9 us without the non-temporal hint (which 256^3 needs: 635 against 681 us).
+// (Small levels in the AB pattern take the one-cell-per-lane form since: 48 x 32 x 32 7.0 us, ONE_BLOCKS.)
 // AA 192 x 160 x 160 FP32, sphere: 340 -> 204 us per step against a pipelined kernel for the blocks off the
 // faces and a one-plane kernel for the rest (a third of the blocks); 5.2 TB/s of the pair's 216 bytes per cell.
 #pragma once
@@ -608,7 +609,7 @@ k_step_two(const StepArgs a) {
         if (is(LF_LIVE_A) && (lma & 0x7ffffffu)) bfl(f, ca, lma, is(LF_OUTLET_A), is(LF_INLET));
     }
     if constexpr (EXTRA == TWO_SPONGE) qa.sponge = spa;
-    collide_cell<float, UNIT, EXTRA == TWO_SPONGE, true>(f, qa, a.cp, rho_o, va[0], va[1], va[2]);
+    collide_cell<float, UNIT, EXTRA == TWO_SPONGE, true, es == 2>(f, qa, a.cp, rho_o, va[0], va[1], va[2]);
     {
         const uint32_t hc = DITH ? round_cell(key, ca - cell0) : 0u;
         for_dirs([&](auto kc) {
@@ -618,7 +619,7 @@ k_step_two(const StepArgs a) {
         if constexpr (es == 2) {
             for_dirs([&](auto kc) {
                 constexpr int K = decltype(kc)::value;
-                s[K] = SP::template put<false>(s[K], f[K], wgt<float>(K), DITH ? round_bits(hc, K) : 0u, DITH);
+                s[K] = SP::template put<false, K>(s[K], f[K], DITH ? round_bits(hc, K) : 0u, DITH);
             });
         }
     }
@@ -636,7 +637,7 @@ k_step_two(const StepArgs a) {
     qb.omega1 = om1b;
     qb.omega4_diag = om4b;
     if constexpr (EXTRA == TWO_SPONGE) qb.sponge = spb;
-    collide_cell<float, UNIT, EXTRA == TWO_SPONGE, true>(f, qb, a.cp, rho_o, vb[0], vb[1], vb[2]);
+    collide_cell<float, UNIT, EXTRA == TWO_SPONGE, true, es == 2>(f, qb, a.cp, rho_o, vb[0], vb[1], vb[2]);
     {
         const uint32_t hc = DITH ? round_cell(key, ca + 1u - cell0) : 0u;
         for_dirs([&](auto kc) {
@@ -646,7 +647,7 @@ k_step_two(const StepArgs a) {
         if constexpr (es == 2) {
             for_dirs([&](auto kc) {
                 constexpr int K = decltype(kc)::value;
-                s[K] = SP::template put<true>(s[K], f[K], wgt<float>(K), DITH ? round_bits(hc, K) : 0u, DITH);
+                s[K] = SP::template put<true, K>(s[K], f[K], DITH ? round_bits(hc, K) : 0u, DITH);
             });
         }
     }

@@ -1,9 +1,10 @@
-"""The two-cells-per-lane step kernel (both patterns) and the FP64 one at the extents where pairs, row ends and rules
-can go wrong, against the oracle bit for bit."""
+"""The one-launch step kernels, two cells per lane (both patterns) and one cell per lane (AB pattern), at the extents
+where pairs, row ends and rules can go wrong, against the oracle bit for bit."""
 import numpy as np
 import pytest
 
-from openaerolab_alpha_01_amd.geometry import sphere_mask, uniform_grid
+from openaerolab_alpha_01_amd import solver
+from openaerolab_alpha_01_amd.geometry import batch_grids, sphere_mask, uniform_grid
 from test_gpu_parity import compare, fields, gpu_plan, oracle_run
 
 pytestmark = pytest.mark.gpu
@@ -24,6 +25,7 @@ CASES = {
 }
 
 
+# (AB: so few blocks take the one-cell-per-lane form)
 @pytest.mark.parametrize("stream", ["ab", "aa"])
 @pytest.mark.parametrize("storage", ["f32", "f16s", "bf16s"])
 @pytest.mark.parametrize("case", list(CASES))
@@ -50,6 +52,36 @@ def test_two_cells_per_lane(oracle, storage, case, stream):
         got = plan.download_f(dtype=np.float32 if storage == "f32" else np.float64)
         want = f_or if storage == "f32" else oracle.to_unshifted(storage, f_or)
         assert np.array_equal(got[..., live], want[..., live])
+    plan.close()
+
+
+@pytest.mark.parametrize("storage", ["f32", "f16s", "bf16s"])
+@pytest.mark.parametrize("case", list(CASES))
+def test_many_copies(oracle, storage, case):
+    """Levels of more than 512 blocks take the two-cells-per-lane kernel in the AB pattern, smaller ones (the
+    test above) the one-cell form: copies of a grid as the domains of one level, each the oracle's bits."""
+    cfg = CASES[case]
+    grid = uniform_grid(cfg["n"], periodic=cfg.get("periodic", (False, False, False)))
+    if "solid" in cfg:
+        grid.solid = sphere_mask(grid, *cfg["solid"])
+    okw = cfg["okw"]
+    rho, u = fields(grid, seed=31, u0=(okw.get("u_inlet", 0.0), 0, 0))
+    f_or, _, _ = oracle_run(oracle, grid, storage, 2, okw, rho, u)
+    copies = 512 // grid.n_blocks + 1
+    big = batch_grids([grid] * copies)
+    dom = {k: okw[k] for k in ("tau", "u_inlet", "body_force", "ymin_wall_bc", "zwall_bc") if k in okw}
+    params = dict(omega_bulk=1.0, omega_3=1.0, omega_4=1.0, lambda_=1 / 6, adaptive_omega4=1, limiter=1, compressible=0,
+                  c_wale=0.0, nu_sgs_background=0.0, inlet_turbulence=0.0)
+    params.update({k: v for k, v in okw.items() if k not in dom})
+    doms = [solver.Domain(extent=grid.n, periodic=grid.periodic, **dom) for _ in range(copies)]
+    plan = solver.Plan(solver.Level(big, doms, block_domain=big.block_domain), storage=storage, stream="ab",
+                       bb_mode="halfway", params=solver.StepParams(**params))
+    plan.init_equilibrium(np.tile(rho, copies), np.tile(u, copies))
+    for t in range(2):
+        plan.level_step(0, t)
+    got = plan.download_f(dtype=np.float32 if storage == "f32" else np.float64).reshape(27, copies, -1)
+    want = f_or if storage == "f32" else oracle.to_unshifted(storage, f_or)
+    assert all(np.array_equal(got[:, i], want) for i in range(copies))
     plan.close()
 
 
