@@ -650,15 +650,18 @@ __global__ void __launch_bounds__(WG) k_xfer_rebuild_row(typename SP::st* f, uin
 //   a pairwise tree: the low bits of j within a DPP row (rotations by 8 and by 4 lanes, the second on
 //   values alike in the first's lanes), the high bits over the wave's four rows through LDS.
 //   Cells: two lanes per cell read its 27 sums, form the moments and write half the directions each.
-// Bound: VALU issue (64 x 27 multiplies and adds per cell, unfused, in a fixed order).  Against 16 lanes per
-// cell with one record per lane, all of them forming the moments: a 75 000-cell fill from FP16 levels 53 -> 43
-// us, a 4-level octree step 1668 -> 1571 us.
+//   Groups: neighbouring entries with the same nodes (a fill's cells between the same coarse centres, four in
+//   a layer on a face) share the records read and decoded once.
+// Bound: VALU issue, some 70 % of the time (64 x 27 multiplies and adds per cell, unfused, in a fixed order: 165
+// to 195 instructions per cell and lane in all, a third of them the moments and the directions).  Against 16
+// lanes per cell with one record per lane, all of them forming the moments: a 4-level octree step 1668 -> 1571
+// us; the groups then 1528 -> 1472 us, a 3-level step with WALE 575 -> 545 us.
 constexpr int XFER_CELLS = 16;   // written cells per wave, at most
 constexpr int XWG = 256;         // lanes of a workgroup
 template <class SP, bool RAW>
 __global__ void __launch_bounds__(XWG) k_xfer_rebuild(typename SP::st* f, uint32_t ncell, const uint32_t* tcells, uint32_t n,
-                                                     uint32_t per, const int32_t* slot, const float* wt, const float* m,
-                                                     float scale, float keep, float* vel) {
+                                                     uint32_t per, const int32_t* slot, const float* wt, const uint8_t* same,
+                                                     const float* m, float scale, float keep, float* vel) {
     constexpr int V = RAW ? 8 : 4;            // directions per lane
     constexpr int NODES = RAW ? 4 : 8;        // nodes per lane
     constexpr int H = NODES / 4;              // partial sums per lane
@@ -676,20 +679,29 @@ __global__ void __launch_bounds__(XWG) k_xfer_rebuild(typename SP::st* f, uint32
     // a quad's lanes read the nodes of its group, one (RAW) or two (lane and lane + 4) each, and pass them on
     // by quad broadcasts
     const uint32_t mine = (uint32_t)(g * NODES + (lane & 3));
-    struct Stencil {
-        uint32_t r[H];        // record in 16-byte units (unused nodes: record 0)
+    struct Stencil {          // of a group's first cell
+        uint32_t r[H];        // record in 16-byte units (0xffffffff: an unused node)
         float w[H];
-        bool some;            // an unused node
+    };
+    auto weights = [&](int d, float (&w)[H]) {
+        const size_t o = (size_t)(i0 + (uint32_t)(d < cnt ? d : cnt - 1)) * 64 + mine;
+#pragma unroll
+        for (int h = 0; h < H; ++h) w[h] = wt[o + 4 * h];
     };
     auto stencil = [&](int d, Stencil& t) {
         const size_t o = (size_t)(i0 + (uint32_t)(d < cnt ? d : cnt - 1)) * 64 + mine;
-        t.some = false;
 #pragma unroll
         for (int h = 0; h < H; ++h) {
             const int32_t sv = slot[o + 4 * h];
             t.r[h] = sv < 0 ? 0xffffffffu : (uint32_t)sv * (RAW ? 4u : 8u);
-            t.w[h] = wt[o + 4 * h];
         }
+        weights(d, t.w);
+    };
+    // groups of cells on the same records: bit d of starts = cell d begins one
+    const uint32_t starts = 1u | (uint32_t)__builtin_amdgcn_ballot_w64(lane < cnt && !(same && same[i0 + (uint32_t)lane]));
+    auto next = [&](int d) {
+        const uint32_t later = d < cnt ? (starts >> d) & ~1u : 0u;
+        return later ? d + __builtin_ctz(later) : cnt;
     };
     const uint4* mq = reinterpret_cast<const uint4*>(m) + q;
     auto records = [&](const Stencil& t, uint4 (&rec)[NODES]) {
@@ -699,12 +711,7 @@ __global__ void __launch_bounds__(XWG) k_xfer_rebuild(typename SP::st* f, uint32
             rec[E] = mq[r == 0xffffffffu ? 0u : r];
         });
     };
-    Stencil sa, sb, sc{};
-    uint4 ra[NODES], rb[NODES];
-    stencil(0, sa);
-    stencil(1, sb);
-    records(sa, ra);
-    auto one = [&](int d, const Stencil& t, uint4 (&rec)[NODES]) {
+    auto one = [&](int d, const Stencil& t, const float (&tw)[H], const float (&x)[NODES][V]) {
         float acc[H][V];
         bool some = false;
 #pragma unroll
@@ -716,17 +723,13 @@ __global__ void __launch_bounds__(XWG) k_xfer_rebuild(typename SP::st* f, uint32
                 for (int e = 0; e < V; ++e) acc[h][e] = 0.0f;
             for_each_dir(std::make_integer_sequence<int, NODES>{}, [&](auto ec) {
                 constexpr int E = decltype(ec)::value;
-                const uint32_t wd[4] = {rec[E].x, rec[E].y, rec[E].z, rec[E].w};
-                const float w = dpp_get<(E & 3) * 0x55>(t.w[E / 4]);
+                const float w = dpp_get<(E & 3) * 0x55>(tw[E / 4]);
                 bool use = true;
                 if constexpr (decltype(check)::value)
                     use = (uint32_t)__builtin_amdgcn_mov_dpp((int)t.r[E / 4], (E & 3) * 0x55, 0xf, 0xf, false) != 0xffffffffu;
 #pragma unroll
                 for (int k = 0; k < V; ++k) {
-                    float x;
-                    if constexpr (RAW) x = SP::from_raw((wd[k >> 1] >> (16 * (k & 1))) & 0xffffu, wk[k]);
-                    else x = __uint_as_float(wd[k]);
-                    const float v = acc[E / 4][k] + w * x;
+                    const float v = acc[E / 4][k] + w * x[E][k];
                     if constexpr (decltype(check)::value) acc[E / 4][k] = use ? v : acc[E / 4][k];
                     else acc[E / 4][k] = v;
                 }
@@ -753,17 +756,51 @@ __global__ void __launch_bounds__(XWG) k_xfer_rebuild(typename SP::st* f, uint32
             for (int k = 0; k < V / 4; ++k) o[k] = make_float4(acc[0][4 * k], acc[0][4 * k + 1], acc[0][4 * k + 2], acc[0][4 * k + 3]);
         }
     };
-    // the next cell's records and the stencil after it are in flight during a cell's sums
-    for (int d = 0; d < cnt; d += 2) {
-        stencil(d + 2, sc);
+    // the cells d0 .. d1 - 1 of a group, the weights of the next one in flight during a cell's sums
+    auto group = [&](int d0, int d1, const Stencil& t, const uint4 (&rec)[NODES]) {
+        float x[NODES][V];
+#pragma unroll
+        for (int e = 0; e < NODES; ++e) {
+            const uint32_t wd[4] = {rec[e].x, rec[e].y, rec[e].z, rec[e].w};
+#pragma unroll
+            for (int k = 0; k < V; ++k) {
+                if constexpr (RAW) x[e][k] = SP::from_raw((wd[k >> 1] >> (16 * (k & 1))) & 0xffffu, wk[k]);
+                else x[e][k] = __uint_as_float(wd[k]);
+            }
+        }
+        float tw[H], tn[H];
+#pragma unroll
+        for (int h = 0; h < H; ++h) tw[h] = t.w[h];
+#pragma unroll 1
+        for (int d = d0; d < d1; ++d) {
+            weights(d + 1, tn);
+            one(d, t, tw, x);
+#pragma unroll
+            for (int h = 0; h < H; ++h) tw[h] = tn[h];
+        }
+    };
+    // the next group's records and the stencil after it are in flight during a group's sums
+    Stencil sa, sb, sc{};
+    uint4 ra[NODES], rb[NODES];
+    int d0 = 0, d1 = next(0), d2 = next(d1);
+    stencil(d0, sa);
+    stencil(d1, sb);
+    records(sa, ra);
+    while (true) {
+        stencil(d2, sc);
         records(sb, rb);
-        one(d, sa, ra);
-        if (d + 1 >= cnt) break;
+        group(d0, d1, sa, ra);
+        if (d1 >= cnt) break;
+        const int d3 = next(d2);
         sa = sc;
-        stencil(d + 3, sc);
+        stencil(d3, sc);
         records(sa, ra);
-        one(d + 1, sb, rb);
+        group(d1, d2, sb, rb);
+        if (d2 >= cnt) break;
         sb = sc;
+        d0 = d2;
+        d1 = d3;
+        d2 = next(d3);
     }
     __builtin_amdgcn_wave_barrier();
     // two lanes per cell, for a direction and its opposite: c c is the same and c u changes its sign
@@ -833,7 +870,7 @@ static hipError_t xfer_sp(const void* fnew, const void* fold, const uint32_t* ce
 }
 template <class SP, bool RAW>
 static hipError_t rebuild_sp(void* f, uint32_t ncell, const uint32_t* tcells, uint32_t n, const int32_t* slot, const float* w,
-                             const void* m, double scale, double keep, void* vel, hipStream_t s) {
+                             const uint8_t* same, const void* m, double scale, double keep, void* vel, hipStream_t s) {
     using T = typename SP::T;
     using st = typename SP::st;
     if (!n) return hipSuccess;
@@ -841,12 +878,21 @@ static hipError_t rebuild_sp(void* f, uint32_t ncell, const uint32_t* tcells, ui
         hipLaunchKernelGGL((k_xfer_rebuild_row<SP>), dim3((n + WG / 16 - 1) / (WG / 16)), dim3(WG), 0, s, (st*)f, ncell, tcells, n,
                            slot, w, (const T*)m, T(scale), T(keep), (T*)vel);
     } else {
-        // written cells per wave: fewer where 32 would leave less than two waves per SIMD (2048 of them)
-        uint32_t per = n / 2048u;
-        per = per < 1u ? 1u : (per > (uint32_t)XFER_CELLS ? (uint32_t)XFER_CELLS : per);
+        // written cells per wave, so that every CU gets the same number k of workgroups (k waves per SIMD): the
+        // cost is k (cells + 7), the rebuild of a wave's cells together counting as 7 more; at least two waves
+        // per SIMD.  Against 16 cells per wave wherever two waves per SIMD are left: a 4-level octree step 1472
+        // -> 1423 us, a 3-level one with WALE 545 -> 513 us (33 800 cells: 11 per wave on three workgroups per
+        // CU, not 16 on two, with a third on a few); from three waves per SIMD on: 1421 and 522 us.
+        uint32_t per = XFER_CELLS, best = 0xffffffffu;
+        for (uint32_t k = 2; k <= 8 || best == 0xffffffffu; ++k) {
+            const uint32_t c = (n + 1024u * k - 1u) / (1024u * k);
+            if (c > (uint32_t)XFER_CELLS || k * (c + 7u) >= best) continue;
+            best = k * (c + 7u);
+            per = c;
+        }
         const uint32_t waves = (n + per - 1) / per;
         hipLaunchKernelGGL((k_xfer_rebuild<SP, RAW>), dim3((waves + XWG / 64 - 1) / (XWG / 64)), dim3(XWG), 0, s, (st*)f, ncell, tcells,
-                           n, per, slot, w, (const float*)m, (float)scale, (float)keep, (float*)vel);
+                           n, per, slot, w, same, (const float*)m, (float)scale, (float)keep, (float*)vel);
     }
     return hipGetLastError();
 }
@@ -866,15 +912,15 @@ hipError_t launch_xfer_gather(int storage, const void* fnew, const void* fold, c
     }
 }
 hipError_t launch_xfer_rebuild(int storage, bool raw, void* f, uint32_t ncell, const uint32_t* tcells, uint32_t n,
-                               const int32_t* slot, const float* w, const void* m, double scale, double keep, void* vel,
-                               hipStream_t s) {
+                               const int32_t* slot, const float* w, const uint8_t* same, const void* m, double scale,
+                               double keep, void* vel, hipStream_t s) {
     switch (storage) {
-        case 0: return rebuild_sp<StF32, false>(f, ncell, tcells, n, slot, w, m, scale, keep, vel, s);
-        case 1: return rebuild_sp<StF64, false>(f, ncell, tcells, n, slot, w, m, scale, keep, vel, s);
-        case 2: return raw ? rebuild_sp<StF16S, true>(f, ncell, tcells, n, slot, w, m, scale, keep, vel, s)
-                           : rebuild_sp<StF16S, false>(f, ncell, tcells, n, slot, w, m, scale, keep, vel, s);
-        case 3: return raw ? rebuild_sp<StBF16S, true>(f, ncell, tcells, n, slot, w, m, scale, keep, vel, s)
-                           : rebuild_sp<StBF16S, false>(f, ncell, tcells, n, slot, w, m, scale, keep, vel, s);
+        case 0: return rebuild_sp<StF32, false>(f, ncell, tcells, n, slot, w, same, m, scale, keep, vel, s);
+        case 1: return rebuild_sp<StF64, false>(f, ncell, tcells, n, slot, w, same, m, scale, keep, vel, s);
+        case 2: return raw ? rebuild_sp<StF16S, true>(f, ncell, tcells, n, slot, w, same, m, scale, keep, vel, s)
+                           : rebuild_sp<StF16S, false>(f, ncell, tcells, n, slot, w, same, m, scale, keep, vel, s);
+        case 3: return raw ? rebuild_sp<StBF16S, true>(f, ncell, tcells, n, slot, w, same, m, scale, keep, vel, s)
+                           : rebuild_sp<StBF16S, false>(f, ncell, tcells, n, slot, w, same, m, scale, keep, vel, s);
         default: return hipErrorInvalidValue;
     }
 }

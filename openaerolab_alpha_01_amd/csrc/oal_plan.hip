@@ -141,6 +141,7 @@ struct Level {
     DevBuf<uint32_t> g_src, g_dst;
     DevBuf<int32_t> g_slot;
     DevBuf<float> g_w;
+    DevBuf<uint8_t> g_same;            // the entry's nodes are those of the entry before
     DevBuf<unsigned char> g_m;
     uint32_t n_gsrc = 0, n_gdst = 0;
     double fill_scale = 0.0, fill_keep = 0.0;
@@ -193,7 +194,7 @@ struct Level {
         rec_tw.release(); rec_ts.release(); rec_tl.release(); rec_tn.release(); blist_xr.release(); blist_xb.release();
         fpart.release(); mpart.release(); red_out.release(); guard.release(); oslot.release(); obuf.release(); blist_rg.release(); blist_in.release(); blist_br.release(); blist_bd.release();
         c8map_d.release(); lslot.release(); lmask.release(); qmap.release(); sponge.release(); sslot.release();
-        g_src.release(); g_dst.release(); g_slot.release(); g_w.release(); g_m.release();
+        g_src.release(); g_dst.release(); g_slot.release(); g_w.release(); g_same.release(); g_m.release();
         r_src.release(); r_dst.release(); r_slot.release(); r_w.release(); r_m.release();
         rf_src.release(); rf_dst.release(); rf_slot.release(); rf_w.release();
         release_surface();
@@ -738,6 +739,35 @@ static std::vector<V> node_to_cell_major(const std::vector<V>& a, size_t n) {
     return b;
 }
 
+// The entries of X (cell-major) in the order of their stencil nodes: the fine cells between the same coarse
+// centres (2 per axis) have the same 64 nodes and become neighbours, which the rebuild reads once.  Returns,
+// per entry, whether its nodes are those of the entry before.
+static std::vector<uint8_t> group_by_nodes(XferHost& X) {
+    const size_t n = X.dst.size();
+    std::vector<uint32_t> order(n);
+    std::iota(order.begin(), order.end(), 0u);
+    const int32_t* sl = X.slot.data();
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) {
+        return std::lexicographical_compare(sl + (size_t)a * 64, sl + (size_t)a * 64 + 64, sl + (size_t)b * 64, sl + (size_t)b * 64 + 64);
+    });
+    XferHost Y;
+    Y.dst.resize(n);
+    Y.slot.resize(64 * n);
+    Y.w.resize(64 * n);
+    std::vector<uint8_t> same(n, 0);
+    for (size_t i = 0; i < n; ++i) {
+        const size_t o = order[i];
+        Y.dst[i] = X.dst[o];
+        std::copy_n(sl + o * 64, 64, Y.slot.data() + i * 64);
+        std::copy_n(X.w.data() + o * 64, 64, Y.w.data() + i * 64);
+        same[i] = i > 0 && std::equal(sl + o * 64, sl + o * 64 + 64, Y.slot.data() + (i - 1) * 64) ? 1 : 0;
+    }
+    X.dst.swap(Y.dst);
+    X.slot.swap(Y.slot);
+    X.w.swap(Y.w);
+    return same;
+}
+
 // written cells inside the destination level, donors inside the source level, slots inside the donor list
 static bool xfer_in_bounds(const XferHost& X, uint64_t ncell_dst, uint64_t ncell_src) {
     for (uint32_t c : X.dst)
@@ -1230,7 +1260,8 @@ int ml_fill(OalPlan* p, int l, double w1, hipStream_t s) {
     if (!F.n_gdst) return OAL_OK;
     OAL_HIP(launch_xfer_gather(p->storage, C.fA.p, w1 == 1.0 ? nullptr : C.fB.p, F.g_src.p, F.n_gsrc, C.ncell, w1,
                                 F.g_m.p, s));
-    OAL_HIP(launch_xfer_rebuild(p->storage, w1 == 1.0, F.fA.p, F.ncell, F.g_dst.p, F.n_gdst, F.g_slot.p, F.g_w.p, F.g_m.p,
+    OAL_HIP(launch_xfer_rebuild(p->storage, w1 == 1.0, F.fA.p, F.ncell, F.g_dst.p, F.n_gdst, F.g_slot.p, F.g_w.p,
+                                F.g_same.p, F.g_m.p,
                                 F.fill_scale, F.fill_keep, p->wale ? (void*)F.velA.p : nullptr, s));
     return OAL_OK;
 }
@@ -1244,7 +1275,7 @@ int ml_restrict(OalPlan* p, int l, hipStream_t s, bool full = false) {
     if (!nd) return OAL_OK;
     OAL_HIP(launch_xfer_gather(p->storage, F.fA.p, nullptr, full ? C.rf_src.p : C.r_src.p, ns, F.ncell, 1.0, C.r_m.p, s));
     OAL_HIP(launch_xfer_rebuild(p->storage, true, C.fA.p, C.ncell, full ? C.rf_dst.p : C.r_dst.p, nd,
-                                full ? C.rf_slot.p : C.r_slot.p, full ? C.rf_w.p : C.r_w.p, C.r_m.p, C.restrict_scale,
+                                full ? C.rf_slot.p : C.r_slot.p, full ? C.rf_w.p : C.r_w.p, nullptr, C.r_m.p, C.restrict_scale,
                                 C.restrict_keep, p->wale ? (void*)C.velA.p : nullptr, s));
     return OAL_OK;
 }
@@ -1776,12 +1807,13 @@ int oal_plan_create(const OalPlanDesc* desc, OalPlan** out) {
                 X->slot = node_to_cell_major(X->slot, X->dst.size());
                 X->w = node_to_cell_major(X->w, X->dst.size());
             }
+            const std::vector<uint8_t> same = group_by_nodes(fillX[l]);
             const XferHost& F = fillX[l];
             const XferHost& R = restX[l];
             const XferHost& RF = restFull[l];
             int r2;
             if ((r2 = upload(L.g_src, F.src)) || (r2 = upload(L.g_dst, F.dst)) || (r2 = upload(L.g_slot, F.slot)) ||
-                (r2 = upload(L.g_w, F.w)) || (r2 = upload(L.r_src, R.src)) || (r2 = upload(L.r_dst, R.dst)) ||
+                (r2 = upload(L.g_w, F.w)) || (r2 = upload(L.g_same, same)) || (r2 = upload(L.r_src, R.src)) || (r2 = upload(L.r_dst, R.dst)) ||
                 (r2 = upload(L.r_slot, R.slot)) || (r2 = upload(L.r_w, R.w)) || (r2 = upload(L.rf_src, RF.src)) ||
                 (r2 = upload(L.rf_dst, RF.dst)) || (r2 = upload(L.rf_slot, RF.slot)) || (r2 = upload(L.rf_w, RF.w)))
                 return bail(r2);

@@ -1,5 +1,5 @@
-"""Level transfers on enough cells that a wave of the rebuild takes several of them (5 per wave in the fill,
-3 in the full restriction, the last wave short), with complete stencils and, around the sphere, incomplete
+"""Level transfers on enough cells that a wave of the rebuild takes several of them (6 per wave in the fill,
+4 in the full restriction), some on the same stencil nodes, with complete stencils and, around the sphere, incomplete
 ones: every level's populations bit for bit the oracle's refined run."""
 import pytest
 import test_gpu_octree as T
