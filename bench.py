@@ -656,7 +656,7 @@ def main(argv=None) -> int:
     cd = float(F[0] / (0.5 * U_IN ** 2 * area))
 
     # (the collision's unit-rate form: the reference's default rates omega_bulk = omega_3 = omega_4 = 1)
-    kernel = "k_step_two<StF32, true, false, 0>" if ab else "k_step_two<StF32, true, false, 0, odd>"
+    kernel = "k_step_two<StF32, true, false, 0, false, 0>" if ab else "k_step_two<StF32, true, false, 0, false, 2>"
     traffic = measured_traffic(kernel)
 
     out = {
@@ -694,7 +694,7 @@ def main(argv=None) -> int:
         bulk16 = bulk_cells
         a16 = bytes_per_lup("f16s") * bulk16 / (ms_k16 * 1e-3) / 1e9
         s16 = bytes_per_lup("f16s") * n_fluid / (ms_t16 / args.steps * 1e-3) / 1e9
-        k16 = "k_step_two<StF16S, true, false, 0>" if ab else "k_step_two<StF16S, true, false, 0, odd>"
+        k16 = "k_step_two<StF16S, true, false, 0, true, 0>" if ab else "k_step_two<StF16S, true, false, 0, true, 2>"
         traffic16 = measured_traffic(k16, "step_f16_256_hbm_traffic.md")
         out["fp16_shifted"] = {"value": round(m16, 1), "unit": "MLUPS", "ms_per_step": round(ms_t16 / args.steps, 4),
                                "speedup_vs_f32": round(m16 / mlups, 3), "tuning": tun16,
@@ -731,7 +731,7 @@ def main(argv=None) -> int:
         bulkw = bulk_cells
         bw = bytes_per_lup("f32", wale=True)
         aw = bw * bulkw / (ms_kw * 1e-3) / 1e9
-        kw = "k_step_two<StF32, true, true, 0>" if ab else "k_step<StF32, regular, wale>"
+        kw = "k_step_two<StF32, true, true, 0, false, 0>" if ab else "k_step_two<StF32, true, true, 0, false, 2>"
         out["wale_on"] = {"value": round(mw, 1), "unit": "MLUPS", "ms_per_step": round(ms_tw / args.steps, 4),
                           "vs_wale_off": round(mw / mlups, 3), "c_wale": 0.2, "inlet_turbulence": 0.01,
                           "tuning": tunw, "cd_transient": round(float(Fw[0] / (0.5 * U_IN ** 2 * area)), 5),
