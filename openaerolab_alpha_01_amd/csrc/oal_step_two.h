@@ -26,19 +26,21 @@
 // Bound and shape.  The plane's 27 words are all in flight together and nothing is kept for a next plane,
 // so a lane needs 97 to 125 registers and four waves share a SIMD; their loads overlap other waves'
 // collisions.  That needs the rare limiter out of the registers (collide_cell's LDS form): with it inline
-// the kernel takes 168 and spills.  Bound: HBM in FP32 (256^3: 5.9 TB/s of 6.0 that a copy reaches counting
-// 216 bytes per cell), in the 16-bit forms VALU and HBM alike (256^3 FP16: about 720 instructions per cell, half of them
-// issued every second cycle, the others every fourth or eighth, some 70 % of the time; 4.9 TB/s).  Measured against walking four planes of a block per workgroup with the next plane's words in
-// flight (two waves per SIMD, a launch per kind of block, the default shape before): 256^3 sphere box FP32
-// 667 -> 633 us per step, FP16 467 -> 370 us; WALE 192 x 160 x 160 FP32 295 -> 232 us, WALE 200 x 120 x 104
-// FP16 200 -> 93 us; WALE 100 x 60 x 44 75 -> 20 us (that shape left 48 workgroups per launch); 12 ragged
-// boxes with solids and sponges FP16 813 -> 460 us.  Blocks run fastest: x-neighbour blocks share the lines
-// of the row ends.  One record per block (TwoRec) in place of a chain of table reads: FP16 256^3 453 -> 372
-// us, 48 x 32 x 32 13.5 -> 10.8 us.  Stores written through at device scope: 48 x 32 x 32 10.8 -> 10.2 us,
-// WALE 100 x 60 x 44 25.3 -> 20.9 us without the non-temporal hint (which 256^3 needs: 635 against 681 us).
-// (Small levels in the AB pattern take the one-cell-per-lane form since: 48 x 32 x 32 7.0 us, ONE_BLOCKS.)
-// AA 192 x 160 x 160 FP32, sphere: 340 -> 204 us per step against a pipelined kernel for the blocks off the
-// faces and a one-plane kernel for the rest (a third of the blocks); 5.2 TB/s of the pair's 216 bytes per cell.
+// the kernel takes 168 and spills.  Bound: HBM in FP32 (256^3: 5.7 TB/s counting 216 bytes per cell, 5.9
+// moved, of 6.0 that a copy reaches), in the 16-bit forms VALU and HBM alike (256^3 FP16: about 720
+// instructions per cell, half of them issued every second cycle, the others every fourth or eighth, some
+// 70 % of the time; 4.9 TB/s).  Measured against walking four planes of a block per workgroup with the
+// next plane's words in flight (two waves per SIMD, a launch per kind of block, the default shape
+// before): 256^3 sphere box FP32 667 -> 633 us per step, FP16 467 -> 370 us; WALE 192 x 160 x 160 FP32
+// 295 -> 232 us, WALE 200 x 120 x 104 FP16 200 -> 93 us; WALE 100 x 60 x 44 75 -> 20 us (that shape left
+// 48 workgroups per launch); 12 ragged boxes with solids and sponges FP16 813 -> 460 us.  Blocks run
+// fastest: x-neighbour blocks share the lines of the row ends.  One record per block (TwoRec) in place of
+// a chain of table reads: FP16 256^3 453 -> 372 us, 48 x 32 x 32 13.5 -> 10.8 us.  Stores written through
+// at device scope: 48 x 32 x 32 10.8 -> 10.2 us, WALE 100 x 60 x 44 25.3 -> 20.9 us without the non-
+// temporal hint (which 256^3 needs: 635 against 681 us). (Small levels in the AB pattern take the one-
+// cell-per-lane form since: 48 x 32 x 32 7.0 us, ONE_BLOCKS.) AA 192 x 160 x 160 FP32, sphere: 340 -> 204
+// us per step against a pipelined kernel for the blocks off the faces and a one-plane kernel for the rest
+// (a third of the blocks); 5.2 TB/s of the pair's 216 bytes per cell.
 #pragma once
 
 #include "oal_step.h"
