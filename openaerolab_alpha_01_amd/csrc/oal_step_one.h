@@ -8,9 +8,9 @@
 //
 // Bound and shape.  FP64: 27 doubles are 54 registers; with the unit-rate collision and without the positivity
 // limiter's branch a lane needs 118 (124 with WALE), so four waves share a SIMD and 64^3 cells are all resident
-// at once.  Bound: HBM (192 x 160 x 160: 5.1 TB/s of 432 bytes per cell), at 64^3 the memory-side cache and one
+// at once.  Bound: HBM (192 x 160 x 160: 5.5 TB/s of 432 bytes per cell), at 64^3 the memory-side cache and one
 // wave's latency.  Measured against a kernel per kind of block, two waves per SIMD, on two streams: 64^3
-// periodic 30.5 -> 18.5 us per step; sphere boxes 192 x 160 x 160 472 -> 416 us, with WALE 568 -> 479 us,
+// periodic 30.5 -> 18.5 us per step; sphere boxes 192 x 160 x 160 472 -> 384 us, with WALE 568 -> 479 us,
 // 100 x 60 x 44 with WALE 94 -> 28.5 us, 48 x 32 x 32 13.1 -> 7.3 us.
 // FP32 and the 16-bit forms: 58 to 62 registers, eight waves per SIMD.  A small level's step is one wave's
 // latency, and here a wave collides one cell per lane instead of two in turn: 48 x 32 x 32 FP32 10.0 -> 7.0 us
@@ -247,13 +247,19 @@ k_step_one(const StepArgs a) {
     }
 }
 
+// Dynamic LDS that no kernel uses, as TWO_HOLD_LDS: two workgroups (eight waves) on a CU where an FP64 level streams
+// through the caches.  Sphere boxes 192 x 160 x 160 418 us per step, 404 with three workgroups, 384 with two;
+// 160 x 128 x 128 with the interpolated wall 250, 228, 225 us.  With WALE it costs (480, 488, 515 us).
+constexpr uint32_t ONE_HOLD_LDS = 70000;
+
 template <class SP>
 static void launch_one_sp(bool wale, const StepArgs& r, hipStream_t stream) {
     const dim3 g(r.n_items);
     auto go = [&](auto unit, auto w, auto dith) {
         constexpr bool U = decltype(unit)::value, W = decltype(w)::value, D = decltype(dith)::value;
-        if (r.cp.limiter == 2) hipLaunchKernelGGL((k_step_one<SP, U, W, true, D>), g, dim3(WG), 0, stream, r);
-        else hipLaunchKernelGGL((k_step_one<SP, U, W, false, D>), g, dim3(WG), 0, stream, r);
+        const uint32_t hold = sizeof(typename SP::T) == 8 && !W && !r.two_keep ? ONE_HOLD_LDS : 0u;
+        if (r.cp.limiter == 2) hipLaunchKernelGGL((k_step_one<SP, U, W, true, D>), g, dim3(WG), hold, stream, r);
+        else hipLaunchKernelGGL((k_step_one<SP, U, W, false, D>), g, dim3(WG), hold, stream, r);
     };
     auto walef = [&](auto unit, auto dith) {
         if (wale) go(unit, std::true_type{}, dith);

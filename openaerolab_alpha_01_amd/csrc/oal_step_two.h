@@ -26,13 +26,13 @@
 // Bound and shape.  The plane's 27 words are all in flight together and nothing is kept for a next plane,
 // so a lane needs 97 to 125 registers and four waves share a SIMD; their loads overlap other waves'
 // collisions.  That needs the rare limiter out of the registers (collide_cell's LDS form): with it inline
-// the kernel takes 168 and spills.  Bound: HBM in FP32 (256^3: 5.7 TB/s counting 216 bytes per cell, 5.9
-// moved, of 6.0 that a copy reaches), in the 16-bit forms VALU and HBM alike (256^3 FP16: about 720
+// the kernel takes 168 and spills.  Bound: HBM in FP32 (256^3: 5.97 TB/s
+// counting 216 bytes per cell, of 6.04 that a copy reaches), in the 16-bit forms VALU and HBM alike (256^3 FP16: about 720
 // instructions per cell, half of them issued every second cycle, the others every fourth or eighth, some
 // 70 % of the time; 4.9 TB/s).  Measured against walking four planes of a block per workgroup with the
 // next plane's words in flight (two waves per SIMD, a launch per kind of block, the default shape
-// before): 256^3 sphere box FP32 667 -> 633 us per step, FP16 467 -> 370 us; WALE 192 x 160 x 160 FP32
-// 295 -> 232 us, WALE 200 x 120 x 104 FP16 200 -> 93 us; WALE 100 x 60 x 44 75 -> 20 us (that shape left
+// before): 256^3 sphere box FP32 667 -> 606 us per step, FP16 467 -> 370 us; WALE 192 x 160 x 160 FP32
+// 295 -> 229 us, WALE 200 x 120 x 104 FP16 200 -> 93 us; WALE 100 x 60 x 44 75 -> 20 us (that shape left
 // 48 workgroups per launch); 12 ragged boxes with solids and sponges FP16 813 -> 460 us.  Blocks run
 // fastest: x-neighbour blocks share the lines of the row ends.  One record per block (TwoRec) in place of
 // a chain of table reads: FP16 256^3 453 -> 372 us, 48 x 32 x 32 13.5 -> 10.8 us.  Stores written through
@@ -705,14 +705,23 @@ k_step_two(const StepArgs a) {
     if (want_force) two_sum3(F0 * force_scale, F1 * force_scale, F2 * force_scale, a.fpart, b * PLANES + (uint32_t)z);
 }
 
+// Dynamic LDS that no kernel uses: it leaves five workgroups (ten waves) on a CU instead of eight where an FP32
+// level streams through the caches.  The loads in flight on an XCD then fit its 4 MB L2 (32 CUs x 5 x 27 KB; eight
+// are 6.9 MB), so the lines at the row ends and of half rows are still there for the neighbouring workgroup.
+// 256^3 FP32: 629.9 us per step, 612 with six workgroups, 605 with five, 615 with four; WALE 192 x 160 x 160: 232,
+// 227.7, 228.2, 237; interpolated wall 160 x 128 x 128 121.9, with five 119.3.  The AA pattern (204, 209, 215 us),
+// the 16-bit forms (256^3 FP16 376, with six 436 us) and levels that stay in the memory-side cache keep all.
+constexpr uint32_t TWO_HOLD_LDS = 18000;
+
 // the blocks of one list, one plane per workgroup
 template <class SP, bool UNIT, bool DITH, bool WALE>
 static void launch_two_w(int extra, dim3 g, hipStream_t s, const StepArgs& r) {
-    if (extra == TWO_SPONGE) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_SPONGE, DITH, PAT_AB>), g, dim3(TWG), 0, s, r);
-    else if (extra == TWO_BFL) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_BFL, DITH, PAT_AB>), g, dim3(TWG), 0, s, r);
+    const uint32_t hold = SP::dithered || r.two_keep ? 0u : TWO_HOLD_LDS;
+    if (extra == TWO_SPONGE) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_SPONGE, DITH, PAT_AB>), g, dim3(TWG), hold, s, r);
+    else if (extra == TWO_BFL) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_BFL, DITH, PAT_AB>), g, dim3(TWG), hold, s, r);
     else if (extra == TWO_AA_EVEN) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_PLAIN, DITH, PAT_AA_EVEN>), g, dim3(TWG), 0, s, r);
     else if (extra == TWO_AA_ODD) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_PLAIN, DITH, PAT_AA_ODD>), g, dim3(TWG), 0, s, r);
-    else hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_PLAIN, DITH, PAT_AB>), g, dim3(TWG), 0, s, r);
+    else hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_PLAIN, DITH, PAT_AB>), g, dim3(TWG), hold, s, r);
 }
 template <class SP>
 static void launch_two_sp(bool wale, int extra, const StepArgs& r, hipStream_t s) {
