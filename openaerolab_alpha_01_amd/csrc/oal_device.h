@@ -347,6 +347,15 @@ __host__ __device__ inline void cell_rates(T nu_eddy, T tau, T amr_scale, T nu_b
     }
 }
 
+// Between a wave's LDS writes and its other lanes' reads of them.  The barrier alone orders the schedule, not
+// memory: the fences keep the accesses on their sides whatever the compiler can show about their addresses.  A
+// wave's LDS instructions run in order, so they cost no instruction.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // 27 words of LDS per lane for the rare branches of the two-cells-per-lane kernel (workgroups of 128 lanes;
 // word k of a lane at [k * 128 + lane]): one array for all of them
 __device__ __forceinline__ uint32_t* two_lds() {

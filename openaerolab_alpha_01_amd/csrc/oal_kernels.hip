@@ -471,7 +471,7 @@ __global__ void __launch_bounds__(WG) k_xfer_gather(const typename SP::st* fnew,
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) sh[wave][lane][p] = make_uint4(w[4 * p], w[4 * p + 1], w[4 * p + 2], w[4 * p + 3]);
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     const uint32_t pieces = (n - i0 < 64u ? n - i0 : 64u) * P;
     uint4* o = reinterpret_cast<uint4*>(out) + (size_t)i0 * P;
 #pragma unroll
@@ -802,7 +802,7 @@ __global__ void __launch_bounds__(XWG) k_xfer_rebuild(typename SP::st* f, uint32
         d1 = d3;
         d2 = next(d3);
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     // two lanes per cell, for a direction and its opposite: c c is the same and c u changes its sign
     const int d = lane >> 1;
     const bool opp = lane & 1;
