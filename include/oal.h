@@ -180,10 +180,10 @@ int oal_level_cells(const OalPlan* plan, int level, int64_t* n_cells);
  * boundary rule or solid link (n_regular; in the AB pattern also whole blocks on a domain face with no
  * solid near), other blocks with no boundary rule (n_interior), boundary blocks of both, and regular
  * blocks that overhang the extent (n_partial) or hold sponge cells (n_sponge).  The AB pattern with FP32
- * arithmetic steps them in one launch of the two-cells-per-lane kernel, but for blocks with an absent
+ * arithmetic steps them in one launch (levels beyond 4 GiB: two) of the two-cells-per-lane kernel, but for blocks with an absent
  * neighbour inside the extent, under the exact specular z wall or the transverse freestream, next to
- * solid cells with OAL_BB_REFERENCE, or whose neighbours lie 4 GiB of populations apart; these, and in
- * FP64 and the AA pattern the boundary blocks, are launched on a second stream that overlaps the bulk
+ * solid cells with OAL_BB_REFERENCE, or whose neighbours in one block layer lie 4 GiB of populations
+ * apart; these, and in FP64 and the AA pattern the boundary blocks, are launched on a second stream that overlaps the bulk
  * launches.  The bulk launches that oal_time_steps times (ms_kernel) are the two-cells-per-lane kernel's,
  * or the n_regular and n_interior blocks'. */
 typedef struct OalLevelInfo {

@@ -5,12 +5,10 @@
 #include <stdint.h>
 
 #include "oal_device.h"
+#include "oal_records.h"
 
 namespace oal {
 
-constexpr int BS = 16;            // cells per block edge
-constexpr int BS2 = BS * BS;
-constexpr int BS3 = BS * BS * BS;
 constexpr int WG = 256;           // threads per workgroup: one 16 x 16 plane of a block
 constexpr int PLANES = BS;        // workgroups per block in the step kernels
 
@@ -40,33 +38,6 @@ struct DevDomain {
     int32_t pad;
 };
 
-// All a workgroup of a one-launch step kernel (k_step_two, k_step_one) reads about its block, one record per entry of a block
-// list: one round of scalar loads in place of a chain (list entry, block tables, domain).  Neighbour
-// offsets are in bytes of populations from the lowest block among the neighbours and the block (absent:
-// the block's own), so that 32 bits reach every one.
-struct TwoRec {
-    uint32_t off[27];          // by (dx + 1) + 3 (dy + 1) + 9 (dz + 1); [13]: the block itself
-    uint32_t base;             // the lowest block
-    uint32_t block;
-    uint32_t flags;            // BF_* and TR_*
-    int32_t org[3];
-    int32_t lslot, sslot, oslot;   // link-mask, sponge and outlet-copy slots
-    int32_t ext[3];
-    float u_in, omega1, omega4d, F[3], tau, amr_scale, force_scale;
-    uint32_t cell0;
-    uint32_t face[6];          // neighbour blocks x+, x-, y+, y-, z+, z- (WALE; absent: the block itself)
-    uint32_t pad0;
-    double omega1_d, omega4d_d;   // FP64 form
-    uint32_t pad[4];
-};
-static_assert(sizeof(TwoRec) == 256, "a record is four cache lines of the scalar cache");
-enum : uint32_t {
-    TR_PER_X = 1u << 8, TR_PER_Y = 1u << 9, TR_PER_Z = 1u << 10,   // periodic axes
-    TR_ZWALL = 1u << 11, TR_YMIN = 1u << 12,                       // no-slip z faces, no-slip y-min face
-    TR_FORCED = 1u << 13,
-    TR_ABSENT = 1u << 16       // shifted by 0..5: the face neighbour is absent
-};
-
 // arguments of the fused stream-collide kernels
 struct StepArgs {
     const void* fin;             // populations read this step
@@ -87,16 +58,17 @@ struct StepArgs {
     const int32_t* blist_boundary_regular;  // [n_boundary_regular] boundary blocks with lexicographic neighbours
     const int32_t* blist_boundary;   // [n_boundary] the other blocks
     uint32_t n_regular, n_interior, n_boundary_regular, n_boundary;
-    // the one-launch kernels' blocks (FP32 arithmetic, and FP64 in the AB pattern; blist_boundary_regular and
-    // blist_boundary then hold the blocks they do not take): without sponge cells, with sponge cells, and
-    // the former split into those with solid links near and the others
+    // the one-launch kernels' blocks (FP32 arithmetic, and FP64 in the AB pattern; blist_interior,
+    // blist_boundary_regular and blist_boundary then hold the blocks they do not take): without sponge cells, with
+    // sponge cells, and the former split into those with solid links near and the others.  Blocks of the WIDE form
+    // follow the n_two records of `two`, those without solid links the n_two_free of two_free.
     const TwoRec* rec;           // the records of this launch (set per launch)
     const TwoRec* two;
     const TwoRec* two_sponge;
     const TwoRec* two_links;
     const TwoRec* two_free;
     int32_t two_keep;            // the level's population buffers stay in the memory-side cache between steps
-    uint32_t n_two, n_two_sponge, n_two_links, n_two_free;
+    uint32_t n_two, n_two_sponge, n_two_links, n_two_free, n_two_wide, n_two_wide_free;
     const int32_t* lslot;        // [nb] link-mask slot of a block with solid cells near, -1 = none
     const uint32_t* lmask;       // [n_lslots * BS3] per cell: bit k source of direction k solid, bit 27 cell solid
     const int32_t* oslot;        // [nb] AA pattern: outlet side-buffer slot of the block, -1 = none
@@ -124,12 +96,6 @@ struct StepArgs {
     CollParams cp;
     __device__ __forceinline__ int32_t step() const { return ts_dev ? ts_dev[0] * ts_mul + ts_add : time_step; }
 };
-
-// Whether the two-cells-per-lane kernel's 32-bit byte offsets span a block's neighbours (block indices lo to
-// hi, populations of `esize` bytes)
-inline bool two_fits(int64_t lo, int64_t hi, uint64_t esize) {
-    return (uint64_t)(hi - lo + 1) * 27ull * BS3 * esize < (1ull << 32);
-}
 
 // Population bytes of a level (both buffers) up to which the two-cells-per-lane kernel's stores are left in
 // the memory-side cache
@@ -179,12 +145,13 @@ void launch_two_f16s(bool wale, int extra, const StepArgs& a, hipStream_t stream
 void launch_two_bf16s(bool wale, int extra, const StepArgs& a, hipStream_t stream);
 // and over the n blocks of a list, by storage code
 void launch_two(int storage, bool wale, int extra, const TwoRec* rec, uint32_t n, hipStream_t stream, const StepArgs& a);
-// likewise the one-cell-per-lane step kernel (AB pattern): oal_one_<storage>.hip
+// likewise the one-cell-per-lane step kernel (AB pattern): oal_one_<storage>.hip; wide: FP64 only (the other forms
+// take small levels here, ONE_BLOCKS, which 32 bits span)
 void launch_one_f32(bool wale, const StepArgs& a, hipStream_t stream);
-void launch_one_f64(bool wale, const StepArgs& a, hipStream_t stream);
+void launch_one_f64(bool wale, bool wide, const StepArgs& a, hipStream_t stream);
 void launch_one_f16s(bool wale, const StepArgs& a, hipStream_t stream);
 void launch_one_bf16s(bool wale, const StepArgs& a, hipStream_t stream);
-void launch_one(int storage, bool wale, const TwoRec* rec, uint32_t n, hipStream_t stream, const StepArgs& a);
+void launch_one(int storage, bool wale, bool wide, const TwoRec* rec, uint32_t n, hipStream_t stream, const StepArgs& a);
 hipError_t launch_copy16(const void* src, void* dst, size_t bytes, hipStream_t stream);
 // Host arrays of init / conversion / macro output cover the first nhost cells of a level (the caller's
 // blocks); the device arrays have ncell cells per direction.

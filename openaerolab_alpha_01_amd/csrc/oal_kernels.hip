@@ -30,15 +30,14 @@ void launch_two(int storage, bool wale, int extra, const TwoRec* rec, uint32_t n
     }
 }
 
-void launch_one(int storage, bool wale, const TwoRec* rec, uint32_t n, hipStream_t stream, const StepArgs& a) {
+void launch_one(int storage, bool wale, bool wide, const TwoRec* rec, uint32_t n, hipStream_t stream, const StepArgs& a) {
     if (!n) return;
     StepArgs r = a;
     r.rec = rec;
-    r.nb = n;
     r.n_items = n * PLANES;
     switch (storage) {
         case 0: launch_one_f32(wale, r, stream); break;
-        case 1: launch_one_f64(wale, r, stream); break;
+        case 1: launch_one_f64(wale, wide, r, stream); break;
         case 2: launch_one_f16s(wale, r, stream); break;
         default: launch_one_bf16s(wale, r, stream); break;
     }

@@ -3,6 +3,6 @@
 
 namespace oal {
 
-void launch_one_f64(bool wale, const StepArgs& a, hipStream_t stream) { launch_one_sp<StF64>(wale, a, stream); }
+void launch_one_f64(bool wale, bool wide, const StepArgs& a, hipStream_t stream) { launch_one_sp<StF64>(wale, a, stream, wide); }
 
 }  // namespace oal

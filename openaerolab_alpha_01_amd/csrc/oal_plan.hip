@@ -106,15 +106,17 @@ struct Level {
     uint32_t n_sponge = 0;             // regular blocks with sponge cells, no solid near (AB)
     uint32_t n_face = 0;               // AB: face cells of the regular-list blocks
     // the one-launch kernels' blocks (FP32 arithmetic, and FP64 in the AB pattern): without and with sponge cells,
-    // the former also split by solid links near (interpolated bounce-back); the boundary blocks it does not
-    // take, with and without lexicographic neighbours
+    // the former also split by solid links near (interpolated bounce-back), blocks of the WIDE form after the others;
+    // the blocks they do not take: without a rule, and boundary blocks with and without lexicographic neighbours
     DevBuf<TwoRec> rec_tw, rec_ts, rec_tl, rec_tn;
-    DevBuf<int32_t> blist_xr, blist_xb;
-    uint32_t n_two = 0, n_two_sponge = 0, n_two_links = 0, n_two_free = 0, n_rest_regular = 0, n_rest = 0;
-    std::vector<char> two_fit_h;       // a block's neighbours lie within that kernel's 32-bit offsets
+    DevBuf<int32_t> blist_xi, blist_xr, blist_xb;
+    uint32_t n_two = 0, n_two_sponge = 0, n_two_links = 0, n_two_free = 0, n_two_wide = 0, n_two_wide_free = 0;
+    uint32_t n_rest_interior = 0, n_rest_regular = 0, n_rest = 0, n_rest_links = 0;
+    std::vector<char> two_fit_h;       // how those kernels' 32-bit offsets span a block's neighbours (FIT_*)
     std::vector<int32_t> nbr_h;        // [32 * nb] neighbour rows (the device's nbr)
     uint32_t esize = 4;                // bytes of a stored population
     bool two() const { return fp32 || ab; }
+    bool bulk() const { return two() ? n_two + n_two_wide + n_two_sponge > 0 : n_regular + n_interior > 0; }
     DevBuf<int32_t> lslot;             // link-mask slot per block
     DevBuf<uint32_t> lmask;            // per-cell solid-link masks of blocks near solid cells
     std::vector<int32_t> lslot_h;      // host copy of lslot
@@ -191,7 +193,7 @@ struct Level {
     void release() {
         nbr.release(); borg.release(); bdom.release(); dom_item0.release(); dom_block0.release();
         bflags.release(); solid.release(); doms.release(); fA.release(); fB.release(); velA.release(); velB.release();
-        rec_tw.release(); rec_ts.release(); rec_tl.release(); rec_tn.release(); blist_xr.release(); blist_xb.release();
+        rec_tw.release(); rec_ts.release(); rec_tl.release(); rec_tn.release(); blist_xi.release(); blist_xr.release(); blist_xb.release();
         fpart.release(); mpart.release(); red_out.release(); guard.release(); oslot.release(); obuf.release(); blist_rg.release(); blist_in.release(); blist_br.release(); blist_bd.release();
         c8map_d.release(); lslot.release(); lmask.release(); qmap.release(); sponge.release(); sslot.release();
         g_src.release(); g_dst.release(); g_slot.release(); g_w.release(); g_same.release(); g_m.release();
@@ -288,7 +290,7 @@ int upload(DevBuf<T>& d, const std::vector<T>& h) {
 // Host tables of one level, built and validated before any device call
 struct HostLevel {
     std::vector<int32_t> borg, bdom, nbr, nbr_bm, oslot, blist_rg, blist_in, blist_br, blist_bd,
-        blist_tw, blist_ts, blist_tl, blist_tn, blist_xr, blist_xb, lslot;
+        blist_tw, blist_ts, blist_tl, blist_tn, blist_ww, blist_wl, blist_wn, blist_xi, blist_xr, blist_xb, lslot;
     std::vector<TwoRec> rec_tw, rec_ts, rec_tl, rec_tn;
     std::vector<uint32_t> lmask;
     int32_t n_oslots = 0;
@@ -301,7 +303,9 @@ struct HostLevel {
 void build_lists(Level& L, HostLevel& H) {
     H.blist_rg.clear(); H.blist_in.clear(); H.blist_br.clear(); H.blist_bd.clear();
     L.n_partial = L.n_sponge = L.n_face = 0;
-    for (auto* l : {&H.blist_tw, &H.blist_ts, &H.blist_tl, &H.blist_tn, &H.blist_xr, &H.blist_xb}) l->clear();
+    for (auto* l : {&H.blist_tw, &H.blist_ts, &H.blist_tl, &H.blist_tn, &H.blist_ww, &H.blist_wl, &H.blist_wn, &H.blist_xi,
+                    &H.blist_xr, &H.blist_xb})
+        l->clear();
     const std::vector<uint32_t>& flags = L.flags_h;
     // blocks on a face whose rule the two-cells kernel does not apply (the exact specular z wall reads
     // another cell of the wall row; the transverse freestream blends): the general kernels step them
@@ -323,13 +327,18 @@ void build_lists(Level& L, HostLevel& H) {
         // the one-launch kernels take every block but those with an absent neighbour inside the
         // extent, those under the exact specular z wall or the transverse freestream, those near solid
         // cells with the reference's reflection, and those whose neighbours their 32-bit offsets do not span
-        // (4 GiB of populations: the wraps of periodic levels and the ghosts of octree levels beyond that)
+        // (4 GiB of populations), all from one base nor, without a sponge, each layer from its own (the wraps
+        // of y-periodic levels and the ghosts of octree levels beyond that)
         // (the FP64 form has none with a sponge)
-        if ((flags[b] & BF_MISSING) || special || !L.two_fit_h[b] || ((flags[b] & BF_SOLID) && !L.bb_halfway) ||
-            (!L.fp32 && (flags[b] & BF_SPONGE))) {
-            (regular ? H.blist_xr : H.blist_xb).push_back((int32_t)b);
+        const char fit = L.two_fit_h[b];
+        if ((flags[b] & BF_MISSING) || special || fit == FIT_NONE || ((flags[b] & BF_SOLID) && !L.bb_halfway) ||
+            ((flags[b] & BF_SPONGE) && (!L.fp32 || fit != FIT_ALL))) {
+            (flags[b] == 0 ? H.blist_xi : regular ? H.blist_xr : H.blist_xb).push_back((int32_t)b);
         } else if (flags[b] & BF_SPONGE) {
             H.blist_ts.push_back((int32_t)b);
+        } else if (fit == FIT_LAYERS) {
+            H.blist_ww.push_back((int32_t)b);
+            ((flags[b] & BF_SOLID) ? H.blist_wl : H.blist_wn).push_back((int32_t)b);
         } else {
             H.blist_tw.push_back((int32_t)b);
             ((flags[b] & BF_SOLID) ? H.blist_tl : H.blist_tn).push_back((int32_t)b);
@@ -371,26 +380,29 @@ void build_lists(Level& L, HostLevel& H) {
     L.n_two_sponge = (uint32_t)H.blist_ts.size();
     L.n_two_links = (uint32_t)H.blist_tl.size();
     L.n_two_free = (uint32_t)H.blist_tn.size();
+    L.n_two_wide = (uint32_t)H.blist_ww.size();
+    L.n_two_wide_free = (uint32_t)H.blist_wn.size();
+    L.n_rest_interior = (uint32_t)H.blist_xi.size();
     L.n_rest_regular = (uint32_t)H.blist_xr.size();
     L.n_rest = (uint32_t)H.blist_xb.size();
-    // FP64 with interpolated bounce-back: the general kernel steps the blocks with solid links too
+    // interpolated bounce-back: in FP64 the general kernel steps the blocks with solid links too, in the other
+    // forms those of the WIDE form
     if (!L.fp32) H.blist_xb.insert(H.blist_xb.end(), H.blist_tl.begin(), H.blist_tl.end());
+    H.blist_xb.insert(H.blist_xb.end(), H.blist_wl.begin(), H.blist_wl.end());
+    L.n_rest_links = (uint32_t)H.blist_xb.size() - L.n_rest;
 }
 
 // The records of the one-launch kernels' block lists; slot: the sponge slots (empty: none)
 void build_two_recs(const Level& L, HostLevel& H, const std::vector<int32_t>& sslot) {
-    auto make = [&](const std::vector<int32_t>& list, std::vector<TwoRec>& out) {
-        out.assign(list.size(), TwoRec{});
-        for (size_t i = 0; i < list.size(); ++i) {
-            const uint32_t b = (uint32_t)list[i];
+    auto make = [&](const std::vector<int32_t>& list, const std::vector<int32_t>& wide, std::vector<TwoRec>& out) {
+        out.assign(list.size() + wide.size(), TwoRec{});
+        for (size_t i = 0; i < out.size(); ++i) {
+            const bool layers = i >= list.size();
+            const uint32_t b = (uint32_t)(layers ? wide[i - list.size()] : list[i]);
             const int32_t* nt = L.nbr_h.data() + (size_t)b * 32;
             const DevDomain& dm = L.doms_h[L.bdom_h[b]];
             TwoRec& r = out[i];
-            uint32_t lo = b;
-            for (int k = 0; k < 27; ++k)
-                if (nt[k] >= 0) lo = std::min(lo, (uint32_t)nt[k]);
-            for (int k = 0; k < 27; ++k) r.off[k] = ((nt[k] < 0 ? b : (uint32_t)nt[k]) - lo) * (27u * BS3 * L.esize);
-            r.base = lo;
+            two_offsets(nt, b, layers, L.esize, r);
             r.block = b;
             r.flags = L.flags_h[b] | (dm.per[0] ? TR_PER_X : 0u) | (dm.per[1] ? TR_PER_Y : 0u) | (dm.per[2] ? TR_PER_Z : 0u) |
                       (dm.zwall != 0 ? TR_ZWALL : 0u) | (dm.ymin_wall == 1 ? TR_YMIN : 0u) | (dm.forced ? TR_FORCED : 0u);
@@ -419,10 +431,10 @@ void build_two_recs(const Level& L, HostLevel& H, const std::vector<int32_t>& ss
         }
     };
     if (!L.two()) return;
-    make(H.blist_tw, H.rec_tw);
-    make(H.blist_ts, H.rec_ts);
-    make(H.blist_tl, H.rec_tl);
-    make(H.blist_tn, H.rec_tn);
+    make(H.blist_tw, H.blist_ww, H.rec_tw);
+    make(H.blist_ts, {}, H.rec_ts);
+    make(H.blist_tl, {}, H.rec_tl);
+    make(H.blist_tn, H.blist_wn, H.rec_tn);
 }
 
 // Host-side construction of one level's tables from the reference-convention descriptor.
@@ -562,8 +574,8 @@ int prepare_level(const OalLevelDesc& d, const OalCollision& coll, bool ab, bool
         dm.nbx = (dm.ext[0] + BS - 1) / BS;
         dm.nby = (dm.ext[1] + BS - 1) / BS;
     }
-    // the in-kernel face rules address by signed 32-bit byte offsets from a block: only domains whose
-    // layer of blocks (plus a row and a block) spans less than 2 GiB may use them
+    // (reported only, OalLevelInfo.n_partial and n_sponge: domains whose layer of blocks, plus a row and a block,
+    // spans less than 2 GiB)
     std::vector<char> near(L.doms_h.size());
     for (size_t i = 0; i < L.doms_h.size(); ++i) {
         const DevDomain& dm = L.doms_h[i];
@@ -586,21 +598,13 @@ int prepare_level(const OalLevelDesc& d, const OalCollision& coll, bool ab, bool
     }
     // block-major copy of the neighbour table: one 32-entry row per block (scalar loads)
     H.nbr_bm.assign((size_t)nb * 32, -1);
-    // (and whether the two-cells-per-lane kernel's 32-bit byte offsets, from the lowest index among them,
-    // reach the highest)
+    // (and how the one-launch kernels' 32-bit byte offsets span its neighbours)
     L.two_fit_h.assign(nb, 0);
     L.esize = (uint32_t)sbytes;
     for (uint32_t b = 0; b < nb; ++b) {
-        int32_t lo = (int32_t)b, hi = (int32_t)b;
-        for (int k = 0; k < 27; ++k) {
-            const int32_t n = k == 13 ? (int32_t)b : nbr[(size_t)k * nb + b];
-            H.nbr_bm[(size_t)b * 32 + k] = n;
-            if (n >= 0) {
-                lo = std::min(lo, n);
-                hi = std::max(hi, n);
-            }
-        }
-        L.two_fit_h[b] = two_fits(lo, hi, (uint64_t)sbytes) ? 1 : 0;
+        int32_t* nt = H.nbr_bm.data() + (size_t)b * 32;
+        for (int k = 0; k < 27; ++k) nt[k] = k == 13 ? (int32_t)b : nbr[(size_t)k * nb + b];
+        L.two_fit_h[b] = two_fit(nt, b, (uint64_t)sbytes);
     }
     if (fp32 || ab) L.nbr_h = H.nbr_bm;
     L.near_h = near;
@@ -1118,8 +1122,8 @@ int upload_level(OalPlan* p, Level& L, const HostLevel& H) {
     if ((rc = upload(L.blist_rg, H.blist_rg)) || (rc = upload(L.blist_in, H.blist_in)) ||
         (rc = upload(L.blist_br, H.blist_br)) || (rc = upload(L.blist_bd, H.blist_bd)) ||
         (rc = upload(L.rec_tw, H.rec_tw)) || (rc = upload(L.rec_ts, H.rec_ts)) || (rc = upload(L.rec_tl, H.rec_tl)) ||
-        (rc = upload(L.rec_tn, H.rec_tn)) || (rc = upload(L.blist_xr, H.blist_xr)) || (rc = upload(L.blist_xb, H.blist_xb)) ||
-        (rc = upload(L.lslot, H.lslot)) || (rc = upload(L.lmask, H.lmask)))
+        (rc = upload(L.rec_tn, H.rec_tn)) || (rc = upload(L.blist_xi, H.blist_xi)) || (rc = upload(L.blist_xr, H.blist_xr)) ||
+        (rc = upload(L.blist_xb, H.blist_xb)) || (rc = upload(L.lslot, H.lslot)) || (rc = upload(L.lmask, H.lmask)))
         return rc;
     if (p->stream_mode == OAL_STREAM_AA) {
         if ((rc = upload(L.oslot, H.oslot))) return rc;
@@ -1198,11 +1202,15 @@ StepArgs make_args(OalPlan* p, Level& L, int32_t time_step, bool want_force) {
     a.n_two_links = L.n_two_links;
     a.two_free = L.rec_tn.p;
     a.n_two_free = L.n_two_free;
-    if (L.two()) {   // the boundary kernels keep the blocks it does not take
+    a.n_two_wide = L.n_two_wide;
+    a.n_two_wide_free = L.n_two_wide_free;
+    if (L.two()) {   // the one-plane kernels keep the blocks it does not take
+        a.blist_interior = L.blist_xi.p;
+        a.n_interior = L.n_rest_interior;
         a.blist_boundary_regular = L.blist_xr.p;
         a.n_boundary_regular = L.n_rest_regular;
         a.blist_boundary = L.blist_xb.p;
-        a.n_boundary = L.n_rest + (!L.fp32 && L.qmap.p ? L.n_two_links : 0);
+        a.n_boundary = L.n_rest + (L.qmap.p ? L.n_rest_links : 0);
     }
     a.qmap = L.qmap.p;
     a.sponge = L.has_sponge ? L.sponge.p : nullptr;
@@ -1222,9 +1230,7 @@ int level_step(OalPlan* p, int level, int32_t time_step, int flags, hipStream_t 
     if (want_force && !L.has_solid) return fail(OAL_ERR_STATE, "force requested on a level without obstacle cells");
     StepArgs a = make_args(p, L, time_step, want_force);
     // side-stream work: the boundary lists
-    const bool split = p->overlap && (L.two() ? a.n_two + a.n_two_sponge > 0 && a.n_boundary_regular + a.n_boundary > 0
-                                              : L.n_regular + L.n_interior > 0 &&
-                                                    L.n_boundary_regular + L.n_boundary > 0);
+    const bool split = p->overlap && L.bulk() && a.n_boundary_regular + a.n_boundary + (L.two() ? a.n_interior : 0) > 0;
     if (split) {
         // fork: the side stream starts after everything queued on s, then s waits for the side stream
         OAL_HIP(hipEventRecord(p->fork, s));
@@ -2184,7 +2190,7 @@ int oal_time_steps(OalPlan* p, int level, int n, int flags, double* ms_total, do
     OAL_HIP(hipSetDevice(p->device));
     OAL_HIP(hipStreamSynchronize(p->stream));
     const Level& L = p->levels[level];
-    const bool bulk = L.two() ? L.n_two + L.n_two_sponge > 0 : L.n_regular + L.n_interior > 0;
+    const bool bulk = L.bulk();
     if (bulk) {
         while (p->bulk_ev.size() < 2 * (size_t)n) {
             hipEvent_t e = nullptr;
@@ -2309,9 +2315,8 @@ static int set_sponge_lib(OalPlan* p, int level, const float* sponge, int32_t bl
     int rc;
     if ((rc = re(L.bflags, L.flags_h)) || (rc = re(L.blist_rg, H.blist_rg)) || (rc = re(L.blist_in, H.blist_in)) ||
         (rc = re(L.blist_br, H.blist_br)) || (rc = re(L.blist_bd, H.blist_bd)) ||
-       
         (rc = re(L.rec_tw, H.rec_tw)) || (rc = re(L.rec_ts, H.rec_ts)) || (rc = re(L.rec_tl, H.rec_tl)) ||
-        (rc = re(L.rec_tn, H.rec_tn)) || (rc = re(L.blist_xr, H.blist_xr)) || (rc = re(L.blist_xb, H.blist_xb)) ||
+        (rc = re(L.rec_tn, H.rec_tn)) || (rc = re(L.blist_xi, H.blist_xi)) || (rc = re(L.blist_xr, H.blist_xr)) || (rc = re(L.blist_xb, H.blist_xb)) ||
         (rc = re(L.sponge, vals)) || (rc = re(L.sslot, slot)))
         return rc;
     L.has_sponge = !vals.empty();

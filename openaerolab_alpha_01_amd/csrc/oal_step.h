@@ -39,8 +39,8 @@ enum : int {
 };
 
 // what a level needs beside the plain step in the two-cells-per-lane kernel
-// (or which half-step of the AA pattern)
-enum : int { TWO_PLAIN = 0, TWO_SPONGE = 1, TWO_BFL = 2, TWO_AA_EVEN = 3, TWO_AA_ODD = 4 };
+// (or which half-step of the AA pattern, or the plain form of blocks with a base per layer)
+enum : int { TWO_PLAIN = 0, TWO_SPONGE = 1, TWO_BFL = 2, TWO_AA_EVEN = 3, TWO_AA_ODD = 4, TWO_WIDE = 5, TWO_AA_ODD_WIDE = 6 };
 
 enum : int { PAT_AB = 0, PAT_AA_EVEN = 1, PAT_AA_ODD = 2 };
 
@@ -662,6 +662,12 @@ template <class SP, int PAT, bool WALE>
 static void launch_boundary(const StepArgs& a, hipStream_t bs) {
     StepArgs r = a;
     const bool bfl = PAT == PAT_AB && a.qmap != nullptr;
+    if constexpr (sizeof(typename SP::T) == 4 || PAT == PAT_AB) {   // blocks without a rule that the one-launch kernels
+        if (a.n_interior) {                                         // do not span
+            r.blist = a.blist_interior;
+            hipLaunchKernelGGL((k_step<SP, PAT, WALE, SEL_INTERIOR>), dim3(a.n_interior * PLANES), dim3(WG), 0, bs, r);
+        }
+    }
     if (a.n_boundary_regular) {
         r.blist = a.blist_boundary_regular;
         const dim3 g(a.n_boundary_regular * PLANES);
@@ -696,7 +702,7 @@ static void launch_boundary(const StepArgs& a, hipStream_t bs) {
 
 // One step of a level: launches over disjoint block lists.
 //   FP32 arithmetic: the two-cells-per-lane kernel for every block but a few kinds, those on the one-plane
-//     boundary kernel; on small levels in the AB pattern the one-cell-per-lane kernel in its place.
+//     interior and boundary kernels; on small levels in the AB pattern the one-cell-per-lane kernel in its place.
 //   FP64, AB pattern: likewise the one-cell-per-lane kernel.
 //   FP64, AA pattern: regular, other interior, regular boundary and boundary blocks, each on a kernel
 //     compiled for its own register budget.
@@ -713,18 +719,25 @@ static hipError_t launch_pat(const StepArgs& a, hipStream_t stream, hipStream_t 
     }
     if constexpr (two) {
         if constexpr (PAT != PAT_AB) {
-            launch_two(SP::code, WALE, PAT == PAT_AA_EVEN ? TWO_AA_EVEN : TWO_AA_ODD, a.two, a.n_two, stream, a);
+            // (the even half-step stays in the block's own slots: its records serve both forms)
+            launch_two(SP::code, WALE, PAT == PAT_AA_EVEN ? TWO_AA_EVEN : TWO_AA_ODD, a.two,
+                       a.n_two + (PAT == PAT_AA_EVEN ? a.n_two_wide : 0), stream, a);
+            if (PAT == PAT_AA_ODD) launch_two(SP::code, WALE, TWO_AA_ODD_WIDE, a.two + a.n_two, a.n_two_wide, stream, a);
         } else if (a.qmap) {   // interpolated bounce-back: its form of the kernel where there are solid links
             launch_two(SP::code, WALE, TWO_BFL, a.two_links, a.n_two_links, stream, a);
             launch_two(SP::code, WALE, TWO_PLAIN, a.two_free, a.n_two_free, stream, a);
+            launch_two(SP::code, WALE, TWO_WIDE, a.two_free + a.n_two_free, a.n_two_wide_free, stream, a);
         } else {
-            if (a.n_two <= (WALE ? ONE_BLOCKS / 2 : ONE_BLOCKS)) launch_one(SP::code, WALE, a.two, a.n_two, stream, a);
+            if (a.n_two <= (WALE ? ONE_BLOCKS / 2 : ONE_BLOCKS)) launch_one(SP::code, WALE, false, a.two, a.n_two, stream, a);
             else launch_two(SP::code, WALE, TWO_PLAIN, a.two, a.n_two, stream, a);
+            launch_two(SP::code, WALE, TWO_WIDE, a.two + a.n_two, a.n_two_wide, stream, a);
             launch_two(SP::code, WALE, TWO_SPONGE, a.two_sponge, a.n_two_sponge, stream, a);
         }
     } else if constexpr (PAT == PAT_AB) {   // (with interpolated bounce-back the boundary lists hold the links)
-        if (a.qmap) launch_one(SP::code, WALE, a.two_free, a.n_two_free, stream, a);
-        else launch_one(SP::code, WALE, a.two, a.n_two, stream, a);
+        const TwoRec* rec = a.qmap ? a.two_free : a.two;
+        const uint32_t n = a.qmap ? a.n_two_free : a.n_two;
+        launch_one(SP::code, WALE, false, rec, n, stream, a);
+        launch_one(SP::code, WALE, true, rec + n, a.qmap ? a.n_two_wide_free : a.n_two_wide, stream, a);
     } else {
         StepArgs r = a;
         if (a.n_regular) {

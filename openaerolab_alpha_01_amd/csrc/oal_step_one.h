@@ -80,7 +80,8 @@ constexpr int one_waves(bool unit, bool wale, bool pos) {
     if (sizeof(typename SP::T) == 8) return pos ? 2 : unit ? 4 : 3;
     return pos ? 3 : unit ? 8 : wale ? 5 : 6;
 }
-template <class SP, bool UNIT, bool WALE, bool POS, bool DITH>
+// WIDE: as in k_step_two (a lane whose rule takes its own population loads it apart)
+template <class SP, bool UNIT, bool WALE, bool POS, bool DITH, bool WIDE = false>
 __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(one_waves<SP>(UNIT, WALE, POS))))
 k_step_one(const StepArgs a) {
     using T = typename SP::T;
@@ -143,6 +144,8 @@ k_step_one(const StepArgs a) {
                 const int dz = sz < 0 ? -1 : (sz >= BS ? 1 : 0);
                 auto boff = [&](int dx, int dy) -> uint32_t { return R.off[(dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)]; };
                 const uint32_t zs = (uint32_t)(sz & (BS - 1)) * (BS2 * es);
+                __amdgpu_buffer_rsrc_t fz = fin;
+                if constexpr (WIDE && cz != 0) fz = buf_layer<WIDE>(a.fin, R, dz, blk);
                 const uint32_t in_row = (uint32_t)((ly - cy) & (BS - 1)) * (BS * es) + (uint32_t)lx * es;
                 const uint32_t c0 = boff(0, 0);
                 // (a row's end is 16 cells from its start: - es becomes + 15 es, and the other way round)
@@ -165,16 +168,26 @@ k_step_one(const StepArgs a) {
                         if constexpr (decltype(rules)::value) {
                             // (whole offsets: a difference of slots would wrap below zero)
                             uint32_t w = o + ((uint32_t)K * slot + zs);
+                            bool ownp = (c.lmask >> K) & 1u;
                             if constexpr (cy != 0 || cz != 0) {
                                 int j;
                                 const bool face = two_row_rule<K>(fc, j);
+                                ownp = ownp || face;
                                 w = face ? own + (uint32_t)j * slot : w;
                             }
                             w = (c.lmask >> K) & 1u ? own + (uint32_t)dopp(K) * slot : w;
-                            if constexpr (cx < 0) w = outlet ? own + (uint32_t)K * slot : w;
-                            s[K] = W::ld(fin, w, 0);
+                            if constexpr (cx < 0) {
+                                ownp = ownp || outlet;
+                                w = outlet ? own + (uint32_t)K * slot : w;
+                            }
+                            if constexpr (WIDE && cz != 0) {
+                                if (ownp) s[K] = W::ld(fin, w, 0);
+                                else s[K] = W::ld(fz, w, 0);
+                            } else {
+                                s[K] = W::ld(fin, w, 0);
+                            }
                         } else {
-                            s[K] = W::ld(fin, o, (uint32_t)K * slot + zs);
+                            s[K] = W::ld(fz, o, (uint32_t)K * slot + zs);
                         }
                     }
                 });
@@ -253,11 +266,21 @@ k_step_one(const StepArgs a) {
 constexpr uint32_t ONE_HOLD_LDS = 70000;
 
 template <class SP>
-static void launch_one_sp(bool wale, const StepArgs& r, hipStream_t stream) {
+static void launch_one_sp(bool wale, const StepArgs& r, hipStream_t stream, bool wide = false) {
     const dim3 g(r.n_items);
     auto go = [&](auto unit, auto w, auto dith) {
         constexpr bool U = decltype(unit)::value, W = decltype(w)::value, D = decltype(dith)::value;
         const uint32_t hold = sizeof(typename SP::T) == 8 && !W && !r.two_keep ? ONE_HOLD_LDS : 0u;
+        if constexpr (sizeof(typename SP::T) == 8) {
+            if (wide && r.cp.limiter == 2) {
+                hipLaunchKernelGGL((k_step_one<SP, U, W, true, D, true>), g, dim3(WG), hold, stream, r);
+                return;
+            }
+            if (wide) {
+                hipLaunchKernelGGL((k_step_one<SP, U, W, false, D, true>), g, dim3(WG), hold, stream, r);
+                return;
+            }
+        }
         if (r.cp.limiter == 2) hipLaunchKernelGGL((k_step_one<SP, U, W, true, D>), g, dim3(WG), hold, stream, r);
         else hipLaunchKernelGGL((k_step_one<SP, U, W, false, D>), g, dim3(WG), hold, stream, r);
     };

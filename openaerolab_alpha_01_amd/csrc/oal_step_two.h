@@ -130,6 +130,12 @@ struct Two<StF32> {
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_at(const void* p) {
     return __builtin_amdgcn_make_buffer_rsrc((char*)p, (short)0, (int)0xffffffff, 0x00020000);
 }
+// the populations that a record's offsets of layer dz (uniform) are counted from
+template <bool WIDE, class REC>
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_layer(const void* p, const REC& R, int dz, uint32_t blk) {
+    const uint32_t base = !WIDE || dz == 0 ? R.base : R.base_z[dz < 0 ? 0 : 1];
+    return buf_at((const char*)p + (size_t)base * blk);
+}
 
 // the rules of a lane's row (both cells share y and z) and of its cells
 struct TwoFaces {
@@ -194,8 +200,8 @@ enum : int { TWO_ST_KEEP = 16, TWO_ST_STREAM = 18, TWO_ST_SCATTER = 0 };
 // evaluated from the fresh state and stored in the own slot J, which the even half-step reads; an inlet
 // link is left to the even half-step.  A lane's rows are its own in both passes, and of the words at the
 // row ends each workgroup reads and writes its own cells only, so no access meets another's.
-template <class SP, class REC, class WORD>
-__device__ __forceinline__ void two_scatter(const REC& R, __amdgpu_buffer_rsrc_t fo, int z, int jx, int ly, bool edge,
+template <class SP, bool WIDE, class REC, class WORD>
+__device__ __forceinline__ void two_scatter(const REC& R, void* fout, __amdgpu_buffer_rsrc_t fown, int z, int jx, int ly, bool edge,
                                             const TwoFaces& fc, uint32_t lf, uint32_t lma, uint32_t lmb, const WORD (&s)[27]) {
     using W = Two<SP>;
     constexpr uint32_t es = W::es, slot = BS3 * es;
@@ -243,6 +249,8 @@ __device__ __forceinline__ void two_scatter(const REC& R, __amdgpu_buffer_rsrc_t
             __builtin_amdgcn_sched_barrier(0);   // (the offsets of one row at a time)
             uint32_t v, e;
             row_of(cy, cz, v, e);
+            __amdgpu_buffer_rsrc_t fo = fown;
+            if constexpr (WIDE && cz != 0) fo = buf_layer<WIDE>(fout, R, z + cz < 0 ? -1 : (z + cz >= BS ? 1 : 0), 27u * slot);
             auto put = [&](const WORD& w, uint32_t lo, uint32_t hi, int k) {
                 if (lo & hi & 1u) W::template st2<AUX>(w, fo, v, (uint32_t)k * slot);
                 else if (lo & 1u) W::template st1<AUX>(W::a(w), fo, v, (uint32_t)k * slot);
@@ -278,14 +286,16 @@ __device__ __forceinline__ void two_scatter(const REC& R, __amdgpu_buffer_rsrc_t
                 const bool wall = (fc.zwall && zf) || (fc.ymin_wall && cyj > 0 && fc.yl);
                 // the rule of direction j: its own population, the opposite one (walls and solid links), the mirrors
                 const int src = outlet && cx > 0 ? j : (wall || !(zf || yf)) ? k : yf ? j - 6 * cyj : j - 18 * czj;
-                if (mine) W::template st1<AUX>(lds[src * TWG], fo, own + (uint32_t)half * es, (uint32_t)j * slot);
+                if (mine) W::template st1<AUX>(lds[src * TWG], fown, own + (uint32_t)half * es, (uint32_t)j * slot);
             }
         }
     }
 }
 
-// DITH: stochastic rounding (the 16-bit forms)
-template <class SP, bool UNIT, bool WALE, int EXTRA, bool DITH, int PAT>
+// DITH: stochastic rounding (the 16-bit forms).  WIDE: each layer of neighbours from its own base.  Only planes 0
+// and 15 of a block have sources (or targets) in another layer, of one cz each, so a plane's buffer is uniform per
+// cz; where a rule takes the own population of a row's lanes instead, those lanes load it apart.
+template <class SP, bool UNIT, bool WALE, int EXTRA, bool DITH, int PAT, bool WIDE = false>
 __global__ void __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(PAT == PAT_AA_ODD && SP::dithered ? 2 : EXTRA == TWO_BFL || PAT == PAT_AA_ODD || (EXTRA == TWO_SPONGE && !(UNIT && !WALE)) ? 3 : 4)))
 k_step_two(const StepArgs a) {
     using W = Two<SP>;
@@ -306,6 +316,12 @@ k_step_two(const StepArgs a) {
     const int jx = (int)(threadIdx.x & 7u), ly = (int)(threadIdx.x >> 3);
     auto boff = [&](int dx, int dy, int dz) -> uint32_t { return R.off[(dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)]; };
     const __amdgpu_buffer_rsrc_t fin = buf_at((const char*)a.fin + (size_t)R.base * blk);
+    // (of the sources of direction cz)
+    auto fin_z = [&](auto czc) {
+        constexpr int cz = decltype(czc)::value;
+        if constexpr (!WIDE || cz == 0) return fin;
+        else return buf_layer<WIDE>(a.fin, R, z - cz < 0 ? -1 : (z - cz >= BS ? 1 : 0), blk);
+    };
     const uint32_t row = (uint32_t)ly * (BS * es) + (uint32_t)jx * (2 * es);
     const uint32_t zown = (uint32_t)z * (BS2 * es);
     const uint32_t own0 = R.off[13];             // uniform
@@ -437,6 +453,11 @@ k_step_two(const StepArgs a) {
             if constexpr (cy != 0 || cz != 0) {
                 int j;
                 const bool face = two_row_rule<K>(fc, j);
+                if constexpr (WIDE && cz != 0) {
+                    if (face) s[K] = W::ld2(fin, own0 + row + rd(j) * slot + zown, 0);
+                    else s[K] = W::ld2(fin_z(dir_c<cz>{}), o, 0);
+                    return;
+                }
                 o = face ? own0 + row + rd(j) * slot + zown : o;
             }
             s[K] = W::ld2(fin, o, 0);
@@ -445,14 +466,14 @@ k_step_two(const StepArgs a) {
         for_dirs([&](auto kc) {
             constexpr int K = decltype(kc)::value;
             constexpr int cy = dcy(K), cz = dcz(K);
-            s[K] = W::ld2(fin, v[cz + 1][cy + 1], rd(K) * slot + zs[cz + 1]);
+            s[K] = W::ld2(fin_z(dir_c<cz>{}), v[cz + 1][cy + 1], rd(K) * slot + zs[cz + 1]);
         });
     }
     if (PAT != PAT_AA_EVEN && (first || last)) {
         for_dirs([&](auto kc) {
             constexpr int K = decltype(kc)::value;
             constexpr int cy = dcy(K), cz = dcz(K);
-            if constexpr (dcx(K) < 0) e9[K / 3] = W::lde(fin, ve[cz + 1][cy + 1] + rd(K) * slot + zs[cz + 1]);
+            if constexpr (dcx(K) < 0) e9[K / 3] = W::lde(fin_z(dir_c<cz>{}), ve[cz + 1][cy + 1] + rd(K) * slot + zs[cz + 1]);
         });
     }
 
@@ -661,7 +682,7 @@ k_step_two(const StepArgs a) {
     const uint32_t vown = own0 + row;
     const bool lva = is(LF_LIVE_A), lvb = is(LF_LIVE_B), both = lva && lvb;
     if constexpr (PAT == PAT_AA_ODD) {
-        two_scatter<SP>(R, fo, z, jx, ly, edge, fc, lf, lma, lmb, s);
+        two_scatter<SP, WIDE>(R, a.fout, fo, z, jx, ly, edge, fc, lf, lma, lmb, s);
     } else {
         // (the even half-step writes population K to the own slot opp K)
         constexpr auto wr = [](int k) { return (uint32_t)(PAT == PAT_AA_EVEN ? dopp(k) : k); };
@@ -721,6 +742,8 @@ static void launch_two_w(int extra, dim3 g, hipStream_t s, const StepArgs& r) {
     else if (extra == TWO_BFL) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_BFL, DITH, PAT_AB>), g, dim3(TWG), hold, s, r);
     else if (extra == TWO_AA_EVEN) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_PLAIN, DITH, PAT_AA_EVEN>), g, dim3(TWG), 0, s, r);
     else if (extra == TWO_AA_ODD) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_PLAIN, DITH, PAT_AA_ODD>), g, dim3(TWG), 0, s, r);
+    else if (extra == TWO_AA_ODD_WIDE) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_PLAIN, DITH, PAT_AA_ODD, true>), g, dim3(TWG), 0, s, r);
+    else if (extra == TWO_WIDE) hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_PLAIN, DITH, PAT_AB, true>), g, dim3(TWG), hold, s, r);
     else hipLaunchKernelGGL((k_step_two<SP, UNIT, WALE, TWO_PLAIN, DITH, PAT_AB>), g, dim3(TWG), hold, s, r);
 }
 template <class SP>

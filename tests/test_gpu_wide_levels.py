@@ -1,0 +1,149 @@
+"""Levels of 4 GiB of populations and more against the oracle, on boxes of 3 blocks a side cut out of them: a box's
+cells further from its cut faces than the steps reach hold the oracle's bits.
+
+A block inside a level of such wide layers reaches its neighbours by a base per layer (the WIDE form of the one-launch
+kernels: f32, f32_aa, f32_wale, f64, f16s), as do the wraps in z of a level of more than 4 GiB (z_wraps).  Where one
+layer is larger than that, the wraps in y take the one-plane kernels (y_wraps).  below: the largest offsets that one
+base spans, between 2 and 4 GiB."""
+import numpy as np
+import pytest
+
+from openaerolab_alpha_01_amd.geometry import sphere_mask, sphere_qmap, uniform_grid
+from test_gpu_parity import gpu_plan
+
+pytestmark = pytest.mark.gpu
+
+STEPS, MARGIN = 4, 6
+FLOW = dict(tau=0.53, u_inlet=0.05)
+# origins of the boxes in blocks (negative: from the far end), a sphere in it or not
+INSIDE, CORNERS = ((0.5, 0.5, 0), True), [((0, 0, 0), True), ((-3, -3, 0), True), ((0, -3, 0), False), ((-3, 0, 0), False)]
+CASES = {
+    # 71 x 70 x 3 blocks (all but the inner layer's span two layers of 2.2 GB), ragged in x, y and z
+    "f32": dict(n=(1130, 1116, 40), storage="f32", boxes=[INSIDE] + CORNERS, force=True),
+    "f32_aa": dict(n=(1130, 1116, 40), storage="f32", stream="aa", boxes=[INSIDE] + CORNERS, force=True,
+                   okw=dict(ymin_wall_bc=1, zwall_bc=2)),
+    "f32_wale": dict(n=(1130, 1116, 40), storage="f32", boxes=[INSIDE] + CORNERS,
+                     okw=dict(c_wale=0.2, omega_3=0.9, omega_4=1.1, adaptive_omega4=0, limiter=2)),
+    "f64": dict(n=(792, 790, 40), storage="f64", boxes=[INSIDE] + CORNERS, force=True, okw=dict(ymin_wall_bc=1)),
+    # 100 x 99 x 3 blocks of 2.2 GB a layer; round to nearest (the random bits of a cell depend on its index)
+    "f16s": dict(n=(1600, 1570, 40), storage="f16s", boxes=[INSIDE] + CORNERS[:2], okw=dict(rounding=1), macro=True),
+    "z_wraps": dict(n=(416, 400, 256), periodic=(False, False, True), storage="f32", force=True,
+                    boxes=[((0.5, 0.5, -1), True), ((0.2, 0.2, -1), False), ((0, 0, -1), True), ((0.5, 0.5, 4), False)]),
+    "z_wraps_aa": dict(n=(416, 400, 256), periodic=(True, False, True), storage="f32", stream="aa", force=True,
+                       boxes=[((0.5, 0.5, -1), True), ((-1, 0.2, -1), False), ((-1, -3, -1), True)]),
+    # the links of blocks in the WIDE form are the general kernel's
+    "z_wraps_bfl": dict(n=(416, 400, 256), periodic=(False, False, True), storage="f32", force=True, qmap=True,
+                        boxes=[((0.5, 0.5, -1), True), ((0.2, 0.2, -1), False)]),
+    "y_wraps": dict(n=(1600, 1600, 16), periodic=(False, True, True), storage="f32", force=True,
+                    boxes=[((0.5, -1, 0), True), ((0.2, -1, 0), False), ((0, -1, 0), False), ((0.2, 0.2, 0), False)]),
+    "y_wraps_aa": dict(n=(1600, 1600, 16), periodic=(False, True, True), storage="f32", stream="aa", force=True,
+                       boxes=[((0.5, -1, 0), True), ((0.2, -1, 0), False), ((-3, -1, 0), False)]),
+    "below": dict(n=(872, 878, 40), storage="f32", boxes=[INSIDE] + CORNERS, force=True),
+}
+
+
+def field(profiles, x, y, z):
+    """[4, ...]: density and velocity at cell coordinates, products of per-axis noise"""
+    fx, fy, fz = profiles
+    out = 0.02 * (fz[:, z] * fy[:, y] * fx[:, x])   # (the order of the whole field below)
+    out[0] += 1.0
+    out[1] += FLOW["u_inlet"]
+    return out
+
+
+def box_of(n, periodic, origin):
+    """(3 x blocks per axis, extent, periodic, [low, high] cut faces) of the box at a block origin"""
+    ids, ext, per, cut = [], [], [], []
+    for a in range(3):
+        nb = -(-n[a] // 16)
+        s = int(origin[a] * nb) if isinstance(origin[a], float) else origin[a] % nb if nb > 3 else 0
+        if nb <= 3:   # the whole axis
+            ids.append(np.arange(nb)), ext.append(n[a]), per.append(periodic[a]), cut.append((False, False))
+        elif periodic[a]:
+            ids.append((s + np.arange(3)) % nb), ext.append(48), per.append(False), cut.append((True, True))
+        else:
+            ids.append(s + np.arange(3)), ext.append(min(48, n[a] - 16 * s)), per.append(False)
+            cut.append((s > 0, s + 3 < nb))
+    return ids, tuple(ext), tuple(per), cut
+
+
+@pytest.mark.timeout(300)
+@pytest.mark.parametrize("case", list(CASES))
+def test_wide_level(oracle, case):
+    cfg = CASES[case]
+    n, periodic, storage, stream = cfg["n"], cfg.get("periodic", (False,) * 3), cfg["storage"], cfg.get("stream", "ab")
+    okw = dict(FLOW, **cfg.get("okw", {}))
+    rng = np.random.default_rng(11)
+    nblk = [-(-v // 16) for v in n]
+    profiles = [rng.uniform(-1, 1, (4, 16 * nb)) for nb in nblk]
+    grid = uniform_grid(n, periodic=periodic)
+    nb, wale = grid.n_blocks, okw.get("c_wale", 0.0) > 0
+    solid = np.zeros((nb, 4096), dtype=np.uint8)
+    qmap = np.zeros((27, nb, 4096), dtype=np.uint16) if cfg.get("qmap") else None
+    npdt = np.float64 if storage == "f64" else np.float32
+    boxes, F = [], np.zeros(3)
+    for origin, sphere in cfg["boxes"]:
+        ids, ext, per, cut = box_of(n, periodic, origin)
+        sub = uniform_grid(ext, periodic=per)
+        bx, by, bz = (ids[a][sub.coords[:, a] - 1] for a in range(3))
+        at = bx + nblk[0] * (by + nblk[1] * bz)
+        q = None
+        if sphere:
+            c, r = (24.3, 23.6, 16.2 if nblk[2] > 1 else 8.2), 4.5
+            sub.solid = sphere_mask(sub, c, r)
+            solid[at] = sub.solid.reshape(-1, 4096)
+        if qmap is not None:
+            q = sphere_qmap(sub, c, r).view(np.uint16) if sphere else np.zeros((27, sub.n_cells), dtype=np.uint16)
+            qmap[:, at] = q.reshape(27, -1, 4096)
+        g = sub.cell_coords()
+        glob = [np.repeat(16 * b, 4096) + g[:, a] % 16 for a, b in enumerate((bx, by, bz))]
+        init = field(profiles, *glob)
+        keep = sub.inside()
+        for a in range(3):
+            keep &= (not cut[a][0]) | (g[:, a] >= MARGIN)
+            keep &= (not cut[a][1]) | (g[:, a] < ext[a] - MARGIN)
+        if stream == "aa" and sphere:
+            keep &= sub.solid == 0
+        G = oracle.Grid(sub, qmap=q)
+        f = oracle.init_eq(storage, G, init[0], init[1:])
+        vel = init[1:].astype(npdt) if wale else None
+        for t in range(STEPS):
+            f, Fb, mac = oracle.step(storage, G, oracle.make_params(time_step=t, arith=oracle.FAST, **okw), f, vel_in=vel,
+                                     want_macro=wale, want_force=t == STEPS - 1 and sphere)
+            vel = mac[1] if wale else None
+        if sphere:
+            F += np.asarray(Fb, dtype=np.float64).reshape(-1, 3)[0]
+        boxes.append((origin, G, at, keep, f))
+    if solid.any():
+        grid.solid = solid.ravel()
+    # [4, blocks z, y, x, cells z, y, x]
+    ax = [p.reshape(4, nb_a, 16) for p, nb_a in zip(profiles, nblk)]
+    init = [0.02 * (ax[2][q][:, None, None, :, None, None] * ax[1][q][None, :, None, None, :, None]
+                    * ax[0][q][None, None, :, None, None, :]) for q in range(4)]
+    rho = (1.0 + init[0]).ravel()
+    u = np.stack([(init[1] + FLOW["u_inlet"]).ravel(), init[2].ravel(), init[3].ravel()])
+    del init
+    plan = gpu_plan(grid, storage, okw, stream)
+    print(f"{case}: {n} {storage} {stream}, {grid.n_cells} cells, {plan.level_info()}", flush=True)
+    if qmap is not None:
+        plan.set_bouzidi(qmap.reshape(27, -1), ff_fallback="halfway_bb")
+        del qmap
+    plan.init_equilibrium(rho, u)
+    del rho, u
+    for t in range(STEPS):
+        plan.level_step(0, t, force=bool(cfg.get("force")) and t == STEPS - 1)
+    if cfg.get("force"):
+        np.testing.assert_allclose(plan.force()[0], F, rtol=1e-11, atol=1e-13)
+    if cfg.get("macro"):
+        rho, u = plan.macro()
+        for origin, G, at, keep, f in boxes:
+            _, r_or, u_or = oracle.moments(storage, G, f)
+            keep = keep & (solid[at].ravel() == 0)
+            assert np.allclose(rho.reshape(nb, 4096)[at].ravel()[keep], r_or[keep], rtol=1e-14, atol=0), origin
+            assert np.allclose(u.reshape(3, nb, 4096)[:, at].reshape(3, -1)[:, keep], u_or[:, keep], rtol=1e-12, atol=1e-15), origin
+    else:
+        got = plan.download_f(dtype=npdt).reshape(27, nb, 4096)
+        for origin, G, at, keep, f in boxes:
+            bad = np.argwhere(got[:, at].reshape(27, -1)[:, keep] != f[:, keep])
+            assert bad.size == 0, (origin, len(bad), bad[:3].tolist())
+    plan.close()
