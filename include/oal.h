@@ -365,7 +365,9 @@ int oal_mass(OalPlan* plan, int level, double* out, void* stream);
 int oal_mass_noalloc(OalPlan* plan, int level, double* out_dev, void* stream);
 
 /* rho [n_cells] and u [3 * n_cells] of the current populations, FP64 host arrays in the reference
- * layout (materialize_current_state_for_io!, src/solver/solver_control.jl:830-851). */
+ * layout (materialize_current_state_for_io!, src/solver/solver_control.jl:830-851).  The plan keeps up to
+ * 24 MiB of pinned memory for it from the first call on; on a host that has none to give, the fields go
+ * through device memory. */
 int oal_download_macro(OalPlan* plan, int level, double* rho, double* u);
 
 /* Stability guard (src/octree_q19/src/io_run.jl:31-65): counts fluid cells with rho <= rho_min,

@@ -3,10 +3,7 @@
 // oal_kernels.hip on its stream.
 #include <hip/hip_runtime.h>
 
-#include <sched.h>
-
 #include <cmath>
-#include <condition_variable>
 #include <cstdio>
 #include <cstring>
 #include <new>
@@ -15,11 +12,11 @@
 #include <array>
 #include <numeric>
 #include <mutex>
-#include <thread>
 #include <unordered_map>
 #include <vector>
 
 #include "../../include/oal.h"
+#include "oal_fields.h"
 #include "oal_kernels.h"
 
 using namespace oal;
@@ -208,8 +205,6 @@ struct Level {
 // Pinned host memory of a plan's field downloads, in slots of one chunk; allocated on the first download,
 // for the largest level downloaded, at most FIELD_SLOTS chunks (24 MiB), and given back with the plan.
 // Pinning costs about 0.25 ms per MiB, once: a small level takes a quarter of its own size.
-constexpr uint32_t FIELD_CHUNK = 65536;   // cells: 2 MiB of rho and u
-constexpr int FIELD_SLOTS = 12;
 struct FieldStage {
     std::mutex mu;                 // one download of a plan at a time
     double* pin = nullptr;
@@ -226,14 +221,17 @@ struct FieldStage {
         if (pin && slot_doubles >= 4 * (size_t)cells && (int)ev.size() >= slots) return hipSuccess;
         release();
         hipError_t e = hipHostMalloc((void**)&pin, (size_t)slots * cells * 32, hipHostMallocDefault);
-        if (e != hipSuccess) { pin = nullptr; return e; }
+        if (e != hipSuccess) pin = nullptr;
         slot_doubles = 4 * (size_t)cells;
         for (int i = 0; i < slots && e == hipSuccess; ++i) {
             hipEvent_t x = nullptr;
             e = hipEventCreateWithFlags(&x, hipEventDisableTiming);
             if (e == hipSuccess) ev.push_back(x);
         }
-        if (e != hipSuccess) release();
+        if (e != hipSuccess) {
+            release();
+            (void)hipGetLastError();   // the download goes on without them: the error is not the next launch's
+        }
         return e;
     }
 };
@@ -2045,13 +2043,33 @@ int oal_mass_noalloc(OalPlan* p, int level, double* out_dev, void* stream) {
     return OAL_OK;
 }
 
-// Density and velocity into pageable host arrays.  The kernel writes chunks of cells into pinned slots over
-// the link, several in flight, while worker threads copy finished slots to the caller's arrays: with one
-// thread that copy (and the first touch of the caller's fresh pages) is the bound, 10 GB/s, against the
-// link's rate.  Up to 4 MiB are copied by the calling thread alone: starting a thread costs about as
-// much as copying half of that.  256^3 (537 MB) 52 -> 12.4 ms, 12 ragged boxes (637 MB) 61 -> 14.6 ms; 8^3 blocks 200 x
-// 120 x 104, regrouped by the kernel instead of the host, 33 -> 2.3 ms; 48 x 32 x 32 0.13 -> 0.10 ms (no
-// device allocation per call).
+// the device side of download_fields
+namespace {
+struct FieldDevice {
+    using error = hipError_t;
+    OalPlan* p;
+    Level& L;
+    DevBuf<double> buf;   // without pinned memory: one chunk
+    error reserve(uint32_t cells, int slots) { return p->fields.reserve(cells, slots); }
+    size_t slots() const { return p->fields.ev.size(); }
+    double* slot(size_t i) const { return p->fields.pin + i * p->fields.slot_doubles; }
+    error issue(size_t i, uint32_t c0, uint32_t n) {
+        const error e = launch_macro_out(p->storage, L.fA.p, L.c8map_d.p, c0, n, permute_of(p), slot(i), p->stream);
+        return e == hipSuccess ? hipEventRecord(p->fields.ev[i], p->stream) : e;
+    }
+    error wait(size_t i) { return hipEventSynchronize(p->fields.ev[i]); }
+    error direct(uint32_t c0, uint32_t n, double* const (&dst)[4]) {
+        error e = buf.n < 4 * (size_t)n ? buf.alloc(4 * (size_t)n) : hipSuccess;   // (the first chunk is the largest)
+        if (e == hipSuccess) e = launch_macro_out(p->storage, L.fA.p, L.c8map_d.p, c0, n, permute_of(p), buf.p, p->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(p->stream);
+        for (int a = 0; a < 4 && e == hipSuccess; ++a)
+            if (dst[a]) e = hipMemcpy(dst[a], buf.p + (size_t)a * n, (size_t)n * 8, hipMemcpyDeviceToHost);
+        return e;
+    }
+    void drain() { (void)hipStreamSynchronize(p->stream); }
+};
+}  // namespace
+
 static int download_macro_impl(OalPlan* p, int level, double* rho, double* u) {
     if (int rc = check_level(p, level)) return rc;
     Level& L = p->levels[level];
@@ -2059,89 +2077,11 @@ static int download_macro_impl(OalPlan* p, int level, double* rho, double* u) {
     OAL_HIP(hipSetDevice(p->device));
     if (int rc = ml_sync_covered(p, p->stream)) return rc;
     const size_t total = L.c8map.empty() ? L.ncell_host : L.c8map.size();
-    const uint32_t chunk = (uint32_t)std::min<size_t>(std::max<size_t>((total + 15) / 16, 4096), FIELD_CHUNK);
-    const size_t nchunk = (total + chunk - 1) / chunk;
     std::lock_guard<std::mutex> hold(p->fields.mu);
-    hipError_t e = p->fields.reserve(chunk, (int)std::min<size_t>((nchunk + 3) / 4 + 1, FIELD_SLOTS));
+    FieldDevice dev{p, L, {}};
+    const hipError_t e = download_fields(dev, total, rho, u);
+    dev.buf.release();
     if (e != hipSuccess) return fail(OAL_ERR_HIP, std::string("oal_download_macro: ") + hipGetErrorString(e));
-    const size_t slots = p->fields.ev.size();
-    auto cells_of = [&](size_t c) { return (uint32_t)std::min<size_t>(chunk, total - c * chunk); };
-    auto copy_out = [&](size_t c) {
-        const size_t n = cells_of(c), at = c * chunk;
-        const double* s = p->fields.pin + (c % slots) * p->fields.slot_doubles;
-        if (rho) std::memcpy(rho + at, s, n * 8);
-        if (u)
-            for (int a = 0; a < 3; ++a) std::memcpy(u + a * total + at, s + (a + 1) * n, n * 8);
-    };
-    // workers: take finished chunks from the queue
-    std::mutex mu;
-    std::condition_variable work, freed;
-    std::vector<size_t> queue;
-    size_t taken = 0;                       // chunks taken from the queue
-    std::vector<char> busy(slots, 0);       // a slot is in flight or being copied
-    bool stop = false;
-    std::vector<std::thread> pool;
-    cpu_set_t set;
-    const int cpus = sched_getaffinity(0, sizeof(set), &set) == 0 ? CPU_COUNT(&set) : 1;
-    const size_t want = total <= 2 * FIELD_CHUNK ? 0 : std::min<size_t>({total / FIELD_CHUNK, 8, (size_t)std::max(cpus - 1, 0)});
-    auto worker = [&] {
-        std::unique_lock<std::mutex> lk(mu);
-        for (;;) {
-            work.wait(lk, [&] { return stop || taken < queue.size(); });
-            if (taken >= queue.size()) return;
-            const size_t c = queue[taken++];
-            lk.unlock();
-            copy_out(c);
-            lk.lock();
-            busy[c % slots] = 0;
-            freed.notify_one();
-        }
-    };
-    try {
-        queue.reserve(nchunk);
-        pool.reserve(want);
-        for (size_t i = 0; i < want; ++i) pool.emplace_back(worker);
-    } catch (...) {   // fewer threads, or none
-    }
-    size_t issued = 0, ready = 0;
-    while (ready < nchunk && e == hipSuccess) {
-        for (;;) {
-            bool open;
-            {
-                std::unique_lock<std::mutex> lk(mu);
-                if (issued == ready && issued < nchunk) freed.wait(lk, [&] { return !busy[issued % slots]; });
-                open = issued < nchunk && !busy[issued % slots];
-                if (open) busy[issued % slots] = 1;
-            }
-            if (!open) break;
-            e = launch_macro_out(p->storage, L.fA.p, L.c8map_d.p, (uint32_t)(issued * chunk), cells_of(issued), permute_of(p),
-                                 p->fields.pin + (issued % slots) * p->fields.slot_doubles, p->stream);
-            if (e == hipSuccess) e = hipEventRecord(p->fields.ev[issued % slots], p->stream);
-            if (e != hipSuccess) break;
-            ++issued;
-        }
-        if (e == hipSuccess) e = hipEventSynchronize(p->fields.ev[ready % slots]);
-        if (e != hipSuccess) break;
-        if (pool.empty()) {
-            copy_out(ready);
-            busy[ready % slots] = 0;
-        } else {
-            std::lock_guard<std::mutex> lk(mu);
-            queue.push_back(ready);
-            work.notify_one();
-        }
-        ++ready;
-    }
-    {
-        std::lock_guard<std::mutex> lk(mu);
-        stop = true;
-    }
-    work.notify_all();
-    for (std::thread& t : pool) t.join();
-    if (e != hipSuccess) {
-        (void)hipStreamSynchronize(p->stream);   // nothing writes the slots any more
-        return fail(OAL_ERR_HIP, std::string("oal_download_macro: ") + hipGetErrorString(e));
-    }
     return OAL_OK;
 }
 
