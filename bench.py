@@ -55,6 +55,14 @@ def bytes_per_lup(storage: str, wale: bool = False) -> int:
     return pops + (2 * 3 * (8 if storage == "f64" else 4) if wale else 0)
 
 
+def tune(plan, level: int = 0):
+    """The autotuner in 20 short rounds, the last one's choice: a GPU that was idle reaches its steady clock after
+    some 150 steps (FP16 0.43 -> 0.38 ms per step), which a single round would time"""
+    for _ in range(20):
+        best, table = plan.autotune(6, level=level)
+    return best, table
+
+
 def gpu_leg(grid, storage: str, stream: str, steps: int, warmup: int, autotune: bool = True, fixed=None,
             qmap=None, wale: bool = False):
     """wale: the reference's production collision (WALE c_wale 0.2 with inlet noise 0.01,
@@ -68,9 +76,8 @@ def gpu_leg(grid, storage: str, stream: str, steps: int, warmup: int, autotune: 
     info = plan.level_info()
     tuning = None
     if autotune:
-        best, table = plan.autotune(6)
-        tuning = dict(best, ms_per_step={f"pipe{pp}_overlap{ov}_face{fk}": round(v, 4)
-                                         for (pp, ov, fk), v in table.items()})
+        best, table = tune(plan)
+        tuning = dict(best, ms_per_step={f"overlap{ov}": round(v, 4) for (_, ov, _), v in table.items()})
     else:
         if fixed:
             plan.set_tuning(**fixed)
@@ -412,7 +419,7 @@ def many_main(args) -> int:
             plan = many_plan(inst, st)
             tun = plan.tuning
             if not args.no_autotune:
-                tun, _ = plan.autotune(6)
+                tun, _ = tune(plan)
             plan.time_steps(args.warmup)
             ms, ker = plan.time_steps(args.steps)
             plan.close()
@@ -472,7 +479,7 @@ def amr_leg(storage: str, steps: int, warmup: int, autotune: bool, graph: int):
     L = len(grids)
     tuning = None
     if autotune:
-        best, _ = plan.autotune(6, level=L - 1)      # the finest level carries most of the work
+        best, _ = tune(plan, L - 1)      # the finest level carries most of the work
         tuning = best
     plan.set_tuning(graph=graph)
     tuning = plan.tuning
@@ -724,7 +731,7 @@ def main(argv=None) -> int:
                              "ms_per_step": round(ms_ta / aa_steps, 4), "vs_ab": round(ma / mlups, 3),
                              "population_bytes": 27 * 4 * n_cells, "population_bytes_ab": 2 * 27 * 4 * n_cells,
                              "step_achieved_gbs": round(sa, 1), "step_frac": round(sa / HBM_PEAK_GBS, 4),
-                             "tuning": {k: tuna[k] for k in ("pipe_planes", "overlap", "face_kernel")},
+                             "tuning": {"overlap": tuna["overlap"]},
                              "blocks": {k: infoa[k] for k in ("n_blocks", "n_regular", "n_boundary_regular", "n_boundary")},
                              "cd_transient": round(float(Fa[0] / (0.5 * U_IN ** 2 * area)), 5)}
     if not args.no_wale_leg:

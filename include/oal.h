@@ -409,7 +409,7 @@ typedef struct {
     int32_t reserved[3];
 } OalTuning;
 
-/* number of launch shapes the autotuner times: pipe_planes {1, 2, 4, 8, 16} x overlap {1, 0} x
+/* number of step times the autotuner reports: pipe_planes {1, 2, 4, 8, 16} x overlap {1, 0} x
  * face_kernel {0, 1} */
 #define OAL_TUNE_SHAPES 20
 
@@ -417,10 +417,11 @@ typedef struct {
 int oal_get_tuning(const OalPlan* plan, OalTuning* tuning);
 int oal_set_tuning(OalPlan* plan, const OalTuning* tuning);
 
-/* The project's autotuner: times every candidate launch shape on `level` for n_steps steps each,
- * keeps the fastest and restores the populations the plan held before; *best receives the choice.
- * ms_per_step[OAL_TUNE_SHAPES] (may be NULL) receives the mean step time of shape i: pipe_planes
- * {1, 2, 4, 8, 16}[i % 5], overlap 1 for (i / 5) even, face_kernel 1 for i >= 10. */
+/* The project's autotuner: times `level` for n_steps steps with overlap 1 and 0 (once where the level has
+ * no launch to overlap), keeps the faster and restores the populations the plan held before; *best receives
+ * the choice, the other fields as they were.  ms_per_step[OAL_TUNE_SHAPES] (may be NULL) receives the mean
+ * step time of shape i, pipe_planes {1, 2, 4, 8, 16}[i % 5], overlap 1 for (i / 5) even, face_kernel 1 for
+ * i >= 10: that of its overlap. */
 int oal_autotune(OalPlan* plan, int level, int n_steps, OalTuning* best, double* ms_per_step);
 
 #ifdef __cplusplus

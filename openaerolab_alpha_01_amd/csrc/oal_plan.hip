@@ -114,6 +114,11 @@ struct Level {
     uint32_t esize = 4;                // bytes of a stored population
     bool two() const { return fp32 || ab; }
     bool bulk() const { return two() ? n_two + n_two_wide + n_two_sponge > 0 : n_regular + n_interior > 0; }
+    // launches beside the bulk launch, which OalTuning.overlap puts on a second stream
+    bool aside() const {
+        return bulk() && (two() ? n_rest_interior + n_rest_regular + n_rest + (qmap.p ? n_rest_links : 0)
+                                : n_boundary_regular + n_boundary) > 0;
+    }
     DevBuf<int32_t> lslot;             // link-mask slot per block
     DevBuf<uint32_t> lmask;            // per-cell solid-link masks of blocks near solid cells
     std::vector<int32_t> lslot_h;      // host copy of lslot
@@ -239,7 +244,7 @@ struct FieldStage {
 struct OalPlan {
     int device = 0;
     bool overlap = true;   // boundary and face launches on the side stream
-    // launch-shape fields kept as the caller set them; no kernel reads them
+    // fields of OalTuning kept as the caller set them; no kernel reads them
     int pipe_planes = 4;
     bool face_kernel = false;
     int pair_kernel = 2;
@@ -1227,8 +1232,7 @@ int level_step(OalPlan* p, int level, int32_t time_step, int flags, hipStream_t 
     const bool want_force = (flags & OAL_STEP_FORCE) != 0;
     if (want_force && !L.has_solid) return fail(OAL_ERR_STATE, "force requested on a level without obstacle cells");
     StepArgs a = make_args(p, L, time_step, want_force);
-    // side-stream work: the boundary lists
-    const bool split = p->overlap && L.bulk() && a.n_boundary_regular + a.n_boundary + (L.two() ? a.n_interior : 0) > 0;
+    const bool split = p->overlap && L.aside();
     if (split) {
         // fork: the side stream starts after everything queued on s, then s waits for the side stream
         OAL_HIP(hipEventRecord(p->fork, s));
@@ -2581,27 +2585,27 @@ int oal_autotune(OalPlan* p, int level, int n_steps, OalTuning* best, double* ms
     const int aa_phase = L.aa_phase;
     OAL_HIP(hipStreamSynchronize(p->stream));
     drop_graphs(p);
-    const int cand[5] = {1, 2, 4, 8, 16};
-    int bestc = p->pipe_planes;
-    bool besto = p->overlap, bestf = p->face_kernel;
-    double bestms = 1e300;
+    // (of the fields of OalTuning only overlap changes a step's launches, on levels with some beside the bulk)
+    const bool had = p->overlap;
+    double ms[2] = {0.0, 0.0};   // whole steps, all launches, by overlap
     int rc = OAL_OK;
     if (e != hipSuccess) rc = fail(OAL_ERR_HIP, std::string("oal_autotune: ") + hipGetErrorString(e));
-    for (int i = 0; i < OAL_TUNE_SHAPES && rc == OAL_OK; ++i) {
-        p->pipe_planes = cand[i % 5];
-        p->overlap = (i / 5) % 2 == 0;
-        p->face_kernel = i >= 10;
+    for (const bool over : {had, !had}) {
+        if (rc != OAL_OK) break;
+        if (over != had && !L.aside()) {
+            ms[over] = ms[had];
+            break;
+        }
+        p->overlap = over;
         double tot = 0.0, ker = 0.0;
         rc = oal_time_steps(p, level, 2, 0, &tot, &ker);   // warm-up of this shape
         if (rc == OAL_OK) rc = oal_time_steps(p, level, n_steps, 0, &tot, &ker);
-        if (rc != OAL_OK) break;
-        const double ms = tot / n_steps;   // whole steps, all launches
-        if (ms_per_step) ms_per_step[i] = ms;
-        if (ms < bestms) { bestms = ms; bestc = cand[i % 5]; besto = p->overlap; bestf = p->face_kernel; }
+        ms[over] = tot / n_steps;
     }
-    p->pipe_planes = bestc;
+    const bool besto = rc == OAL_OK && ms[!had] < ms[had] ? !had : had;
     p->overlap = besto;
-    p->face_kernel = bestf;
+    if (rc == OAL_OK && ms_per_step)
+        for (int i = 0; i < OAL_TUNE_SHAPES; ++i) ms_per_step[i] = ms[(i / 5) % 2 == 0];
     // restore
     if (e == hipSuccess) e = hipMemcpyAsync(L.fA.p, save, L.fA.n, hipMemcpyDeviceToDevice, p->stream);
     if (e == hipSuccess && L.fB.p) e = hipMemcpyAsync(L.fB.p, save, L.fA.n, hipMemcpyDeviceToDevice, p->stream);
@@ -2614,9 +2618,9 @@ int oal_autotune(OalPlan* p, int level, int n_steps, OalTuning* best, double* ms
     if (rc == OAL_OK && e != hipSuccess) rc = fail(OAL_ERR_HIP, std::string("oal_autotune: ") + hipGetErrorString(e));
     if (rc == OAL_OK && best) {
         *best = OalTuning{};
-        best->pipe_planes = bestc;
+        best->pipe_planes = p->pipe_planes;
         best->overlap = besto ? 1 : 0;
-        best->face_kernel = bestf ? 1 : 0;
+        best->face_kernel = p->face_kernel ? 1 : 0;
         best->graph = p->graph ? 1 : 0;
         best->pair_kernel = p->pair_kernel;
     }

@@ -233,8 +233,8 @@ class Plan:
     # -- launch shape ------------------------------------------------------------------------------
     @property
     def tuning(self) -> dict:
-        """Launch shape: pipe_planes (1, 2, 4, 8, 16), overlap (0 or 1), face_kernel (0 or 1), graph (0 or 1:
-        step() replays a captured graph of one coarse step)."""
+        """Launch shape: overlap (0 or 1), graph (0 or 1: step() replays a captured graph of one coarse step), and
+        pipe_planes (1, 2, 4, 8, 16), face_kernel (0 or 1) and pair_kernel (0, 1, 2), which no kernel reads any more."""
         t = _lib.OalTuning()
         check(self.lib.oal_get_tuning(self.h, C.byref(t)), "oal_get_tuning")
         return {"pipe_planes": t.pipe_planes, "overlap": t.overlap, "face_kernel": t.face_kernel, "graph": t.graph,
@@ -311,8 +311,8 @@ class Plan:
         self.set_tuning(pipe_planes=v)
 
     def autotune(self, n_steps: int = 10, level: int = 0) -> tuple[dict, dict]:
-        """Time every launch shape, keep the fastest; the populations are restored afterwards.
-        Returns the choice and {(pipe_planes, overlap, face_kernel): ms per step}."""
+        """Time both settings of overlap, keep the faster; the populations are restored afterwards.
+        Returns the choice and {(pipe_planes, overlap, face_kernel): ms per step}, which overlap alone decides."""
         best = _lib.OalTuning()
         ms = (C.c_double * _lib.OAL_TUNE_SHAPES)()
         check(self.lib.oal_autotune(self.h, level, n_steps, C.byref(best), ms), "oal_autotune")
