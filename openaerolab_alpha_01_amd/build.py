@@ -76,39 +76,54 @@ def build_oracle(verbose: bool = False) -> Path:
 
 
 def scratch_kernels(report: str) -> list[tuple[str, int]]:
-    """(kernel, bytes per lane) of every kernel that the compiler's resource-usage remarks show with
-    scratch (register spills).  A frame no larger than the spilled scalar registers, in a kernel that spills
-    no vector register, holds their slots only: scalars are kept in lanes of a vector register and the
-    frame is never accessed."""
+    """(kernel, bytes per lane) of every kernel that the compiler's resource-usage remarks show with a scratch
+    frame"""
     out = []
     for block in report.split("remark: Function Name: ")[1:]:
-        name = block.split()[0]
         m = re.search(r"ScratchSize \[bytes/lane\]: (\d+)", block)
-        sgpr, vgpr = (int((re.search(rf"{r} Spill: (\d+)", block) or [0, 0])[1]) for r in ("SGPRs", "VGPRs"))
-        if m and int(m.group(1)) > (0 if vgpr else 4 * sgpr):
-            out.append((name, int(m.group(1))))
+        if m and int(m.group(1)) > 0:
+            out.append((block.split()[0], int(m.group(1))))
     return out
+
+
+def scratch_accesses(asm: str) -> set[str]:
+    """the functions of a device assembly that hold an instruction which can reach a scratch frame (gfx950:
+    scratch_* and flat_*).  A kernel whose only spills are scalars kept in lanes of a vector register has a
+    frame for their slots that nothing accesses."""
+    out = set()
+    for name, body in re.findall(r"^(\w+):[ \t]*(?:;[^\n]*)?\n(.*?)^\.Lfunc_end\d+:", asm, re.M | re.S):
+        if re.search(r"^\s+(?:scratch|flat)_", body, re.M):
+            out.add(name)
+    return out
+
+
+def device_assembly(jobs: int | None = None) -> tuple[str, str]:
+    """the resource-usage remarks and the gfx950 assembly of every source, by the library's flags"""
+    jobs = jobs or min(len(SOURCES), max(1, len(os.sched_getaffinity(0))))
+
+    def run(src):
+        cmd = [HIPCC, *HIP_FLAGS, "-Rpass-analysis=kernel-resource-usage", "--cuda-device-only", "-S", "-o", "-", str(src)]
+        return subprocess.run(cmd, cwd=str(CSRC), capture_output=True, text=True, check=True)
+
+    with ThreadPoolExecutor(jobs) as pool:
+        results = list(pool.map(run, SOURCES))
+    return "".join(r.stderr for r in results), "".join(r.stdout for r in results)
 
 
 def main(argv: list[str]) -> int:
     verbose = "-v" in argv
     if "--resources" in argv:
-        # every kernel's registers and scratch; fails when any kernel spills to scratch
-        import io
-        import contextlib
-        err = io.StringIO()
-        with contextlib.redirect_stderr(err):
-            build_library(verbose=verbose, extra=["-Rpass-analysis=kernel-resource-usage"])
-        report = err.getvalue()
+        # every kernel's registers and scratch, from the assembly (no library is built); fails when a kernel accesses
+        # its frame
+        report, asm = device_assembly()
         sys.stderr.write(report)
-        spills = scratch_kernels(report)
-        for name, b in spills:
-            print(f"scratch: {b} B/lane in {name}")
-        print(f"{report.count('Function Name: ')} kernels, {len(spills)} with scratch")
-        if spills:
-            return 1
-    else:
-        build_library(verbose=verbose)
+        frames, accessed = scratch_kernels(report), scratch_accesses(asm)
+        spills = [n for n, _ in frames if n in accessed]
+        for name, b in frames:
+            print(f"scratch: {b} B/lane in {name}, {'accessed' if name in accessed else 'not accessed'}")
+        print(f"{report.count('Function Name: ')} kernels, {len(frames)} with a frame, {len(spills)} that access it")
+        return 1 if spills else 0
+    build_library(verbose=verbose)
     if "--no-oracle" not in argv:
         build_oracle(verbose=verbose)
     return 0
