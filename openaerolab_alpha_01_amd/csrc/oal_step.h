@@ -421,8 +421,8 @@ __device__ __forceinline__ void step_cell(const StepArgs& a, const CellCtx& c, c
         if constexpr (REG && !GEN && PAT == PAT_AA_EVEN) {
             val = SP::ld((const st*)(ra.base(fi, K, c.z, 0) + ra.v[1][1]), w);
         } else if constexpr (REG && !GEN) {
-            constexpr int slot = PAT == PAT_AB ? K : dopp(K);
-            val = SP::ld((const st*)(ra.base(fi, slot, c.z, dcz(K)) + ra.v[dcx(K) + 1][dcy(K) + 1]), w);
+            static_assert(PAT == PAT_AA_ODD, "the AB pattern's regular blocks without a rule are the one-launch kernels'");
+            val = SP::ld((const st*)(ra.base(fi, dopp(K), c.z, dcz(K)) + ra.v[dcx(K) + 1][dcy(K) + 1]), w);
         } else if constexpr (PAT == PAT_AA_EVEN) {
             // every direction loads the own slot K, so the 27 loads are in flight together; an inlet
             // link's value replaces it afterwards, evaluated in full precision as the pull step does
@@ -602,10 +602,9 @@ __device__ __forceinline__ void step_cell(const StepArgs& a, const CellCtx& c, c
     });
 }
 
-// SEL: which blocks a launch covers.  SEL_ALL dispatches on the block flags inside one launch;
-// SEL_INTERIOR / SEL_BOUNDARY run the interior and the boundary block lists as separate launches, so
-// that the interior kernel is compiled for its own (smaller) register budget.
-enum : int { SEL_ALL = 0, SEL_INTERIOR = 1, SEL_BOUNDARY = 2, SEL_REGULAR = 3, SEL_BOUNDARY_REGULAR = 4 };
+// SEL: which block list a launch covers: blocks without a rule or boundary blocks, each also with lexicographic
+// neighbours (regular), on a kernel of its own register budget.
+enum : int { SEL_INTERIOR = 1, SEL_BOUNDARY = 2, SEL_REGULAR = 3, SEL_BOUNDARY_REGULAR = 4 };
 
 #ifndef OAL_STEP_WAVES
 #define OAL_STEP_WAVES 3
@@ -618,11 +617,11 @@ constexpr int step_waves() {
     return sizeof(typename SP::T) == 8 && PAT != PAT_AB ? 1 : sizeof(typename SP::T) == 8 || PAT != PAT_AB || WALE ? 2 : OAL_STEP_WAVES;
 }
 
-template <class SP, int PAT, bool WALE, int SEL = SEL_ALL, bool BFL = false, bool SPONGE = false, bool FX = true>
+template <class SP, int PAT, bool WALE, int SEL, bool BFL = false, bool SPONGE = false, bool FX = true>
 __global__ void __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(step_waves<SP, PAT, WALE>()))) k_step(const StepArgs a) {
     const uint32_t litem = xcd_item(blockIdx.x, gridDim.x);
     const uint32_t lb = litem / PLANES;
-    const uint32_t b = a.blist ? (uint32_t)a.blist[lb] : lb;
+    const uint32_t b = (uint32_t)a.blist[lb];
     const uint32_t item = b * PLANES + litem % PLANES;
     CellCtx c;
     c.b = b;
