@@ -52,7 +52,7 @@ struct StepArgs {
     void* vel_out;               // [3 * ncell] velocity written (WALE, macro output)
     void* rho_out;               // [ncell] density written (macro output) or null
     double* fpart;               // [n_items * 4] per-workgroup force partials or null
-    const int32_t* blist;        // blocks of this launch (item / PLANES -> block), null = all in order
+    const int32_t* blist;        // k_step: blocks of this launch (item / PLANES -> block; set per launch)
     const int32_t* blist_regular;    // [n_regular] interior blocks whose neighbours sit at lexicographic offsets
     const int32_t* blist_interior;   // [n_interior] other blocks with all flags clear
     const int32_t* blist_boundary_regular;  // [n_boundary_regular] boundary blocks with lexicographic neighbours
@@ -103,10 +103,12 @@ constexpr uint64_t TWO_KEEP_BYTES = 192ull << 20;
 
 // Blocks up to which a level in the AB pattern with FP32 arithmetic takes the one-cell-per-lane kernel (half as
 // many with WALE): twice the waves with half the work each.  128 blocks fill the chip's wave slots in either
-// form; measured (us per step, one against two cells per lane), FP32: 8 blocks 6.7 / 9.6, 64 11.0 / 13.2,
-// 216 31.6 / 34.3, 512 84 / 87, 1000 161 / 162, 4096 653 / 634; FP16: 8 7.3 / 13.4, 216 26.8 / 29.4,
-// 512 56.9 / 63.4, 640 68.6 / 67.8, 4096 385 / 370; WALE FP32: 8 9.4 / 11.6, 216 38.9 / 40.9, 294 63.4 / 62.2,
-// 1000 202 / 193; WALE FP16: 216 35.5 / 37.3, 343 49.9 / 49.0, 1000 146 / 126.
+// form; measured (us per step of a box around a sphere, with the events that time it, one against two cells per
+// lane), FP32: 8 blocks 13.8 / 16.6, 216 37.4 / 41.4, 343 64.2 / 66.2, 512 90.7 / 93.1, 576 101.2 / 101.7, 640 111.0 /
+// 110.1, 1000 168.6 / 164.2, 4096 663 / 617; FP16: 8 14.3 / 20.1, 216 28.5 / 35.7, 343 39 / 44, 512 60 / 71, 576 66 / 67,
+// 1000 104 / 105, 4096 391 / 376 (BF16 alike); WALE FP32: 8 16.5 / 18.9, 216 44.0 / 48.2, 252 62.3 / 61.8, 294 70.0 / 69.0,
+// 1000 209 / 199; WALE FP16: 216 38.8 / 43.0, 294 46.4 / 49.8, 448 63.3 / 68.6, 512 84.4 / 86.0, 576 92.0 / 84.3, 1000 148 /
+// 134 (its own line would lie at 512).
 constexpr uint32_t ONE_BLOCKS = 512;
 
 struct ReduceArgs {

@@ -727,11 +727,13 @@ k_step_two(const StepArgs a) {
 }
 
 // Dynamic LDS that no kernel uses: it leaves five workgroups (ten waves) on a CU instead of eight where an FP32
-// level streams through the caches.  The loads in flight on an XCD then fit its 4 MB L2 (32 CUs x 5 x 27 KB; eight
-// are 6.9 MB), so the lines at the row ends and of half rows are still there for the neighbouring workgroup.
-// 256^3 FP32: 629.9 us per step, 612 with six workgroups, 605 with five, 615 with four; WALE 192 x 160 x 160: 232,
-// 227.7, 228.2, 237; interpolated wall 160 x 128 x 128 121.9, with five 119.3.  The AA pattern (204, 209, 215 us),
-// the 16-bit forms (256^3 FP16 376, with six 436 us) and levels that stay in the memory-side cache keep all.
+// level streams through the caches.  The number is measured.  The loads in flight on an XCD (27 KB a workgroup, 32
+// CUs) are 7.1 MB with eight against its 4 MB L2, so that lines at the row ends and of half rows leave it before
+// the neighbouring workgroup reads them; with five they are 4.4 MB, and reads fall from 1.076 to 1.039 of
+// algorithmic; with four too few are in flight.  256^3 FP32: 629.9 us per step, 612 with six workgroups, 605 with
+// five, 615 with four; WALE 192 x 160 x 160: 232, 227.7 and 228.2 (no difference), 237; interpolated wall 160 x 128 x
+// 128 121.9, with five 119.3.  The AA pattern (204, 209, 215 us), the 16-bit forms (256^3 FP16 376, with six 436
+// us) and levels that stay in the memory-side cache keep all.
 constexpr uint32_t TWO_HOLD_LDS = 18000;
 
 // the blocks of one list, one plane per workgroup
