@@ -585,11 +585,12 @@ int prepare_level(const OalLevelDesc& d, const OalCollision& coll, bool ab, bool
         near[i] = ((uint64_t)dm.nbx * dm.nby + dm.nbx + 1) * 27u * BS3 * (uint64_t)sbytes < (1ull << 31);
     }
     // (a boundary block qualifies when no neighbour inside the extent is absent and every present one is
-    // at its lexicographic offset: its out-of-extent sources take the face rules and are never read)
+    // at its lexicographic offset: its out-of-extent sources take the face rules and are never read; and when
+    // 32 bits reach the rows before and after)
     L.regular_h.assign(nb, 0);
     for (uint32_t b = 0; b < nb; ++b) {
         const DevDomain& dm = L.doms_h[bdom[b]];
-        bool regular = !(flags[b] & BF_MISSING);
+        bool regular = !(flags[b] & BF_MISSING) && row_fits(dm.nbx, (uint64_t)sbytes);
         for (int k = 0; k < 27 && regular; ++k) {
             const int ox = k % 3 - 1, oy = (k / 3) % 3 - 1, oz = k / 9 - 1;
             const int64_t want = (int64_t)b + ox + (int64_t)oy * dm.nbx + (int64_t)oz * dm.nbx * dm.nby;

@@ -51,6 +51,17 @@ enum : uint32_t {
 // scalar registers.
 enum : char { FIT_NONE = 0, FIT_ALL = 1, FIT_LAYERS = 2 };
 
+// Byte offset, from a block's start, of the cell `local` of its neighbour (dx, dy) in a row of nbx blocks: k_step's
+// regular forms keep it in signed 32 bits per lane (RegAddr) ...
+inline int64_t row_offset(int dx, int dy, int64_t nbx, int64_t local, uint64_t esize) {
+    return ((dx + dy * nbx) * (27 * BS3) + local) * (int64_t)esize;
+}
+// ... which hold the blocks of the rows before and after where a row spans less than 2 GiB (4853 blocks in FP32, 77 648
+// cells; FP64 2426); blocks of longer rows are not regular: the general forms' addresses have 64 bits
+inline bool row_fits(int64_t nbx, uint64_t esize) {
+    return row_offset(1, 1, nbx, BS3, esize) < (1ll << 31) && row_offset(-1, -1, nbx, 0, esize) >= -(1ll << 31);
+}
+
 // The block that a record counts the offsets of each layer of neighbours from (nt: the block's row of neighbours,
 // -1 = absent): the lowest of all of them, or (by layers) of the layer, which the block itself stands for where it
 // has none

@@ -20,6 +20,8 @@ def records(tmp_path_factory):
     d = tmp_path_factory.mktemp("records")
     (d / "r.cpp").write_text('''#include "oal_records.h"
 extern "C" int fit(const int32_t* nt, uint32_t b, uint64_t es) { return oal::two_fit(nt, b, es); }
+extern "C" int row_fits(int64_t nbx, uint64_t es) { return oal::row_fits(nbx, es); }
+extern "C" int64_t row_offset(int dx, int dy, int64_t nbx, int64_t local, uint64_t es) { return oal::row_offset(dx, dy, nbx, local, es); }
 extern "C" void offsets(const int32_t* nt, uint32_t b, int layers, uint32_t es, uint32_t* off, uint32_t* base) {
     oal::TwoRec r{};
     oal::two_offsets(nt, b, layers != 0, es, r);
@@ -45,6 +47,7 @@ extern "C" void offsets(const int32_t* nt, uint32_t b, int layers, uint32_t es, 
         assert f == LAYERS or base[0] == base[1] == base[2]
         assert (off.astype(np.int64) + blk <= 2 ** 32).all() and (off % blk == 0).all()
         return f, np.repeat(base, 9).astype(np.int64) + off // blk
+    row.lib = lib
     return row
 
 
@@ -112,3 +115,23 @@ def test_any_order(records):
         else:
             assert nt.max() - nt[nt >= 0].min() + 1 > 9709
     assert seen == {NONE, ALL, LAYERS}
+
+
+@pytest.mark.parametrize("storage", list(ESIZE))
+def test_rows_reached_by_signed_offsets(records, storage):
+    """the regular one-plane forms keep the offset of a cell in the next row of blocks in 32 signed bits: every one
+    of them is exact up to the longest row that counts as regular, and the next longer row has one that is not"""
+    es = ESIZE[storage]
+    fits = lambda n: bool(records.lib.row_fits(ctypes.c_int64(n), ctypes.c_uint64(es)))
+    records.lib.row_offset.restype = ctypes.c_int64
+
+    def exact(n):
+        got = [records.lib.row_offset(dx, dy, ctypes.c_int64(n), ctypes.c_int64(c), ctypes.c_uint64(es))
+               for dx in (-1, 0, 1) for dy in (-1, 0, 1) for c in (0, 4095)]
+        assert got == [((dx + dy * n) * 27 * 4096 + c) * es for dx in (-1, 0, 1) for dy in (-1, 0, 1) for c in (0, 4095)]
+        return all(np.int64(v).astype(np.int32) == v for v in got)
+
+    last = max(n for n in range(1, 10000) if fits(n))
+    assert last == {"f32": 4853, "f64": 2426, "16": 9707}[storage]
+    assert all(fits(n) and exact(n) for n in (1, 2, 16, last // 2, last - 1, last))
+    assert not any(fits(n) or exact(n) for n in (last + 2, 2 * last, 38836))

@@ -3,8 +3,8 @@ cells further from its cut faces than the steps reach hold the oracle's bits.
 
 A block inside a level of such wide layers reaches its neighbours by a base per layer (the WIDE form of the one-launch
 kernels: f32, f32_aa, f32_wale, f64, f16s), as do the wraps in z of a level of more than 4 GiB (z_wraps).  Where one
-layer is larger than that, the wraps in y take the one-plane kernels (y_wraps).  below: the largest offsets that one
-base spans, between 2 and 4 GiB."""
+layer is larger than that, the wraps in y take the one-plane kernels (y_wraps), as do rows of 2 GiB where a rule or two
+rows do (rows_*).  below: the largest offsets that one base spans, between 2 and 4 GiB."""
 import numpy as np
 import pytest
 
@@ -38,6 +38,14 @@ CASES = {
                     boxes=[((0.5, -1, 0), True), ((0.2, -1, 0), False), ((0, -1, 0), False), ((0.2, 0.2, 0), False)]),
     "y_wraps_aa": dict(n=(1600, 1600, 16), periodic=(False, True, True), storage="f32", stream="aa", force=True,
                        boxes=[((0.5, -1, 0), True), ((0.2, -1, 0), False), ((-3, -1, 0), False)]),
+    # rows of 2 GiB of blocks and more: beyond the signed offsets of the regular one-plane forms (FP64 in the AA pattern,
+    # the exact specular z wall), and beyond two rows of unsigned ones (rows_f32)
+    "rows_f64_aa": dict(n=(38900, 32, 16), storage="f64", stream="aa", force=True,
+                        boxes=[((0.5, 0, 0), True), ((0, 0, 0), False), ((-3, 0, 0), False)]),
+    "rows_zwall": dict(n=(77700, 32, 16), storage="f32", force=True, okw=dict(zwall_bc=1),
+                       boxes=[((0.5, 0, 0), True), ((0, 0, 0), False), ((-3, 0, 0), False)]),
+    "rows_f32": dict(n=(77700, 64, 16), storage="f32", force=True,
+                     boxes=[((0.5, 0, 0), True), ((0.2, -3, 0), False), ((-3, -3, 0), True)]),
     "below": dict(n=(872, 878, 40), storage="f32", boxes=[INSIDE] + CORNERS, force=True),
 }
 
