@@ -46,7 +46,7 @@ enum : uint32_t {
 // layers of the domain's blocks, which cease to fit beyond 1114 x 1114 cells per layer in FP32 (FP64 788 x 788,
 // 16 bits 1576 x 1576), and the wraps of a z-periodic level span the whole of it; by layers it spans two rows.
 // Against the general kernel, which steps whatever no 32 bits span (ms per step): 1136 x 1120 x 96 FP32 5.64 ->
-// 4.42, with WALE 7.60 -> 5.30, AA 7.74 -> 5.50; 800 x 800 x 112 FP64 5.87 -> 5.39; 1600 x 1600 x 48 FP16 3.97 ->
+// 4.42, with WALE 7.60 -> 5.30, AA 7.74 -> 5.50; 800 x 800 x 112 FP64 5.85 -> 5.50; 1600 x 1600 x 48 FP16 3.97 ->
 // 2.54; 400 x 416 x 416 FP32 periodic 2.62 -> 2.52.  A form of its own, so that the narrow one keeps its
 // scalar registers.
 enum : char { FIT_NONE = 0, FIT_ALL = 1, FIT_LAYERS = 2 };

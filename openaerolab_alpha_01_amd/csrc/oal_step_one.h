@@ -144,6 +144,7 @@ k_step_one(const StepArgs a) {
                 const int dz = sz < 0 ? -1 : (sz >= BS ? 1 : 0);
                 auto boff = [&](int dx, int dy) -> uint32_t { return R.off[(dx + 1) + 3 * (dy + 1) + 9 * (dz + 1)]; };
                 const uint32_t zs = (uint32_t)(sz & (BS - 1)) * (BS2 * es);
+                [[maybe_unused]] const __amdgpu_buffer_rsrc_t fz = buf_layer<WIDE>(a.fin, R, dz, blk);   // (WIDE, cz != 0)
                 const uint32_t in_row = (uint32_t)((ly - cy) & (BS - 1)) * (BS * es) + (uint32_t)lx * es;
                 const uint32_t c0 = boff(0, 0);
                 // (a row's end is 16 cells from its start: - es becomes + 15 es, and the other way round)
@@ -177,12 +178,12 @@ k_step_one(const StepArgs a) {
                                 int j;
                                 const bool ownp = two_row_rule<K>(fc, j) || ((c.lmask >> K) & 1u) || (cx < 0 && outlet);
                                 if (ownp) s[K] = W::ld(fin, w, 0);
-                                else s[K] = W::ld(buf_layer<WIDE>(a.fin, R, dz, blk), w, 0);
+                                else s[K] = W::ld(fz, w, 0);
                             } else {
                                 s[K] = W::ld(fin, w, 0);
                             }
                         } else {
-                            if constexpr (WIDE && cz != 0) s[K] = W::ld(buf_layer<WIDE>(a.fin, R, dz, blk), o, (uint32_t)K * slot + zs);
+                            if constexpr (WIDE && cz != 0) s[K] = W::ld(fz, o, (uint32_t)K * slot + zs);
                             else s[K] = W::ld(fin, o, (uint32_t)K * slot + zs);
                         }
                     }
